@@ -252,5 +252,8 @@ def work(case):
 def tolerance(case):
     """Four times the largest difference seen between the kernels and attention computed in float32 (2.5e-3 in bf16,
     3.2e-4 in fp16 where every key counts; single values near zero in the sum of many differ by up to 0.07 and 0.01 of the
-    root mean square)."""
+    root mean square).  A whole model rounds to bf16 after each of its own operations as well: the same model with its dense
+    rows computed in float32 differs by 9e-3."""
+    if case["kind"] == "model":
+        return {"rel": 3e-2, "max": 0.3}
     return {"rel": 1.5e-3, "max": 0.05} if case["dtype"] == "fp16" else {"rel": 1e-2, "max": 0.3}
