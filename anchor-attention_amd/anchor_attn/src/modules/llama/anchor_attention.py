@@ -19,7 +19,8 @@ from typing import Optional, Tuple
 import torch
 import torch.nn.functional as F
 
-from anchor_attn.src.ops.anchor_attn_v4 import LOG2E, _anchor_attn, anchor_attn, dense_causal_attention
+from anchor_attn.src.ops.anchor_attn_v4 import (LOG2E, _anchor_attn, anchor_attn, dense_causal_attention, dense_rows_attention,
+                                                dense_rows_supported)
 
 ATTN_NAME = "anchor_attn"
 DENSE_ATTN_NAME = "anchor_attn_dense"
@@ -33,15 +34,28 @@ record_ratio: bool = False
 last_ratio: Optional[torch.Tensor] = None
 
 
-def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[int]):
+def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[int], out=None):
     """Dense attention for the parts the sparse operator does not cover (tail rows, decode, padded batches).
-    ``causal_offset``: query row i may see keys ``<= causal_offset + i`` (None: use ``attention_mask`` as is)."""
+    ``causal_offset``: query row i may see keys ``<= causal_offset + i`` (None: use ``attention_mask`` as is).  Writes into
+    ``out`` where it is given and the own kernel runs, otherwise returns a new tensor; either way the result is returned.
+    The own kernel takes bf16/fp16 inference on the GPU; the framework's attention does everything else (other types and
+    head dimensions, gradients, the CPU)."""
     groups = query.shape[1] // key.shape[1]
+    wants_grad = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
+    if (attention_mask is None and causal_offset is not None and causal_offset >= 0 and not wants_grad
+            and (scaling is None or scaling > 0) and dense_rows_supported(query, key, value)):
+        return dense_rows_attention(query, key, value, causal_offset, sm_scale=scaling, out=out)
     mask = attention_mask
     if causal_offset is not None and mask is None and query.shape[2] > 1:
         rows = torch.arange(query.shape[2], device=query.device)[:, None] + causal_offset
         mask = torch.arange(key.shape[2], device=query.device)[None, :] <= rows
     return F.scaled_dot_product_attention(query, key, value, attn_mask=mask, scale=scaling, enable_gqa=groups > 1)
+
+
+def _dense_into(out, query, key, value, attention_mask, scaling, causal_offset):
+    got = _dense(query, key, value, attention_mask, scaling, causal_offset, out)
+    if got is not out:
+        out.copy_(got)
 
 
 def anchor_attention_forward(module, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
@@ -58,7 +72,7 @@ def anchor_attention_forward(module, query: torch.Tensor, key: torch.Tensor, val
     # Prefill of a fresh sequence without padding is the case the operator is defined for.
     sparse_ok = N > 1 and n_kv == N and attention_mask is None and N >= big and query.dtype in (torch.bfloat16, torch.float16)
     if not sparse_ok:
-        out_bhnd.copy_(_dense(query, key, value, attention_mask, scaling, n_kv - N if attention_mask is None else None))
+        _dense_into(out_bhnd, query, key, value, attention_mask, scaling, n_kv - N if attention_mask is None else None)
         return out, None
     pad = N % big
     main = N - pad
@@ -71,7 +85,7 @@ def anchor_attention_forward(module, query: torch.Tensor, key: torch.Tensor, val
                     block_size=block_size, step=step, difference=theta,
                     return_computational_ratio=False, out=out_bhnd[:, :, :main])
     if pad:
-        out_bhnd[:, :, main:].copy_(_dense(query[:, :, main:], key, value, None, scaling, main))
+        _dense_into(out_bhnd[:, :, main:], query[:, :, main:], key, value, None, scaling, main)
     return out, None
 
 
@@ -89,10 +103,10 @@ def dense_attention_forward(module, query: torch.Tensor, key: torch.Tensor, valu
     out_bhnd = out.transpose(1, 2)
     kernel_ok = N >= 128 and n_kv == N and attention_mask is None and query.dtype in (torch.bfloat16, torch.float16) and query.is_cuda
     if not kernel_ok:
-        out_bhnd.copy_(_dense(query, key, value, attention_mask, scaling, n_kv - N if attention_mask is None else None))
+        _dense_into(out_bhnd, query, key, value, attention_mask, scaling, n_kv - N if attention_mask is None else None)
         return out, None
     main = N - N % 128
     dense_causal_attention(query[:, :, :main], key[:, :, :main], value[:, :, :main], sm_scale=scaling, out=out_bhnd[:, :, :main])
     if main < N:
-        out_bhnd[:, :, main:].copy_(_dense(query[:, :, main:], key, value, None, scaling, main))
+        _dense_into(out_bhnd[:, :, main:], query[:, :, main:], key, value, None, scaling, main)
     return out, None

@@ -158,6 +158,38 @@ def anchor_attn_test_time(Q, K, V, sm_scale: float = None, block_size: int = 128
     return output, search_time, compute_time
 
 
+def dense_rows_supported(Q, K, V) -> bool:
+    """Whether :func:`dense_rows_attention` takes these tensors (its kernels' types, head dimensions, alignment and
+    32-bit addressing of one head)."""
+    if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype):
+        return False
+    D = Q.shape[3]
+    if D not in (64, 128) or K.shape != V.shape or K.shape[3] != D or K.shape[0] != Q.shape[0] or Q.shape[1] % K.shape[1]:
+        return False
+    for t in (Q, K, V):
+        if t.stride(3) != 1 or t.data_ptr() % 16 or t.stride(0) % 8 or t.stride(1) % 8 or t.stride(2) % 8:
+            return False
+        if not D <= t.stride(2) <= 1 << 14 or not 0 < t.shape[2] <= 1 << 20 or t.shape[2] * t.stride(2) * 2 >= 1 << 32:
+            return False
+    return True
+
+
+def dense_rows_attention(Q, K, V, causal_offset: int, sm_scale: float = None, out: torch.Tensor = None):
+    """Causal attention of ``Q`` ``[B,H,n_rows,D]`` over ``K``/``V`` ``[B,H_kv,n_keys,D]`` on the same MFMA core: query row
+    ``i`` sees keys ``0 .. causal_offset + i``.  Any row and key count (:func:`dense_rows_supported` names the rest)."""
+    B, H, N, D = Q.shape
+    sm_scale = sm_scale if sm_scale else 1.0 / (D ** 0.5)
+    output = torch.empty_like(Q) if out is None else out
+    lib = _hip.lib()
+    sizes = (B, H, K.shape[1], N, K.shape[2], D, int(causal_offset))
+    nbytes = lib.aa_dense_rows_workspace_bytes(*sizes)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=Q.device) if nbytes else None
+    _hip.check(lib.aa_dense_rows_fwd(*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output),
+                                     ws.data_ptr() if nbytes else None, nbytes, *sizes,
+                                     float(sm_scale), _hip.dtype_code(Q), _stream()))
+    return output
+
+
 def dense_causal_attention(Q, K, V, sm_scale: float = None, out: torch.Tensor = None):
     """Plain causal attention on the same MFMA core (the dense baseline the sparse operator is
     compared with; GQA-aware like the reference's flash_attn_triton.py:129-132)."""

@@ -451,4 +451,86 @@ int aa_dense_causal_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   return check_launch(run_flash(a, 2, (hipStream_t)stream), who);
 }
 
+// Sizes of a rows-mode problem, checked and planned: what aa_dense_rows_workspace_bytes and aa_dense_rows_fwd share.
+static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim,
+                           int causal_offset) {
+  if (batch <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_rows <= 0 || n_keys <= 0 || causal_offset < 0) {
+    set_error("%s: batch, head counts, n_rows and n_keys must be positive and causal_offset not negative (got %d, %d, %d, %d, %d, %d)", who,
+              batch, n_q_heads, n_kv_heads, n_rows, n_keys, causal_offset);
+    return AA_EBADARG;
+  }
+  if (n_q_heads % n_kv_heads != 0) {
+    set_error("%s: n_kv_heads (%d) must divide n_q_heads (%d)", who, n_kv_heads, n_q_heads);
+    return AA_EBADARG;
+  }
+  if (head_dim != 128 && head_dim != 64) {
+    set_error("%s: head_dim %d is not supported (128 or 64)", who, head_dim);
+    return AA_EUNSUPPORTED;
+  }
+  if (n_keys > (1 << 20) || n_rows > (1 << 20) || causal_offset > (1 << 20)) {
+    set_error("%s: %d rows, %d keys or causal offset %d is more than 2^20", who, n_rows, n_keys, causal_offset);
+    return AA_EUNSUPPORTED;
+  }
+  // (up to 64 chunks of every column block)
+  if ((int64_t)n_rows * (n_q_heads / n_kv_heads) > 0x3fffffffLL ||
+      (int64_t)batch * n_kv_heads * (((int64_t)n_rows * (n_q_heads / n_kv_heads) + 127) / 128) * 64 > 0x7fffffffLL) {
+    set_error("%s: problem too large for one launch", who);
+    return AA_EUNSUPPORTED;
+  }
+  a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_rows = n_rows; a.n_ctx = n_keys; a.head_dim = head_dim;
+  a.causal_offset = causal_offset;
+  a.big_block = n_keys; a.block_size = 128;  // (unused in this mode; not zero)
+  plan_rows(a);
+  return AA_OK;
+}
+
+static int64_t rows_state_columns(const FlashArgs& a) {
+  return a.n_chunks > 1 ? (int64_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks * 128 : 0;
+}
+
+size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset) {
+  FlashArgs a = {};
+  if (plan_dense_rows("aa_dense_rows_workspace_bytes", a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset)) return 0;
+  return (size_t)rows_state_columns(a) * (head_dim + 2) * 4;  // accumulators, maxima, sums
+}
+
+int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                      const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                      const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                      void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                      void* workspace, size_t workspace_bytes,
+                      int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
+                      float sm_scale, int dtype, void* stream) {
+  const char* who = "aa_dense_rows_fwd";
+  FlashArgs a = {};
+  int rc;
+  if ((rc = check_dtype(dtype, who))) return rc;
+  if ((rc = plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset))) return rc;
+  if ((rc = check_tensor(q, q_sb, q_sh, q_sn, n_rows, head_dim, who, "q"))) return rc;
+  if ((rc = check_tensor(k, k_sb, k_sh, k_sn, n_keys, head_dim, who, "k"))) return rc;
+  if ((rc = check_tensor(v, v_sb, v_sh, v_sn, n_keys, head_dim, who, "v"))) return rc;
+  if ((rc = check_tensor(out, o_sb, o_sh, o_sn, n_rows, head_dim, who, "out"))) return rc;
+  if (!(sm_scale > 0.f)) {  // the running maxima are those of the raw dot products
+    set_error("%s: sm_scale %g must be positive", who, (double)sm_scale);
+    return AA_EUNSUPPORTED;
+  }
+  const int64_t cols = rows_state_columns(a);
+  if (cols > 0) {
+    if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
+    if (workspace_bytes < (size_t)cols * (head_dim + 2) * 4) {
+      set_error("%s: workspace has %zu bytes, %zu needed", who, workspace_bytes, (size_t)cols * (head_dim + 2) * 4);
+      return AA_EBADARG;
+    }
+  }
+  a.q = (const uint16_t*)q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_sn = q_sn;
+  a.k = (const uint16_t*)k; a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
+  a.v = (const uint16_t*)v; a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn;
+  a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
+  a.acc_out = (float*)workspace; a.M_out = a.acc_out + cols * head_dim; a.L_out = a.M_out + cols;
+  a.acc_frag = a.acc_out; a.M = a.M_out; a.L = a.L_out;
+  a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
+  if ((rc = check_launch(run_flash(a, 3, (hipStream_t)stream), who))) return rc;
+  return a.n_chunks > 1 ? check_launch(launch_rows_combine(a, (hipStream_t)stream), who) : AA_OK;
+}
+
 }  // extern "C"

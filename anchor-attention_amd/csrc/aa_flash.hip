@@ -1,7 +1,9 @@
-// MFMA flash-attention core for gfx950, used three ways:
+// MFMA flash-attention core for gfx950, used four ways:
 //   kAnchor : stage 1 - windowed causal attention over [0,S) U [bb*S, r]; emits M, L, Acc
 //   kSparse : stage 3 - resumes from (M, L, Acc) over K/V rows gathered at selected indices
 //   kDense  : plain causal attention (baseline)
+//   kRows   : causal attention of any number of query rows over any number of keys (the rows that the sparse operator does
+//             not cover: ragged tails, short prompts, prompts continued on a cache), the keys split over work-groups
 //
 // Formulation.  A wave owns 32 query rows and computes the TRANSPOSED score tile
 //   S^T[key][query] = K[key][:] . Q[query][:]      (MFMA A = K rows from LDS, B = Q from registers)
@@ -47,7 +49,7 @@ constexpr int kTileBytes = kBN * kRowBytes;
 constexpr int kDist = 4;         // MFMA operands are fetched from LDS this many MFMAs ahead of their use
 constexpr int kIdxWin = 1024;    // selected-key indices held in LDS at a time (16 tiles)
 
-enum FlashMode : int { kAnchor = 0, kSparse = 1, kDense = 2 };
+enum FlashMode : int { kAnchor = 0, kSparse = 1, kDense = 2, kRows = 3 };
 
 // Timing-only ablations.  A build with -DAA_ABLATE=n (`make ablations`) leaves out one ingredient of the kernel so
 // that its cost can be measured (bench_ablations.py); such a build computes WRONG results on purpose, reports
@@ -138,6 +140,11 @@ __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, cons
     const uint32_t key = gather_keys[j];  // this lane's row of the tile's j-th block of 16 rows
     if ((n & 1) == 0) load16_to_lds(kb, __umul24(key, k_row_bytes) + k_col, lds_k + 16 * j * kRowBytes);
     else load16_to_lds(vb, __umul24(key, v_row_bytes) + v_col, lds_v + 16 * j * kRowBytes);
+  } else if (MODE == kRows) {
+    // consecutive keys up to a key count that need not fill the last tile: the caller's per-lane offsets (gather_keys: four
+    // for K, four for V, from the tile's first row) are loop-invariant except that they are clamped for that tile
+    if ((n & 1) == 0) load16_to_lds(kb + (uint64_t)(uint32_t)key0 * k_row_bytes, gather_keys[j], lds_k + 16 * j * kRowBytes);
+    else load16_to_lds(vb + (uint64_t)(uint32_t)key0 * v_row_bytes, gather_keys[4 + j], lds_v + 16 * j * kRowBytes);
   } else {
     // consecutive keys: the first row of the tile's j-th block of 16 rows goes into the (scalar) base address, the
     // thread's row inside the block and its chunk are one loop-invariant vector offset - no vector arithmetic per tile
@@ -175,9 +182,10 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   // list's round trip to memory and the wait for its stores.
   const int group = p.n_q_heads / p.n_kv_heads;
   const int nq = MODE == kSparse ? p.q_blocks_per_wg : 1;
-  const int n_qunit = p.n_ctx / (BM * nq);
+  const int n_qunit = MODE == kRows ? 1 : p.n_ctx / (BM * nq);
   const int S = p.big_block;
   int g, qunit, kvh, b;
+  int chunk = 0;  // (rows) which chunk of the keys
   const uint32_t n_pairs = (uint32_t)(p.batch * p.n_kv_heads) * (uint32_t)(p.n_ctx / S);
   if (MODE == kSparse && n_pairs % 8u == 0u) {
     // Stage 3's work per (KV head, big block) pair is the length of the pair's index lists, which depends on the data:
@@ -196,6 +204,16 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     qunit = bb_ * (S / (BM * nq)) + (int)(within / group);
     kvh = unit % p.n_kv_heads;
     b = unit / p.n_kv_heads;
+  } else if (MODE == kRows) {
+    // A work-group owns 128 columns of one KV head - a column is one (query row, head of the group) pair, heads running
+    // fastest, so all heads of a group use the same K/V tile - and one chunk of the keys.  Work-groups of one chunk are
+    // neighbours on one XCD (they read the same K/V rows), latest columns, which see the most keys, first.
+    uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, p.n_col_blocks * p.n_chunks, 1);
+    qunit = p.n_col_blocks - 1 - (int)(vid % p.n_col_blocks);  vid /= p.n_col_blocks;
+    chunk = vid % p.n_chunks;  vid /= p.n_chunks;
+    kvh = vid % p.n_kv_heads;
+    b = vid / p.n_kv_heads;
+    g = 0;
   } else {
     uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, group * n_qunit, group);
     g = vid % group;  vid /= group;
@@ -265,30 +283,44 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   for (int qb = 0; qb < nq; ++qb) {
   const int R0 = (qunit * nq + qb) * BM;
   const int wr0 = R0 + wave * 32;
-  const int my_row = wr0 + c32;
+  // (rows) this lane's column, as (row, head of the group): columns past the last one repeat it and are not stored
+  const int n_cols = MODE == kRows ? p.n_rows * group : 0;
+  const int my_col = min(wr0 + c32, n_cols - 1);
+  const int my_row = MODE == kRows ? my_col / group : wr0 + c32;
+  // (rows) the last key this lane's row sees, and the smallest such key of the wave (rows ascend with the lane)
+  const int my_last_key = MODE == kRows ? min(p.causal_offset + my_row, p.n_ctx - 1) : my_row;
+  const int wave_last_key = MODE == kRows ? __builtin_amdgcn_readfirstlane(my_last_key) : wr0;
 
   // ---- sparse mode: the queries and the softmax statistics are requested first ----------------------
   // They depend on nothing, whereas the first K/V tile needs the index list, which needs its own round trip to
   // memory.  The 64 KB of accumulator state follow the first tile's loads (further down) and are not waited for
   // before the first scores are computed.
   float m_run, l_run;
-  const uint16_t* qrow = qp + (int64_t)my_row * p.q_sn + 8 * half;
+  const uint16_t* qrow = qp + (int64_t)my_row * p.q_sn + 8 * half + (MODE == kRows ? (my_col - my_row * group) * p.q_sh : 0);
   if (MODE == kSparse && !have_queries) request_queries(my_row);
   const bool feeds_next = list_chains && qb + 1 < nq;  // the next block takes its first tile from this one
 
   // ---- tile schedule -------------------------------------------------------------------------
   const bool pool = MODE == kAnchor && p.qbar_out != nullptr;
   int n_tiles, n_init = 0;
+  int key_base = 0;  // (rows) first key of the chunk
   if (MODE == kAnchor) {
     n_init = min(S, R0 + BM) / kBN;
     n_tiles = n_init + (bb >= 1 ? (R0 + BM - bb * S) / kBN : 0);
   } else if (MODE == kDense) {
     n_tiles = (R0 + BM) / kBN;
+  } else if (MODE == kRows) {
+    const int last_row = min(R0 + BM, n_cols) - 1;
+    const int seen = min(p.causal_offset + last_row / group, p.n_ctx - 1) / kBN + 1;  // tiles up to the last key any column sees
+    key_base = chunk * p.chunk_tiles * kBN;
+    n_tiles = min(seen - chunk * p.chunk_tiles, p.chunk_tiles);
+    if (n_tiles <= 0) return;  // (never chunk 0: every row sees at least one key)
   } else {
     n_tiles = sparse_tiles;
   }
   // first key (anchor, dense) or first list position (sparse) of tile i
-#define AA_TILE_KEY0(i) ((MODE == kAnchor) ? ((i) < n_init ? (i) * kBN : bb * S + ((i) - n_init) * kBN) : (i) * kBN)
+#define AA_TILE_KEY0(i) \
+  ((MODE == kAnchor) ? ((i) < n_init ? (i) * kBN : bb * S + ((i) - n_init) * kBN) : (MODE == kRows ? key_base : 0) + (i) * kBN)
 
   // sparse mode: list positions [w0, w0 + kIdxWin) -> LDS (zeros past the count).  The load is bounded by the list's
   // capacity, not by its count, so that it does not have to wait for the count to arrive; what lies past the count is
@@ -326,19 +358,32 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   const char* qblock = reinterpret_cast<const char*>(qp + (int64_t)R0 * p.q_sn);
   const uint32_t q_row_bytes = (uint32_t)p.q_sn * 2u;
   const uint32_t q_voff = (uint32_t)(tid >> 4) * q_row_bytes + (uint32_t)((tid & 15) & (D / 8 - 1)) * 16u;
+  // (rows) per-lane offsets of a tile's four blocks of 16 K rows and 16 V rows from the tile's first row, of which
+  // `rows_left` lie inside the tensor: lanes past the last key read it again and are masked
+  uint32_t row_offs[8];
+  auto set_row_offs = [&](const int rows_left) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t r = (uint32_t)min((tid >> 4) + 16 * j, rows_left - 1);
+      row_offs[j] = __umul24(r, k_row_bytes) + k_col;
+      row_offs[4 + j] = __umul24(r, v_row_bytes) + v_col;
+    }
+  };
+  if (MODE == kRows) set_row_offs(p.n_ctx - key_base);
   if (n_tiles > 0 && !chained) {
     const uint32_t first = MODE == kSparse ? (uint32_t)cur * kTileBytes : 0u;
     uint32_t keys0[4] = {0u, 0u, 0u, 0u};
     if (MODE == kSparse) tile_gather_keys(keys0, sm.idx, 0, tid);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      tile_fetch_one<MODE>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(0), keys0, lds_k0 + first,
-                           lds_v0 + first, k_voff, v_voff);
+      tile_fetch_one<MODE>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(0), MODE == kRows ? row_offs : keys0,
+                           lds_k0 + first, lds_v0 + first, k_voff, v_voff);
   }
   // the accumulator state: the youngest loads in flight, first needed by the first P.V product
   if (MODE == kSparse && !chained) request_state(my_row);
 
-  // ---- queries: B operand, pre-scaled into the exp2 domain -----------------------------------
+  // ---- queries: B operand, pre-scaled into the exp2 domain (rows: as they are, the scores are scaled in float32) -----
+  const float score_scale = MODE == kRows ? p.sm_scale * kLog2e : 1.f;
   vec8 qreg[kKS];
   {
     const bool chain = (MODE == kAnchor) && (p.scale_mode == 0);
@@ -347,7 +392,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
       for (int ks = 0; ks < kKS; ++ks) qraw[ks] = *reinterpret_cast<const u32x4*>(qrow + 16 * ks);
     }
 #pragma unroll
-    for (int ks = 0; ks < kKS; ++ks) qreg[ks] = scale_q8<T>(qraw[ks], p.sm_scale, chain);
+    for (int ks = 0; ks < kKS; ++ks) qreg[ks] = MODE == kRows ? *reinterpret_cast<const vec8*>(&qraw[ks]) : scale_q8<T>(qraw[ks], p.sm_scale, chain);
   }
 
   // ---- running state (sparse mode loaded it at the top) -----------------------------------------
@@ -415,9 +460,9 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   // causal / list-end mask of one 32-key half (only tiles on the diagonal or at the end of a list need it)
 #define AA_MASK(sx, kb)                                                              \
   if (MODE != kSparse) {                                                             \
-    if (key0 + 32 * (kb) + 31 > wr0) {                                               \
+    if (key0 + 32 * (kb) + 31 > wave_last_key) {                                     \
       _Pragma("unroll") for (int r = 0; r < 16; ++r)                                 \
-        if (AA_KEY_OF(kb, r) > my_row) sx[r] = -INFINITY;                            \
+        if (AA_KEY_OF(kb, r) > my_last_key) sx[r] = -INFINITY;                       \
     }                                                                                \
   } else if (key0 + 32 * (kb) + 32 > cnt) {                                          \
     _Pragma("unroll") for (int r = 0; r < 16; ++r)                                   \
@@ -434,7 +479,8 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     t0 = fmaxf(t0, t3);                                                              \
     mx = max_with_other_half(t0);                                                     \
   }
-#define AA_EXP2(x) ((AA_ABLATE == 1 || AA_ABLATE == 2) ? (x) : fast_exp2(x))
+  // (rows: maxima and scores are kept as raw dot products; the scale is applied to the difference, in float32)
+#define AA_EXP2(x) ((AA_ABLATE == 1 || AA_ABLATE == 2) ? (x) : fast_exp2(MODE == kRows ? (x) * score_scale : (x)))
   // p = exp2(s) for accumulator registers 4c .. 4c+3 of one half, summed and rounded into the P^T fragment words
 #define AA_EXP_CHUNK(sx, pw, sum, c)                                                 \
   {                                                                                  \
@@ -491,6 +537,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     const uint32_t k_voff_sel = fetch_queries ? q_voff : k_voff, v_voff_sel = fetch_queries ? q_voff : v_voff;
     uint32_t keys_next[4] = {0u, 0u, 0u, 0u};  // (sparse) row numbers of the next tile, read before the tile's first load is issued
     if (MODE == kSparse) tile_gather_keys(keys_next, sm.idx, key0_next, tid);
+    if (MODE == kRows && p.n_ctx - key0_next < kBN) set_row_offs(p.n_ctx - key0_next);
 #define AA_FETCH_ONE(n)                                                                                               \
   if (MODE == kAnchor) {                                                                                              \
     const int j_ = (n) >> 1;                                                                                          \
@@ -500,8 +547,8 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     load16_to_lds(fetch_queries ? q_ : kv_, ((n) & 1) ? v_voff_sel : k_voff_sel,                                      \
                   (((n) & 1) ? lds_v0 : lds_k0) + (buf ^ 1) * kTileBytes + 16 * j_ * kRowBytes);                      \
   } else {                                                                                                            \
-    tile_fetch_one<MODE>(n, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, key0_next, keys_next,               \
-                         lds_k0 + (buf ^ 1) * kTileBytes, lds_v0 + (buf ^ 1) * kTileBytes, k_voff, v_voff);           \
+    tile_fetch_one<MODE>(n, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, key0_next,                          \
+                         MODE == kRows ? row_offs : keys_next, lds_k0 + (buf ^ 1) * kTileBytes, lds_v0 + (buf ^ 1) * kTileBytes, k_voff, v_voff);           \
   }
     // (a wave whose rows all lie above this tile - two of the four waves on the last tile of a causal work-group -
     // runs it fully masked: it would only wait at the barrier for the others anyway)
@@ -561,16 +608,18 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
       if (moved0) {
         // slow path: some row's max grew.  Lanes whose max did not move get shift 0 and alpha 1 (exact).
         // S1 is being accumulated on top of the old -m_ref and is shifted once it is complete.
+        // (rows: a chunk may hold no key of a row's so far - its max stays -inf and its reference 0)
         const float m_new = fmaxf(m_run, m_ref + mx0);
-        const float alpha = fast_exp2(m_run - m_new);
-        shift0 = m_new - m_ref;
+        const float m_base = MODE == kRows && m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = AA_EXP2(m_run - m_base);
+        shift0 = m_base - m_ref;
         m_run = m_new;
-        m_ref = m_new;
+        m_ref = m_base;
         l_run *= alpha;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s0[r] -= shift0;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) negm[r] = -m_new;
+        for (int r = 0; r < 16; ++r) negm[r] = -m_base;
 #pragma unroll
         for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -614,15 +663,16 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
       if (moved1) {
         // as above, except that O^T is rescaled only after the P0 V0 products in flight have been added
         const float m_new = fmaxf(m_run, m_ref + mx1);
-        alpha1 = fast_exp2(m_run - m_new);
-        const float shift = m_new - m_ref;
+        const float m_base = MODE == kRows && m_new == -INFINITY ? 0.f : m_new;
+        alpha1 = AA_EXP2(m_run - m_base);
+        const float shift = m_base - m_ref;
         m_run = m_new;
-        m_ref = m_new;
+        m_ref = m_base;
         l_run *= alpha1;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s1[r] -= shift;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) negm[r] = -m_new;
+        for (int r = 0; r < 16; ++r) negm[r] = -m_base;
       }
       AA_FENCE;
 #pragma unroll
@@ -677,9 +727,10 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   if (MODE == kSparse) {
     for (int i = 0; i < n_tiles; ++i) run_tile(std::integral_constant<int, -1>{}, i);
   } else {
-    // 128 query rows and 64-key tiles: the window of a query block always holds an even number of tiles
+    // (anchor, dense: 128 query rows and 64-key tiles, so the window of a query block holds an even number of tiles)
     for (int i = 0; i < n_tiles; i += 2) {
       run_tile(std::integral_constant<int, 0>{}, i);
+      if (MODE == kRows && i + 1 == n_tiles) break;
       run_tile(std::integral_constant<int, 1>{}, i + 1);
     }
   }
@@ -687,6 +738,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
 #undef AA_KEY_OF
 #undef AA_MASK
 #undef AA_ROWMAX
+#undef AA_EXP2
 #undef AA_EXP_CHUNK
 #undef AA_V_SRC
 #undef AA_V_FETCH
@@ -750,6 +802,24 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
         reinterpret_cast<uint16_t*>(p.abar_out)[bh * n_pr + R0 / bs + pp] = (uint16_t)(T::pack(am / d, 0.f) & 0xffffu);
       }
     }
+  } else if (MODE == kRows && p.n_chunks > 1) {
+    // one of several chunks: the unnormalised state goes to the workspace, in fragment order as in anchor mode, and
+    // rows_combine_kernel merges the chunks
+    const int64_t slot = ((((int64_t)b * p.n_kv_heads + kvh) * p.n_col_blocks + qunit) * p.n_chunks + chunk) * 4 + wave;
+    if (half == 0) {
+      p.M_out[slot * 32 + c32] = m_run;
+      p.L_out[slot * 32 + c32] = l_tot;
+    }
+    float* af = p.acc_out + slot * (kDB * 4 * 256) + lane * 4;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        floatx4 t;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = acc[db][rg * 4 + c];
+        *reinterpret_cast<floatx4*>(af + (db * 4 + rg) * 256) = t;
+      }
   } else {
     // out = bf16(acc / l): the wave stages its [32][D] tile in LDS - 32 rows of the tile pitch, 16-byte chunks swizzled
     // with the row like a K tile - and writes whole rows.  The staging area is private to the wave (only a wave-local wait
@@ -785,7 +855,12 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     for (int it = 0; it < 32 / kRowsPerStore; ++it) {
       const int r = it * kRowsPerStore + lane_e / kLanesPerRow, c = lane_e % kLanesPerRow;
       const u32x4 w = *reinterpret_cast<const u32x4*>(ob + r * kRowBytes + ((c ^ (r & kChunkMask)) << 4));
-      __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(op + (int64_t)(wr0 + r) * p.o_sn + 8 * c));
+      if (MODE == kRows) {
+        const int col = wr0 + r, row = col / group;
+        if (col < n_cols) *reinterpret_cast<u32x4*>(op + (col - row * group) * p.o_sh + (int64_t)row * p.o_sn + 8 * c) = w;
+      } else {
+        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(op + (int64_t)(wr0 + r) * p.o_sn + 8 * c));
+      }
     }
     chained = more && list_chains;
     have_queries = more;
@@ -805,7 +880,8 @@ static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
     const int per_big_block = a.big_block / 128;  // even for every supported geometry
     a.q_blocks_per_wg = per_big_block % AA_SPARSE_QBLOCKS == 0 ? AA_SPARSE_QBLOCKS : (per_big_block % 2 == 0 ? 2 : 1);
   }
-  const dim3 grid((uint32_t)a.batch * a.n_q_heads * (a.n_ctx / (128 * a.q_blocks_per_wg))), block(256);
+  const dim3 grid(MODE == kRows ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
+                                : (uint32_t)a.batch * a.n_q_heads * (a.n_ctx / (128 * a.q_blocks_per_wg))), block(256);
   if (a.head_dim == 128) {
     if (a.dtype == 0) hipLaunchKernelGGL((flash_kernel<MODE, Bf16, 128>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((flash_kernel<MODE, F16, 128>), grid, block, 0, stream, a);
@@ -819,6 +895,7 @@ static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
 hipError_t launch_flash(const FlashArgs& a, int mode, hipStream_t stream) {
   if (mode == kAnchor) return launch<kAnchor>(a, stream);
   if (mode == kSparse) return launch<kSparse>(a, stream);
+  if (mode == kRows) return launch<kRows>(a, stream);
   return launch<kDense>(a, stream);
 }
 

@@ -20,11 +20,20 @@ struct FlashArgs {
   int big_block, block_size;
   float sm_scale; int scale_mode;
   int q_blocks_per_wg;  // set by the launcher
+  // rows mode: n_rows query rows over n_ctx keys, row i sees keys 0 .. causal_offset + i.  The (row, head) columns of a
+  // KV head come in blocks of 128, the keys in chunks of chunk_tiles 64-key tiles; with more than one chunk the work-groups
+  // write M_out, L_out, acc_out [batch, n_kv_heads, n_col_blocks, n_chunks, 128 columns] for rows_combine_kernel
+  int n_rows, causal_offset, n_col_blocks, n_chunks, chunk_tiles;
   int dtype;            // AA_DTYPE_BF16 / AA_DTYPE_F16: what the 16-bit elements of q, k, v, out, qbar, abar are
 };
 
-// mode: 0 anchor (stage 1), 1 sparse (stage 3), 2 dense causal
+// mode: 0 anchor (stage 1), 1 sparse (stage 3), 2 dense causal, 3 rows
 hipError_t launch_flash(const FlashArgs& a, int mode, hipStream_t stream);
+
+// rows mode with several chunks: merges the chunks of `a` (the arguments of the launch that wrote them) into a.out
+hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream);
+// rows mode: sets n_col_blocks, n_chunks and chunk_tiles from the sizes
+void plan_rows(FlashArgs& a);
 
 struct PoolArgs {
   const uint16_t* q; int64_t q_sb, q_sh, q_sn;

@@ -1,0 +1,122 @@
+// Dense attention of any number of query rows over any number of keys on gfx950: the planning of the flash kernel's rows
+// mode (aa_flash.hip) and the kernel that merges its key chunks.
+//
+// Why rows have a kernel of their own: library attention takes a ragged causal window only as an explicit boolean mask,
+// and then multiplies, masks and soft-maxes the whole score matrix in float32 in memory.  1089 rows over 40001 keys with
+// 32/8 heads of 128 took 18.7 ms that way and take 0.80 ms + 0.03 ms (combine) here, 0.9 PFLOP/s; 777 rows over 777 keys
+// took 403 us and take 21 us.
+#include "aa_common.h"
+#include "aa_kernels.h"
+
+namespace aa {
+
+// Merges the key chunks of rows mode: out = sum_c w_c acc_c / sum_c w_c l_c with w_c = exp2((m_c - max m) * scale).
+// One work-group per 128-column block and 32-column piece of the head dimension; lane layout and order of the state are
+// those of the flash kernel that wrote it, so every load moves one contiguous KiB per wave.  Bound by reading the state,
+// which the flash kernel has just written (L2 / memory-side cache).
+template <typename T, int D>
+__global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
+  constexpr int kDB = D / 32;
+  const int lane = threadIdx.x & 63, half = lane >> 5, c32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t id = blockIdx.x;
+  const int db = id % kDB;  id /= kDB;
+  const int block = id % p.n_col_blocks;  id /= p.n_col_blocks;
+  const int kvh = id % p.n_kv_heads, b = id / p.n_kv_heads;
+  const int group = p.n_q_heads / p.n_kv_heads, n_cols = p.n_rows * group;
+  // the chunks that hold keys of this block (the others were not written)
+  const int last_row = (min(128 * block + 128, n_cols) - 1) / group;
+  const int tiles = min(p.causal_offset + last_row, p.n_ctx - 1) / 64 + 1;
+  const int n_chunks = (tiles + p.chunk_tiles - 1) / p.chunk_tiles;
+  const int64_t slot0 = ((((int64_t)b * p.n_kv_heads + kvh) * p.n_col_blocks + block) * p.n_chunks) * 4 + wave;
+  const float scale = p.sm_scale * kLog2e;
+
+  float m_all = -INFINITY;
+#pragma unroll 4
+  for (int c = 0; c < n_chunks; ++c) m_all = fmaxf(m_all, p.M[(slot0 + 4 * c) * 32 + c32]);
+  floatx4 acc[4];
+  float l_all = 0.f;
+#pragma unroll
+  for (int rg = 0; rg < 4; ++rg) acc[rg] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int c = 0; c < n_chunks; ++c) {
+    const int64_t slot = slot0 + 4 * c;
+    const float w = fast_exp2((p.M[slot * 32 + c32] - m_all) * scale);
+    l_all += w * p.L[slot * 32 + c32];
+    const float* af = p.acc_frag + (slot * kDB + db) * (4 * 256) + lane * 4;
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) {
+      const floatx4 t = *reinterpret_cast<const floatx4*>(af + rg * 256);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[rg][e] += w * t[e];
+    }
+  }
+  const float inv = 1.f / l_all;
+  uint32_t w[4][2];
+#pragma unroll
+  for (int rg = 0; rg < 4; ++rg) {
+    w[rg][0] = T::pack(acc[rg][0] * inv, acc[rg][1] * inv);
+    w[rg][1] = T::pack(acc[rg][2] * inv, acc[rg][3] * inv);
+  }
+  // a lane holds columns 8*rg + 4*half .. +3 of the piece: the two halves of the wave trade register groups, so that each
+  // lane stores whole 16-byte chunks (half 0 the even groups, half 1 the odd ones)
+  const int col = 128 * block + 32 * wave + c32;
+  const int row = min(col, n_cols - 1) / group;
+  uint16_t* op = p.out + b * p.o_sb + (int64_t)(kvh * group + min(col, n_cols - 1) - row * group) * p.o_sh + (int64_t)row * p.o_sn + 32 * db;
+#pragma unroll
+  for (int pr = 0; pr < 2; ++pr) {
+    const uint32_t r0 = __shfl_xor(half ? w[2 * pr][0] : w[2 * pr + 1][0], 32, 64);
+    const uint32_t r1 = __shfl_xor(half ? w[2 * pr][1] : w[2 * pr + 1][1], 32, 64);
+    uint4 o;
+    if (half == 0) o = uint4{w[2 * pr][0], w[2 * pr][1], r0, r1};
+    else o = uint4{r0, r1, w[2 * pr + 1][0], w[2 * pr + 1][1]};
+    if (col < n_cols) *reinterpret_cast<uint4*>(op + 8 * (2 * pr + half)) = o;
+  }
+}
+
+hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream) {
+  const dim3 grid((uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * (a.head_dim / 32)), block(256);
+  if (a.head_dim == 128) {
+    if (a.dtype == 0) hipLaunchKernelGGL((rows_combine_kernel<Bf16, 128>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((rows_combine_kernel<F16, 128>), grid, block, 0, stream, a);
+  } else {
+    if (a.dtype == 0) hipLaunchKernelGGL((rows_combine_kernel<Bf16, 64>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((rows_combine_kernel<F16, 64>), grid, block, 0, stream, a);
+  }
+  return hipGetLastError();
+}
+
+// How the keys of a rows-mode problem are cut into chunks.  The chip holds 512 work-groups (two per CU).  A tile takes a
+// work-group about 1.9 us with a neighbour on its CU and 1.1 us alone; several chunks cost a write and a read of the state
+// (64 KB per column block and chunk at head dimension 128) and one more launch.  Every number of chunks up to 64 is priced with that
+// and the cheapest is taken.
+void plan_rows(FlashArgs& a) {
+  const int group = a.n_q_heads / a.n_kv_heads;
+  a.n_col_blocks = (a.n_rows * group + 127) / 128;
+  const int64_t units = (int64_t)a.batch * a.n_kv_heads;
+  const int max_tiles = (min(a.causal_offset + a.n_rows, a.n_ctx) + 63) / 64;
+  int64_t total = 0;  // tiles of one unit
+  for (int i = 0; i < a.n_col_blocks; ++i)
+    total += min(a.causal_offset + (min(128 * (i + 1), a.n_rows * group) - 1) / group, a.n_ctx - 1) / 64 + 1;
+  double best = 1e30;
+  a.n_chunks = 1;
+  a.chunk_tiles = max_tiles;
+  for (int n = 1; n <= 64 && n <= max_tiles; ++n) {
+    const int len = (max_tiles + n - 1) / n, chunks = (max_tiles + len - 1) / len;
+    int64_t wgs = 0;
+    for (int i = 0; i < a.n_col_blocks; ++i)
+      wgs += (min(a.causal_offset + (min(128 * (i + 1), a.n_rows * group) - 1) / group, a.n_ctx - 1) / 64 + len) / len;
+    wgs *= units;
+    const double t_tile = wgs <= 256 ? 1.1 : 1.9;
+    const double rounds = (double)((wgs + 511) / 512) * ((double)total * units / wgs);
+    double us = t_tile * (rounds > len ? rounds : len) * a.head_dim / 128;
+    if (chunks > 1) us += 6.0 + (double)wgs * 128 * a.head_dim * 8 / 4e6;
+    if (us < best) {
+      best = us;
+      a.n_chunks = chunks;
+      a.chunk_tiles = len;
+    }
+  }
+}
+
+}  // namespace aa

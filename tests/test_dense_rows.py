@@ -1,0 +1,60 @@
+"""Dense attention of any query rows over any keys (``dense_rows_attention``: ragged tails, short prompts, continued prompts)
+against float64 attention, at the sizes where tiles, column blocks and key chunks end.
+
+Bound: probabilities are rounded to the 16-bit type (unit roundoff u) before the second product, so the sum is off by at most
+u * max|v|, and the result is rounded once more, u * |out|; five per cent on top covers the float32 sums and exp2."""
+import pytest
+import torch
+
+
+def _reference(q, k, v, scale, keep):
+    """float64 attention, head by head; ``keep`` [B,n_rows,n_keys] says which keys a row sees (a row without any gives 0)."""
+    group = q.shape[1] // k.shape[1]
+    out = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    for h in range(q.shape[1]):
+        kt = k[:, h // group].double().transpose(1, 2).contiguous()
+        s = torch.matmul(q[:, h].double(), kt) * scale
+        p = torch.nan_to_num(s.masked_fill(~keep, float("-inf")).softmax(-1))
+        out[:, h] = torch.matmul(p, v[:, h // group].double())
+    return out
+
+
+def _check(out, want, v, dtype):
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    err, bound = (out.double() - want).abs(), 1.05 * u * (v.double().abs().max() + want.abs())
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+def _qkv(batch, hq, hkv, n_rows, n_keys, d, dtype, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    # queries in the [B,N,H,D] storage a model hands over, keys and values as a cache holds them; large scores (a spread of
+    # about 4) so that single keys matter
+    q = (4.0 * torch.randn(batch, n_rows, hq, d, generator=g, device="cuda")).to(dtype).transpose(1, 2)
+    k = torch.randn(batch, hkv, n_keys, d, generator=g, device="cuda").to(dtype)
+    v = torch.randn(batch, hkv, n_keys, d, generator=g, device="cuda").to(dtype)
+    return q, k, v
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,hq,hkv,n_rows,offset,d,dtype", [
+    (1, 4, 2, 77, 4096, 128, torch.bfloat16),     # a tail: several chunks, the last of them ragged
+    (1, 32, 8, 127, 0, 128, torch.bfloat16),      # a short prompt: fewer keys in the early column blocks
+    (2, 14, 2, 65, 0, 64, torch.bfloat16),        # a group of seven: column blocks that cut a row's heads
+    (1, 28, 4, 64, 12345, 128, torch.float16),    # many chunks; rows whose last chunk holds no key of theirs
+    (3, 8, 8, 130, 63, 64, torch.float16),        # no groups, two column blocks, chunk and tile edges
+    (1, 7, 1, 33, 0, 128, torch.bfloat16),        # fewer keys than a tile
+    (1, 2, 1, 2047, 2048, 64, torch.bfloat16),    # the longest tail
+])
+def test_dense_rows_against_float64(batch, hq, hkv, n_rows, offset, d, dtype):
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention, dense_rows_supported
+    n_keys = offset + n_rows
+    q, k, v = _qkv(batch, hq, hkv, n_rows, n_keys, d, dtype, n_rows + offset)
+    assert dense_rows_supported(q, k, v)
+    out = torch.full((batch, n_rows, hq, d), float("nan"), dtype=dtype, device="cuda").transpose(1, 2)
+    got = dense_rows_attention(q, k, v, offset, out=out)
+    assert got is out
+    keys, rows = torch.arange(n_keys, device="cuda"), torch.arange(n_rows, device="cuda") + offset
+    keep = (keys[None, :] <= rows[:, None]).expand(batch, -1, -1)
+    _check(out, _reference(q, k, v, d ** -0.5, keep), v, dtype)
+    again = dense_rows_attention(q.contiguous(), k, v, offset, sm_scale=d ** -0.5)
+    assert torch.equal(again, out)
