@@ -174,17 +174,24 @@ def dense_rows_supported(Q, K, V) -> bool:
     return True
 
 
-def dense_rows_attention(Q, K, V, causal_offset: int, sm_scale: float = None, out: torch.Tensor = None):
-    """Causal attention of ``Q`` ``[B,H,n_rows,D]`` over ``K``/``V`` ``[B,H_kv,n_keys,D]`` on the same MFMA core: query row
-    ``i`` sees keys ``0 .. causal_offset + i``.  Any row and key count (:func:`dense_rows_supported` names the rest)."""
+def dense_rows_attention(Q, K, V, causal_offset: int = 0, sm_scale: float = None, out: torch.Tensor = None, mask: torch.Tensor = None):
+    """Attention of ``Q`` ``[B,H,n_rows,D]`` over ``K``/``V`` ``[B,H_kv,n_keys,D]`` on the same MFMA core: query row ``i``
+    sees keys ``0 .. causal_offset + i``, or, with a boolean ``mask`` ``[B or 1, 1, n_rows, n_keys]``, the keys it is True for.
+    Any row and key count (:func:`dense_rows_supported` names the rest)."""
     B, H, N, D = Q.shape
+    n_keys = K.shape[2]
     sm_scale = sm_scale if sm_scale else 1.0 / (D ** 0.5)
     output = torch.empty_like(Q) if out is None else out
+    mask_args = (None, 0, 0)
+    if mask is not None:
+        assert mask.dtype == torch.bool and mask.shape[0] in (1, B) and tuple(mask.shape[1:]) == (1, N, n_keys)
+        mask = mask if mask.stride(3) == 1 else mask.contiguous()
+        mask_args = (mask.data_ptr(), mask.stride(0) if mask.shape[0] > 1 else 0, mask.stride(2))
     lib = _hip.lib()
-    sizes = (B, H, K.shape[1], N, K.shape[2], D, int(causal_offset))
-    nbytes = lib.aa_dense_rows_workspace_bytes(*sizes)
+    sizes = (B, H, K.shape[1], N, n_keys, D, int(causal_offset))
+    nbytes = lib.aa_dense_rows_workspace_bytes(*sizes, mask is not None)
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=Q.device) if nbytes else None
-    _hip.check(lib.aa_dense_rows_fwd(*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output),
+    _hip.check(lib.aa_dense_rows_fwd(*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output), *mask_args,
                                      ws.data_ptr() if nbytes else None, nbytes, *sizes,
                                      float(sm_scale), _hip.dtype_code(Q), _stream()))
     return output

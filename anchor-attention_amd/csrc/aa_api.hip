@@ -451,9 +451,9 @@ int aa_dense_causal_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   return check_launch(run_flash(a, 2, (hipStream_t)stream), who);
 }
 
-// Sizes of a rows-mode problem, checked and planned: what aa_dense_rows_workspace_bytes and aa_dense_rows_fwd share.
+// Sizes of a rows-mode problem, checked and planned; `masked`: with a boolean mask in the place of the causal rule.
 static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim,
-                           int causal_offset) {
+                           int causal_offset, bool masked) {
   if (batch <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_rows <= 0 || n_keys <= 0 || causal_offset < 0) {
     set_error("%s: batch, head counts, n_rows and n_keys must be positive and causal_offset not negative (got %d, %d, %d, %d, %d, %d)", who,
               batch, n_q_heads, n_kv_heads, n_rows, n_keys, causal_offset);
@@ -471,33 +471,47 @@ static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_hea
     set_error("%s: %d rows, %d keys or causal offset %d is more than 2^20", who, n_rows, n_keys, causal_offset);
     return AA_EUNSUPPORTED;
   }
-  // (up to 64 chunks of every column block)
-  if ((int64_t)n_rows * (n_q_heads / n_kv_heads) > 0x3fffffffLL ||
-      (int64_t)batch * n_kv_heads * (((int64_t)n_rows * (n_q_heads / n_kv_heads) + 127) / 128) * 64 > 0x7fffffffLL) {
+  const int64_t col_blocks = ((int64_t)n_rows * (n_q_heads / n_kv_heads) + 127) / 128;
+  // (up to 64 chunks of every column block in one launch; the mask kernel counts column blocks and batch in its grid's y and z, and a row's packed mask has a 32-bit byte offset)
+  if (col_blocks > 0x7fffff || (int64_t)batch * n_kv_heads * col_blocks * 64 > 0x7fffffffLL || (masked && (col_blocks > 65535 || batch > 65535 || (int64_t)n_rows * ((n_keys + 63) / 64) * 8 > 0xffffffffLL))) {
     set_error("%s: problem too large for one launch", who);
     return AA_EUNSUPPORTED;
   }
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_rows = n_rows; a.n_ctx = n_keys; a.head_dim = head_dim;
-  a.causal_offset = causal_offset;
+  a.causal_offset = masked ? n_keys : causal_offset;
+  a.mask_words_per_row = masked ? (n_keys + 63) / 64 : 0;
   a.big_block = n_keys; a.block_size = 128;  // (unused in this mode; not zero)
   plan_rows(a);
   return AA_OK;
 }
 
-static int64_t rows_state_columns(const FlashArgs& a) {
-  return a.n_chunks > 1 ? (int64_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks * 128 : 0;
+// Scratch of a rows-mode problem: the state of its chunks, then the packed mask and its tile flags.
+struct RowsScratch {
+  int64_t state_columns;
+  size_t words, flags, total;
+};
+static RowsScratch carve_rows(const FlashArgs& a) {
+  RowsScratch r;
+  r.state_columns = a.n_chunks > 1 ? (int64_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks * 128 : 0;
+  r.words = align256((size_t)r.state_columns * (a.head_dim + 2) * 4);  // accumulators, maxima, sums
+  r.flags = r.words + align256((size_t)a.batch * a.n_rows * a.mask_words_per_row * 8);
+  r.total = r.flags + (size_t)a.batch * a.n_col_blocks * a.mask_words_per_row;
+  return r;
 }
 
-size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset) {
+size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
+                                     int masked) {
   FlashArgs a = {};
-  if (plan_dense_rows("aa_dense_rows_workspace_bytes", a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset)) return 0;
-  return (size_t)rows_state_columns(a) * (head_dim + 2) * 4;  // accumulators, maxima, sums
+  if (plan_dense_rows("aa_dense_rows_workspace_bytes", a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, masked != 0))
+    return 0;
+  return carve_rows(a).total;
 }
 
 int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                       const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                       const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                       void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                      const uint8_t* mask, int64_t mask_sb, int64_t mask_sn,
                       void* workspace, size_t workspace_bytes,
                       int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
                       float sm_scale, int dtype, void* stream) {
@@ -505,7 +519,7 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   FlashArgs a = {};
   int rc;
   if ((rc = check_dtype(dtype, who))) return rc;
-  if ((rc = plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset))) return rc;
+  if ((rc = plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, mask != nullptr))) return rc;
   if ((rc = check_tensor(q, q_sb, q_sh, q_sn, n_rows, head_dim, who, "q"))) return rc;
   if ((rc = check_tensor(k, k_sb, k_sh, k_sn, n_keys, head_dim, who, "k"))) return rc;
   if ((rc = check_tensor(v, v_sb, v_sh, v_sn, n_keys, head_dim, who, "v"))) return rc;
@@ -514,11 +528,11 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
     set_error("%s: sm_scale %g must be positive", who, (double)sm_scale);
     return AA_EUNSUPPORTED;
   }
-  const int64_t cols = rows_state_columns(a);
-  if (cols > 0) {
+  const RowsScratch r = carve_rows(a);
+  if (r.total > 0) {
     if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
-    if (workspace_bytes < (size_t)cols * (head_dim + 2) * 4) {
-      set_error("%s: workspace has %zu bytes, %zu needed", who, workspace_bytes, (size_t)cols * (head_dim + 2) * 4);
+    if (workspace_bytes < r.total) {
+      set_error("%s: workspace has %zu bytes, %zu needed", who, workspace_bytes, r.total);
       return AA_EBADARG;
     }
   }
@@ -526,10 +540,16 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   a.k = (const uint16_t*)k; a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
   a.v = (const uint16_t*)v; a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn;
   a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
-  a.acc_out = (float*)workspace; a.M_out = a.acc_out + cols * head_dim; a.L_out = a.M_out + cols;
+  char* ws = static_cast<char*>(workspace);
+  a.acc_out = (float*)ws; a.M_out = a.acc_out + r.state_columns * head_dim; a.L_out = a.M_out + r.state_columns;
   a.acc_frag = a.acc_out; a.M = a.M_out; a.L = a.L_out;
   a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
-  if ((rc = check_launch(run_flash(a, 3, (hipStream_t)stream), who))) return rc;
+  if (mask != nullptr) {
+    a.mask_words = (const uint64_t*)(ws + r.words);
+    a.tile_flags = (const uint8_t*)(ws + r.flags);
+    if ((rc = check_launch(launch_mask_pack(a, mask, mask_sb, mask_sn, (hipStream_t)stream), who))) return rc;
+  }
+  if ((rc = check_launch(run_flash(a, mask != nullptr ? 4 : 3, (hipStream_t)stream), who))) return rc;
   return a.n_chunks > 1 ? check_launch(launch_rows_combine(a, (hipStream_t)stream), who) : AA_OK;
 }
 

@@ -4,6 +4,7 @@
 //   kDense  : plain causal attention (baseline)
 //   kRows   : causal attention of any number of query rows over any number of keys (the rows that the sparse operator does
 //             not cover: ragged tails, short prompts, prompts continued on a cache), the keys split over work-groups
+//   kMasked : the same with a boolean mask (padded batches, sliding windows) instead of the causal rule
 //
 // Formulation.  A wave owns 32 query rows and computes the TRANSPOSED score tile
 //   S^T[key][query] = K[key][:] . Q[query][:]      (MFMA A = K rows from LDS, B = Q from registers)
@@ -48,8 +49,9 @@ constexpr int kRowBytes = 256;   // pitch of a K/V row in LDS (128 16-bit elemen
 constexpr int kTileBytes = kBN * kRowBytes;
 constexpr int kDist = 4;         // MFMA operands are fetched from LDS this many MFMAs ahead of their use
 constexpr int kIdxWin = 1024;    // selected-key indices held in LDS at a time (16 tiles)
+constexpr int32_t kMixedTile = 1 << 30;  // (masked) flag of a listed tile of which some pairs are masked
 
-enum FlashMode : int { kAnchor = 0, kSparse = 1, kDense = 2, kRows = 3 };
+enum FlashMode : int { kAnchor = 0, kSparse = 1, kDense = 2, kRows = 3, kMasked = 4 };
 
 // Timing-only ablations.  A build with -DAA_ABLATE=n (`make ablations`) leaves out one ingredient of the kernel so
 // that its cost can be measured (bench_ablations.py); such a build computes WRONG results on purpose, reports
@@ -73,13 +75,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
-template <bool WITH_IDX>
+template <int MODE>
 struct FlashSmem {
   struct {
     char k[2][kTileBytes];
     char v[2][kTileBytes];
   } t;  // (the epilogue stages the output in the tile space)
-  int32_t idx[WITH_IDX ? kIdxWin : 4];  // sparse mode: window of the big block's index list
+  // sparse mode: window of the big block's index list; masked mode: the chunk's tiles that hold a visible key, and their number
+  int32_t idx[MODE == kSparse ? kIdxWin : MODE == kMasked ? kMaskedTiles + 4 : 4];
 };
 
 // Query pre-scaling into the exp2 domain, eight elements at a time.  `chain`: both constants and both products rounded
@@ -140,7 +143,7 @@ __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, cons
     const uint32_t key = gather_keys[j];  // this lane's row of the tile's j-th block of 16 rows
     if ((n & 1) == 0) load16_to_lds(kb, __umul24(key, k_row_bytes) + k_col, lds_k + 16 * j * kRowBytes);
     else load16_to_lds(vb, __umul24(key, v_row_bytes) + v_col, lds_v + 16 * j * kRowBytes);
-  } else if (MODE == kRows) {
+  } else if (MODE == kRows || MODE == kMasked) {
     // consecutive keys up to a key count that need not fill the last tile: the caller's per-lane offsets (gather_keys: four
     // for K, four for V, from the tile's first row) are loop-invariant except that they are clamped for that tile
     if ((n & 1) == 0) load16_to_lds(kb + (uint64_t)(uint32_t)key0 * k_row_bytes, gather_keys[j], lds_k + 16 * j * kRowBytes);
@@ -161,8 +164,9 @@ template <int MODE, typename T, int D>
 __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   typedef typename T::vec8 vec8;
   typedef __attribute__((address_space(3))) vec8 lds_vec8;
-  __shared__ __attribute__((aligned(16))) FlashSmem<MODE == kSparse> sm;
+  __shared__ __attribute__((aligned(16))) FlashSmem<MODE> sm;
   constexpr int BM = 128;
+  constexpr bool kAnyRows = MODE == kRows || MODE == kMasked;
   static_assert(D == 128 || D == 64, "head dimension");
   constexpr int kKS = D / 16;       // MFMAs per 32-key block of S^T = K Q^T
   constexpr int kDB = D / 32;       // 32-column blocks of the head dimension: accumulators of O^T
@@ -182,7 +186,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   // list's round trip to memory and the wait for its stores.
   const int group = p.n_q_heads / p.n_kv_heads;
   const int nq = MODE == kSparse ? p.q_blocks_per_wg : 1;
-  const int n_qunit = MODE == kRows ? 1 : p.n_ctx / (BM * nq);
+  const int n_qunit = kAnyRows ? 1 : p.n_ctx / (BM * nq);
   const int S = p.big_block;
   int g, qunit, kvh, b;
   int chunk = 0;  // (rows) which chunk of the keys
@@ -204,7 +208,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     qunit = bb_ * (S / (BM * nq)) + (int)(within / group);
     kvh = unit % p.n_kv_heads;
     b = unit / p.n_kv_heads;
-  } else if (MODE == kRows) {
+  } else if (kAnyRows) {
     // A work-group owns 128 columns of one KV head - a column is one (query row, head of the group) pair, heads running
     // fastest, so all heads of a group use the same K/V tile - and one chunk of the keys.  Work-groups of one chunk are
     // neighbours on one XCD (they read the same K/V rows), latest columns, which see the most keys, first.
@@ -284,19 +288,19 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   const int R0 = (qunit * nq + qb) * BM;
   const int wr0 = R0 + wave * 32;
   // (rows) this lane's column, as (row, head of the group): columns past the last one repeat it and are not stored
-  const int n_cols = MODE == kRows ? p.n_rows * group : 0;
+  const int n_cols = kAnyRows ? p.n_rows * group : 0;
   const int my_col = min(wr0 + c32, n_cols - 1);
-  const int my_row = MODE == kRows ? my_col / group : wr0 + c32;
+  const int my_row = kAnyRows ? my_col / group : wr0 + c32;
   // (rows) the last key this lane's row sees, and the smallest such key of the wave (rows ascend with the lane)
-  const int my_last_key = MODE == kRows ? min(p.causal_offset + my_row, p.n_ctx - 1) : my_row;
-  const int wave_last_key = MODE == kRows ? __builtin_amdgcn_readfirstlane(my_last_key) : wr0;
+  const int my_last_key = kAnyRows ? min(p.causal_offset + my_row, p.n_ctx - 1) : my_row;
+  const int wave_last_key = kAnyRows ? __builtin_amdgcn_readfirstlane(my_last_key) : wr0;
 
   // ---- sparse mode: the queries and the softmax statistics are requested first ----------------------
   // They depend on nothing, whereas the first K/V tile needs the index list, which needs its own round trip to
   // memory.  The 64 KB of accumulator state follow the first tile's loads (further down) and are not waited for
   // before the first scores are computed.
   float m_run, l_run;
-  const uint16_t* qrow = qp + (int64_t)my_row * p.q_sn + 8 * half + (MODE == kRows ? (my_col - my_row * group) * p.q_sh : 0);
+  const uint16_t* qrow = qp + (int64_t)my_row * p.q_sn + 8 * half + (kAnyRows ? (my_col - my_row * group) * p.q_sh : 0);
   if (MODE == kSparse && !have_queries) request_queries(my_row);
   const bool feeds_next = list_chains && qb + 1 < nq;  // the next block takes its first tile from this one
 
@@ -304,23 +308,50 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   const bool pool = MODE == kAnchor && p.qbar_out != nullptr;
   int n_tiles, n_init = 0;
   int key_base = 0;  // (rows) first key of the chunk
+  int entry_next = 0;  // (masked) list entry of the tile to be fetched next
+  u32x2 mask_word_next = {0u, 0u};  // (masked) which of that tile's 64 keys this lane's row sees, if the tile is a mixed one
+  const uint32_t mask_row_off = MODE == kMasked ? (uint32_t)my_row * (uint32_t)p.mask_words_per_row * 8u : 0u;  // (below 2^32: checked on the host)
+  auto request_mask_word = [&]() __attribute__((always_inline)) {
+    if (MODE == kMasked && (entry_next & kMixedTile)) {
+      const char* w = reinterpret_cast<const char*>(p.mask_words + ((int64_t)b * p.n_rows * p.mask_words_per_row + (entry_next & (kMixedTile - 1))));
+      mask_word_next = *reinterpret_cast<const u32x2*>(w + mask_row_off);
+    }
+  };
   if (MODE == kAnchor) {
     n_init = min(S, R0 + BM) / kBN;
     n_tiles = n_init + (bb >= 1 ? (R0 + BM - bb * S) / kBN : 0);
   } else if (MODE == kDense) {
     n_tiles = (R0 + BM) / kBN;
-  } else if (MODE == kRows) {
+  } else if (kAnyRows) {
     const int last_row = min(R0 + BM, n_cols) - 1;
     const int seen = min(p.causal_offset + last_row / group, p.n_ctx - 1) / kBN + 1;  // tiles up to the last key any column sees
     key_base = chunk * p.chunk_tiles * kBN;
     n_tiles = min(seen - chunk * p.chunk_tiles, p.chunk_tiles);
     if (n_tiles <= 0) return;  // (never chunk 0: every row sees at least one key)
+    if (MODE == kMasked) {
+      // list the chunk's tiles in which any row of the work-group sees a key
+      if (wave == 0) {
+        const uint8_t* flags = p.tile_flags + ((int64_t)b * p.n_col_blocks + qunit) * p.mask_words_per_row + chunk * p.chunk_tiles;
+        int listed = 0;
+        for (int t = 0; t < n_tiles; t += 64) {
+          const int flag = t + lane < n_tiles ? flags[t + lane] : 0;
+          const uint64_t some = __ballot(flag != 0);
+          if (flag) sm.idx[listed + __popcll(some & ((1ull << lane) - 1))] = (chunk * p.chunk_tiles + t + lane) | (flag == 1 ? kMixedTile : 0);
+          listed += __popcll(some);
+        }
+        if (lane == 0) sm.idx[kMaskedTiles] = listed;
+      }
+      __syncthreads();
+      n_tiles = __builtin_amdgcn_readfirstlane(sm.idx[kMaskedTiles]);
+      entry_next = n_tiles > 0 ? __builtin_amdgcn_readfirstlane(sm.idx[0]) : 0;
+    }
   } else {
     n_tiles = sparse_tiles;
   }
   // first key (anchor, dense) or first list position (sparse) of tile i
 #define AA_TILE_KEY0(i) \
-  ((MODE == kAnchor) ? ((i) < n_init ? (i) * kBN : bb * S + ((i) - n_init) * kBN) : (MODE == kRows ? key_base : 0) + (i) * kBN)
+  (MODE == kMasked ? (entry_next & (kMixedTile - 1)) * kBN \
+   : (MODE == kAnchor) ? ((i) < n_init ? (i) * kBN : bb * S + ((i) - n_init) * kBN) : (kAnyRows ? key_base : 0) + (i) * kBN)
 
   // sparse mode: list positions [w0, w0 + kIdxWin) -> LDS (zeros past the count).  The load is bounded by the list's
   // capacity, not by its count, so that it does not have to wait for the count to arrive; what lies past the count is
@@ -361,29 +392,36 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   // (rows) per-lane offsets of a tile's four blocks of 16 K rows and 16 V rows from the tile's first row, of which
   // `rows_left` lie inside the tensor: lanes past the last key read it again and are masked
   uint32_t row_offs[8];
+  // (from an opaque copy of the thread number: the pieces would otherwise occupy registers throughout the tile loop for
+  // the one time that the offsets are clamped)
   auto set_row_offs = [&](const int rows_left) __attribute__((always_inline)) {
+    int t = tid;
+    asm volatile("" : "+v"(t));
+    const uint32_t kc = (uint32_t)(((t & 15) ^ ((t >> 4) & 15)) & (D / 8 - 1)) * 16u;
+    const uint32_t vc = (uint32_t)(((t & 15) ^ (((t >> 4) & 7) << 1)) & (D / 8 - 1)) * 16u;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const uint32_t r = (uint32_t)min((tid >> 4) + 16 * j, rows_left - 1);
-      row_offs[j] = __umul24(r, k_row_bytes) + k_col;
-      row_offs[4 + j] = __umul24(r, v_row_bytes) + v_col;
+      const uint32_t r = (uint32_t)min((t >> 4) + 16 * j, rows_left - 1);
+      row_offs[j] = __umul24(r, k_row_bytes) + kc;
+      row_offs[4 + j] = __umul24(r, v_row_bytes) + vc;
     }
   };
-  if (MODE == kRows) set_row_offs(p.n_ctx - key_base);
+  if (kAnyRows) set_row_offs(p.n_ctx - AA_TILE_KEY0(0));
+  request_mask_word();
   if (n_tiles > 0 && !chained) {
     const uint32_t first = MODE == kSparse ? (uint32_t)cur * kTileBytes : 0u;
     uint32_t keys0[4] = {0u, 0u, 0u, 0u};
     if (MODE == kSparse) tile_gather_keys(keys0, sm.idx, 0, tid);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      tile_fetch_one<MODE>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(0), MODE == kRows ? row_offs : keys0,
+      tile_fetch_one<MODE>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(0), kAnyRows ? row_offs : keys0,
                            lds_k0 + first, lds_v0 + first, k_voff, v_voff);
   }
   // the accumulator state: the youngest loads in flight, first needed by the first P.V product
   if (MODE == kSparse && !chained) request_state(my_row);
 
   // ---- queries: B operand, pre-scaled into the exp2 domain (rows: as they are, the scores are scaled in float32) -----
-  const float score_scale = MODE == kRows ? p.sm_scale * kLog2e : 1.f;
+  const float score_scale = kAnyRows ? p.sm_scale * kLog2e : 1.f;
   vec8 qreg[kKS];
   {
     const bool chain = (MODE == kAnchor) && (p.scale_mode == 0);
@@ -392,7 +430,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
       for (int ks = 0; ks < kKS; ++ks) qraw[ks] = *reinterpret_cast<const u32x4*>(qrow + 16 * ks);
     }
 #pragma unroll
-    for (int ks = 0; ks < kKS; ++ks) qreg[ks] = MODE == kRows ? *reinterpret_cast<const vec8*>(&qraw[ks]) : scale_q8<T>(qraw[ks], p.sm_scale, chain);
+    for (int ks = 0; ks < kKS; ++ks) qreg[ks] = kAnyRows ? *reinterpret_cast<const vec8*>(&qraw[ks]) : scale_q8<T>(qraw[ks], p.sm_scale, chain);
   }
 
   // ---- running state (sparse mode loaded it at the top) -----------------------------------------
@@ -459,7 +497,14 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
 #define AA_KEY_OF(kb, r) (key0 + 32 * (kb) + 8 * ((r) >> 2) + 4 * half + ((r) & 3))
   // causal / list-end mask of one 32-key half (only tiles on the diagonal or at the end of a list need it)
 #define AA_MASK(sx, kb)                                                              \
-  if (MODE != kSparse) {                                                             \
+  if (MODE == kMasked) {                                                             \
+    if (mixed) {                                                                     \
+      uint32_t seen_ = mask_word[kb];                                                \
+      asm volatile("" : "+v"(seen_)); /* (the bits are taken apart here, not earlier) */ \
+      _Pragma("unroll") for (int r = 0; r < 16; ++r)                                 \
+        if (!((seen_ >> (8 * (r >> 2) + (r & 3))) & 1u)) sx[r] = -INFINITY;          \
+    }                                                                                \
+  } else if (MODE != kSparse) {                                                             \
     if (key0 + 32 * (kb) + 31 > wave_last_key) {                                     \
       _Pragma("unroll") for (int r = 0; r < 16; ++r)                                 \
         if (AA_KEY_OF(kb, r) > my_last_key) sx[r] = -INFINITY;                       \
@@ -480,7 +525,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     mx = max_with_other_half(t0);                                                     \
   }
   // (rows: maxima and scores are kept as raw dot products; the scale is applied to the difference, in float32)
-#define AA_EXP2(x) ((AA_ABLATE == 1 || AA_ABLATE == 2) ? (x) : fast_exp2(MODE == kRows ? (x) * score_scale : (x)))
+#define AA_EXP2(x) ((AA_ABLATE == 1 || AA_ABLATE == 2) ? (x) : fast_exp2(kAnyRows ? (x) * score_scale : (x)))
   // p = exp2(s) for accumulator registers 4c .. 4c+3 of one half, summed and rounded into the P^T fragment words
 #define AA_EXP_CHUNK(sx, pw, sum, c)                                                 \
   {                                                                                  \
@@ -509,13 +554,15 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   // One tile.  The LDS buffer it reads (BUF) is a compile-time constant - the loop below is unrolled by two - so that
   // the buffer's offset is part of every LDS instruction's immediate offset and the read addresses are loop-invariant.
   // Sparse mode, whose tile counts can be odd, keeps one copy of the tile (BUF = -1): the buffer is i & 1 and the read
-  // addresses step back and forth between the two buffers.
+  // addresses step back and forth between the two buffers.  So does masked mode, for which two copies spill 25 registers.
   int32_t buf_step = (MODE == kSparse && cur) ? -kTileBytes : kTileBytes;
   auto run_tile = [&](auto buf_const, const int i) __attribute__((always_inline)) {
     constexpr int kBuf = decltype(buf_const)::value;
     constexpr uint32_t rd_off = kBuf > 0 ? kBuf * kTileBytes : 0;  // immediate part of the LDS read addresses
     const int buf = kBuf >= 0 ? kBuf : cur;
-    const int key0 = AA_TILE_KEY0(i);
+    const int key0 = AA_TILE_KEY0(i);  // (masked: entry_next is still this tile's)
+    const bool mixed = MODE == kMasked && (entry_next & kMixedTile);
+    const u32x2 mask_word = {mask_word_next[0] >> (4 * half), mask_word_next[1] >> (4 * half)};
     if (MODE == kSparse && i + 1 < n_tiles && ((i + 1) & (kIdxWin / kBN - 1)) == 0) {
       // tile i+1 opens the next window; everyone finished reading the old one before the last barrier
       fill_index_window((i + 1) * kBN);
@@ -530,6 +577,10 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     // chunks in place)
     // (sparse, chained: the last tile of a block fetches the list's first tile, for the next block)
     const int i_next = i + 1 < n_tiles ? i + 1 : (feeds_next ? 0 : i);
+    if (MODE == kMasked) {
+      entry_next = __builtin_amdgcn_readfirstlane(sm.idx[i_next]);
+      request_mask_word();
+    }
     const int key0_next = AA_TILE_KEY0(i_next);
     const bool fetch_queries = MODE == kAnchor && pool && i + 1 == n_tiles;  // wave-uniform
     // (selects, not branches: the eight slots stay straight-line code; the base address is scalar, and the vector offset
@@ -537,7 +588,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     const uint32_t k_voff_sel = fetch_queries ? q_voff : k_voff, v_voff_sel = fetch_queries ? q_voff : v_voff;
     uint32_t keys_next[4] = {0u, 0u, 0u, 0u};  // (sparse) row numbers of the next tile, read before the tile's first load is issued
     if (MODE == kSparse) tile_gather_keys(keys_next, sm.idx, key0_next, tid);
-    if (MODE == kRows && p.n_ctx - key0_next < kBN) set_row_offs(p.n_ctx - key0_next);
+    if (kAnyRows && p.n_ctx - key0_next < kBN) set_row_offs(p.n_ctx - key0_next);
 #define AA_FETCH_ONE(n)                                                                                               \
   if (MODE == kAnchor) {                                                                                              \
     const int j_ = (n) >> 1;                                                                                          \
@@ -548,7 +599,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
                   (((n) & 1) ? lds_v0 : lds_k0) + (buf ^ 1) * kTileBytes + 16 * j_ * kRowBytes);                      \
   } else {                                                                                                            \
     tile_fetch_one<MODE>(n, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, key0_next,                          \
-                         MODE == kRows ? row_offs : keys_next, lds_k0 + (buf ^ 1) * kTileBytes, lds_v0 + (buf ^ 1) * kTileBytes, k_voff, v_voff);           \
+                         kAnyRows ? row_offs : keys_next, lds_k0 + (buf ^ 1) * kTileBytes, lds_v0 + (buf ^ 1) * kTileBytes, k_voff, v_voff);           \
   }
     // (a wave whose rows all lie above this tile - two of the four waves on the last tile of a causal work-group -
     // runs it fully masked: it would only wait at the barrier for the others anyway)
@@ -610,7 +661,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
         // S1 is being accumulated on top of the old -m_ref and is shifted once it is complete.
         // (rows: a chunk may hold no key of a row's so far - its max stays -inf and its reference 0)
         const float m_new = fmaxf(m_run, m_ref + mx0);
-        const float m_base = MODE == kRows && m_new == -INFINITY ? 0.f : m_new;
+        const float m_base = kAnyRows && m_new == -INFINITY ? 0.f : m_new;
         const float alpha = AA_EXP2(m_run - m_base);
         shift0 = m_base - m_ref;
         m_run = m_new;
@@ -663,7 +714,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
       if (moved1) {
         // as above, except that O^T is rescaled only after the P0 V0 products in flight have been added
         const float m_new = fmaxf(m_run, m_ref + mx1);
-        const float m_base = MODE == kRows && m_new == -INFINITY ? 0.f : m_new;
+        const float m_base = kAnyRows && m_new == -INFINITY ? 0.f : m_new;
         alpha1 = AA_EXP2(m_run - m_base);
         const float shift = m_base - m_ref;
         m_run = m_new;
@@ -722,15 +773,17 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
       cur ^= 1;
     }
     if (AA_ABLATE != 9) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile i+1 has landed in LDS
+    // (so has the mask word: named here, or the compiler would wait for it behind the next tile's loads)
+    if (MODE == kMasked) asm volatile("" : "+v"(mask_word_next[0]), "+v"(mask_word_next[1]));
     if (AA_ABLATE != 8 && AA_ABLATE != 9) __syncthreads();
   };
-  if (MODE == kSparse) {
+  if (MODE == kSparse || MODE == kMasked) {
     for (int i = 0; i < n_tiles; ++i) run_tile(std::integral_constant<int, -1>{}, i);
   } else {
     // (anchor, dense: 128 query rows and 64-key tiles, so the window of a query block holds an even number of tiles)
     for (int i = 0; i < n_tiles; i += 2) {
       run_tile(std::integral_constant<int, 0>{}, i);
-      if (MODE == kRows && i + 1 == n_tiles) break;
+      if (kAnyRows && i + 1 == n_tiles) break;
       run_tile(std::integral_constant<int, 1>{}, i + 1);
     }
   }
@@ -802,7 +855,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
         reinterpret_cast<uint16_t*>(p.abar_out)[bh * n_pr + R0 / bs + pp] = (uint16_t)(T::pack(am / d, 0.f) & 0xffffu);
       }
     }
-  } else if (MODE == kRows && p.n_chunks > 1) {
+  } else if (kAnyRows && p.n_chunks > 1) {
     // one of several chunks: the unnormalised state goes to the workspace, in fragment order as in anchor mode, and
     // rows_combine_kernel merges the chunks
     const int64_t slot = ((((int64_t)b * p.n_kv_heads + kvh) * p.n_col_blocks + qunit) * p.n_chunks + chunk) * 4 + wave;
@@ -836,7 +889,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
     const int c32_e = lane_e & 31, half_e = lane_e >> 5;
-    const float inv = 1.0f / l_tot;
+    const float inv = MODE == kMasked && l_tot == 0.f ? 0.f : 1.0f / l_tot;  // (a row that sees no key gives 0)
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -855,7 +908,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     for (int it = 0; it < 32 / kRowsPerStore; ++it) {
       const int r = it * kRowsPerStore + lane_e / kLanesPerRow, c = lane_e % kLanesPerRow;
       const u32x4 w = *reinterpret_cast<const u32x4*>(ob + r * kRowBytes + ((c ^ (r & kChunkMask)) << 4));
-      if (MODE == kRows) {
+      if (kAnyRows) {
         const int col = wr0 + r, row = col / group;
         if (col < n_cols) *reinterpret_cast<u32x4*>(op + (col - row * group) * p.o_sh + (int64_t)row * p.o_sn + 8 * c) = w;
       } else {
@@ -880,7 +933,7 @@ static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
     const int per_big_block = a.big_block / 128;  // even for every supported geometry
     a.q_blocks_per_wg = per_big_block % AA_SPARSE_QBLOCKS == 0 ? AA_SPARSE_QBLOCKS : (per_big_block % 2 == 0 ? 2 : 1);
   }
-  const dim3 grid(MODE == kRows ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
+  const dim3 grid(MODE == kRows || MODE == kMasked ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
                                 : (uint32_t)a.batch * a.n_q_heads * (a.n_ctx / (128 * a.q_blocks_per_wg))), block(256);
   if (a.head_dim == 128) {
     if (a.dtype == 0) hipLaunchKernelGGL((flash_kernel<MODE, Bf16, 128>), grid, block, 0, stream, a);
@@ -896,6 +949,7 @@ hipError_t launch_flash(const FlashArgs& a, int mode, hipStream_t stream) {
   if (mode == kAnchor) return launch<kAnchor>(a, stream);
   if (mode == kSparse) return launch<kSparse>(a, stream);
   if (mode == kRows) return launch<kRows>(a, stream);
+  if (mode == kMasked) return launch<kMasked>(a, stream);
   return launch<kDense>(a, stream);
 }
 

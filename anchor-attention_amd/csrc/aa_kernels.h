@@ -24,16 +24,23 @@ struct FlashArgs {
   // KV head come in blocks of 128, the keys in chunks of chunk_tiles 64-key tiles; with more than one chunk the work-groups
   // write M_out, L_out, acc_out [batch, n_kv_heads, n_col_blocks, n_chunks, 128 columns] for rows_combine_kernel
   int n_rows, causal_offset, n_col_blocks, n_chunks, chunk_tiles;
+  // masked mode (rows mode whose causal_offset lets every row see every key, and a boolean mask): the mask as bits
+  // [batch, n_rows, mask_words_per_row] (bit j of word t: key 64 t + j), and what each tile of each column block holds,
+  // tile_flags [batch, n_col_blocks, mask_words_per_row]: 0 nothing visible, 1 some, 2 every key to every row
+  const uint64_t* mask_words; const uint8_t* tile_flags; int mask_words_per_row;
   int dtype;            // AA_DTYPE_BF16 / AA_DTYPE_F16: what the 16-bit elements of q, k, v, out, qbar, abar are
 };
 
-// mode: 0 anchor (stage 1), 1 sparse (stage 3), 2 dense causal, 3 rows
+// mode: 0 anchor (stage 1), 1 sparse (stage 3), 2 dense causal, 3 rows, 4 masked
 hipError_t launch_flash(const FlashArgs& a, int mode, hipStream_t stream);
 
 // rows mode with several chunks: merges the chunks of `a` (the arguments of the launch that wrote them) into a.out
 hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream);
 // rows mode: sets n_col_blocks, n_chunks and chunk_tiles from the sizes
 void plan_rows(FlashArgs& a);
+constexpr int kMaskedTiles = 1024;  // most tiles in a chunk of masked mode (the list of a chunk's visible tiles lives in LDS)
+// masked mode: fills mask_words and tile_flags of `a` from a byte mask [batch, n_rows, n_ctx] with strides (mask_sb, mask_sn, 1)
+hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mask_sb, int64_t mask_sn, hipStream_t stream);
 
 struct PoolArgs {
   const uint16_t* q; int64_t q_sb, q_sh, q_sn;

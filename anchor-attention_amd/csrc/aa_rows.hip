@@ -4,7 +4,8 @@
 // Why rows have a kernel of their own: library attention takes a ragged causal window only as an explicit boolean mask,
 // and then multiplies, masks and soft-maxes the whole score matrix in float32 in memory.  1089 rows over 40001 keys with
 // 32/8 heads of 128 took 18.7 ms that way and take 0.80 ms + 0.03 ms (combine) here, 0.9 PFLOP/s; 777 rows over 777 keys
-// took 403 us and take 21 us.
+// took 403 us and take 21 us.  A left-padded batch of 3 x 2500 tokens with its boolean mask took 7.66 ms and takes 0.26 ms:
+// the mask is packed to bits once, and tiles in which no row of a work-group sees a key are not visited.
 #include "aa_common.h"
 #include "aa_kernels.h"
 
@@ -41,7 +42,8 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
 #pragma unroll 2
   for (int c = 0; c < n_chunks; ++c) {
     const int64_t slot = slot0 + 4 * c;
-    const float w = fast_exp2((p.M[slot * 32 + c32] - m_all) * scale);
+    const float m = p.M[slot * 32 + c32];
+    const float w = m == -INFINITY ? 0.f : fast_exp2((m - m_all) * scale);  // (a chunk without a key of this row's)
     l_all += w * p.L[slot * 32 + c32];
     const float* af = p.acc_frag + (slot * kDB + db) * (4 * 256) + lane * 4;
 #pragma unroll
@@ -51,7 +53,7 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
       for (int e = 0; e < 4; ++e) acc[rg][e] += w * t[e];
     }
   }
-  const float inv = 1.f / l_all;
+  const float inv = l_all == 0.f ? 0.f : 1.f / l_all;  // (masked mode: a row that sees no key gives 0)
   uint32_t w[4][2];
 #pragma unroll
   for (int rg = 0; rg < 4; ++rg) {
@@ -86,6 +88,58 @@ hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Masked mode: packs the byte mask of one column block's rows, 64 keys to a word, and notes for each 64-key tile whether any
+// and whether every one of the rows sees it.  A work-group takes 4096 keys of the block's rows, a wave 1024 of them, a lane 16.
+// Bound by reading the mask once; rows that two column blocks share are packed twice, to the same words.
+__global__ void __launch_bounds__(256) mask_pack_kernel(const FlashArgs p, const uint8_t* mask, const int64_t mask_sb, const int64_t mask_sn) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int block = blockIdx.y, b = blockIdx.z;
+  const int group = p.n_q_heads / p.n_kv_heads, n_cols = p.n_rows * group;
+  const int row0 = 128 * block / group, row1 = (min(128 * block + 128, n_cols) - 1) / group;  // first and last row of the block
+  const int key0 = (blockIdx.x * 4 + wave) * 1024 + 16 * lane;
+  const int tile = key0 / 64;
+  if (__all(tile >= p.mask_words_per_row)) return;
+  const int keys = max(0, min(16, p.n_ctx - key0));  // of this lane's 16
+  const uint8_t* src = mask + b * mask_sb + key0;
+  uint64_t* words = const_cast<uint64_t*>(p.mask_words) + (int64_t)b * p.n_rows * p.mask_words_per_row;
+  uint32_t any = 0u, all = 0xffffu;
+#pragma unroll 4
+  for (int row = row0; row <= row1; ++row) {
+    uint32_t bits = 0u;
+    const uint8_t* at = src + (int64_t)row * mask_sn;
+    if (keys == 16) {
+      uint32_t x[4];
+      __builtin_memcpy(x, at, 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // bytes 0/1 -> four bits: the products meet at bits 24..27 without carries
+        const uint32_t ones = (x[i] | (x[i] >> 4)) | ((x[i] | (x[i] >> 4)) >> 2);  // any bit of a byte counts as true
+        bits |= ((((ones | (ones >> 1)) & 0x01010101u) * 0x01020408u) >> 24 & 0xfu) << (4 * i);
+      }
+    } else {
+      for (int i = 0; i < keys; ++i) bits |= at[i] ? 1u << i : 0u;
+    }
+    any |= bits;
+    all &= bits;
+    // four lanes make a word
+    const uint32_t pair = bits | (__shfl_down(bits, 1, 64) << 16);
+    const uint32_t high = __shfl_down(pair, 2, 64);
+    if ((lane & 3) == 0 && tile < p.mask_words_per_row) words[(int64_t)row * p.mask_words_per_row + tile] = (uint64_t)pair | (uint64_t)high << 32;
+  }
+  any |= __shfl_xor(any, 1, 64);
+  any |= __shfl_xor(any, 2, 64);
+  all &= __shfl_xor(all, 1, 64);
+  all &= __shfl_xor(all, 2, 64);
+  if ((lane & 3) == 0 && tile < p.mask_words_per_row)
+    const_cast<uint8_t*>(p.tile_flags)[((int64_t)b * p.n_col_blocks + block) * p.mask_words_per_row + tile] = all == 0xffffu ? 2 : any ? 1 : 0;
+}
+
+hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mask_sb, int64_t mask_sn, hipStream_t stream) {
+  const dim3 grid((a.n_ctx + 4095) / 4096, a.n_col_blocks, a.batch);
+  hipLaunchKernelGGL(mask_pack_kernel, grid, dim3(256), 0, stream, a, mask, mask_sb, mask_sn);
+  return hipGetLastError();
+}
+
 // How the keys of a rows-mode problem are cut into chunks.  The chip holds 512 work-groups (two per CU).  A tile takes a
 // work-group about 1.9 us with a neighbour on its CU and 1.1 us alone; several chunks cost a write and a read of the state
 // (64 KB per column block and chunk at head dimension 128) and one more launch.  Every number of chunks up to 64 is priced with that
@@ -101,7 +155,8 @@ void plan_rows(FlashArgs& a) {
   double best = 1e30;
   a.n_chunks = 1;
   a.chunk_tiles = max_tiles;
-  for (int n = 1; n <= 64 && n <= max_tiles; ++n) {
+  const int n_min = a.mask_words_per_row > 0 ? (max_tiles + kMaskedTiles - 1) / kMaskedTiles : 1;
+  for (int n = n_min; n <= 64 && n <= max_tiles; ++n) {
     const int len = (max_tiles + n - 1) / n, chunks = (max_tiles + len - 1) / len;
     int64_t wgs = 0;
     for (int i = 0; i < a.n_col_blocks; ++i)

@@ -186,12 +186,17 @@ int aa_dense_causal_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
  * modules/llama/anchor_attention.py:101-109): query row i of n_rows sees keys 0 .. causal_offset + i of n_keys
  * (causal_offset >= 0); neither count has to be a multiple of anything.  q and out have n_rows rows, k and v n_keys.
  * out = round16(softmax(q k^T * sm_scale) v), the scores scaled in float32; sm_scale must be positive.
+ * mask, if not NULL, takes the place of the causal rule: byte [b, i, j] of [batch, n_rows, n_keys] with element strides
+ * (mask_sb, mask_sn, 1), which may be 0, says whether row i sees key j (0: no), for every head; a row that sees no key
+ * gives 0.  (Padded batches and sliding windows; the reference unpads with flash_attn_varlen_func.)
  * workspace: aa_dense_rows_workspace_bytes() bytes of device scratch, which may be none (contents undefined afterwards). */
-size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset);
+size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
+                                     int masked);
 int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                       const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                       const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                       void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                      const uint8_t* mask, int64_t mask_sb, int64_t mask_sn,
                       void* workspace, size_t workspace_bytes,
                       int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
                       float sm_scale, int dtype, void* stream);

@@ -58,3 +58,31 @@ def test_dense_rows_against_float64(batch, hq, hkv, n_rows, offset, d, dtype):
     _check(out, _reference(q, k, v, d ** -0.5, keep), v, dtype)
     again = dense_rows_attention(q.contiguous(), k, v, offset, sm_scale=d ** -0.5)
     assert torch.equal(again, out)
+
+
+def _mask(kind, batch, n_rows, n_keys):
+    rows, keys = torch.arange(n_rows, device="cuda") + n_keys - n_rows, torch.arange(n_keys, device="cuda")
+    causal = keys[None, :] <= rows[:, None]
+    if kind == "padded":  # left-padded prompts: whole tiles nobody sees, rows without any key
+        pads = torch.tensor([(37 * b) % n_keys + 70 * b for b in range(batch)], device="cuda")
+        return (causal[None] & (keys[None, None, :] >= pads[:, None, None]))[:, None]
+    if kind == "window":  # one mask for the whole batch
+        return (causal & (keys[None, :] > rows[:, None] - 100))[None, None]
+    g = torch.Generator(device="cuda").manual_seed(n_keys)
+    return torch.rand(batch, 1, n_rows, n_keys, generator=g, device="cuda") < 0.4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,hq,hkv,n_rows,n_keys,d,dtype,kind", [
+    (3, 8, 2, 333, 333, 128, torch.bfloat16, "padded"),
+    (2, 7, 1, 129, 1025, 64, torch.float16, "random"),   # a group of seven; one key past a tile
+    (2, 4, 4, 65, 4161, 128, torch.bfloat16, "padded"),  # more keys than one work-group of the mask kernel packs; chunks
+    (2, 4, 2, 300, 300, 64, torch.bfloat16, "window"),
+    (1, 2, 1, 5, 67000, 128, torch.bfloat16, "random"),  # more tiles than one chunk may list
+])
+def test_masked_rows_against_float64(batch, hq, hkv, n_rows, n_keys, d, dtype, kind):
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
+    q, k, v = _qkv(batch, hq, hkv, n_rows, n_keys, d, dtype, n_rows + n_keys)
+    mask = _mask(kind, batch, n_rows, n_keys)
+    out = dense_rows_attention(q, k, v, mask=mask)
+    _check(out, _reference(q, k, v, d ** -0.5, mask[:, 0].expand(batch, -1, -1)), v, dtype)
