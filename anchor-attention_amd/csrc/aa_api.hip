@@ -481,7 +481,12 @@ static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_hea
   a.causal_offset = masked ? n_keys : causal_offset;
   a.mask_words_per_row = masked ? (n_keys + 63) / 64 : 0;
   a.big_block = n_keys; a.block_size = 128;  // (unused in this mode; not zero)
-  plan_rows(a);
+  if (decode_takes(n_rows, n_q_heads / n_kv_heads, masked)) {
+    a.mask_words_per_row = 0;  // (the decode kernel reads the byte mask itself)
+    plan_decode(a);
+  } else {
+    plan_rows(a);
+  }
   return AA_OK;
 }
 
@@ -490,9 +495,10 @@ struct RowsScratch {
   int64_t state_columns;
   size_t words, flags, total;
 };
-static RowsScratch carve_rows(const FlashArgs& a) {
+static RowsScratch carve_rows(const FlashArgs& a, bool decode) {
   RowsScratch r;
-  r.state_columns = a.n_chunks > 1 ? (int64_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks * 128 : 0;
+  const int columns = decode ? a.n_rows * (a.n_q_heads / a.n_kv_heads) : 128 * a.n_col_blocks;
+  r.state_columns = a.n_chunks > 1 ? (int64_t)a.batch * a.n_kv_heads * a.n_chunks * columns : 0;
   r.words = align256((size_t)r.state_columns * (a.head_dim + 2) * 4);  // accumulators, maxima, sums
   r.flags = r.words + align256((size_t)a.batch * a.n_rows * a.mask_words_per_row * 8);
   r.total = r.flags + (size_t)a.batch * a.n_col_blocks * a.mask_words_per_row;
@@ -504,7 +510,7 @@ size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, i
   FlashArgs a = {};
   if (plan_dense_rows("aa_dense_rows_workspace_bytes", a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, masked != 0))
     return 0;
-  return carve_rows(a).total;
+  return carve_rows(a, decode_takes(n_rows, n_q_heads / n_kv_heads, masked != 0)).total;
 }
 
 int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
@@ -528,7 +534,8 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
     set_error("%s: sm_scale %g must be positive", who, (double)sm_scale);
     return AA_EUNSUPPORTED;
   }
-  const RowsScratch r = carve_rows(a);
+  const bool decode = decode_takes(n_rows, n_q_heads / n_kv_heads, mask != nullptr);
+  const RowsScratch r = carve_rows(a, decode);
   if (r.total > 0) {
     if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
     if (workspace_bytes < r.total) {
@@ -544,6 +551,10 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   a.acc_out = (float*)ws; a.M_out = a.acc_out + r.state_columns * head_dim; a.L_out = a.M_out + r.state_columns;
   a.acc_frag = a.acc_out; a.M = a.M_out; a.L = a.L_out;
   a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
+  if (decode) {
+    a.mask_bytes = mask; a.mask_sb = mask_sb;
+    return check_launch(launch_decode(a, (hipStream_t)stream), who);
+  }
   if (mask != nullptr) {
     a.mask_words = (const uint64_t*)(ws + r.words);
     a.tile_flags = (const uint8_t*)(ws + r.flags);

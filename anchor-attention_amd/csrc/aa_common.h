@@ -81,6 +81,17 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // the barrier stay in flight across it.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+typedef __attribute__((address_space(3))) char lds_char;
+__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(lds_char*)p; }
+
+// 64 lanes x 16 bytes, global -> LDS without passing through registers: lane L's bytes land at
+// lds_dst + 16*L (lds_dst is wave-uniform and travels in M0).  Completion is tracked by vmcnt.
+__device__ __forceinline__ void load16_to_lds(const char* base, const uint32_t byte_off, const uint32_t lds_dst) {
+  // the LDS base is bound to M0 by the constraint, so the compiler knows that M0 is written here; the nop covers the
+  // wait state an LDS-DMA instruction needs after a scalar write of M0 (the compiler does not look inside the asm)
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(lds_dst), "v"(byte_off), "s"(base) : "memory");
+}
+
 // value held by the lane 32 positions away (the two halves of a wave share MFMA columns)
 __device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32, 64); }
 

@@ -28,6 +28,8 @@ struct FlashArgs {
   // [batch, n_rows, mask_words_per_row] (bit j of word t: key 64 t + j), and what each tile of each column block holds,
   // tile_flags [batch, n_col_blocks, mask_words_per_row]: 0 nothing visible, 1 some, 2 every key to every row
   const uint64_t* mask_words; const uint8_t* tile_flags; int mask_words_per_row;
+  // decode kernel with a mask (one query row): the byte mask itself
+  const uint8_t* mask_bytes; int64_t mask_sb;
   int dtype;            // AA_DTYPE_BF16 / AA_DTYPE_F16: what the 16-bit elements of q, k, v, out, qbar, abar are
 };
 
@@ -41,6 +43,13 @@ void plan_rows(FlashArgs& a);
 constexpr int kMaskedTiles = 1024;  // most tiles in a chunk of masked mode (the list of a chunk's visible tiles lives in LDS)
 // masked mode: fills mask_words and tile_flags of `a` from a byte mask [batch, n_rows, n_ctx] with strides (mask_sb, mask_sn, 1)
 hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mask_sb, int64_t mask_sn, hipStream_t stream);
+
+// A few query rows over many keys (decode steps): the arguments of rows mode, one column block, chunk_tiles counted in 32-key
+// tiles, and the chunks' state as M_out, L_out [batch, n_kv_heads, n_chunks, columns] and acc_out [..., columns, head_dim].
+constexpr int kDecMaxChunks = 256;
+bool decode_takes(int n_rows, int group, bool masked);
+void plan_decode(FlashArgs& a);
+hipError_t launch_decode(const FlashArgs& a, hipStream_t stream);
 
 struct PoolArgs {
   const uint16_t* q; int64_t q_sb, q_sh, q_sn;

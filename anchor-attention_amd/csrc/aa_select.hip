@@ -142,13 +142,7 @@ constexpr int kSelRowBytes = 256; // one pooled row in LDS
 #define AA_SEL_WGS 2              // work-groups per CU the kernel is compiled for
 #endif
 
-typedef __attribute__((address_space(3))) char sel_lds_char;
-__device__ __forceinline__ uint32_t sel_lds_addr(const void* p) { return (uint32_t)(uintptr_t)(sel_lds_char*)p; }
-// 64 lanes x 16 bytes (or x 4 bytes) global -> LDS; lane L's bytes land at lds_dst + 16*L (4*L).  lds_dst is wave-uniform
-// and travels in M0; the nop covers the wait state an LDS-DMA instruction needs after a scalar write of M0.
-__device__ __forceinline__ void sel_load16_to_lds(const char* base, const uint32_t byte_off, const uint32_t lds_dst) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(lds_dst), "v"(byte_off), "s"(base) : "memory");
-}
+// load16_to_lds for 4 bytes a lane
 __device__ __forceinline__ void sel_load4_to_lds(const char* base, const uint32_t byte_off, const uint32_t lds_dst) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dword %1, %2" : : "{m0}"(lds_dst), "v"(byte_off), "s"(base) : "memory");
 }
@@ -225,8 +219,8 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
   const char* qbar_base = reinterpret_cast<const char*>(p.qbar);
   const char* thr_base = reinterpret_cast<const char*>(p.thr);
   const int64_t head0 = ((int64_t)b * p.n_q_heads + kvh * group) * n_pr;  // first pooled row of the group's first head
-  const uint32_t a_lds0 = sel_lds_addr(a_lds[0]) + wave * kRowsPerWave * kSelRowBytes;
-  const uint32_t thr_lds0 = sel_lds_addr(thr_lds[0]);
+  const uint32_t a_lds0 = lds_addr(a_lds[0]) + wave * kRowsPerWave * kSelRowBytes;
+  const uint32_t thr_lds0 = lds_addr(thr_lds[0]);
   auto item_first_row = [&](const int item_unclamped) {  // pooled-row number, within the whole qbar array, of an item's first row
     const int item = min(item_unclamped, n_items - 1);   // past the end: repeat the last item
     const int q = item_bb_off(item);
@@ -241,7 +235,7 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
       const int r = 4 * j + (lane >> 4);  // row inside the wave's share
       const uint32_t prow = item_row0[r / STEP] + (uint32_t)(r % STEP);
       const uint32_t chunk = (uint32_t)(((lane & 15) ^ (r & 15)) & (D / 8 - 1));
-      sel_load16_to_lds(qbar_base, prow * (uint32_t)(2 * D) + chunk * 16u, a_lds0 + buf * (ROWS * kSelRowBytes) + 4 * j * kSelRowBytes);
+      load16_to_lds(qbar_base, prow * (uint32_t)(2 * D) + chunk * 16u, a_lds0 + buf * (ROWS * kSelRowBytes) + 4 * j * kSelRowBytes);
     }
     if (wave < ROWS / 64) {  // thresholds of block rows 64*wave + lane
       const int r = 64 * wave + lane;
@@ -255,7 +249,7 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
   // A operand of MFMA step ks: row c32 of the group, chunk 2*ks + half, swizzled with the row's low four bits
   uint32_t a_rd[kKS];
 #pragma unroll
-  for (int ks = 0; ks < kKS; ++ks) a_rd[ks] = sel_lds_addr(a_lds[0]) + c32 * kSelRowBytes + (((2 * ks + half) ^ (c32 & 15)) << 4);
+  for (int ks = 0; ks < kKS; ++ks) a_rd[ks] = lds_addr(a_lds[0]) + c32 * kSelRowBytes + (((2 * ks + half) ^ (c32 & 15)) << 4);
   typedef __attribute__((address_space(3))) vec8 lds_vec8_t;
   typedef __attribute__((address_space(3))) floatx4 lds_floatx4_t;
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));

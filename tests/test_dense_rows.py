@@ -44,6 +44,14 @@ def _qkv(batch, hq, hkv, n_rows, n_keys, d, dtype, seed):
     (3, 8, 8, 130, 63, 64, torch.float16),        # no groups, two column blocks, chunk and tile edges
     (1, 7, 1, 33, 0, 128, torch.bfloat16),        # fewer keys than a tile
     (1, 2, 1, 2047, 2048, 64, torch.bfloat16),    # the longest tail
+    # at most 32 (row, head) columns: the decode kernel
+    (1, 32, 8, 1, 33000, 128, torch.bfloat16),    # a decode step: a chunk per CU, the last tile ragged
+    (3, 14, 2, 1, 0, 64, torch.float16),          # one key
+    (2, 8, 1, 4, 61, 128, torch.float16),         # all 32 columns, rows that end in the same tile
+    (5, 4, 4, 3, 1021, 64, torch.bfloat16),       # no groups
+    (40, 16, 8, 1, 300, 128, torch.bfloat16),     # more units than CUs: one chunk, written without a merge
+    (1, 4, 4, 9, 500, 64, torch.bfloat16),        # nine columns
+    (1, 33, 1, 1, 700, 64, torch.bfloat16),       # one column too many for it
 ])
 def test_dense_rows_against_float64(batch, hq, hkv, n_rows, offset, d, dtype):
     from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention, dense_rows_supported
@@ -79,6 +87,9 @@ def _mask(kind, batch, n_rows, n_keys):
     (2, 4, 4, 65, 4161, 128, torch.bfloat16, "padded"),  # more keys than one work-group of the mask kernel packs; chunks
     (2, 4, 2, 300, 300, 64, torch.bfloat16, "window"),
     (1, 2, 1, 5, 67000, 128, torch.bfloat16, "random"),  # more tiles than one chunk may list
+    (4, 28, 4, 1, 2501, 128, torch.bfloat16, "padded"),  # a padded batch's decode step: tiles that are skipped
+    (1, 2, 2, 1, 9000, 64, torch.float16, "random"),
+    (40, 16, 8, 1, 8193, 64, torch.bfloat16, "window"),  # a second chunk of one key, since the first may hold no more
 ])
 def test_masked_rows_against_float64(batch, hq, hkv, n_rows, n_keys, d, dtype, kind):
     from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
