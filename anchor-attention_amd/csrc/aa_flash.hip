@@ -32,11 +32,12 @@
 // Work-group = 4 waves = 128 query rows; keys are consumed 64 at a time through a
 // double-buffered LDS tile that the memory system fills directly (global_load_lds_dwordx4: no staging
 // registers, no LDS store instructions).  Such a load writes lane L's 16 bytes at M0 + 16*L, so LDS rows
-// are unpadded 256 bytes; bank conflicts are avoided by XOR-swizzling the 16-byte chunks of a row, which
+// are unpadded; bank conflicts are avoided by XOR-swizzling the 16-byte chunks of a row, which
 // costs nothing on the load side (a lane simply fetches the chunk that belongs in its slot):
-//   K row r, chunk c  ->  slot c ^ (r & 15)          (row-per-lane 16-byte reads)
-//   V row r, chunk c  ->  slot c ^ ((r & 7) << 1)    (transposing 8-byte reads)
-// Both choices measure conflict-free for their read pattern (and each is 2-way conflicted for the other's).
+//                             head dimension 128                64
+//   K row r, chunk c  ->  slot c ^ (r & 15)          c ^ ((r & 7) ^ (r >> 3 & 1))   (row-per-lane 16-byte reads)
+//   V row r, chunk c  ->  slot c ^ ((r & 7) << 1)    c ^ ((r & 3) << 1)             (transposing 8-byte reads)
+// These choices measure conflict-free for their read pattern (and each is 2-way conflicted for the other's).
 #include <type_traits>
 
 #include "aa_common.h"
@@ -45,8 +46,7 @@
 namespace aa {
 
 constexpr int kBN = 64;        // keys per LDS tile
-constexpr int kRowBytes = 256;   // pitch of a K/V row in LDS (128 16-bit elements, unpadded, chunks swizzled; head dimension 64 fills half)
-constexpr int kTileBytes = kBN * kRowBytes;
+constexpr int kLoadBytes = 4096; // what one LDS-DMA instruction of the work-group brings (256 threads x 16 bytes)
 constexpr int kDist = 4;         // MFMA operands are fetched from LDS this many MFMAs ahead of their use
 constexpr int kIdxWin = 1024;    // selected-key indices held in LDS at a time (16 tiles)
 constexpr int32_t kMixedTile = 1 << 30;  // (masked) flag of a listed tile of which some pairs are masked
@@ -75,11 +75,17 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
-template <int MODE>
+// Swizzle of the 16-byte chunks of LDS row r (see the top of the file); both have a period of 32 rows or less.
+template <int D>
+__device__ __forceinline__ int k_swizzle(const int r) { return D == 128 ? r & 15 : (r & 7) ^ ((r >> 3) & 1); }
+template <int D>
+__device__ __forceinline__ int v_swizzle(const int r) { return D == 128 ? (r & 7) << 1 : (r & 3) << 1; }
+
+template <int MODE, int D>
 struct FlashSmem {
   struct {
-    char k[2][kTileBytes];
-    char v[2][kTileBytes];
+    char k[2][kBN * 2 * D];
+    char v[2][kBN * 2 * D];
   } t;  // (the epilogue stages the output in the tile space)
   // sparse mode: window of the big block's index list; masked mode: the chunk's tiles that hold a visible key, and their number
   int32_t idx[MODE == kSparse ? kIdxWin : MODE == kMasked ? kMaskedTiles + 4 : 4];
@@ -107,53 +113,59 @@ __device__ __forceinline__ typename T::vec8 scale_q8(const u32x4 raw, const floa
   return *reinterpret_cast<const typename T::vec8*>(&packed);
 }
 
-// One K/V tile: wave w fills LDS rows 16*j + 4*w .. +3 (j = 0..3), i.e. thread t brings the chunk that belongs in
-// slot (t & 15) of row (t >> 4) + 16*j; tile_fetch_one issues one of the tile's eight loads.  `kb`/`vb` are the
+// One K/V tile: a row has D/8 slots of 16 bytes and one load instruction of the work-group fills 2048/D rows, thread t slot
+// t % (D/8) of row t / (D/8) + (2048/D)*j (j = 0..3 at head dimension 128, 0..1 at 64); tile_fetch_one issues one of the
+// tile's eight (four) loads.  `kb`/`vb` are the
 // wave-uniform head bases, `k_col`/`v_col` the byte offset of this thread's (swizzled) chunk inside a row,
-// `lds_k`/`lds_v` the LDS address of row 4*w of the destination tile.  Gathered tiles take their row numbers from
+// `lds_k`/`lds_v` the LDS address of wave w's first slot in the destination tile.  Gathered tiles take their row numbers from
 // the LDS window of the index list (a dependent global load per tile would put a full memory latency on the
-// critical path of every tile); the caller reads a tile's four row numbers per lane (`gather_keys`, see tile_gather_keys)
+// critical path of every tile); the caller reads a tile's row numbers (`gather_keys`, see tile_gather_keys)
 // before it issues the tile's first load: a wave's LDS reads are served in order with its global -> LDS loads, so a row
 // number read after a load would arrive only when that load's data has.
 // the row numbers lane `tid` needs for the gathered tile at list position key0 (positions past the count hold 0: row 0,
 // masked later)
-__device__ __forceinline__ void tile_gather_keys(uint32_t (&keys)[4], const int32_t* idx_win, const int key0, const int tid) {
+template <int D>
+__device__ __forceinline__ void tile_gather_keys(uint32_t (&keys)[D / 32], const int32_t* idx_win, const int key0, const int tid) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) keys[j] = (uint32_t)idx_win[(key0 + (tid >> 4) + 16 * j) & (kIdxWin - 1)];
+  for (int j = 0; j < D / 32; ++j) keys[j] = (uint32_t)idx_win[(key0 + tid / (D / 8) + (2048 / D) * j) & (kIdxWin - 1)];
 }
 
-template <int MODE>
+template <int MODE, int D>
 __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, const char* vb, const uint32_t k_row_bytes,
                                                const uint32_t v_row_bytes, const uint32_t k_col, const uint32_t v_col, const int key0,
                                                const uint32_t* gather_keys, const uint32_t lds_k, const uint32_t lds_v,
                                                const uint32_t k_voff, const uint32_t v_voff) {
-  const int j = n >> 1;  // load n: K (even n) or V (odd n) rows 16*j + ...
+  constexpr int kLoadRows = 2048 / D;  // rows that one load instruction fills
+  const int j = n >> 1;  // load n: K (even n) or V (odd n) rows kLoadRows*j + ...
   if (MODE == kSparse) {
-    const uint32_t key = gather_keys[j];  // this lane's row of the tile's j-th block of 16 rows
-    if ((n & 1) == 0) load16_to_lds(kb, __umul24(key, k_row_bytes) + k_col, lds_k + 16 * j * kRowBytes);
-    else load16_to_lds(vb, __umul24(key, v_row_bytes) + v_col, lds_v + 16 * j * kRowBytes);
+    const uint32_t key = gather_keys[j];  // this lane's row of the tile's j-th block of kLoadRows rows
+    if ((n & 1) == 0) load16_to_lds(kb, __umul24(key, k_row_bytes) + k_col, lds_k + j * kLoadBytes);
+    else load16_to_lds(vb, __umul24(key, v_row_bytes) + v_col, lds_v + j * kLoadBytes);
   } else if (MODE == kRows || MODE == kMasked) {
-    // consecutive keys up to a key count that need not fill the last tile: the caller's per-lane offsets (gather_keys: four
-    // for K, four for V, from the tile's first row) are loop-invariant except that they are clamped for that tile
-    if ((n & 1) == 0) load16_to_lds(kb + (uint64_t)(uint32_t)key0 * k_row_bytes, gather_keys[j], lds_k + 16 * j * kRowBytes);
-    else load16_to_lds(vb + (uint64_t)(uint32_t)key0 * v_row_bytes, gather_keys[4 + j], lds_v + 16 * j * kRowBytes);
+    // consecutive keys up to a key count that need not fill the last tile: the caller's per-lane offsets (gather_keys: D/32
+    // for K, D/32 for V, from the tile's first row) are loop-invariant except that they are clamped for that tile
+    if ((n & 1) == 0) load16_to_lds(kb + (uint64_t)(uint32_t)key0 * k_row_bytes, gather_keys[j], lds_k + j * kLoadBytes);
+    else load16_to_lds(vb + (uint64_t)(uint32_t)key0 * v_row_bytes, gather_keys[D / 32 + j], lds_v + j * kLoadBytes);
   } else {
-    // consecutive keys: the first row of the tile's j-th block of 16 rows goes into the (scalar) base address, the
+    // consecutive keys: the first row of the tile's j-th block of kLoadRows rows goes into the (scalar) base address, the
     // thread's row inside the block and its chunk are one loop-invariant vector offset - no vector arithmetic per tile
-    if ((n & 1) == 0) load16_to_lds(kb + (uint64_t)(uint32_t)(key0 + 16 * j) * k_row_bytes, k_voff, lds_k + 16 * j * kRowBytes);
-    else load16_to_lds(vb + (uint64_t)(uint32_t)(key0 + 16 * j) * v_row_bytes, v_voff, lds_v + 16 * j * kRowBytes);
+    if ((n & 1) == 0) load16_to_lds(kb + (uint64_t)(uint32_t)(key0 + kLoadRows * j) * k_row_bytes, k_voff, lds_k + j * kLoadBytes);
+    else load16_to_lds(vb + (uint64_t)(uint32_t)(key0 + kLoadRows * j) * v_row_bytes, v_voff, lds_v + j * kLoadBytes);
   }
 }
 
-// D is the head dimension, 128 or 64.  With 64 the LDS tiles keep their 256-byte row pitch and their swizzles - a row
-// then fills eight of its sixteen 16-byte slots, the lanes of a tile load that would bring the other eight fetch a
-// duplicate that is never read - so every LDS address below is the same for both sizes, and only the number of MFMA steps
-// over the head dimension (kKS per 32 keys of Q.K^T) and of 32-column output blocks (kDB) changes.
+// D is the head dimension, 128 or 64: it sets the LDS row pitch, the number of tile loads, of MFMA steps over the head
+// dimension (kKS per 32 keys of Q.K^T) and of 32-column output blocks (kDB).
+//
+// Work-groups per CU: with 128 two (248 registers, 64 KB of LDS).  With 64 a tile has half the MFMAs but the same soft-max,
+// so the vector ALU bounds it, and a third wave per SIMD (168 registers; 2 and 8 of them spill around the tile loop in anchor
+// and sparse mode) keeps that busy: 69 % of the cycles, matrix pipe 49 %.  16384 tokens, 32/8 heads of 64: stage 1 470 -> 413 us
+// against two work-groups per CU and 256-byte LDS rows of which half was filled.
 template <int MODE, typename T, int D>
-__global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
+__global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const FlashArgs p) {
   typedef typename T::vec8 vec8;
   typedef __attribute__((address_space(3))) vec8 lds_vec8;
-  __shared__ __attribute__((aligned(16))) FlashSmem<MODE> sm;
+  __shared__ __attribute__((aligned(16))) FlashSmem<MODE, D> sm;
   constexpr int BM = 128;
   constexpr bool kAnyRows = MODE == kRows || MODE == kMasked;
   static_assert(D == 128 || D == 64, "head dimension");
@@ -161,6 +173,11 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   constexpr int kDB = D / 32;       // 32-column blocks of the head dimension: accumulators of O^T
   constexpr int kNS = 2 * kKS;      // S^T slots of a 64-key tile
   constexpr int kNV = 4 * kDB;      // O^T slots of a 64-key tile (two 16-key steps per 32-key block)
+  constexpr int kRowBytes = 2 * D;  // pitch of a K/V row in LDS (unpadded, chunks swizzled)
+  constexpr int kTileBytes = kBN * kRowBytes;
+  constexpr int kSlots = D / 8;              // 16-byte slots of a row
+  constexpr int kLoadRows = 256 / kSlots;    // rows that one load instruction of the work-group fills
+  constexpr int kHalfLoads = kBN / kLoadRows;  // load instructions of a K (or V) tile
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -368,42 +385,41 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   }
 
   // this thread's chunk of a row (swizzled: see the top of the file) and the wave's slice of the LDS tiles
-  // (head dimension 64: a row has eight chunks; the lanes whose slot belongs to none of them fetch a duplicate)
-  const uint32_t k_col = (uint32_t)(((tid & 15) ^ ((tid >> 4) & 15)) & (D / 8 - 1)) * 16u;
-  const uint32_t v_col = (uint32_t)(((tid & 15) ^ (((tid >> 4) & 7) << 1)) & (D / 8 - 1)) * 16u;
-  const uint32_t lds_k0 = lds_addr(sm.t.k[0]) + wave * 4 * kRowBytes, lds_v0 = lds_addr(sm.t.v[0]) + wave * 4 * kRowBytes;
-  // byte offset of this thread's chunk of row (tid >> 4) of a block of 16 tile rows from the block's first row
-  const uint32_t k_voff = (tid >> 4) * k_row_bytes + k_col, v_voff = (tid >> 4) * v_row_bytes + v_col;
+  const uint32_t k_col = (uint32_t)((tid % kSlots) ^ k_swizzle<D>(tid / kSlots)) * 16u;
+  const uint32_t v_col = (uint32_t)((tid % kSlots) ^ v_swizzle<D>(tid / kSlots)) * 16u;
+  const uint32_t lds_k0 = lds_addr(sm.t.k[0]) + wave * 1024, lds_v0 = lds_addr(sm.t.v[0]) + wave * 1024;
+  // byte offset of this thread's chunk of row tid / kSlots of a block of kLoadRows tile rows from the block's first row
+  const uint32_t k_voff = (tid / kSlots) * k_row_bytes + k_col, v_voff = (tid / kSlots) * v_row_bytes + v_col;
   // (anchor mode with pooling) the work-group's raw query rows, fetched like a tile by the last tile's load slots
   const char* qblock = reinterpret_cast<const char*>(qp + (int64_t)R0 * p.q_sn);
   const uint32_t q_row_bytes = (uint32_t)p.q_sn * 2u;
-  const uint32_t q_voff = (uint32_t)(tid >> 4) * q_row_bytes + (uint32_t)((tid & 15) & (D / 8 - 1)) * 16u;
-  // (rows) per-lane offsets of a tile's four blocks of 16 K rows and 16 V rows from the tile's first row, of which
+  const uint32_t q_voff = (uint32_t)(tid / kSlots) * q_row_bytes + (uint32_t)(tid % kSlots) * 16u;
+  // (rows) per-lane offsets of a tile's blocks of kLoadRows K rows and V rows from the tile's first row, of which
   // `rows_left` lie inside the tensor: lanes past the last key read it again and are masked
-  uint32_t row_offs[8];
+  uint32_t row_offs[2 * kHalfLoads];
   // (from an opaque copy of the thread number: the pieces would otherwise occupy registers throughout the tile loop for
   // the one time that the offsets are clamped)
   auto set_row_offs = [&](const int rows_left) __attribute__((always_inline)) {
     int t = tid;
     asm volatile("" : "+v"(t));
-    const uint32_t kc = (uint32_t)(((t & 15) ^ ((t >> 4) & 15)) & (D / 8 - 1)) * 16u;
-    const uint32_t vc = (uint32_t)(((t & 15) ^ (((t >> 4) & 7) << 1)) & (D / 8 - 1)) * 16u;
+    const uint32_t kc = (uint32_t)((t % kSlots) ^ k_swizzle<D>(t / kSlots)) * 16u;
+    const uint32_t vc = (uint32_t)((t % kSlots) ^ v_swizzle<D>(t / kSlots)) * 16u;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t r = (uint32_t)min((t >> 4) + 16 * j, rows_left - 1);
+    for (int j = 0; j < kHalfLoads; ++j) {
+      const uint32_t r = (uint32_t)min(t / kSlots + kLoadRows * j, rows_left - 1);
       row_offs[j] = __umul24(r, k_row_bytes) + kc;
-      row_offs[4 + j] = __umul24(r, v_row_bytes) + vc;
+      row_offs[kHalfLoads + j] = __umul24(r, v_row_bytes) + vc;
     }
   };
   if (kAnyRows) set_row_offs(p.n_ctx - AA_TILE_KEY0(0));
   request_mask_word();
   if (n_tiles > 0 && !chained) {
     const uint32_t first = MODE == kSparse ? (uint32_t)cur * kTileBytes : 0u;
-    uint32_t keys0[4] = {0u, 0u, 0u, 0u};
-    if (MODE == kSparse) tile_gather_keys(keys0, sm.idx, 0, tid);
+    uint32_t keys0[kHalfLoads] = {};
+    if (MODE == kSparse) tile_gather_keys<D>(keys0, sm.idx, 0, tid);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      tile_fetch_one<MODE>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(0), kAnyRows ? row_offs : keys0,
+    for (int j = 0; j < 2 * kHalfLoads; ++j)
+      tile_fetch_one<MODE, D>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(0), kAnyRows ? row_offs : keys0,
                            lds_k0 + first, lds_v0 + first, k_voff, v_voff);
   }
   // the accumulator state: the youngest loads in flight, first needed by the first P.V product
@@ -459,7 +475,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     __syncthreads();
   }
 
-  // per-lane LDS byte offsets.  K: row c32 (+32*kb), chunk 2*ks + half, swizzled with the row's low four bits.
+  // per-lane LDS byte offsets.  K: row c32 (+32*kb), chunk 2*ks + half, swizzled.
   // (absolute LDS addresses into the current buffer; the 32-key half and the row steps are immediate offsets)
   const uint32_t first_buf = MODE == kSparse ? (uint32_t)cur * kTileBytes : 0u;  // (sparse) where this block's first tile lies
   // (sparse: formed per block from an opaque copy of the lane number - hoisted out of the loop over the work-group's
@@ -469,16 +485,16 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
   const int c32_t = lane_t & 31, half_t = lane_t >> 5;
   uint32_t k_rd[kKS];
 #pragma unroll
-  for (int ks = 0; ks < kKS; ++ks) k_rd[ks] = lds_addr(sm.t.k[0]) + first_buf + c32_t * kRowBytes + (((2 * ks + half_t) ^ (c32_t & 15)) << 4);
+  for (int ks = 0; ks < kKS; ++ks) k_rd[ks] = lds_addr(sm.t.k[0]) + first_buf + c32_t * kRowBytes + (((2 * ks + half_t) ^ k_swizzle<D>(c32_t)) << 4);
   // transposing V read i: a group of 16 lanes covers 16 head-dim columns; lane points at row r0 = 4*half + (lane%16)/4
-  // (+ multiples of 8, which leave r0 = row & 7 alone), bf16 columns 32*(i&3) + 16*((lane>>4)&1) + 4*(lane&3): chunk
-  // 4*(i&3) + y0 with y0 < 4, swizzled with r0 << 1 -> one offset per value of i & 3
+  // (+ multiples of 8, which the swizzle does not see), bf16 columns 32*(i&3) + 16*((lane>>4)&1) + 4*(lane&3): chunk
+  // 4*(i&3) + y0 with y0 < 4, swizzled -> one offset per value of i & 3
   uint32_t v_rd[kDB];
   {
     const int r0 = 4 * half_t + ((lane_t & 15) >> 2);
     const int y0 = 2 * ((lane_t >> 4) & 1) + ((lane_t & 3) >> 1);
 #pragma unroll
-    for (int m = 0; m < kDB; ++m) v_rd[m] = lds_addr(sm.t.v[0]) + first_buf + r0 * kRowBytes + (((4 * m + y0) ^ (r0 << 1)) << 4) + 8 * (lane_t & 1);
+    for (int m = 0; m < kDB; ++m) v_rd[m] = lds_addr(sm.t.v[0]) + first_buf + r0 * kRowBytes + (((4 * m + y0) ^ v_swizzle<D>(r0)) << 4) + 8 * (lane_t & 1);
   }
 
 
@@ -575,19 +591,19 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
     // (selects, not branches: the eight slots stay straight-line code; the base address is scalar, and the vector offset
     // is chosen once per tile and operand kind)
     const uint32_t k_voff_sel = fetch_queries ? q_voff : k_voff, v_voff_sel = fetch_queries ? q_voff : v_voff;
-    uint32_t keys_next[4] = {0u, 0u, 0u, 0u};  // (sparse) row numbers of the next tile, read before the tile's first load is issued
-    if (MODE == kSparse) tile_gather_keys(keys_next, sm.idx, key0_next, tid);
+    uint32_t keys_next[kHalfLoads] = {};  // (sparse) row numbers of the next tile, read before the tile's first load is issued
+    if (MODE == kSparse) tile_gather_keys<D>(keys_next, sm.idx, key0_next, tid);
     if (kAnyRows && p.n_ctx - key0_next < kBN) set_row_offs(p.n_ctx - key0_next);
 #define AA_FETCH_ONE(n)                                                                                               \
   if (MODE == kAnchor) {                                                                                              \
     const int j_ = (n) >> 1;                                                                                          \
-    const char* kv_ = ((n) & 1) ? vbase + (uint64_t)(uint32_t)(key0_next + 16 * j_) * v_row_bytes                     \
-                                : kbase + (uint64_t)(uint32_t)(key0_next + 16 * j_) * k_row_bytes;                    \
-    const char* q_ = qblock + (uint64_t)(64 * ((n) & 1) + 16 * j_) * q_row_bytes;                                     \
+    const char* kv_ = ((n) & 1) ? vbase + (uint64_t)(uint32_t)(key0_next + kLoadRows * j_) * v_row_bytes                     \
+                                : kbase + (uint64_t)(uint32_t)(key0_next + kLoadRows * j_) * k_row_bytes;                    \
+    const char* q_ = qblock + (uint64_t)(64 * ((n) & 1) + kLoadRows * j_) * q_row_bytes;                                     \
     load16_to_lds(fetch_queries ? q_ : kv_, ((n) & 1) ? v_voff_sel : k_voff_sel,                                      \
-                  (((n) & 1) ? lds_v0 : lds_k0) + (buf ^ 1) * kTileBytes + 16 * j_ * kRowBytes);                      \
+                  (((n) & 1) ? lds_v0 : lds_k0) + (buf ^ 1) * kTileBytes + j_ * kLoadBytes);                      \
   } else {                                                                                                            \
-    tile_fetch_one<MODE>(n, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, key0_next,                          \
+    tile_fetch_one<MODE, D>(n, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, key0_next,                          \
                          kAnyRows ? row_offs : keys_next, lds_k0 + (buf ^ 1) * kTileBytes, lds_v0 + (buf ^ 1) * kTileBytes, k_voff, v_voff);           \
   }
     // (a wave whose rows all lie above this tile - two of the four waves on the last tile of a causal work-group -
@@ -626,7 +642,7 @@ __global__ void __launch_bounds__(256, 2) flash_kernel(const FlashArgs p) {
         AA_S_MFMA(s0, n);
         if (AA_ABLATE != 3) {
 #pragma unroll
-          for (int u = 0; u < 8 / kKS; ++u) { AA_FETCH_ONE(n * (8 / kKS) + u) }
+          for (int u = 0; u < 2 * kHalfLoads / kKS; ++u) { AA_FETCH_ONE(n * (2 * kHalfLoads / kKS) + u) }
         }
         AA_FENCE;
       }

@@ -140,8 +140,8 @@ hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mas
   return hipGetLastError();
 }
 
-// How the keys of a rows-mode problem are cut into chunks.  The chip holds 512 work-groups (two per CU).  A tile takes a
-// work-group about 1.9 us with a neighbour on its CU and 1.1 us alone; several chunks cost a write and a read of the state
+// How the keys of a rows-mode problem are cut into chunks.  The chip holds 512 work-groups (two per CU) at head dimension
+// 128 and 768 at 64.  A tile takes a work-group about 1.9 us (64: 1.7 us) when the CUs are full and 1.1 us (1.0 us) alone; several chunks cost a write and a read of the state
 // (64 KB per column block and chunk at head dimension 128) and one more launch.  Every number of chunks up to 64 is priced with that
 // and the cheapest is taken.
 void plan_rows(FlashArgs& a) {
@@ -152,6 +152,7 @@ void plan_rows(FlashArgs& a) {
   int64_t total = 0;  // tiles of one unit
   for (int i = 0; i < a.n_col_blocks; ++i)
     total += min(a.causal_offset + (min(128 * (i + 1), a.n_rows * group) - 1) / group, a.n_ctx - 1) / 64 + 1;
+  const int slots = a.head_dim == 128 ? 512 : 768;
   double best = 1e30;
   a.n_chunks = 1;
   a.chunk_tiles = max_tiles;
@@ -162,9 +163,9 @@ void plan_rows(FlashArgs& a) {
     for (int i = 0; i < a.n_col_blocks; ++i)
       wgs += (min(a.causal_offset + (min(128 * (i + 1), a.n_rows * group) - 1) / group, a.n_ctx - 1) / 64 + len) / len;
     wgs *= units;
-    const double t_tile = wgs <= 256 ? 1.1 : 1.9;
-    const double rounds = (double)((wgs + 511) / 512) * ((double)total * units / wgs);
-    double us = t_tile * (rounds > len ? rounds : len) * a.head_dim / 128;
+    const double t_tile = a.head_dim == 128 ? (wgs <= 256 ? 1.1 : 1.9) : (wgs <= 256 ? 1.0 : 1.7);
+    const double rounds = (double)((wgs + slots - 1) / slots) * ((double)total * units / wgs);
+    double us = t_tile * (rounds > len ? rounds : len);
     if (chunks > 1) us += 6.0 + (double)wgs * 128 * a.head_dim * 8 / 4e6;
     if (us < best) {
       best = us;
