@@ -39,14 +39,12 @@ def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[i
     ``causal_offset``: query row i may see keys ``<= causal_offset + i`` (None: use ``attention_mask`` as is).  Writes into
     ``out`` where it is given and the own kernel runs, otherwise returns a new tensor; either way the result is returned.
     The own kernel takes bf16/fp16 inference on the GPU; the framework's attention does everything else (other types and
-    head dimensions, gradients, the CPU)."""
+    head dimensions, gradients and tangents, vmap, tracing, the CPU)."""
     groups = query.shape[1] // key.shape[1]
     wants_grad = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
-    by_mask = (attention_mask is not None and causal_offset is None and attention_mask.dtype == torch.bool and attention_mask.dim() == 4
-               and attention_mask.shape[0] in (1, query.shape[0])
-               and tuple(attention_mask.shape[1:]) == (1, query.shape[2], key.shape[2]))
+    by_mask = attention_mask is not None and causal_offset is None
     by_offset = attention_mask is None and causal_offset is not None and causal_offset >= 0
-    if ((by_mask or by_offset) and not wants_grad and (scaling is None or scaling > 0) and dense_rows_supported(query, key, value)):
+    if (by_mask or by_offset) and not wants_grad and (scaling is None or scaling > 0) and dense_rows_supported(query, key, value, attention_mask):
         return dense_rows_attention(query, key, value, causal_offset or 0, sm_scale=scaling, out=out, mask=attention_mask)
     mask = attention_mask
     if causal_offset is not None and mask is None and query.shape[2] > 1:

@@ -103,4 +103,5 @@ def dtype_code(t) -> int:
 def t3(t):
     """(data_ptr, stride_b, stride_h, stride_n) of a [B,H,N,D] tensor whose last stride is 1."""
     assert t.dim() == 4 and t.stride(3) == 1
-    return (t.data_ptr(), t.stride(0), t.stride(1), t.stride(2))
+    sb, sh, sn, _ = t.stride()
+    return (t.data_ptr(), sb, sh, sn)

@@ -158,18 +158,37 @@ def anchor_attn_test_time(Q, K, V, sm_scale: float = None, block_size: int = 128
     return output, search_time, compute_time
 
 
-def dense_rows_supported(Q, K, V) -> bool:
-    """Whether :func:`dense_rows_attention` takes these tensors (its kernels' types, head dimensions, alignment and
-    32-bit addressing of one head)."""
-    if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype):
+def _called_plainly() -> bool:
+    """False while something other than eager execution watches the operations (vmap, forward-mode differentiation, tracing,
+    compilation, a dispatch mode): it would not see what happens behind the C interface."""
+    return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def dense_rows_supported(Q, K, V, mask=None) -> bool:
+    """Whether :func:`dense_rows_attention` takes these tensors (its kernels' types, head dimensions, alignment, sizes of
+    one launch and 32-bit addressing of one head)."""
+    if not (type(Q) is type(K) is type(V) is torch.Tensor and _called_plainly()):
         return False
-    D = Q.shape[3]
-    if D not in (64, 128) or K.shape != V.shape or K.shape[3] != D or K.shape[0] != Q.shape[0] or Q.shape[1] % K.shape[1]:
+    if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype and K.device == V.device == Q.device):
         return False
-    for t in (Q, K, V):
-        if t.stride(3) != 1 or t.data_ptr() % 16 or t.stride(0) % 8 or t.stride(1) % 8 or t.stride(2) % 8:
+    B, H, N, D = Q.shape
+    if D not in (64, 128) or K.shape != V.shape or K.shape[3] != D or K.shape[0] != B or not B or not K.shape[1] or H % K.shape[1] or not H:
+        return False
+    n_keys = K.shape[2]
+    for t, rows in ((Q, N), (K, n_keys), (V, n_keys)):
+        sb, sh, sn, sd = t.stride()
+        if sd != 1 or (sb | sh | sn) & 7 or t.data_ptr() & 15 or not D <= sn <= 1 << 14 or not 0 < rows <= 1 << 20 or rows * sn * 2 >= 1 << 32:
             return False
-        if not D <= t.stride(2) <= 1 << 14 or not 0 < t.shape[2] <= 1 << 20 or t.shape[2] * t.stride(2) * 2 >= 1 << 32:
+    col_blocks = (N * (H // K.shape[1]) + 127) // 128
+    if B * K.shape[1] * col_blocks * 64 >= 1 << 31:
+        return False
+    if mask is not None:
+        if type(mask) is not torch.Tensor or mask.device != Q.device or mask.dtype != torch.bool or mask.dim() != 4:
+            return False
+        if mask.shape[0] not in (1, B) or tuple(mask.shape[1:]) != (1, N, n_keys):
+            return False
+        if B >= 1 << 16 or col_blocks >= 1 << 16 or N * ((n_keys + 63) // 64) * 8 >= 1 << 32:
             return False
     return True
 
@@ -191,9 +210,13 @@ def dense_rows_attention(Q, K, V, causal_offset: int = 0, sm_scale: float = None
     sizes = (B, H, K.shape[1], N, n_keys, D, int(causal_offset))
     nbytes = lib.aa_dense_rows_workspace_bytes(*sizes, mask is not None)
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=Q.device) if nbytes else None
-    _hip.check(lib.aa_dense_rows_fwd(*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output), *mask_args,
-                                     ws.data_ptr() if nbytes else None, nbytes, *sizes,
-                                     float(sm_scale), _hip.dtype_code(Q), _stream()))
+    args = (*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output), *mask_args, ws.data_ptr() if nbytes else None, nbytes, *sizes,
+            float(sm_scale), _hip.dtype_code(Q))
+    if Q.device.index == torch.cuda.current_device():
+        _hip.check(lib.aa_dense_rows_fwd(*args, _stream()))
+    else:  # (a pipeline's later layers lie on other GPUs than the current one)
+        with torch.cuda.device(Q.device):
+            _hip.check(lib.aa_dense_rows_fwd(*args, _stream()))
     return output
 
 

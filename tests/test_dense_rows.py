@@ -97,3 +97,40 @@ def test_masked_rows_against_float64(batch, hq, hkv, n_rows, n_keys, d, dtype, k
     mask = _mask(kind, batch, n_rows, n_keys)
     out = dense_rows_attention(q, k, v, mask=mask)
     _check(out, _reference(q, k, v, d ** -0.5, mask[:, 0].expand(batch, -1, -1)), v, dtype)
+
+
+def test_own_kernels_are_left_out_of_transformed_and_traced_calls():
+    """Their work is invisible to vmap, forward-mode differentiation, tracing and dispatch modes."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from anchor_attn.src.ops.anchor_attn_v4 import _called_plainly
+    assert _called_plainly()
+    seen = []
+
+    def probe(x):
+        seen.append(_called_plainly())
+        return x * 2
+
+    x = torch.ones(2, 3)
+    torch.func.vmap(probe)(x)
+    torch.func.jvp(probe, (x,), (x,))
+    with torch.autograd.forward_ad.dual_level():
+        probe(torch.autograd.forward_ad.make_dual(x, x))
+    make_fx(probe)(x)
+    torch.jit.trace(probe, (x,), check_trace=False)
+    with FlopCounterMode(display=False):
+        probe(x)
+    assert len(seen) >= 6 and not any(seen)
+    assert _called_plainly()
+
+
+@pytest.mark.gpu
+def test_calls_that_stay_with_library_attention():
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_supported
+    q, k, v = _qkv(2, 4, 2, 1, 40, 64, torch.bfloat16, 1)
+    assert dense_rows_supported(q, k, v)
+    assert not dense_rows_supported(q[:0], k[:0], v[:0])  # an empty batch
+    mask = torch.ones(2, 1, 1, 40, dtype=torch.bool, device="cuda")
+    assert dense_rows_supported(q, k, v, mask)
+    assert not dense_rows_supported(q, k, v, mask.cpu()) and not dense_rows_supported(q, k.cpu(), v.cpu())
