@@ -222,11 +222,13 @@ size_t aa_workspace_bytes(int batch, int n_q_heads, int n_ctx, int head_dim, int
   return carve(batch, n_q_heads, n_ctx, head_dim, block_size, step).total;
 }
 
-// Stage 1; with qbar/abar non-null (block_size <= 128) the kernel also emits the pooled queries and anchors.
+// Stage 1; with qbar/abar non-null (block_size <= 128) the kernel also emits the pooled queries and anchors, with `out`
+// non-null the output of big block 0, whose rows select no keys, in the place of their state and pooled rows.
 static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                        const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                        float* M, float* L, float* acc_frag, void* qbar, void* abar,
+                       void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
                        int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                        int block_size, int step, float sm_scale, int scale_mode, int dtype, void* stream) {
   int rc;
@@ -245,6 +247,7 @@ static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_s
   a.k = (const uint16_t*)k; a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
   a.v = (const uint16_t*)v; a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn;
   a.M_out = M; a.L_out = L; a.acc_out = acc_frag;
+  a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
   a.qbar_out = (uint16_t*)qbar; a.abar_out = (uint16_t*)abar;
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size;
@@ -259,7 +262,7 @@ int aa_stage1_anchor_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
                          int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                          int block_size, int step, float sm_scale, int scale_mode, int dtype, void* stream) {
   return stage1_impl("aa_stage1_anchor_fwd", q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc_frag, nullptr,
-                     nullptr, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, scale_mode, dtype, stream);
+                     nullptr, nullptr, 0, 0, 0, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, scale_mode, dtype, stream);
 }
 
 int aa_pool_q_anchor(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn, const float* M,
@@ -316,8 +319,10 @@ int aa_stage2_select(const void* qbar, const void* abar,
               who, n_q_heads / n_kv_heads, n_ctx / (block_size * step), (long long)batch * n_q_heads * (n_ctx / block_size));
     return AA_EUNSUPPORTED;
   }
-  if ((rc = check_launch(launch_select_thresholds(a, (hipStream_t)stream), who))) return rc;
-  if ((rc = check_launch(launch_select_scores(a, (hipStream_t)stream), who))) return rc;
+  if (n_ctx > block_size * step) {  // (a single big block has no candidates: its counts are 0)
+    if ((rc = check_launch(launch_select_thresholds(a, (hipStream_t)stream), who))) return rc;
+    if ((rc = check_launch(launch_select_scores(a, (hipStream_t)stream), who))) return rc;
+  }
   return check_launch(launch_select_compact(a, (hipStream_t)stream), who);
 }
 
@@ -342,7 +347,9 @@ int aa_stage2_select_static(const void* qbar, const void* abar,
                           n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream);
 }
 
-int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+// Stage 3 for the rows from big block `first_big_block` (0 or 1) on.
+static int stage3_impl(const char* who, int first_big_block,
+                       const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                          const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                          const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                          const int32_t* coords, const int32_t* counts,
@@ -350,7 +357,6 @@ int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
                          void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
                          int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                          int block_size, int step, float sm_scale, int dtype, void* stream) {
-  const char* who = "aa_stage3_sparse_fwd";
   int rc;
   if ((rc = check_dtype(dtype, who))) return rc;
   if ((rc = check_dims({batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step}, who))) return rc;
@@ -370,9 +376,21 @@ int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
   a.coords = coords; a.counts = counts;
   a.coords_per_head = aa_coords_entries_per_head(n_ctx, block_size, step);
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
-  a.big_block = block_size * step; a.block_size = block_size;
+  a.big_block = block_size * step; a.block_size = block_size; a.first_big_block = first_big_block;
   a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
   return check_launch(run_flash(a, 1, (hipStream_t)stream), who);
+}
+
+int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                         const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                         const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                         const int32_t* coords, const int32_t* counts,
+                         const float* M, const float* L, const float* acc_frag,
+                         void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                         int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                         int block_size, int step, float sm_scale, int dtype, void* stream) {
+  return stage3_impl("aa_stage3_sparse_fwd", 0, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc_frag,
+                     out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, dtype, stream);
 }
 
 int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
@@ -400,25 +418,30 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   void* abar = ws + w.abar;
   uint32_t* mask = (uint32_t*)(ws + w.mask);
   int32_t* coords = (int32_t*)(ws + w.coords);
-  int32_t* counts = (int32_t*)(ws + w.counts);
+  // (stage 2 writes the counts where the caller wants them; a pointer that is not aligned for that gets a copy)
+  const bool counts_direct = counts_out != nullptr && (reinterpret_cast<uintptr_t>(counts_out) & 15u) == 0;
+  int32_t* counts = counts_direct ? counts_out : (int32_t*)(ws + w.counts);
+  if ((rc = check_tensor(out, o_sb, o_sh, o_sn, n_ctx, head_dim, who, "out"))) return rc;
   // A stage-1 work-group holds 128 query rows: whole pooled rows when block_size <= 128, and then it pools them itself
   // (same arithmetic as aa_pool_q_anchor, bit for bit) instead of a separate pass over the queries.
   const bool fused_pool = block_size <= 128;
   if ((rc = stage1_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc, fused_pool ? qbar : nullptr,
-                        fused_pool ? abar : nullptr, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step,
+                        fused_pool ? abar : nullptr, out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step,
                         (float)sm_scale, scale_mode, dtype, stream)))
     return rc;
-  if (!fused_pool &&
+  // Big block 0 selects nothing and is finished by now; stages 2 and 3 are for the others.
+  const bool selects = n_ctx > block_size * step;
+  if (!fused_pool && selects &&
       (rc = aa_pool_q_anchor(q, q_sb, q_sh, q_sn, M, qbar, abar, batch, n_q_heads, n_ctx, head_dim, block_size, dtype, stream)))
     return rc;
   if ((rc = aa_stage2_select(qbar, abar, k, k_sb, k_sh, k_sn, mask, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
                              head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream)))
     return rc;
-  if ((rc = aa_stage3_sparse_fwd(q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc, out,
+  if ((rc = stage3_impl(who, 1, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc, out,
                                  o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, (float)sm_scale,
                                  dtype, stream)))
     return rc;
-  if (counts_out != nullptr) {
+  if (counts_out != nullptr && !counts_direct) {
     const size_t bytes = (size_t)batch * n_q_heads * (n_ctx / (block_size * step)) * 4;
     hipError_t e = hipMemcpyAsync(counts_out, counts, bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream);
     if ((rc = check_launch(e, who))) return rc;

@@ -192,11 +192,12 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   // list's round trip to memory and the wait for its stores.
   const int group = p.n_q_heads / p.n_kv_heads;
   const int nq = MODE == kSparse ? p.q_blocks_per_wg : 1;
-  const int n_qunit = kAnyRows ? 1 : p.n_ctx / (BM * nq);
   const int S = p.big_block;
+  // (sparse mode may leave out the first big block, whose rows select nothing)
+  const int n_qunit = kAnyRows ? 1 : (p.n_ctx - (MODE == kSparse ? p.first_big_block * S : 0)) / (BM * nq);
   int g, qunit, kvh, b;
   int chunk = 0;  // (rows) which chunk of the keys
-  const uint32_t n_pairs = (uint32_t)(p.batch * p.n_kv_heads) * (uint32_t)(p.n_ctx / S);
+  const uint32_t n_pairs = (uint32_t)(p.batch * p.n_kv_heads) * (uint32_t)(p.n_ctx / S - p.first_big_block);
   if (MODE == kSparse && n_pairs % 8u == 0u) {
     // Stage 3's work per (KV head, big block) pair is the length of the pair's index lists, which depends on the data:
     // a head whose queries select many keys would keep its XCD busy long after the others have finished if whole
@@ -230,7 +231,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     qunit = vid % n_qunit;  vid /= n_qunit;
     kvh = vid % p.n_kv_heads;
     b = vid / p.n_kv_heads;
-    qunit = n_qunit - 1 - qunit;  // longest rows first (later big blocks also carry the longest index lists)
+    qunit = p.n_ctx / (BM * nq) - 1 - qunit;  // longest rows first (later big blocks also carry the longest index lists)
   }
   const int hq = kvh * group + g;
   const int bb = qunit * nq * BM / S;  // (all blocks of a work-group lie in one big block: the host picks q_blocks_per_wg so)
@@ -311,7 +312,9 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   const bool feeds_next = list_chains && qb + 1 < nq;  // the next block takes its first tile from this one
 
   // ---- tile schedule -------------------------------------------------------------------------
-  const bool pool = MODE == kAnchor && p.qbar_out != nullptr;
+  // (anchor) the first big block's rows select no keys further on: where the caller gives the output, they are done here
+  const bool finishes = MODE == kAnchor && p.out != nullptr && bb == 0;
+  const bool pool = MODE == kAnchor && p.qbar_out != nullptr && !finishes;
   int n_tiles, n_init = 0;
   int key_base = 0;  // (rows) first key of the chunk
   int entry_next = 0;  // (masked) list entry of the tile to be fetched next
@@ -805,7 +808,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 
   // ---- epilogue --------------------------------------------------------------------------------
   const float l_tot = l_run + xor32(l_run);
-  if (MODE == kAnchor) {
+  if (MODE == kAnchor && !finishes) {
     if (half == 0) {
       p.M_out[bh * p.n_ctx + my_row] = m_run;
       p.L_out[bh * p.n_ctx + my_row] = l_tot;
@@ -927,19 +930,29 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 }
 
 #ifndef AA_SPARSE_QBLOCKS
-#define AA_SPARSE_QBLOCKS 4  // 128-row query blocks a stage-3 work-group handles one after the other (when the big block allows)
+#define AA_SPARSE_QBLOCKS 4  // most 128-row query blocks a stage-3 work-group handles one after the other
 #endif
 
 template <int MODE>
 static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
   FlashArgs a = args;
   a.q_blocks_per_wg = 1;
+  int64_t blocks = (int64_t)a.batch * a.n_q_heads * (a.n_ctx / 128);
   if (MODE == kSparse) {
-    const int per_big_block = a.big_block / 128;  // even for every supported geometry
-    a.q_blocks_per_wg = per_big_block % AA_SPARSE_QBLOCKS == 0 ? AA_SPARSE_QBLOCKS : (per_big_block % 2 == 0 ? 2 : 1);
+    const int per_big_block = a.big_block / 128;
+    blocks -= (int64_t)a.batch * a.n_q_heads * a.first_big_block * per_big_block;
+    if (blocks == 0) return hipSuccess;
+    // Chained blocks save a work-group's start and the list's round trip, but few work-groups leave CUs idle: as many as
+    // still fill the chip twice (two work-groups per CU at head dimension 128, three at 64).  Four at any size against this
+    // rule, operator: 14/2 heads of 64, 8192 tokens, every key selected 491 -> 288 us; 32/8 heads of 128, 4096 tokens
+    // 353 -> 288 us, 16384 tokens 2661 -> 2568 us (filling the chip once: 2649); 32768 tokens, few keys: within 0.3 %.
+    const int fills_twice = 2 * (a.head_dim == 128 ? 512 : 768);
+    int nq = AA_SPARSE_QBLOCKS;
+    while (nq > 1 && (per_big_block % nq != 0 || blocks / nq < fills_twice)) nq /= 2;
+    a.q_blocks_per_wg = nq;
   }
   const dim3 grid(MODE == kRows || MODE == kMasked ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
-                                : (uint32_t)a.batch * a.n_q_heads * (a.n_ctx / (128 * a.q_blocks_per_wg))), block(256);
+                                : (uint32_t)(blocks / a.q_blocks_per_wg)), block(256);
   if (a.head_dim == 128) {
     if (a.dtype == 0) hipLaunchKernelGGL((flash_kernel<MODE, Bf16, 128>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((flash_kernel<MODE, F16, 128>), grid, block, 0, stream, a);

@@ -8,7 +8,7 @@ struct FlashArgs {
   const uint16_t* q; int64_t q_sb, q_sh, q_sn;
   const uint16_t* k; int64_t k_sb, k_sh, k_sn;
   const uint16_t* v; int64_t v_sb, v_sh, v_sn;
-  uint16_t* out;     int64_t o_sb, o_sh, o_sn;   // sparse / dense modes
+  uint16_t* out;     int64_t o_sb, o_sh, o_sn;   // all modes (anchor mode, optional: the first big block's rows, which select no keys, are finished there)
   float* M_out; float* L_out; float* acc_out;  // anchor mode
   // anchor mode, optional (both or neither; block_size <= 128): the work-group also mean-pools its 128 raw query rows
   // and anchors into qbar [B,Hq,N/block_size,head_dim] and abar [B,Hq,N/block_size], bit for bit what pool_kernel computes
@@ -18,6 +18,7 @@ struct FlashArgs {
   int batch, n_q_heads, n_kv_heads, n_ctx;
   int head_dim;  // 128 or 64
   int big_block, block_size;
+  int first_big_block;  // sparse mode: 1 leaves out the rows of big block 0 (anchor mode has finished them), 0 takes all rows
   float sm_scale; int scale_mode;
   int q_blocks_per_wg;  // set by the launcher
   // rows mode: n_rows query rows over n_ctx keys, row i sees keys 0 .. causal_offset + i.  The (row, head) columns of a
