@@ -24,7 +24,12 @@ LOG2E = 1.44269504
 
 def _ratio(true_counts, B, H, N, block_size, step):
     # same expression as the reference (anchor_attn_v4.py:271); stays a 0-dim device tensor
-    return true_counts.sum() / (B * H * N * N / (block_size * step) // 2)
+    denominator = B * H * N * N / (block_size * step) // 2
+    if torch.get_default_dtype() != torch.float32 or not true_counts.is_contiguous():
+        return true_counts.sum() / denominator  # (the quotient of whole numbers has the default type)
+    ratio = torch.empty((), dtype=torch.float32, device=true_counts.device)
+    _hip.check(_hip.lib().aa_sparsity_ratio(true_counts.data_ptr(), true_counts.numel(), denominator, ratio.data_ptr(), _stream()))
+    return ratio
 
 
 def _log_ratio(sparse_ratio):

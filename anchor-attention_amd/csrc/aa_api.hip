@@ -449,6 +449,15 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   return AA_OK;
 }
 
+int aa_sparsity_ratio(const int32_t* counts, int64_t n, double denominator, float* ratio, void* stream) {
+  const char* who = "aa_sparsity_ratio";
+  if (counts == nullptr || ratio == nullptr || n <= 0 || !(denominator > 0.0)) {
+    set_error("%s: counts and ratio must not be NULL, n (%lld) and denominator (%g) must be positive", who, (long long)n, denominator);
+    return AA_EBADARG;
+  }
+  return check_launch(launch_ratio(counts, n, 1.f / (float)denominator, ratio, (hipStream_t)stream), who);
+}
+
 int aa_dense_causal_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                         const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                         const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,

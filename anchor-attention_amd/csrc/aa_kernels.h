@@ -78,5 +78,6 @@ struct SelectArgs {
 hipError_t launch_select_thresholds(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_select_scores(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream);
+hipError_t launch_ratio(const int32_t* counts, int64_t n, float inverse, float* ratio, hipStream_t stream);
 
 }  // namespace aa

@@ -381,4 +381,23 @@ hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// The share of selected keys: a few KB of counts summed by one work-group, bound by its launch.  The framework's sum and
+// division of the same counts were four launches (conversion, sum, a scalar's copy, division), 14 us of the 207 us that the
+// operator took on 4096 tokens with 32/8 heads of 128.
+__global__ void __launch_bounds__(256) ratio_kernel(const int32_t* counts, const int64_t n, const float inverse, float* ratio) {
+  __shared__ long long part[4];
+  long long sum = 0;
+  for (int64_t i = threadIdx.x; i < n; i += 256) sum += counts[i];
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) *ratio = (float)(part[0] + part[1] + part[2] + part[3]) * inverse;
+}
+
+hipError_t launch_ratio(const int32_t* counts, int64_t n, float inverse, float* ratio, hipStream_t stream) {
+  hipLaunchKernelGGL(ratio_kernel, dim3(1), dim3(256), 0, stream, counts, n, inverse, ratio);
+  return hipGetLastError();
+}
+
 }  // namespace aa

@@ -170,6 +170,10 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
                        int dtype, void* stream);
 
+/* sum(counts[0 .. n)) / denominator as one float32 on the device: the sparsity ratio of anchor_attn_v4.py:270-272, with the
+ * sum in 64-bit integers, rounded to float32 and multiplied by float32(1 / denominator). */
+int aa_sparsity_ratio(const int32_t* counts, int64_t n, double denominator, float* ratio, void* stream);
+
 /* ---- dense causal baseline on the same MFMA core --------------------------------------------
  * Counterpart of the reference's dense comparison path (flash_attn_triton.py:83-211, GQA mapping
  * :129-132): plain causal softmax attention, out = round16(softmax(q k^T * sm_scale) v).

@@ -27,3 +27,14 @@ def test_operator_equals_its_stages(batch, hq, hkv, n_big, d, block, step, theta
     want, want_ratio = anchor_attn_without_anchor(q, k, v, block_size=block, step=step, difference=theta)
     assert got is out and torch.equal(out, want) and torch.equal(ratio, want_ratio)
     assert n_big > 1 or float(ratio) == 0.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,n_ctx", [(1, 2048), (255, 6144), (256, 10240), (8192, 131072), (70001, 126976)])
+def test_ratio_equals_the_expression_in_torch(n, n_ctx):
+    """The same operations on the same whole numbers, so the same float; sums beyond 2^31 among them."""
+    from anchor_attn.src.ops.anchor_attn_v4 import _ratio
+    counts = torch.randint(0, n_ctx, (n, 1, 1, 1), dtype=torch.int32, generator=torch.Generator().manual_seed(n)).cuda()
+    got = _ratio(counts, 3, 7, n_ctx, 128, 16)
+    want = counts.sum() / (3 * 7 * n_ctx * n_ctx / (128 * 16) // 2)
+    assert got.dtype == want.dtype and got.shape == want.shape and torch.equal(got, want)
