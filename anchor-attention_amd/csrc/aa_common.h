@@ -115,7 +115,8 @@ __host__ __device__ inline int64_t coords_tri(int64_t bb, int64_t S, int64_t bs)
 // with its own L2).  The work consists of `n_units` units (a KV head of one batch element) of `per_unit`
 // work-groups each, ordered heaviest first inside a unit; work-groups of one unit read the same K/V rows or pooled
 // queries.  Returns the logical index unit * per_unit + idx such that
-//   n_units % 8 == 0 : every XCD owns n_units / 8 whole units, in order;
+//   n_units % 8 == 0 : every XCD owns n_units / 8 whole units, every eighth one: the units of one batch element, whose work
+//                      differs from another's where prompts are padded, are spread over the XCDs;
 //   8 % n_units == 0 : s = 8 / n_units XCDs share a unit and take its rows alternately (row = idx / inner, the
 //                      `inner` work-groups of a row stay together), so that each gets the same mix of heavy and light;
 //   otherwise        : the hardware order is kept.
@@ -123,7 +124,7 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uin
   const uint32_t total = n_units * per_unit;
   const uint32_t xcd = wg % 8u, k = wg / 8u;
   if (total % 8u != 0u) return wg;
-  if (n_units % 8u == 0u) return xcd * (total / 8u) + k;
+  if (n_units % 8u == 0u) return (k / per_unit * 8u + xcd) * per_unit + k % per_unit;
   if (8u % n_units == 0u) {
     const uint32_t s = 8u / n_units;
     if ((per_unit / inner) % s == 0u) return (xcd / s) * per_unit + ((k / inner) * s + xcd % s) * inner + k % inner;

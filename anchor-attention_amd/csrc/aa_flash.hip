@@ -318,6 +318,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   int n_tiles, n_init = 0;
   int key_base = 0;  // (rows) first key of the chunk
   int entry_next = 0;  // (masked) list entry of the tile to be fetched next
+  int entry_after = 0;  // (masked) and of the one after that, read from LDS a whole tile before it is needed
   u32x2 mask_word_next = {0u, 0u};  // (masked) which of that tile's 64 keys this lane's row sees, if the tile is a mixed one
   const uint32_t mask_row_off = MODE == kMasked ? (uint32_t)my_row * (uint32_t)p.mask_words_per_row * 8u : 0u;  // (below 2^32: checked on the host)
   auto request_mask_word = [&]() __attribute__((always_inline)) {
@@ -353,6 +354,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
       __syncthreads();
       n_tiles = __builtin_amdgcn_readfirstlane(sm.idx[kMaskedTiles]);
       entry_next = n_tiles > 0 ? __builtin_amdgcn_readfirstlane(sm.idx[0]) : 0;
+      entry_after = sm.idx[n_tiles > 1 ? 1 : 0];
     }
   } else {
     n_tiles = sparse_tiles;
@@ -586,8 +588,9 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // (sparse, chained: the last tile of a block fetches the list's first tile, for the next block)
     const int i_next = i + 1 < n_tiles ? i + 1 : (feeds_next ? 0 : i);
     if (MODE == kMasked) {
-      entry_next = __builtin_amdgcn_readfirstlane(sm.idx[i_next]);
+      entry_next = __builtin_amdgcn_readfirstlane(entry_after);
       request_mask_word();
+      entry_after = sm.idx[min(i + 2, n_tiles - 1)];
     }
     const int key0_next = AA_TILE_KEY0(i_next);
     const bool fetch_queries = MODE == kAnchor && pool && i + 1 == n_tiles;  // wave-uniform

@@ -69,7 +69,7 @@ def test_dense_rows_against_float64(batch, hq, hkv, n_rows, offset, d, dtype):
 
 
 def _mask(kind, batch, n_rows, n_keys):
-    rows, keys = torch.arange(n_rows, device="cuda") + n_keys - n_rows, torch.arange(n_keys, device="cuda")
+    rows, keys = torch.arange(n_rows, device="cuda") + max(n_keys - n_rows, 0), torch.arange(n_keys, device="cuda")
     causal = keys[None, :] <= rows[:, None]
     if kind == "padded":  # left-padded prompts: whole tiles nobody sees, rows without any key
         pads = torch.tensor([(37 * b) % n_keys + 70 * b for b in range(batch)], device="cuda")
@@ -87,6 +87,9 @@ def _mask(kind, batch, n_rows, n_keys):
     (2, 4, 4, 65, 4161, 128, torch.bfloat16, "padded"),  # more keys than one work-group of the mask kernel packs; chunks
     (2, 4, 2, 300, 300, 64, torch.bfloat16, "window"),
     (1, 2, 1, 5, 67000, 128, torch.bfloat16, "random"),  # more tiles than one chunk may list
+    (2, 4, 2, 40, 13, 64, torch.bfloat16, "random"),     # fewer keys than a lane of the mask kernel packs
+    (1, 2, 2, 150, 16, 128, torch.float16, "random"),    # and as many; more rows than it loads at once
+    (2, 3, 1, 30, 1023, 64, torch.bfloat16, "padded"),   # a ragged end of one work-group's keys
     (4, 28, 4, 1, 2501, 128, torch.bfloat16, "padded"),  # a padded batch's decode step: tiles that are skipped
     (1, 2, 2, 1, 9000, 64, torch.float16, "random"),
     (40, 16, 8, 1, 8193, 64, torch.bfloat16, "window"),  # a second chunk of one key, since the first may hold no more
