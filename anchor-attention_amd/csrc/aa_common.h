@@ -31,6 +31,8 @@ struct Bf16 {
     bf16x2 h = __builtin_convertvector(f, bf16x2);
     return *reinterpret_cast<uint32_t*>(&h);
   }
+  // the pair that rounding to `packed` took from a and b
+  static __device__ __forceinline__ uint32_t pack_rest(float a, float b, uint32_t packed) { return pack(a - lo(packed), b - hi(packed)); }
   static __device__ __forceinline__ float round(float a) { return lo(pack(a, 0.f)); }  // float -> nearest bf16 -> float
   // (a * b).to(bf16) as the operator's definition compiles: a float32 product, then the rounding
   static __device__ __forceinline__ float round_product(float a, float b) { return round(a * b); }
@@ -50,6 +52,7 @@ struct F16 {
     f16x2 h = __builtin_convertvector(f, f16x2);
     return *reinterpret_cast<uint32_t*>(&h);
   }
+  static __device__ __forceinline__ uint32_t pack_rest(float a, float b, uint32_t packed) { return pack(a - lo(packed), b - hi(packed)); }
   static __device__ __forceinline__ float round(float a) { return lo(pack(a, 0.f)); }
   // (a * b).to(fp16) as the operator's definition compiles: ONE rounding of the exact product (the multiply and the
   // cast become a single mixed-precision instruction).  Written out so that it does not depend on what this compiler

@@ -9,7 +9,9 @@
 // (S^T = K Q^T with the scores scaled in float32, online soft-max, O^T += V^T P^T); the waves' states are merged
 // through LDS, the chunks' by decode_combine_kernel.
 //
-// One row, 32/8 heads of 128, 33001 keys (135 MB): 25.8 us = 5.2 TB/s, the rate of a large copy, and 4.1 us for the merge.
+// (P enters the product as two 16-bit numbers, its rounding and the rest: the precision of float32 for 0.5 us.)
+//
+// One row, 32/8 heads of 128, 33001 keys (135 MB): 26.3 us = 5.1 TB/s, the rate of a large copy, and 4.1 us for the merge.
 // The rows mode, which moves the state of 128 columns through its workspace, took 30.1 + 15.0 us; library attention, one
 // work-group per head, 1164 us.
 #include "aa_common.h"
@@ -167,7 +169,7 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
         for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
       m_run = m_new;
     }
-    u32x4 pw[2];
+    u32x4 pw[2], pw_rest[2];  // P^T and what its rounding left, both 16 bits wide: the sum has the precision of P in float32
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       float e[4];
@@ -178,6 +180,8 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
       }
       pw[c >> 1][2 * (c & 1) + 0] = T::pack(e[0], e[1]);
       pw[c >> 1][2 * (c & 1) + 1] = T::pack(e[2], e[3]);
+      pw_rest[c >> 1][2 * (c & 1) + 0] = T::pack_rest(e[0], e[1], pw[c >> 1][2 * (c & 1) + 0]);
+      pw_rest[c >> 1][2 * (c & 1) + 1] = T::pack_rest(e[2], e[3], pw[c >> 1][2 * (c & 1) + 1]);
     }
 #pragma unroll
     for (int st = 0; st < 2; ++st)
@@ -187,6 +191,7 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
         const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)(uintptr_t)(v_rd[db] + off + (16 * st + 8) * kPitch));
         const shortx8 a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         acc[db] = T::mfma(*reinterpret_cast<const vec8*>(&a), *reinterpret_cast<const vec8*>(&pw[st]), acc[db]);
+        acc[db] = T::mfma(*reinterpret_cast<const vec8*>(&a), *reinterpret_cast<const vec8*>(&pw_rest[st]), acc[db]);
       }
     const int t_after = t_next < n_tiles ? next_tile(t_next) : n_tiles;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this slot has been read

@@ -12,7 +12,7 @@
 // of a query are then plain per-lane scalars (one exchange with the lane 32 positions away
 // completes the row max).  The second product is computed transposed as well,
 //   O^T[d][query] += V^T[d][key] . P^T[key][query]  (A = V^T, B = P^T straight from the S^T
-// accumulator registers, rounded to bf16) - P never travels through LDS.
+// accumulator registers, rounded to bf16; rows and masked: as two such numbers) - P never travels through LDS.
 // The contraction slot k = 8*(lane/32) + e of MFMA step st of key block kb is fed from accumulator
 // register 8*st + e, i.e. key 32*kb + 16*st + 8*(e/4) + 4*(lane/32) + e%4: two runs of four
 // consecutive keys.  V sits row-major in LDS exactly as it is in memory, and each run of four keys
@@ -544,6 +544,10 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     if (AA_ABLATE != 2) { sum += e0; sum += e1; sum += e2; sum += e3; }              \
     pw[(c) >> 1][2 * ((c) & 1) + 0] = T::pack(e0, e1);                                 \
     pw[(c) >> 1][2 * ((c) & 1) + 1] = T::pack(e2, e3);                                 \
+    if (kAnyRows) { /* what the rounding left, as a second 16-bit number */            \
+      pw##_rest[(c) >> 1][2 * ((c) & 1) + 0] = T::pack_rest(e0, e1, pw[(c) >> 1][2 * ((c) & 1) + 0]);  \
+      pw##_rest[(c) >> 1][2 * ((c) & 1) + 1] = T::pack_rest(e2, e3, pw[(c) >> 1][2 * ((c) & 1) + 1]);  \
+    }                                                                                  \
   }
   // V operand fetch i (two transposing reads): i = (kb*2 + st)*kDB + db
 #define AA_V_SRC(i) (v_rd[(i) % kDB] + (uint32_t)(rd_off + (32 * ((i) / (2 * kDB)) + 16 * (((i) / kDB) & 1)) * kRowBytes))
@@ -558,6 +562,8 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     const shortx8 av = __builtin_shufflevector(vlo[i], vhi[i], 0, 1, 2, 3, 4, 5, 6, 7);                \
     acc[(i) % kDB] = T::mfma(*reinterpret_cast<const vec8*>(&av),                                      \
                              AA_ABLATE == 10 ? qreg[(i) % kKS] : *reinterpret_cast<const vec8*>(&pw[((i) / kDB) & 1]), acc[(i) % kDB]); \
+    if (kAnyRows) acc[(i) % kDB] = T::mfma(*reinterpret_cast<const vec8*>(&av),                        \
+                                           *reinterpret_cast<const vec8*>(&pw##_rest[((i) / kDB) & 1]), acc[(i) % kDB]); \
   }
 #define AA_FENCE __builtin_amdgcn_sched_barrier(0)
 
@@ -619,6 +625,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
       vec8 ka[kNS];                // K operand of slot n = kb*kKS + ks
       shortx4 vlo[kNV], vhi[kNV];  // V operand of slot kNS + i, i = (kb*2 + st)*kDB + db
       u32x4 pw0[2], pw1[2];        // P^T fragments (bf16 pairs) of the two halves
+      u32x4 pw0_rest[2], pw1_rest[2];  // (rows) and of what their rounding left
       float mx0, mx1, sum0 = 0.f, sum1 = 0.f, shift0 = 0.f, alpha1 = 1.f;
 #define AA_K_FETCH(t) ka[t] = *(const lds_vec8*)(uintptr_t)(k_rd[(t) % kKS] + (uint32_t)(rd_off + 32 * ((t) / kKS) * kRowBytes))
 

@@ -1,8 +1,9 @@
 """Dense attention of any query rows over any keys (``dense_rows_attention``: ragged tails, short prompts, continued prompts)
 against float64 attention, at the sizes where tiles, column blocks and key chunks end.
 
-Bound: probabilities are rounded to the 16-bit type (unit roundoff u) before the second product, so the sum is off by at most
-u * max|v|, and the result is rounded once more, u * |out|; five per cent on top covers the float32 sums and exp2."""
+Bound (loose; the tight one is with the test of the probabilities' precision): probabilities rounded to the 16-bit type (unit
+roundoff u) before the second product would put the sum off by at most u * max|v|, and the result is rounded once more,
+u * |out|; five per cent on top covers the float32 sums and exp2."""
 import pytest
 import torch
 
@@ -66,6 +67,29 @@ def test_dense_rows_against_float64(batch, hq, hkv, n_rows, offset, d, dtype):
     _check(out, _reference(q, k, v, d ** -0.5, keep), v, dtype)
     again = dense_rows_attention(q.contiguous(), k, v, offset, sm_scale=d ** -0.5)
     assert torch.equal(again, out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_rows,offset,d,masked", [
+    (77, 1000, 128, False), (130, 63, 64, False), (129, 0, 128, True), (65, 0, 64, True), (1, 3000, 128, False), (2, 517, 64, False),
+    (1, 777, 128, True),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_probabilities_keep_float32_precision(n_rows, offset, d, masked, dtype):
+    """Bound: a probability enters the second product as two 16-bit numbers, off by u^2 of itself; its score is a float32 sum
+    over d, off by at most d * 2^-24 * |q||k| * scale, and the probability by as much of itself; the result is rounded once."""
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
+    n_keys, scale = offset + n_rows, d ** -0.5
+    q, k, v = _qkv(2, 4, 2, n_rows, n_keys, d, dtype, 3 * n_rows + offset)
+    keys, rows = torch.arange(n_keys, device="cuda"), torch.arange(n_rows, device="cuda") + offset
+    keep = (keys[None, :] <= rows[:, None]).expand(2, -1, -1)
+    out = dense_rows_attention(q, k, v, mask=keep[:, None]) if masked else dense_rows_attention(q, k, v, offset)
+    want = _reference(q, k, v, scale, keep)
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    score = d * 2.0 ** -24 * scale * float(q.double().norm(dim=-1).max() * k.double().norm(dim=-1).max())
+    bound = 1.05 * (u * want.abs() + (u * u + score) * v.double().abs().max())
+    err = (out.double() - want).abs()
+    assert bool((err <= bound).all()), float((err - bound).max())
 
 
 def _mask(kind, batch, n_rows, n_keys):
