@@ -171,9 +171,11 @@ hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mas
 }
 
 // How the keys of a rows-mode problem are cut into chunks.  The chip holds 512 work-groups (two per CU) at head dimension
-// 128 and 768 at 64.  A tile takes a work-group about 1.9 us (64: 1.7 us) when the CUs are full and 1.1 us (1.0 us) alone; several chunks cost a write and a read of the state
-// (64 KB per column block and chunk at head dimension 128) and one more launch.  Every number of chunks up to 64 is priced with that
-// and the cheapest is taken.
+// 128 and 768 at 64.  A tile takes a work-group about 1.9 us (64: 1.7 us) when the CUs are full and 1.1 us (1.0 us) alone,
+// measured with one MFMA per V operand; several chunks cost a write and a read of the state (64 KB per column block and
+// chunk at head dimension 128) and one more launch.  Every number of chunks up to 64 is priced with that and the cheapest
+// is taken.  (Prices raised by the 1.3 that the second MFMA costs a full chip cut short prompts into more chunks: fourteen
+// prompts and batches level, one 20.7 -> 25.8 us.)
 void plan_rows(FlashArgs& a) {
   const int group = a.n_q_heads / a.n_kv_heads;
   a.n_col_blocks = (a.n_rows * group + 127) / 128;
