@@ -3,7 +3,7 @@
 //
 // Why rows have a kernel of their own: library attention takes a ragged causal window only as an explicit boolean mask,
 // and then multiplies, masks and soft-maxes the whole score matrix in float32 in memory.  1089 rows over 40001 keys with
-// 32/8 heads of 128 took 18.7 ms that way and take 1.03 ms + 0.03 ms (combine) here, 0.7 PFLOP/s of scores and P.V; 777 rows
+// 32/8 heads of 128 took 18.7 ms that way and take 0.97 ms + 0.03 ms (combine) here, 0.7 PFLOP/s of scores and P.V; 777 rows
 // over 777 keys took 403 us and take 22 us.  A left-padded batch of 3 x 2500 tokens with its boolean mask took 7.66 ms and
 // takes 0.22 ms: the mask is packed to bits once, and tiles in which no row of a work-group sees a key are not visited.
 // Probabilities keep the float32 precision they had there: each enters P.V as two 16-bit numbers.  That costs a second MFMA
