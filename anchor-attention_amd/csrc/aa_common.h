@@ -20,8 +20,14 @@ constexpr float kLog2e = 1.44269504f;  // the literal the operator's definition 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
+// kProbLog2: where a probability p <= 1 is kept as two 16-bit numbers (its rounding and the rest), 2^kProbLog2 * p is formed
+// instead; the sums of probabilities carry the same factor and it cancels in the quotient.  fp16 needs it: p and its rest lie
+// on the grid of the subnormals, 2^-24, as soon as p is below 2^-14 - the keys that lose to an attention sink by ten
+// nats.  2^15 * p (at most 32768) puts the rest's grid at 2^-39 of the sum's scale: the pair is off by 2^-22 of p down to
+// p = 2^-18, by 2^-16 down to 2^-24 (17 nats below the largest), by 2^-11, a result's own rounding, at 2^-29 (20 nats).
 struct Bf16 {
   typedef bf16x8 vec8;
+  static constexpr float kProbLog2 = 0.f;
   static __device__ __forceinline__ float lo(uint32_t u) { return __uint_as_float(u << 16); }
   static __device__ __forceinline__ float hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
   static __device__ __forceinline__ float from16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
@@ -43,6 +49,7 @@ struct Bf16 {
 
 struct F16 {
   typedef f16x8 vec8;
+  static constexpr float kProbLog2 = 15.f;
   static __device__ __forceinline__ float lo(uint32_t u) { return (float)(*reinterpret_cast<f16x2*>(&u))[0]; }
   static __device__ __forceinline__ float hi(uint32_t u) { return (float)(*reinterpret_cast<f16x2*>(&u))[1]; }
   static __device__ __forceinline__ float from16(uint16_t h) { return lo((uint32_t)h); }
@@ -78,6 +85,11 @@ struct F16 {
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+// 2^(x * scale + kProbLog2): a probability that is to be kept as two 16-bit numbers (bf16: without the addition of 0)
+template <typename T>
+__device__ __forceinline__ float prob_exp2(float x, float scale) {
+  return fast_exp2(T::kProbLog2 != 0.f ? __builtin_fmaf(x, scale, T::kProbLog2) : x * scale);
+}
 
 // Work-group barrier for LDS hand-over only: waits for this wave's LDS traffic, then synchronises.
 // Unlike __syncthreads() it does not wait for outstanding global loads, so prefetches issued before

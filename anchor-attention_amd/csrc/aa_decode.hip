@@ -9,7 +9,7 @@
 // (S^T = K Q^T with the scores scaled in float32, online soft-max, O^T += V^T P^T); the waves' states are merged
 // through LDS, the chunks' by decode_combine_kernel.
 //
-// (P enters the product as two 16-bit numbers, its rounding and the rest: the precision of float32 for 0.5 us.)
+// (P enters the product as two 16-bit numbers, its rounding and the rest, as in the rows mode: 0.5 us.)
 //
 // One row, 32/8 heads of 128, 33001 keys (135 MB): 26.3 us = 5.1 TB/s, the rate of a large copy, and 4.1 us for the merge.
 // The rows mode, which moves the state of 128 columns through its workspace, took 30.1 + 15.0 us; library attention, one
@@ -169,13 +169,13 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
         for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
       m_run = m_new;
     }
-    u32x4 pw[2], pw_rest[2];  // P^T and what its rounding left, both 16 bits wide: the sum has the precision of P in float32
+    u32x4 pw[2], pw_rest[2];  // P^T and what its rounding left, both 16 bits wide
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       float e[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        e[i] = fast_exp2((s[4 * c + i] - m_base) * scale);
+        e[i] = prob_exp2<T>(s[4 * c + i] - m_base, scale);
         l_run += e[i];
       }
       pw[c >> 1][2 * (c & 1) + 0] = T::pack(e[0], e[1]);

@@ -536,11 +536,12 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   }
   // (rows: maxima and scores are kept as raw dot products; the scale is applied to the difference, in float32)
 #define AA_EXP2(x) ((AA_ABLATE == 1 || AA_ABLATE == 2) ? (x) : fast_exp2(kAnyRows ? (x) * score_scale : (x)))
-  // p = exp2(s) for accumulator registers 4c .. 4c+3 of one half, summed and rounded into the P^T fragment words
+#define AA_PROB(x) (kAnyRows && AA_ABLATE != 1 && AA_ABLATE != 2 ? prob_exp2<T>(x, score_scale) : AA_EXP2(x))
+  // p = exp2(s) (rows: 2^kProbLog2 times that) for accumulator registers 4c .. 4c+3 of one half, summed and rounded into the P^T fragment words
 #define AA_EXP_CHUNK(sx, pw, sum, c)                                                 \
   {                                                                                  \
-    const float e0 = AA_EXP2(sx[4 * (c) + 0]), e1 = AA_EXP2(sx[4 * (c) + 1]);        \
-    const float e2 = AA_EXP2(sx[4 * (c) + 2]), e3 = AA_EXP2(sx[4 * (c) + 3]);        \
+    const float e0 = AA_PROB(sx[4 * (c) + 0]), e1 = AA_PROB(sx[4 * (c) + 1]);        \
+    const float e2 = AA_PROB(sx[4 * (c) + 2]), e3 = AA_PROB(sx[4 * (c) + 3]);        \
     if (AA_ABLATE != 2) { sum += e0; sum += e1; sum += e2; sum += e3; }              \
     pw[(c) >> 1][2 * ((c) & 1) + 0] = T::pack(e0, e1);                                 \
     pw[(c) >> 1][2 * ((c) & 1) + 1] = T::pack(e2, e3);                                 \
@@ -810,6 +811,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 #undef AA_MASK
 #undef AA_ROWMAX
 #undef AA_EXP2
+#undef AA_PROB
 #undef AA_EXP_CHUNK
 #undef AA_V_SRC
 #undef AA_V_FETCH

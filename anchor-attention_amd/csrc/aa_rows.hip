@@ -6,7 +6,8 @@
 // 32/8 heads of 128 took 18.7 ms that way and take 0.97 ms + 0.03 ms (combine) here, 0.7 PFLOP/s of scores and P.V; 777 rows
 // over 777 keys took 403 us and take 22 us.  A left-padded batch of 3 x 2500 tokens with its boolean mask took 7.66 ms and
 // takes 0.22 ms: the mask is packed to bits once, and tiles in which no row of a work-group sees a key are not visited.
-// Probabilities keep the float32 precision they had there: each enters P.V as two 16-bit numbers.  That costs a second MFMA
+// Probabilities were float32 there: each enters P.V as two 16-bit numbers (bf16: 16 bits of it; fp16: 22, formed with a
+// factor that keeps small ones off the subnormals' grid, see kProbLog2).  That costs a second MFMA
 // per V operand (with one: 0.80 ms, 20 us and 0.19 ms) and brings the error against float64 from up to 1.02 times that of
 // library attention to the same (1.460e-3, 1.468e-3 with one, padded 3 x 1000, bf16).
 #include "aa_common.h"

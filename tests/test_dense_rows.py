@@ -69,27 +69,81 @@ def test_dense_rows_against_float64(batch, hq, hkv, n_rows, offset, d, dtype):
     assert torch.equal(again, out)
 
 
+SINK_CASES = [(77, 1000, 128, False), (130, 63, 64, False), (129, 0, 128, True), (65, 0, 64, True), (1, 3000, 128, False), (2, 517, 64, False),
+              (1, 777, 128, True), (1, 901, 64, True)]  # rows, masked, decode and masked decode kernels
+
+
+def _as_kept(p, dtype, how):
+    """What is left of probabilities kept as one 16-bit number, as two, or as two formed as 2^15 p (fp16's subnormals)."""
+    factor = 2.0 ** 15 if how != "plain pair" and dtype == torch.float16 else 1.0
+    x = (p * factor).float()
+    hi = x.to(dtype).float()
+    return (hi if how == "one" else hi + (x - hi).to(dtype).float()).double() / factor
+
+
+def _sink_scores(gap, dtype):
+    """The number of nats in [gap, gap + 1), a multiple of 1/16, whose exp(-x) the poorer ways of keeping it hit worst."""
+    x = gap + torch.arange(16, dtype=torch.float64) / 16
+    p = torch.exp(-x)
+    worst = (_as_kept(p, dtype, "one") / p - 1).abs()
+    if dtype == torch.float16 and gap >= 10:
+        worst = torch.minimum(worst, (_as_kept(p, dtype, "plain pair") / p - 1).abs())
+    return float(x[worst.argmax()])
+
+
+def _sink_inputs(n_rows, n_keys, d, dtype, gap, device):
+    """An attention sink: key 0 with a value of 0, and all others ``gap`` nats below it with values of one sign, so that the
+    output is their sum and a probability's error shows in full.  Scores are exact (one product of whole sixteenths, scale 1/8)."""
+    g = torch.Generator().manual_seed(n_rows + n_keys + d)
+    q, k = torch.zeros(2, 4, n_rows, d, dtype=dtype), torch.zeros(2, 2, n_keys, d, dtype=dtype)
+    q[..., 0] = 8.0
+    k[:, :, 1:, 0] = -_sink_scores(gap, dtype)
+    v = (0.5 + torch.rand(2, 2, n_keys, d, generator=g)).to(dtype)
+    v[:, :, 0] = 0.0
+    keys, rows = torch.arange(n_keys), torch.arange(n_rows) + n_keys - n_rows
+    return [x.to(device) for x in (q, k, v, (keys[None, :] <= rows[:, None]).expand(2, -1, -1))]
+
+
+def _beyond_rounding(out, want, n_keys):
+    """How far ``out`` is past the bound: half a unit of the 16-bit result, and of the result 2^-16 for a probability kept as two
+    numbers (bf16: 2^-17, fp16: 2^-22) with its score's exponential, and n_keys * 2^-24 for the float32 sums."""
+    digits, smallest = (8, -133) if out.dtype == torch.bfloat16 else (11, -24)
+    exponent = torch.frexp(want)[1].double()
+    half_unit = 0.5 * torch.exp2((exponent - digits).clamp(min=smallest))
+    return (out.double() - want).abs() - half_unit - (2.0 ** -16 + n_keys * 2.0 ** -24) * want.abs()
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_rows,offset,d,masked", [
-    (77, 1000, 128, False), (130, 63, 64, False), (129, 0, 128, True), (65, 0, 64, True), (1, 3000, 128, False), (2, 517, 64, False),
-    (1, 777, 128, True),
-])
+@pytest.mark.parametrize("n_rows,offset,d,masked", SINK_CASES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_probabilities_keep_float32_precision(n_rows, offset, d, masked, dtype):
-    """Bound: a probability enters the second product as two 16-bit numbers, off by u^2 of itself; its score is a float32 sum
-    over d, off by at most d * 2^-24 * |q||k| * scale, and the probability by as much of itself; the result is rounded once."""
     from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
-    n_keys, scale = offset + n_rows, d ** -0.5
-    q, k, v = _qkv(2, 4, 2, n_rows, n_keys, d, dtype, 3 * n_rows + offset)
-    keys, rows = torch.arange(n_keys, device="cuda"), torch.arange(n_rows, device="cuda") + offset
-    keep = (keys[None, :] <= rows[:, None]).expand(2, -1, -1)
-    out = dense_rows_attention(q, k, v, mask=keep[:, None]) if masked else dense_rows_attention(q, k, v, offset)
-    want = _reference(q, k, v, scale, keep)
-    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-    score = d * 2.0 ** -24 * scale * float(q.double().norm(dim=-1).max() * k.double().norm(dim=-1).max())
-    bound = 1.05 * (u * want.abs() + (u * u + score) * v.double().abs().max())
-    err = (out.double() - want).abs()
-    assert bool((err <= bound).all()), float((err - bound).max())
+    n_keys = offset + n_rows
+    for gap in (1, 10, 12, 14):
+        q, k, v, keep = _sink_inputs(n_rows, n_keys, d, dtype, gap, "cuda")
+        how = {"mask": keep[:, None]} if masked else {"causal_offset": offset}
+        out = dense_rows_attention(q, k, v, sm_scale=0.125, **how)
+        past = _beyond_rounding(out, _reference(q, k, v, 0.125, keep), n_keys)
+        assert bool((past <= 0).all()), (gap, float(past.max()))
+
+
+@pytest.mark.parametrize("n_rows,offset,d,masked", SINK_CASES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_poorer_probabilities_are_seen(n_rows, offset, d, masked, dtype):
+    """The bound above lets two numbers pass and, on the same inputs, neither a single 16-bit number nor - fp16 - a pair whose
+    small members fall among the subnormals."""
+    n_keys = offset + n_rows
+    for gap in (1, 10, 12, 14):
+        q, k, v, keep = _sink_inputs(n_rows, n_keys, d, dtype, gap, "cpu")
+        s = torch.matmul(q.double(), k.double().repeat_interleave(2, 1).transpose(2, 3)) * 0.125
+        p = torch.exp(s.masked_fill(~keep[:, None], float("-inf")))
+        want = _reference(q, k, v, 0.125, keep)
+        fails = {}
+        for how in ("one", "pair", "plain pair"):
+            out = (torch.matmul(_as_kept(p, dtype, how), v.double().repeat_interleave(2, 1)) / p.sum(-1, keepdim=True)).to(dtype)
+            fails[how] = bool((_beyond_rounding(out, want, n_keys) > 0).any())
+        assert fails["one"] and not fails["pair"], (gap, fails)
+        assert fails["plain pair"] == (dtype == torch.float16 and gap >= 10), (gap, fails)
 
 
 def _mask(kind, batch, n_rows, n_keys):
