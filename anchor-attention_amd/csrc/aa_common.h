@@ -28,6 +28,7 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 struct Bf16 {
   typedef bf16x8 vec8;
   static constexpr float kProbLog2 = 0.f;
+  static constexpr uint16_t kExponent = 0x7f80;  // its bits, all of them set in infinities and NaN
   static __device__ __forceinline__ float lo(uint32_t u) { return __uint_as_float(u << 16); }
   static __device__ __forceinline__ float hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
   static __device__ __forceinline__ float from16(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
@@ -50,6 +51,7 @@ struct Bf16 {
 struct F16 {
   typedef f16x8 vec8;
   static constexpr float kProbLog2 = 15.f;
+  static constexpr uint16_t kExponent = 0x7c00;
   static __device__ __forceinline__ float lo(uint32_t u) { return (float)(*reinterpret_cast<f16x2*>(&u))[0]; }
   static __device__ __forceinline__ float hi(uint32_t u) { return (float)(*reinterpret_cast<f16x2*>(&u))[1]; }
   static __device__ __forceinline__ float from16(uint16_t h) { return lo((uint32_t)h); }

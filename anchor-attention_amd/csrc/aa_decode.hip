@@ -16,6 +16,7 @@
 // work-group per head, 1164 us.
 #include "aa_common.h"
 #include "aa_kernels.h"
+#include "aa_nonfinite.h"
 
 namespace aa {
 
@@ -199,6 +200,20 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
     t = t_next;
     t_next = t_after;
     slot ^= 1;
+  }
+
+  if (__builtin_expect(__any(holds_nan(acc) && !is_nan(l_run)), 0)) {
+    // V holds infinities or NaN: the wave's sums once more (see aa_nonfinite.h)
+    const float m_base = m_run == -INFINITY ? 0.f : m_run;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+    for (t = next_tile(wave - 4); t < n_tiles; t = next_tile(t)) {
+      const int key0 = key_lo + t * kDecTile, count = my_last_key + 1 - key0;
+      const uint32_t seen = MASKED ? tile_bits(t) : count >= 32 ? ~0u : count <= 0 ? 0u : (1u << count) - 1u;
+      exact_pv_tile<T, D>(acc, qreg, kbase, vbase, k_row, v_row, key0, key_hi, seen, m_base, scale, lane);
+    }
   }
 
   // ---- the four waves' states -> one -----------------------------------------------------------

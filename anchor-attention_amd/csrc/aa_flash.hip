@@ -42,6 +42,7 @@
 
 #include "aa_common.h"
 #include "aa_kernels.h"
+#include "aa_nonfinite.h"
 
 namespace aa {
 
@@ -817,6 +818,33 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 #undef AA_V_FETCH
 #undef AA_PV_MFMA
 #undef AA_FENCE
+
+  if (kAnyRows && __builtin_expect(__any(holds_nan(acc) && !is_nan(l_run)), 0)) {
+    // V holds infinities or NaN: the wave's sums once more (see aa_nonfinite.h)
+    const float m_base = m_run == -INFINITY ? 0.f : m_run;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+    for (int i = 0; i < 2 * n_tiles; ++i) {  // 32 keys at a time
+      int key0 = key_base + 32 * i;
+      uint32_t seen;
+      if (MODE == kMasked) {
+        const int32_t entry = __builtin_amdgcn_readfirstlane(sm.idx[i >> 1]);
+        const int tile = entry & (kMixedTile - 1);
+        key0 = tile * kBN + 32 * (i & 1);
+        seen = ~0u;
+        if (entry & kMixedTile) {
+          const char* w = reinterpret_cast<const char*>(p.mask_words + ((int64_t)b * p.n_rows * p.mask_words_per_row + tile));
+          seen = *reinterpret_cast<const uint32_t*>(w + mask_row_off + 4 * (i & 1));
+        }
+      } else {
+        const int count = my_last_key + 1 - key0;
+        seen = count >= 32 ? ~0u : count <= 0 ? 0u : (1u << count) - 1u;
+      }
+      exact_pv_tile<T, D>(acc, qreg, kbase, vbase, k_row_bytes, v_row_bytes, key0, p.n_ctx, seen, m_base, score_scale, lane);
+    }
+  }
 
   // ---- epilogue --------------------------------------------------------------------------------
   const float l_tot = l_run + xor32(l_run);

@@ -146,6 +146,53 @@ def test_poorer_probabilities_are_seen(n_rows, offset, d, masked, dtype):
         assert fails["plain pair"] == (dtype == torch.float16 and gap >= 10), (gap, fails)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,hq,hkv,n_rows,offset,d,masked", [
+    (1, 8, 2, 77, 9000, 128, False),   # chunks, a ragged last tile
+    (1, 4, 4, 150, 0, 64, False),      # one chunk
+    (2, 4, 2, 129, 0, 128, True), (1, 2, 1, 5, 67000, 64, True),
+    (1, 8, 2, 1, 3000, 128, False), (2, 8, 1, 4, 61, 64, False),
+    (2, 8, 2, 1, 777, 64, True), (1, 4, 4, 1, 2500, 128, True),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_values_that_are_not_finite(batch, hq, hkv, n_rows, offset, d, masked, dtype):
+    """A row that sees an infinite value gives that infinity, NaN for infinities of both signs and for NaN, in the columns of
+    these values and in no other.  (A row that does not see the key gives NaN there too or what it would without: 0 times
+    infinity is NaN where its tile is multiplied.)  A key that is NaN makes every row NaN that sees it."""
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
+    n_keys = offset + n_rows
+    q, k, v = _qkv(batch, hq, hkv, n_rows, n_keys, d, dtype, 7 * n_rows + offset)
+    q /= 4.0
+    inf, mid, last = float("inf"), n_keys // 2, n_keys - 1
+    spots = [(0, 1, inf), (mid, 3, -inf), (last, 5, inf), (mid, 40, inf), (last, 40, -inf), (mid, 41, float("nan")), (0, d - 1, -inf)]
+    for key, col, x in spots:
+        v[:, :, key, col] = x
+    rows, keys = torch.arange(n_rows, device="cuda") + offset, torch.arange(n_keys, device="cuda")
+    keep = (keys[None, :] <= rows[:, None]).expand(batch, -1, -1)
+    if masked:
+        keep = keep & ((keys % 5 != 3) | (keys == 0) | (keys == mid) | (keys == last))
+    how = {"mask": keep[:, None]} if masked else {"causal_offset": offset}
+    out = dense_rows_attention(q, k, v, **how).double()
+    finite = torch.where(v.isfinite(), v, torch.zeros_like(v))
+    want = _reference(q, k, finite, d ** -0.5, keep)
+    special = torch.zeros(batch, n_rows, d, dtype=torch.float64, device="cuda")
+    unseen = torch.zeros(batch, n_rows, d, dtype=torch.bool, device="cuda")
+    for key, col, x in spots:
+        special[:, :, col] += torch.where(keep[:, :, key], x, 0.0)
+        unseen[:, :, col] |= ~keep[:, :, key]
+    want = want + special[:, None]
+    same = (out == want) | (out.isnan() & want.isnan()) | (want.isfinite() & ((out - want).abs() <= 1.05 * 2.0 ** -7 * (6 + want.abs())))
+    assert bool((same | (out.isnan() & unseen[:, None])).all())
+    assert bool(out[..., :1].isfinite().all()) and bool((out[:, :, -1, 1] == inf).all()) and bool((out[:, :, -1, 5] == inf).all())
+    k[:, :, mid] = float("nan")
+    out = dense_rows_attention(q, k, finite, **how)
+    sees = keep[:, None, :, mid, None]
+    assert bool((out.isnan() == sees).all())
+    q[:, 1, 0] = float("nan")
+    out = dense_rows_attention(q, torch.nan_to_num(k), finite, **how)
+    assert bool(out[:, 1, 0].isnan().all()) and bool(out[:, 0].isfinite().all()) and bool(out[:, 1, 1:].isfinite().all())
+
+
 def _mask(kind, batch, n_rows, n_keys):
     rows, keys = torch.arange(n_rows, device="cuda") + max(n_keys - n_rows, 0), torch.arange(n_keys, device="cuda")
     causal = keys[None, :] <= rows[:, None]
