@@ -170,9 +170,9 @@ def _called_plainly() -> bool:
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0)
 
 
-def dense_rows_supported(Q, K, V, mask=None) -> bool:
+def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
     """Whether :func:`dense_rows_attention` takes these tensors (its kernels' types, head dimensions, alignment, sizes of
-    one launch and 32-bit addressing of one head)."""
+    one launch and 32-bit addressing of one head; all of them hold for ``out`` too, whose strides can be wider than ``Q``'s)."""
     if not (type(Q) is type(K) is type(V) is torch.Tensor and _called_plainly()):
         return False
     if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype and K.device == V.device == Q.device):
@@ -181,7 +181,7 @@ def dense_rows_supported(Q, K, V, mask=None) -> bool:
     if D not in (64, 128) or K.shape != V.shape or K.shape[3] != D or K.shape[0] != B or not B or not K.shape[1] or H % K.shape[1] or not H:
         return False
     n_keys = K.shape[2]
-    for t, rows in ((Q, N), (K, n_keys), (V, n_keys)):
+    for t, rows in ((Q, N), (K, n_keys), (V, n_keys), (Q if out is None else out, N)):
         sb, sh, sn, sd = t.stride()
         if sd != 1 or (sb | sh | sn) & 7 or t.data_ptr() & 15 or not D <= sn <= 1 << 14 or not 0 < rows <= 1 << 20 or rows * sn * 2 >= 1 << 32:
             return False

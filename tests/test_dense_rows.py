@@ -254,6 +254,22 @@ def test_own_kernels_are_left_out_of_transformed_and_traced_calls():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,n_rows,n_keys", [(160, 8, 1, 300), (136, 136, 40, 40), (128, 8, 1, 300)])
+def test_plug_with_an_output_too_wide_for_the_kernels(hq, hkv, n_rows, n_keys):
+    """The plug's output has rows of all heads, n_heads * D elements, also where the queries' rows are D apart (every one-token
+    step); beyond 16384 the kernels do not address them (the last case is the widest that they do)."""
+    import types
+
+    from anchor_attn.src.modules.llama.anchor_attention import anchor_attention_forward
+    q, k, v = _qkv(2, hq, hkv, n_rows, n_keys, 128, torch.bfloat16, hq)
+    module = types.SimpleNamespace(config=types.SimpleNamespace(block_size_M=128, step=16, theta=12.0))
+    out, _ = anchor_attention_forward(module, q.clone(memory_format=torch.contiguous_format), k, v, None, scaling=128 ** -0.5)
+    rows, keys = torch.arange(n_rows, device="cuda") + n_keys - n_rows, torch.arange(n_keys, device="cuda")
+    keep = (keys[None, :] <= rows[:, None]).expand(2, -1, -1)
+    _check(out.transpose(1, 2), _reference(q, k, v, 128 ** -0.5, keep), v, torch.bfloat16)
+
+
+@pytest.mark.gpu
 def test_calls_that_stay_with_library_attention():
     from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_supported
     q, k, v = _qkv(2, 4, 2, 1, 40, 64, torch.bfloat16, 1)
