@@ -163,11 +163,22 @@ def anchor_attn_test_time(Q, K, V, sm_scale: float = None, block_size: int = 128
     return output, search_time, compute_time
 
 
+def _function_modes():
+    """The ``TorchFunctionMode`` stack without ``torch.device(...)`` blocks, which only concern factory functions."""
+    return [m for m in torch.overrides._get_current_function_mode_stack() if type(m) is not torch.utils._device.DeviceContext]
+
+
 def _called_plainly() -> bool:
     """False while something other than eager execution watches the operations (vmap, forward-mode differentiation, tracing,
-    compilation, a dispatch mode): it would not see what happens behind the C interface."""
-    return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing() and torch._C._len_torch_dispatch_stack() == 0)
+    compilation, a dispatch or function mode): it would not see what happens behind the C interface.  The framework has no
+    public names for most of these; a release in which they have moved counts as watched."""
+    try:
+        return (not torch.compiler.is_compiling() and torch._C._functorch.peek_interpreter_stack() is None
+                and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing()
+                and torch._C._len_torch_dispatch_stack() == 0
+                and (torch._C._len_torch_function_stack() == 0 or not _function_modes()))
+    except AttributeError:
+        return False
 
 
 def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:

@@ -228,7 +228,7 @@ def test_masked_rows_against_float64(batch, hq, hkv, n_rows, n_keys, d, dtype, k
 
 
 def test_own_kernels_are_left_out_of_transformed_and_traced_calls():
-    """Their work is invisible to vmap, forward-mode differentiation, tracing and dispatch modes."""
+    """Their work is invisible to vmap, forward-mode differentiation, tracing, dispatch and function modes."""
     from torch.fx.experimental.proxy_tensor import make_fx
     from torch.utils.flop_counter import FlopCounterMode
 
@@ -249,8 +249,25 @@ def test_own_kernels_are_left_out_of_transformed_and_traced_calls():
     torch.jit.trace(probe, (x,), check_trace=False)
     with FlopCounterMode(display=False):
         probe(x)
-    assert len(seen) >= 6 and not any(seen)
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Watch():
+        probe(x)
+    with Watch(), torch.device("cpu"):
+        probe(x)
+    assert len(seen) >= 8 and not any(seen)
+    with torch.device("cpu"):  # (says where new tensors go, no more)
+        assert _called_plainly()
     assert _called_plainly()
+
+
+def test_own_kernels_are_left_out_where_the_framework_lacks_a_name(monkeypatch):
+    from anchor_attn.src.ops.anchor_attn_v4 import _called_plainly
+    assert _called_plainly()
+    monkeypatch.delattr(torch._C, "_len_torch_dispatch_stack")
+    assert not _called_plainly()
 
 
 @pytest.mark.gpu
