@@ -181,10 +181,16 @@ def _called_plainly() -> bool:
         return False
 
 
+def _no_backend_chosen() -> bool:
+    """Whether all of library attention's backends are allowed: who rules one out (``torch.nn.attention.sdpa_kernel``,
+    ``torch.backends.cuda.enable_*_sdp``) has chosen what computes the attention."""
+    return torch.backends.cuda.flash_sdp_enabled() and torch.backends.cuda.mem_efficient_sdp_enabled() and torch.backends.cuda.math_sdp_enabled()
+
+
 def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
     """Whether :func:`dense_rows_attention` takes these tensors (its kernels' types, head dimensions, alignment, sizes of
     one launch and 32-bit addressing of one head; all of them hold for ``out`` too, whose strides can be wider than ``Q``'s)."""
-    if not (type(Q) is type(K) is type(V) is torch.Tensor and _called_plainly()):
+    if not (type(Q) is type(K) is type(V) is torch.Tensor and _called_plainly() and _no_backend_chosen()):
         return False
     if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype and K.device == V.device == Q.device):
         return False

@@ -263,6 +263,36 @@ def test_own_kernels_are_left_out_of_transformed_and_traced_calls():
     assert _called_plainly()
 
 
+def _spy_on_library_attention(monkeypatch):
+    from anchor_attn.src.modules.llama import anchor_attention
+    calls, library = [], torch.nn.functional.scaled_dot_product_attention
+    monkeypatch.setattr(anchor_attention.F, "scaled_dot_product_attention", lambda *a, **kw: calls.append(a[0].dtype) or library(*a, **kw))
+    return calls
+
+
+def _plug(q, k, v, mask=None, scaling=0.125):
+    import types
+
+    from anchor_attn.src.modules.llama.anchor_attention import anchor_attention_forward
+    module = types.SimpleNamespace(config=types.SimpleNamespace(block_size_M=128, step=16, theta=12.0))
+    return anchor_attention_forward(module, q, k, v, mask, scaling=scaling)[0].transpose(1, 2)
+
+
+@pytest.mark.gpu
+def test_a_chosen_backend_of_library_attention_is_used(monkeypatch):
+    from torch.nn.attention import SDPBackend, sdpa_kernel
+    calls = _spy_on_library_attention(monkeypatch)
+    q, k, v = _qkv(1, 4, 2, 5, 40, 64, torch.bfloat16, 1)
+    own = _plug(q, k, v)
+    assert not calls
+    with sdpa_kernel(SDPBackend.MATH):
+        got = _plug(q, k, v)
+    assert len(calls) == 1
+    _check(got, own.double(), 2 * v, torch.bfloat16)
+    _plug(q, k, v)
+    assert len(calls) == 1
+
+
 def test_own_kernels_are_left_out_where_the_framework_lacks_a_name(monkeypatch):
     from anchor_attn.src.ops.anchor_attn_v4 import _called_plainly
     assert _called_plainly()
@@ -275,15 +305,11 @@ def test_own_kernels_are_left_out_where_the_framework_lacks_a_name(monkeypatch):
 def test_plug_with_an_output_too_wide_for_the_kernels(hq, hkv, n_rows, n_keys):
     """The plug's output has rows of all heads, n_heads * D elements, also where the queries' rows are D apart (every one-token
     step); beyond 16384 the kernels do not address them (the last case is the widest that they do)."""
-    import types
-
-    from anchor_attn.src.modules.llama.anchor_attention import anchor_attention_forward
     q, k, v = _qkv(2, hq, hkv, n_rows, n_keys, 128, torch.bfloat16, hq)
-    module = types.SimpleNamespace(config=types.SimpleNamespace(block_size_M=128, step=16, theta=12.0))
-    out, _ = anchor_attention_forward(module, q.clone(memory_format=torch.contiguous_format), k, v, None, scaling=128 ** -0.5)
+    out = _plug(q.clone(memory_format=torch.contiguous_format), k, v, scaling=128 ** -0.5)
     rows, keys = torch.arange(n_rows, device="cuda") + n_keys - n_rows, torch.arange(n_keys, device="cuda")
     keep = (keys[None, :] <= rows[:, None]).expand(2, -1, -1)
-    _check(out.transpose(1, 2), _reference(q, k, v, 128 ** -0.5, keep), v, torch.bfloat16)
+    _check(out, _reference(q, k, v, 128 ** -0.5, keep), v, torch.bfloat16)
 
 
 @pytest.mark.gpu
