@@ -194,6 +194,8 @@ def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
         return False
     if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype and K.device == V.device == Q.device):
         return False
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != Q.dtype:  # (attention is computed in that type)
+        return False
     B, H, N, D = Q.shape
     if D not in (64, 128) or K.shape != V.shape or K.shape[3] != D or K.shape[0] != B or not B or not K.shape[1] or H % K.shape[1] or not H:
         return False

@@ -293,6 +293,18 @@ def test_a_chosen_backend_of_library_attention_is_used(monkeypatch):
     assert len(calls) == 1
 
 
+@pytest.mark.gpu
+def test_autocast_says_which_type_attention_is_computed_in(monkeypatch):
+    calls = _spy_on_library_attention(monkeypatch)
+    q, k, v = _qkv(1, 4, 2, 5, 40, 64, torch.bfloat16, 1)
+    with torch.autocast("cuda", torch.float16):
+        assert _plug(q, k, v).dtype == torch.bfloat16
+    assert len(calls) == 1
+    with torch.autocast("cuda", torch.bfloat16):
+        _plug(q, k, v)
+    assert len(calls) == 1
+
+
 def test_own_kernels_are_left_out_where_the_framework_lacks_a_name(monkeypatch):
     from anchor_attn.src.ops.anchor_attn_v4 import _called_plainly
     assert _called_plainly()
