@@ -44,7 +44,8 @@ def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[i
     wants_grad = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
     by_mask = attention_mask is not None and causal_offset is None
     by_offset = attention_mask is None and causal_offset is not None and causal_offset >= 0
-    if (by_mask or by_offset) and not wants_grad and (scaling is None or scaling > 0) and dense_rows_supported(query, key, value, attention_mask, out):
+    # (the own kernel scales raw scores in float32: by a positive number whose product with them neither vanishes nor overflows)
+    if (by_mask or by_offset) and not wants_grad and (scaling is None or 1e-30 < scaling < 1e30) and dense_rows_supported(query, key, value, attention_mask, out):
         return dense_rows_attention(query, key, value, causal_offset or 0, sm_scale=scaling, out=out, mask=attention_mask)
     mask = attention_mask
     if causal_offset is not None and mask is None and query.shape[2] > 1:

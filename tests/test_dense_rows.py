@@ -305,6 +305,17 @@ def test_autocast_says_which_type_attention_is_computed_in(monkeypatch):
     assert len(calls) == 1
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("scaling", [0.0, -0.125, 1e-46, 1e-40, 1e-20])
+def test_scales_beyond_the_kernels_range(scaling):
+    """0 and negative ones, and one that is 0 or not normal as a float32; the last is computed by the kernels.  The result but
+    for the negative one is the mean of the values that a row sees."""
+    q, k, v = _qkv(2, 4, 2, 5, 40, 64, torch.bfloat16, 1)
+    rows, keys = torch.arange(5, device="cuda") + 35, torch.arange(40, device="cuda")
+    keep = (keys[None, :] <= rows[:, None]).expand(2, -1, -1)
+    _check(_plug(q, k, v, scaling=scaling), _reference(q, k, v, scaling, keep), v, torch.bfloat16)
+
+
 def test_own_kernels_are_left_out_where_the_framework_lacks_a_name(monkeypatch):
     from anchor_attn.src.ops.anchor_attn_v4 import _called_plainly
     assert _called_plainly()
