@@ -19,7 +19,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn.functional as F
 
-from anchor_attn.src.ops.anchor_attn_v4 import (LOG2E, _anchor_attn, anchor_attn, dense_causal_attention, dense_rows_attention,
+from anchor_attn.src.ops.anchor_attn_v4 import (LOG2E, _anchor_attn, _dense_rows, anchor_attn, dense_causal_attention,
                                                 dense_rows_supported)
 
 ATTN_NAME = "anchor_attn"
@@ -46,7 +46,7 @@ def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[i
     by_offset = attention_mask is None and causal_offset is not None and causal_offset >= 0
     # (the own kernel scales raw scores in float32: by a positive number whose product with them neither vanishes nor overflows)
     if (by_mask or by_offset) and not wants_grad and (scaling is None or 1e-30 < scaling < 1e30) and dense_rows_supported(query, key, value, attention_mask, out):
-        return dense_rows_attention(query, key, value, causal_offset or 0, sm_scale=scaling, out=out, mask=attention_mask)
+        return _dense_rows(query, key, value, causal_offset or 0, scaling, out, attention_mask)
     mask = attention_mask
     if causal_offset is not None and mask is None and query.shape[2] > 1:
         rows = torch.arange(query.shape[2], device=query.device)[:, None] + causal_offset

@@ -187,20 +187,22 @@ def _no_backend_chosen() -> bool:
     return torch.backends.cuda.flash_sdp_enabled() and torch.backends.cuda.mem_efficient_sdp_enabled() and torch.backends.cuda.math_sdp_enabled()
 
 
-def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
-    """Whether :func:`dense_rows_attention` takes these tensors (its kernels' types, head dimensions, alignment, sizes of
-    one launch and 32-bit addressing of one head; all of them hold for ``out`` too, whose strides can be wider than ``Q``'s)."""
-    if not (type(Q) is type(K) is type(V) is torch.Tensor and _called_plainly() and _no_backend_chosen()):
-        return False
+def _rows_kernels_take(Q, K, V, mask=None, out=None) -> bool:
+    """The kernels' types, head dimensions, alignment, sizes of one launch and 32-bit addressing of one head; all of them hold
+    for ``out`` too, whose strides can be wider than ``Q``'s."""
     if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype and K.device == V.device == Q.device):
         return False
-    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != Q.dtype:  # (attention is computed in that type)
+    if not Q.dim() == K.dim() == V.dim() == 4:
         return False
     B, H, N, D = Q.shape
     if D not in (64, 128) or K.shape != V.shape or K.shape[3] != D or K.shape[0] != B or not B or not K.shape[1] or H % K.shape[1] or not H:
         return False
+    if out is None:
+        out = Q
+    elif out.shape != Q.shape or out.dtype != Q.dtype or out.device != Q.device:
+        return False
     n_keys = K.shape[2]
-    for t, rows in ((Q, N), (K, n_keys), (V, n_keys), (Q if out is None else out, N)):
+    for t, rows in ((Q, N), (K, n_keys), (V, n_keys), (out, N)):
         sb, sh, sn, sd = t.stride()
         if sd != 1 or (sb | sh | sn) & 7 or t.data_ptr() & 15 or not D <= sn <= 1 << 14 or not 0 < rows <= 1 << 20 or rows * sn * 2 >= 1 << 32:
             return False
@@ -217,17 +219,34 @@ def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
     return True
 
 
+def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
+    """Whether the attention of these tensors is to be computed by :func:`dense_rows_attention`: its kernels take them, and
+    nothing about the call asks for the framework's own operations."""
+    if not (type(Q) is type(K) is type(V) is torch.Tensor and _called_plainly() and _no_backend_chosen()):
+        return False
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != Q.dtype:  # (attention is computed in that type)
+        return False
+    return _rows_kernels_take(Q, K, V, mask, out)
+
+
 def dense_rows_attention(Q, K, V, causal_offset: int = 0, sm_scale: float = None, out: torch.Tensor = None, mask: torch.Tensor = None):
     """Attention of ``Q`` ``[B,H,n_rows,D]`` over ``K``/``V`` ``[B,H_kv,n_keys,D]`` on the same MFMA core: query row ``i``
     sees keys ``0 .. causal_offset + i``, or, with a boolean ``mask`` ``[B or 1, 1, n_rows, n_keys]``, the keys it is True for.
-    Any row and key count (:func:`dense_rows_supported` names the rest)."""
+    Any row and key count (:func:`_rows_kernels_take` names the rest)."""
+    if not _rows_kernels_take(Q, K, V, mask, out):
+        raise _hip.AnchorAttnHipError("dense_rows_attention: unsupported tensors (bf16 or fp16 on one GPU, head dimension 64 or 128, rows of at "
+                                      "most 16384 elements on 16-byte boundaries, a boolean mask [B or 1, 1, n_rows, n_keys], out like Q)")
+    return _dense_rows(Q, K, V, causal_offset, sm_scale, out, mask)
+
+
+def _dense_rows(Q, K, V, causal_offset, sm_scale, out, mask):
+    # (the tensors have been looked at: the launch trusts their shapes)
     B, H, N, D = Q.shape
     n_keys = K.shape[2]
     sm_scale = sm_scale if sm_scale else 1.0 / (D ** 0.5)
     output = torch.empty_like(Q) if out is None else out
     mask_args = (None, 0, 0)
     if mask is not None:
-        assert mask.dtype == torch.bool and mask.shape[0] in (1, B) and tuple(mask.shape[1:]) == (1, N, n_keys)
         mask = mask if mask.stride(3) == 1 else mask.contiguous()
         mask_args = (mask.data_ptr(), mask.stride(0) if mask.shape[0] > 1 else 0, mask.stride(2))
     lib = _hip.lib()

@@ -336,6 +336,22 @@ def test_plug_with_an_output_too_wide_for_the_kernels(hq, hkv, n_rows, n_keys):
 
 
 @pytest.mark.gpu
+def test_tensors_that_the_kernels_would_misread_are_refused():
+    """On the host, before anything is launched: nothing behind this call looks at shapes again."""
+    from anchor_attn.src.ops._hip import AnchorAttnHipError
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
+    q, k, v = _qkv(2, 4, 2, 3, 40, 64, torch.bfloat16, 1)
+    mask = torch.ones(2, 1, 3, 40, dtype=torch.bool, device="cuda")
+    dense_rows_attention(q, k, v, 37)
+    for bad in [dict(V=v[:, :, :39]), dict(K=k[:1], V=v[:1]), dict(K=k.half()), dict(K=k.cpu(), V=v.cpu()), dict(Q=q.cpu()), dict(Q=q[0]),
+                dict(K=k[..., :32], V=v[..., :32]), dict(out=torch.empty_like(q)[:, :, :2]), dict(out=torch.empty_like(q).half()),
+                dict(out=torch.empty_like(q).cpu()), dict(mask=mask[..., :39]), dict(mask=mask[:, :, :2]), dict(mask=mask.to(torch.uint8)),
+                dict(mask=mask.cpu()), dict(mask=mask.expand(2, 4, 3, 40))]:
+        with pytest.raises(AnchorAttnHipError, match="unsupported tensors"):
+            dense_rows_attention(**{"Q": q, "K": k, "V": v, "causal_offset": 37, **bad})
+
+
+@pytest.mark.gpu
 def test_calls_that_stay_with_library_attention():
     from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_supported
     q, k, v = _qkv(2, 4, 2, 1, 40, 64, torch.bfloat16, 1)
