@@ -79,6 +79,22 @@ int check_dims(const Dims& d, const char* who) {
   return AA_OK;
 }
 
+// What stage 2 asks beyond that: the score kernel numbers (query head of the KV group, big block) pairs with 16 bits and
+// addresses the pooled queries with 32-bit byte offsets.
+int check_select(const Dims& d, int geometry, const char* who) {
+  if (geometry != AA_GEOMETRY_AS_RUN && geometry != AA_GEOMETRY_INTENDED) {
+    set_error("%s: geometry %d is neither AA_GEOMETRY_AS_RUN nor AA_GEOMETRY_INTENDED", who, geometry);
+    return AA_EBADARG;
+  }
+  if ((int64_t)(d.n_q_heads / d.n_kv_heads) * (d.n_ctx / (d.block_size * d.step)) >= 65536 ||
+      (int64_t)d.batch * d.n_q_heads * (d.n_ctx / d.block_size) * 2 * d.head_dim > 0xffffffffLL) {
+    set_error("%s: too many (head, big block) pairs or pooled rows for one launch (heads per KV head %d, big blocks %d, pooled rows %lld)",
+              who, d.n_q_heads / d.n_kv_heads, d.n_ctx / (d.block_size * d.step), (long long)d.batch * d.n_q_heads * (d.n_ctx / d.block_size));
+    return AA_EUNSUPPORTED;
+  }
+  return AA_OK;
+}
+
 int check_tensor(const void* ptr, int64_t sb, int64_t sh, int64_t sn, int n_ctx, int head_dim, const char* who, const char* name) {
   if (ptr == nullptr) {
     set_error("%s: %s is NULL", who, name);
@@ -289,11 +305,8 @@ int aa_stage2_select(const void* qbar, const void* abar,
   const char* who = "aa_stage2_select";
   int rc;
   if ((rc = check_dtype(dtype, who))) return rc;
-  if (geometry != AA_GEOMETRY_AS_RUN && geometry != AA_GEOMETRY_INTENDED) {
-    set_error("%s: geometry %d is neither AA_GEOMETRY_AS_RUN nor AA_GEOMETRY_INTENDED", who, geometry);
-    return AA_EBADARG;
-  }
-  if ((rc = check_dims({batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step}, who))) return rc;
+  const Dims dims = {batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step};
+  if ((rc = check_dims(dims, who)) || (rc = check_select(dims, geometry, who))) return rc;
   if ((rc = check_tensor(k, k_sb, k_sh, k_sn, n_ctx, head_dim, who, "k"))) return rc;
   if ((rc = check_ptr(qbar, who, "qbar")) || (rc = check_ptr(abar, who, "abar")) || (rc = check_ptr(mask_ws, who, "mask_ws")) ||
       (rc = check_ptr(coords, who, "coords")) || (rc = check_ptr(counts, who, "counts")))
@@ -311,14 +324,6 @@ int aa_stage2_select(const void* qbar, const void* abar,
   a.dtype = dtype;
   a.key_lo = geometry == AA_GEOMETRY_AS_RUN ? block_size : block_size * step;
   a.key_slack = geometry == AA_GEOMETRY_AS_RUN ? block_size : 0;
-  // the score kernel numbers (query head of the KV group, big block) pairs with 16 bits and addresses the pooled
-  // queries with 32-bit byte offsets
-  if ((int64_t)(n_q_heads / n_kv_heads) * (n_ctx / (block_size * step)) >= 65536 ||
-      (int64_t)batch * n_q_heads * (n_ctx / block_size) * 2 * head_dim > 0xffffffffLL) {
-    set_error("%s: too many (head, big block) pairs or pooled rows for one launch (heads per KV head %d, big blocks %d, pooled rows %lld)",
-              who, n_q_heads / n_kv_heads, n_ctx / (block_size * step), (long long)batch * n_q_heads * (n_ctx / block_size));
-    return AA_EUNSUPPORTED;
-  }
   if (n_ctx > block_size * step) {  // (a single big block has no candidates: its counts are 0)
     if ((rc = check_launch(launch_select_thresholds(a, (hipStream_t)stream), who))) return rc;
     if ((rc = check_launch(launch_select_scores(a, (hipStream_t)stream), who))) return rc;
@@ -403,7 +408,9 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        int dtype, void* stream) {
   const char* who = "aa_anchor_attn_fwd";
   int rc;
-  if ((rc = check_dims({batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step}, who))) return rc;
+  // (all that a later stage could refuse is looked at first: stage 1 already writes the first big block's output)
+  const Dims dims = {batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step};
+  if ((rc = check_dims(dims, who)) || (rc = check_select(dims, geometry, who))) return rc;
   if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
   const Workspace w = carve(batch, n_q_heads, n_ctx, head_dim, block_size, step);
   if (workspace_bytes < w.total) {

@@ -79,6 +79,21 @@ def test_error_codes_without_touching_the_gpu():
     assert lib.aa_version() == 3
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="host pointers: the call must not get as far as a launch")
+def test_the_operator_refuses_before_its_first_launch():
+    """Stage 1 writes rows of the output, so a refusal by a later stage would leave them changed."""
+    lib = _hip.lib()
+    buf = ctypes.create_string_buffer(4096 + 64)
+    p = (ctypes.addressof(buf) + 63) & ~63
+
+    def call(hq, hkv, n, bs, geometry):
+        s = (n * 64 * hq, n * 64, 64)
+        return lib.aa_anchor_attn_fwd(p, *s, p, *s, p, *s, p, *s, p, 1 << 60, None, 1, hq, hkv, n, 64, bs, 16, 0.1, 12.0, 0, geometry, 0, None)
+
+    assert call(2, 2, 2048, 128, 7) == 1 and b"geometry" in lib.aa_last_error()
+    assert call(32, 1, 1 << 20, 16, 0) == 2 and b"pairs" in lib.aa_last_error()  # 32 x 4096 (head, big block) pairs
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_hip, "_lib", None)
     monkeypatch.setattr(_hip, "library_path", lambda: str(tmp_path / "nope.so"))
