@@ -207,7 +207,8 @@ def _rows_kernels_take(Q, K, V, mask=None, out=None) -> bool:
         if sd != 1 or (sb | sh | sn) & 7 or t.data_ptr() & 15 or not D <= sn <= 1 << 14 or not 0 < rows <= 1 << 20 or rows * sn * 2 >= 1 << 32:
             return False
     col_blocks = (N * (H // K.shape[1]) + 127) // 128
-    if B * K.shape[1] * col_blocks * 64 >= 1 << 31:
+    # (that many column blocks are one chunk each; but a decode step's chunk holds 2^13 keys, a masked one 2^16)
+    if B * K.shape[1] * col_blocks * (1 if col_blocks > 1 and mask is None else (n_keys >> 13) + 1) >= 1 << 24:
         return False
     if mask is not None:
         if type(mask) is not torch.Tensor or mask.device != Q.device or mask.dtype != torch.bool or mask.dim() != 4:

@@ -511,8 +511,9 @@ static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_hea
     return AA_EUNSUPPORTED;
   }
   const int64_t col_blocks = ((int64_t)n_rows * (n_q_heads / n_kv_heads) + 127) / 128;
-  // (up to 64 chunks of every column block in one launch; the mask kernel counts column blocks and batch in its grid's y and z, and a row's packed mask has a 32-bit byte offset)
-  if (col_blocks > 0x7fffff || (int64_t)batch * n_kv_heads * col_blocks * 64 > 0x7fffffffLL || (masked && (col_blocks > 65535 || batch > 65535 || (int64_t)n_rows * ((n_keys + 63) / 64) * 8 > 0xffffffffLL))) {
+  // (the mask kernel counts column blocks and batch in its grid's y and z, and a row's packed mask has a 32-bit byte offset)
+  const int64_t blocks = (int64_t)batch * n_kv_heads * col_blocks;
+  if (blocks > 0xffffff || (masked && (col_blocks > 65535 || batch > 65535 || (int64_t)n_rows * ((n_keys + 63) / 64) * 8 > 0xffffffffLL))) {
     set_error("%s: problem too large for one launch", who);
     return AA_EUNSUPPORTED;
   }
@@ -525,6 +526,11 @@ static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_hea
     plan_decode(a);
   } else {
     plan_rows(a);
+  }
+  // (a launch takes less than 2^32 threads, 256 to a column block and chunk)
+  if (blocks * a.n_chunks > 0xffffff) {
+    set_error("%s: problem too large for one launch", who);
+    return AA_EUNSUPPORTED;
   }
   return AA_OK;
 }

@@ -94,6 +94,22 @@ def test_the_operator_refuses_before_its_first_launch():
     assert call(32, 1, 1 << 20, 16, 0) == 2 and b"pairs" in lib.aa_last_error()  # 32 x 4096 (head, big block) pairs
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="host pointers: the call must not get as far as a launch")
+def test_dense_rows_refuse_more_work_groups_than_a_launch_takes():
+    """2^24 work-groups of 256 threads."""
+    lib = _hip.lib()
+    buf = ctypes.create_string_buffer(4096 + 64)
+    p = (ctypes.addressof(buf) + 63) & ~63
+
+    def call(batch, rows, keys):
+        s = (0, 0, 64)
+        return lib.aa_dense_rows_fwd(p, *s, p, *s, p, *s, p, *s, None, 0, 0, p, 1 << 60, batch, 1, 1, rows, keys, 64, 0, 0.1, 0, None)
+
+    for batch, rows, keys in [(1 << 24, 1, 8), (1 << 20, 2048, 8), (1 << 22, 1, 40000)]:
+        assert call(batch, rows, keys) == 2 and b"too large" in lib.aa_last_error()
+    assert lib.aa_dense_rows_workspace_bytes(1 << 20, 1, 1, 1, 9000, 64, 0, 0) > 0  # (two chunks)
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_hip, "_lib", None)
     monkeypatch.setattr(_hip, "library_path", lambda: str(tmp_path / "nope.so"))

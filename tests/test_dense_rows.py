@@ -357,6 +357,9 @@ def test_calls_that_stay_with_library_attention():
     q, k, v = _qkv(2, 4, 2, 1, 40, 64, torch.bfloat16, 1)
     assert dense_rows_supported(q, k, v)
     assert not dense_rows_supported(q[:0], k[:0], v[:0])  # an empty batch
+    many = [x[:1, :2].expand(1 << 23, -1, -1, -1) for x in (q, k, v)]
+    assert not dense_rows_supported(*many)  # more work-groups than a launch takes
+    assert dense_rows_supported(*[x[1:] for x in many])
     mask = torch.ones(2, 1, 1, 40, dtype=torch.bool, device="cuda")
     assert dense_rows_supported(q, k, v, mask)
     assert not dense_rows_supported(q, k, v, mask.cpu()) and not dense_rows_supported(q, k.cpu(), v.cpu())
