@@ -2,9 +2,10 @@
 // group) columns per KV head.
 //
 // Bound by reading K and V once.  The keys of a (batch, KV head) unit are cut into chunks, one work-group each, so that
-// about one work-group per CU is at work; inside a work-group each of the four waves streams its own 32-key tiles (tile
-// t of the chunk to wave t % 4) through two private LDS slots filled by LDS-DMA, with no barrier until the end: a wave
-// waits for its own loads only, and a CU has up to 128 KB in flight (head dimension 128).  All heads of a group are columns
+// about one work-group per CU is at work; inside a work-group each of the four waves (or the only one: many units with short
+// caches) streams its own 32-key tiles (tile t of the chunk to wave t % 4) through two private LDS slots filled by LDS-DMA,
+// with no barrier until the end: a wave waits for its own loads only, and a CU has up to 128 KB in flight (head dimension
+// 128).  All heads of a group are columns
 // of the same products, so K and V are read once per KV head.  The arithmetic is that of the flash kernel's rows mode
 // (S^T = K Q^T with the scores scaled in float32, online soft-max, O^T += V^T P^T); the waves' states are merged
 // through LDS, the chunks' by decode_combine_kernel.
@@ -29,8 +30,8 @@ constexpr int kDecCols = 32;       // columns of a unit: query rows x heads of t
 constexpr int kDecTile = 32;       // keys a wave takes at a time
 constexpr int kDecMaxChunk = 8192; // keys of a chunk (masked: the chunk's mask bits live in LDS)
 
-template <typename T, int D, bool MASKED>
-__global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
+template <typename T, int D, bool MASKED, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) decode_kernel(const FlashArgs p) {
   typedef typename T::vec8 vec8;
   typedef __attribute__((address_space(3))) vec8 lds_vec8;
   constexpr int kKS = D / 16, kDB = D / 32;
@@ -40,9 +41,12 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
   constexpr int kLoads = kDecTile / kRowsPerLoad; // load instructions of a K (or V) tile
   constexpr int kTile = kDecTile * kPitch;        // bytes of a K (or V) tile
   constexpr int kAccPitch = D + 4;                // floats of a column's accumulator when the waves are merged
-  static_assert(4 * kDecCols * kAccPitch * 4 <= 16 * kTile, "the waves' accumulators fit where their tiles were");
-  __shared__ __attribute__((aligned(16))) char tiles[4][2][2][kTile];  // wave, slot, K/V
-  __shared__ float stats[2][4][kDecCols];
+  static_assert(kDecCols * kAccPitch * 4 <= 4 * kTile, "the waves' accumulators fit where their tiles were");
+  // tiles by wave, slot and K/V.  (A single wave with a single tile is given one slot, see launch_decode_for)
+  __shared__ __attribute__((aligned(16))) char fixed[WAVES > 1 ? WAVES * 4 * kTile : 16];
+  extern __shared__ __attribute__((aligned(16))) char sized[];
+  char* const tiles = WAVES > 1 ? fixed : sized;
+  __shared__ float stats[2][WAVES][kDecCols];
   __shared__ uint64_t seen[MASKED ? kDecMaxChunk / 64 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, c32 = lane & 31;
@@ -64,7 +68,7 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
     const int key0 = key_lo + t * kDecTile, left = key_hi - key0;
     const char* kb = kbase + (uint64_t)(uint32_t)key0 * k_row;
     const char* vb = vbase + (uint64_t)(uint32_t)key0 * v_row;
-    const uint32_t dst = lds_addr(tiles[wave][slot][0]);
+    const uint32_t dst = lds_addr(tiles) + (2 * wave + slot) * (2 * kTile);
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const int row = j * kRowsPerLoad + lane / kChunks;
@@ -81,7 +85,7 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
 
   if (MASKED) {  // the chunk's mask bits, 64 keys to a word (a single row: the same for every column)
     const uint8_t* m = p.mask_bytes + b * p.mask_sb + key_lo;
-    for (int i = 64 * wave; i < key_hi - key_lo; i += 256) {
+    for (int i = 64 * wave; i < key_hi - key_lo; i += 64 * WAVES) {
       const uint64_t w = __ballot(i + lane < key_hi - key_lo && m[i + lane] != 0);
       if (lane == 0) seen[i / 64] = w;
     }
@@ -91,11 +95,11 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
     return MASKED ? (uint32_t)(__builtin_amdgcn_readfirstlane(reinterpret_cast<const uint32_t*>(seen)[t])) : ~0u;
   };
   auto next_tile = [&](int t) {  // this wave's next tile in which a key is seen
-    for (t += 4; MASKED && t < n_tiles && tile_bits(t) == 0u;) t += 4;
+    for (t += WAVES; MASKED && t < n_tiles && tile_bits(t) == 0u;) t += WAVES;
     return t;
   };
 
-  int t = next_tile(wave - 4), t_next = n_tiles;
+  int t = next_tile(wave - WAVES), t_next = n_tiles;
   if (t < n_tiles) {
     issue(t, 0);
     t_next = next_tile(t);
@@ -120,7 +124,7 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
 
   // LDS offsets inside a tile, as in the flash kernel: K row c32, chunk 2*ks + half; V by transposing reads
-  const uint32_t tile0 = lds_addr(tiles[wave][0][0]);
+  const uint32_t tile0 = lds_addr(tiles) + wave * (4 * kTile);
   uint32_t k_rd[kKS], v_rd[kDB];
 #pragma unroll
   for (int ks = 0; ks < kKS; ++ks) k_rd[ks] = tile0 + c32 * kPitch + 16 * k_slot(c32, 2 * ks + half);
@@ -209,21 +213,21 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
-    for (t = next_tile(wave - 4); t < n_tiles; t = next_tile(t)) {
+    for (t = next_tile(wave - WAVES); t < n_tiles; t = next_tile(t)) {
       const int key0 = key_lo + t * kDecTile, count = my_last_key + 1 - key0;
       const uint32_t seen = MASKED ? tile_bits(t) : count >= 32 ? ~0u : count <= 0 ? 0u : (1u << count) - 1u;
       exact_pv_tile<T, D>(acc, qreg, kbase, vbase, k_row, v_row, key0, key_hi, seen, m_base, scale, lane);
     }
   }
 
-  // ---- the four waves' states -> one -----------------------------------------------------------
+  // ---- the waves' states -> one ------------------------------------------------------------------
   const float l_tot = l_run + xor32(l_run);
   if (half == 0) {
     stats[0][wave][c32] = m_run;
     stats[1][wave][c32] = l_tot;
   }
   __syncthreads();  // (everyone is done with the tiles: the accumulators take their place)
-  float* accs = reinterpret_cast<float*>(&tiles[0][0][0][0]);
+  float* accs = reinterpret_cast<float*>(tiles);
   if (c32 < n_cols) {
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
@@ -236,15 +240,15 @@ __global__ void __launch_bounds__(256) decode_kernel(const FlashArgs p) {
       }
   }
   __syncthreads();
-  for (int i = tid; i < n_cols * (D / 4); i += 256) {
+  for (int i = tid; i < n_cols * (D / 4); i += 64 * WAVES) {
     const int col = i / (D / 4), d = 4 * (i % (D / 4));
     float m = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) m = fmaxf(m, stats[0][w][col]);
+    for (int w = 0; w < WAVES; ++w) m = fmaxf(m, stats[0][w][col]);
     float l = 0.f;
     floatx4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const float mw = stats[0][w][col];
       const float f = mw == -INFINITY ? 0.f : fast_exp2((mw - m) * scale);
       l += f * stats[1][w][col];
@@ -326,26 +330,43 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const FlashArgs p) 
 bool decode_takes(int n_rows, int group, bool masked) { return n_rows * (int64_t)group <= kDecCols && (!masked || n_rows == 1); }
 
 // One work-group per CU (256; head dimension 64, whose tiles are half as large: two) as far as the units allow, each with
-// at least 256 keys - a wave's two tiles - since below that the merge costs more than the reading.
+// at least 256 keys - a wave's two tiles - and one up to 640 keys, below which the merge costs more than the reading (8 to 64 units: 384
+// keys 8.2 us against 10.1 in two chunks, 512 9.6 against 10.5, 640 10.8 against 11.5, 768 12.0 against 11.3 in three).
+//
+// A work-group is four waves, whose tiles fill a CU's LDS, or a single one.  Four leave the CU to one unit, most of whose time goes
+// by in starting, waiting for the first tile and merging, as soon as the units outnumber the CUs; of the single waves five (64:
+// ten; nine and eighteen where there is one tile) share it.  8192 units of head dimension 128, one head each: 32 keys 118 us
+// with four waves and 26 with one (library attention, which took such steps before: 72, and 16 keys 121, 22 and 19), 128 keys 159 and 98, 512 391 and
+// 385, 1024 711 and 726; of 64: 32 keys 44 and 15, 192 79 and 75, 256 95 and 100.  256 units of 128: 64 keys 5.3 and 6.1, 32 keys 5.3 and 4.8.
 void plan_decode(FlashArgs& a) {
   const int units = a.batch * a.n_kv_heads, slots = a.head_dim == 128 ? 256 : 512;
   int n = slots / units;
   n = n > (a.n_ctx + 255) / 256 ? (a.n_ctx + 255) / 256 : n;
   n = n > kDecMaxChunks ? kDecMaxChunks : n;
+  if (a.n_ctx <= 640) n = 1;
   const int least = (a.n_ctx + kDecMaxChunk - 1) / kDecMaxChunk;
   n = n < least ? least : n;
   const int tiles = (a.n_ctx + kDecTile - 1) / kDecTile;
   a.chunk_tiles = (tiles + n - 1) / n;
   a.n_chunks = (tiles + a.chunk_tiles - 1) / a.chunk_tiles;
   a.n_col_blocks = 1;
+  a.decode_waves = tiles == 1 || (units > slots && a.n_ctx <= (a.head_dim == 128 ? 512 : 192)) ? 1 : 4;
 }
 
 template <typename T, int D>
 static void launch_decode_for(const FlashArgs& a, hipStream_t stream) {
   const int units = a.batch * a.n_kv_heads, group = a.n_q_heads / a.n_kv_heads;
   const dim3 grid((uint32_t)units * a.n_chunks), block(256);
-  if (a.mask_bytes) hipLaunchKernelGGL((decode_kernel<T, D, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((decode_kernel<T, D, false>), grid, block, 0, stream, a);
+  if (a.decode_waves == 1) {
+    // LDS for one tile where there is one (at least what the accumulators take): nine work-groups on a CU instead of five
+    const int tile = kDecTile * 2 * D, accs = kDecCols * (D + 4) * 4;
+    const size_t lds = a.n_ctx > kDecTile ? 4 * tile : 2 * tile > accs ? 2 * tile : accs;
+    if (a.mask_bytes) hipLaunchKernelGGL((decode_kernel<T, D, true, 1>), grid, dim3(64), lds, stream, a);
+    else hipLaunchKernelGGL((decode_kernel<T, D, false, 1>), grid, dim3(64), lds, stream, a);
+  } else {
+    if (a.mask_bytes) hipLaunchKernelGGL((decode_kernel<T, D, true, 4>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((decode_kernel<T, D, false, 4>), grid, block, 0, stream, a);
+  }
   if (a.n_chunks > 1) hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((uint32_t)units * a.n_rows * group), block, 0, stream, a);
 }
 

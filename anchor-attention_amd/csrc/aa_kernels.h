@@ -29,6 +29,7 @@ struct FlashArgs {
   // [batch, n_rows, mask_words_per_row] (bit j of word t: key 64 t + j), and what each tile of each column block holds,
   // tile_flags [batch, n_col_blocks, mask_words_per_row]: 0 nothing visible, 1 some, 2 every key to every row
   const uint64_t* mask_words; const uint8_t* tile_flags; int mask_words_per_row;
+  int decode_waves;  // decode kernel: waves of a work-group, 4 or 1
   // decode kernel with a mask (one query row): the byte mask itself
   const uint8_t* mask_bytes; int64_t mask_sb;
   int dtype;            // AA_DTYPE_BF16 / AA_DTYPE_F16: what the 16-bit elements of q, k, v, out, qbar, abar are

@@ -50,7 +50,14 @@ def _qkv(batch, hq, hkv, n_rows, n_keys, d, dtype, seed):
     (3, 14, 2, 1, 0, 64, torch.float16),          # one key
     (2, 8, 1, 4, 61, 128, torch.float16),         # all 32 columns, rows that end in the same tile
     (5, 4, 4, 3, 1021, 64, torch.bfloat16),       # no groups
-    (40, 16, 8, 1, 300, 128, torch.bfloat16),     # more units than CUs: one chunk, written without a merge
+    (40, 16, 8, 1, 300, 128, torch.bfloat16),     # more units than CUs: one wave to a unit, written without a merge
+    (40, 32, 16, 2, 190, 64, torch.float16),      # the same, two rows
+    (40, 16, 8, 1, 512, 128, torch.float16),      # and its largest cache; one key more and four waves share a unit
+    (40, 16, 8, 1, 513, 128, torch.float16),      # (513 + 1 keys: the last tile holds two)
+    (300, 2, 1, 1, 31, 128, torch.bfloat16),      # a single full tile
+    (300, 2, 1, 1, 32, 128, torch.bfloat16),      # and a second one of one key
+    (2, 8, 2, 1, 639, 128, torch.bfloat16),       # the most keys of a single chunk
+    (2, 8, 2, 1, 640, 64, torch.bfloat16),        # and the fewest of several
     (1, 4, 4, 9, 500, 64, torch.bfloat16),        # nine columns
     (1, 33, 1, 1, 700, 64, torch.bfloat16),       # one column too many for it
 ])
@@ -153,6 +160,7 @@ def test_poorer_probabilities_are_seen(n_rows, offset, d, masked, dtype):
     (2, 4, 2, 129, 0, 128, True), (1, 2, 1, 5, 67000, 64, True),
     (1, 8, 2, 1, 3000, 128, False), (2, 8, 1, 4, 61, 64, False),
     (2, 8, 2, 1, 777, 64, True), (1, 4, 4, 1, 2500, 128, True),
+    (40, 8, 8, 1, 70, 128, False), (80, 8, 8, 1, 27, 64, True),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_values_that_are_not_finite(batch, hq, hkv, n_rows, offset, d, masked, dtype):
@@ -217,6 +225,8 @@ def _mask(kind, batch, n_rows, n_keys):
     (2, 3, 1, 30, 1023, 64, torch.bfloat16, "padded"),   # a ragged end of one work-group's keys
     (4, 28, 4, 1, 2501, 128, torch.bfloat16, "padded"),  # a padded batch's decode step: tiles that are skipped
     (1, 2, 2, 1, 9000, 64, torch.float16, "random"),
+    (40, 16, 8, 1, 70, 128, torch.float16, "padded"),    # one wave to a unit; prompts of a few keys, one of none
+    (80, 8, 8, 1, 25, 64, torch.bfloat16, "random"),
     (40, 16, 8, 1, 8193, 64, torch.bfloat16, "window"),  # a second chunk of one key, since the first may hold no more
 ])
 def test_masked_rows_against_float64(batch, hq, hkv, n_rows, n_keys, d, dtype, kind):
