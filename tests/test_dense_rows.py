@@ -326,6 +326,19 @@ def test_scales_beyond_the_kernels_range(scaling):
     _check(_plug(q, k, v, scaling=scaling), _reference(q, k, v, scaling, keep), v, torch.bfloat16)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,hq,hkv,n,library", [(65, 32, 32, 31, True), (64, 32, 32, 31, False), (65, 32, 32, 32, False), (65, 32, 16, 31, False)])
+def test_many_padded_prompts_of_a_few_tokens(monkeypatch, batch, hq, hkv, n, library):
+    calls = _spy_on_library_attention(monkeypatch)
+    q, k, v = _qkv(batch, hq, hkv, n, n, 64, torch.bfloat16, n)
+    pads, pos = torch.arange(batch, device="cuda") % (n // 2), torch.arange(n, device="cuda")
+    mask = (pos[None, None, :] >= pads[:, None, None]) & (pos[None, None, :] <= pos[None, :, None])
+    got = _plug(q, k, v, mask[:, None])
+    assert bool(calls) == library
+    rows = mask.any(-1)[:, None, :, None]  # (what a row that sees nothing gives is not looked at here)
+    _check(torch.where(rows, got, 0.0), _reference(q, k, v, 0.125, mask), v, torch.bfloat16)
+
+
 def test_own_kernels_are_left_out_where_the_framework_lacks_a_name(monkeypatch):
     from anchor_attn.src.ops.anchor_attn_v4 import _called_plainly
     assert _called_plainly()
