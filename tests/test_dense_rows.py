@@ -207,6 +207,8 @@ def _mask(kind, batch, n_rows, n_keys):
     if kind == "padded":  # left-padded prompts: whole tiles nobody sees, rows without any key
         pads = torch.tensor([(37 * b) % n_keys + 70 * b for b in range(batch)], device="cuda")
         return (causal[None] & (keys[None, None, :] >= pads[:, None, None]))[:, None]
+    if kind == "causal":
+        return causal[None, None]
     if kind == "window":  # one mask for the whole batch
         return (causal & (keys[None, :] > rows[:, None] - 100))[None, None]
     g = torch.Generator(device="cuda").manual_seed(n_keys)
@@ -271,6 +273,108 @@ def test_own_kernels_are_left_out_of_transformed_and_traced_calls():
     with torch.device("cpu"):  # (says where new tensors go, no more)
         assert _called_plainly()
     assert _called_plainly()
+
+
+def _layouts(q, k, v):
+    """The same keys and values in other storage: [B,N,H,D], slices of a longer and wider cache, rows of different pitch."""
+    batch, hkv, n_keys, d = k.shape
+    yield "as they are", q, k, v
+    yield "B,N,H,D", q, *[x.transpose(1, 2).contiguous().transpose(1, 2) for x in (k, v)]
+    cache = torch.full((2, batch + 1, hkv + 1, n_keys + 77, d), float("nan"), dtype=k.dtype, device=k.device)
+    cache[0, 1:, 1:, 5:5 + n_keys], cache[1, 1:, 1:, 5:5 + n_keys] = k, v
+    yield "a sliced cache", q, cache[0, 1:, 1:, 5:5 + n_keys], cache[1, 1:, 1:, 5:5 + n_keys]
+    wide = torch.full((batch, n_keys, hkv, 3 * d), float("nan"), dtype=k.dtype, device=k.device)
+    wide[..., d:2 * d] = k.transpose(1, 2)
+    yield "different pitches", q, wide[..., d:2 * d].transpose(1, 2), v.transpose(1, 2).contiguous().transpose(1, 2)
+    packed = torch.full((batch, q.shape[2], q.shape[1], 2 * d), float("nan"), dtype=q.dtype, device=q.device)
+    packed[..., d:] = q.transpose(1, 2)
+    yield "queries of a packed projection", packed[..., d:].transpose(1, 2), k, v
+
+
+KERNELS = [(2, 8, 2, 77, 1300, 128, False), (1, 4, 4, 130, 130, 64, False), (2, 8, 2, 129, 1301, 64, True), (2, 6, 2, 65, 65, 128, True),
+           (2, 8, 2, 1, 1301, 128, False), (40, 8, 8, 2, 90, 64, False), (2, 8, 2, 1, 1301, 64, True), (40, 8, 8, 1, 90, 128, True)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,hq,hkv,n_rows,n_keys,d,masked", KERNELS)
+def test_storage_of_keys_values_and_queries(batch, hq, hkv, n_rows, n_keys, d, masked):
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention, dense_rows_supported
+    mask = _mask("padded", batch, n_rows, n_keys) if masked else None
+    first = None
+    for name, q, k, v in _layouts(*_qkv(batch, hq, hkv, n_rows, n_keys, d, torch.bfloat16, n_keys)):
+        assert dense_rows_supported(q, k, v, mask), name
+        out = dense_rows_attention(q, k, v, n_keys - n_rows, mask=mask)
+        first = out if first is None else first
+        assert torch.equal(out, first), name
+    keep = mask[:, 0] if masked else _mask("causal", batch, n_rows, n_keys)[:, 0].expand(batch, -1, -1)
+    _check(first, _reference(q, k, v, d ** -0.5, keep), v, torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,hq,hkv,n_rows,n_keys,d,masked", [x for x in KERNELS if x[-1]])
+def test_storage_of_masks(batch, hq, hkv, n_rows, n_keys, d, masked):
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
+    q, k, v = _qkv(batch, hq, hkv, n_rows, n_keys, d, torch.bfloat16, n_keys)
+
+    def strided(mask):  # rows wider than the mask, from an odd byte on; last dimension not the fastest; every second byte
+        wide = torch.ones(batch, 1, n_rows, n_keys + 39, dtype=torch.bool, device="cuda")
+        wide[..., 3:3 + n_keys] = mask
+        return [wide[..., 3:3 + n_keys], mask.transpose(2, 3).contiguous().transpose(2, 3), torch.repeat_interleave(mask, 2, dim=3)[..., ::2]]
+
+    mask = _mask("padded", batch, n_rows, n_keys)
+    want = dense_rows_attention(q, k, v, mask=mask)
+    _check(want, _reference(q, k, v, d ** -0.5, mask[:, 0]), v, torch.bfloat16)
+    for m in strided(mask):
+        assert torch.equal(dense_rows_attention(q, k, v, mask=m), want)
+    # one row for all rows, one mask for the whole batch (strides of 0), and both
+    for m in (mask[:, :, -1:].expand(-1, -1, n_rows, -1), mask[:1].expand(batch, -1, -1, -1), mask[:1], mask[:1, :, -1:].expand(batch, -1, n_rows, -1)):
+        assert torch.equal(dense_rows_attention(q, k, v, mask=m), dense_rows_attention(q, k, v, mask=m.expand(batch, 1, n_rows, n_keys).clone()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,hq,hkv,n_rows,n_keys,d,masked", KERNELS)
+def test_rows_on_other_streams_in_graphs_and_from_another_device(monkeypatch, batch, hq, hkv, n_rows, n_keys, d, masked):
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
+    sets = [(*_qkv(batch, hq, hkv, n_rows, n_keys, d, torch.bfloat16, seed),
+             _mask(kind, batch, n_rows, n_keys).expand(batch, -1, -1, -1) if masked else None)
+            for seed, kind in ((1, "padded"), (2, "random"), (3, "window"))]
+    offset = n_keys - n_rows
+    eager = [dense_rows_attention(q, k, v, offset, mask=m) for q, k, v, m in sets]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for (q, k, v, m), want in zip(sets, eager):
+            assert torch.equal(dense_rows_attention(q, k, v, offset, mask=m), want)
+    torch.cuda.synchronize()
+    fixed = [x.clone() if x is not None else None for x in sets[0]]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = dense_rows_attention(*fixed[:3], offset, mask=fixed[3])
+    for i in (1, 2, 0, 1):  # every replay against the eager result, with eager work between
+        for dst, src in zip(fixed, sets[i]):
+            if dst is not None:
+                dst.copy_(src)
+        out.fill_(float("nan"))
+        graph.replay()
+        q, k, v, m = sets[(i + 1) % 3]
+        assert torch.equal(dense_rows_attention(q, k, v, offset, mask=m), eager[(i + 1) % 3])
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[i]), i
+    # with another device current than that of the tensors (a pipeline's later layers): pretended, there is one
+    entered = []
+
+    class Device(torch.cuda.device):
+        def __init__(self, device):
+            entered.append(device)
+            super().__init__(device)
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0 if entered else 1)
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    q, k, v, m = sets[0]
+    got = dense_rows_attention(q, k, v, offset, mask=m)
+    assert entered == [q.device]
+    monkeypatch.undo()
+    assert torch.equal(got, eager[0])
 
 
 def _spy_on_library_attention(monkeypatch):
