@@ -172,11 +172,16 @@ hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mas
 }
 
 // How the keys of a rows-mode problem are cut into chunks.  The chip holds 512 work-groups (two per CU) at head dimension
-// 128 and 768 at 64.  A tile takes a work-group about 1.9 us (64: 1.7 us) when the CUs are full and 1.1 us (1.0 us) alone,
-// measured with one MFMA per V operand; several chunks cost a write and a read of the state (64 KB per column block and
-// chunk at head dimension 128) and one more launch.  Every number of chunks up to 64 is priced with that and the cheapest
-// is taken.  (Prices raised by the 1.3 that the second MFMA costs a full chip cut short prompts into more chunks: fourteen
-// prompts and batches level, one 20.7 -> 25.8 us.)
+// 128 and 768 at 64.  Every number of chunks up to 64 is priced and the cheapest taken: the longest chain of tiles, or all tiles
+// over the chip's places, at a price per tile, and for several chunks one more launch and a write and a read of the state (64 KB per
+// column block and chunk at head dimension 128).
+//
+// The prices are not the tile's times (a work-group alone on its CU takes 1.45 us a tile at head dimension 128 and 1.1 at 64, each
+// work-group of a full chip 3.1 and 2.9): the form knows nothing of how uneven column blocks fill the last round, and with these times it
+// takes counts that are 3.9 and 7.2 % slower than the best.  They are those for which it comes closest: with 75 sizes of each head dimension (40 to 5000
+// rows, up to 40000 keys, 1 to 16 KV heads, 1 to 8 heads a group) the count taken is 0.9 % slower than the best of fifteen on
+// average and 6.6 % at worst, 64: 2.7 and 15 %.  (Prices from the kernel with one MFMA per V operand, 1.1 and 1.9, 1.0 and 1.7 us a tile and
+// 6 us + 4 MB/us for the state: 1.8 and 17 %, 5.2 and 29 %: they cut 2047 rows with 32/8 heads of 64, 61.8 us against 48.3 whole.)
 void plan_rows(FlashArgs& a) {
   const int group = a.n_q_heads / a.n_kv_heads;
   a.n_col_blocks = (a.n_rows * group + 127) / 128;
@@ -196,10 +201,10 @@ void plan_rows(FlashArgs& a) {
     for (int i = 0; i < a.n_col_blocks; ++i)
       wgs += (min(a.causal_offset + (min(128 * (i + 1), a.n_rows * group) - 1) / group, a.n_ctx - 1) / 64 + len) / len;
     wgs *= units;
-    const double t_tile = a.head_dim == 128 ? (wgs <= 256 ? 1.1 : 1.9) : (wgs <= 256 ? 1.0 : 1.7);
+    const double t_tile = a.head_dim == 128 ? (wgs <= 256 ? 1.5 : 1.8) : (wgs <= 256 ? 1.2 : 1.45);
     const double rounds = (double)((wgs + slots - 1) / slots) * ((double)total * units / wgs);
     double us = t_tile * (rounds > len ? rounds : len);
-    if (chunks > 1) us += 6.0 + (double)wgs * 128 * a.head_dim * 8 / 4e6;
+    if (chunks > 1) us += a.head_dim == 128 ? 4.0 + (double)wgs * 128 * 128 * 8 / 4e6 : 2.0 + (double)wgs * 128 * 64 * 8 / 2e6;
     if (us < best) {
       best = us;
       a.n_chunks = chunks;
