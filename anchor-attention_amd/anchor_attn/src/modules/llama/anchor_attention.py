@@ -19,8 +19,8 @@ from typing import Optional, Tuple
 import torch
 import torch.nn.functional as F
 
-from anchor_attn.src.ops.anchor_attn_v4 import (LOG2E, _anchor_attn, _dense_rows, anchor_attn, dense_causal_attention,
-                                                dense_rows_supported)
+from anchor_attn.src.ops.anchor_attn_v4 import (LOG2E, _anchor_attn, _dense_rows, _rows_dispatch, anchor_attn,
+                                                dense_causal_attention)
 
 ATTN_NAME = "anchor_attn"
 DENSE_ATTN_NAME = "anchor_attn_dense"
@@ -45,8 +45,10 @@ def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[i
     by_mask = attention_mask is not None and causal_offset is None
     by_offset = attention_mask is None and causal_offset is not None and causal_offset >= 0
     # (the own kernel scales raw scores in float32: by a positive number whose product with them neither vanishes nor overflows)
-    if (by_mask or by_offset) and not wants_grad and (scaling is None or 1e-30 < scaling < 1e30) and dense_rows_supported(query, key, value, attention_mask, out):
-        return _dense_rows(query, key, value, causal_offset or 0, scaling, out, attention_mask)
+    if (by_mask or by_offset) and not wants_grad and (scaling is None or 1e-30 < scaling < 1e30):
+        tensors = _rows_dispatch(query, key, value, attention_mask, out)
+        if tensors is not None:
+            return _dense_rows(tensors, query, key, causal_offset or 0, scaling, out, attention_mask)
     mask = attention_mask
     if causal_offset is not None and mask is None and query.shape[2] > 1:
         rows = torch.arange(query.shape[2], device=query.device)[:, None] + causal_offset
@@ -98,7 +100,7 @@ def dense_attention_forward(module, query: torch.Tensor, key: torch.Tensor, valu
     the same kernels" that the sparse operator is compared with.  Counterpart of the reference's ``"flash"`` pattern
     (modules/patch.py:128-130 -> modules/llama/flash_attention.py, ops/flash_attn_triton.py:641-657), with the same
     division of labour as the sparse plug: a fresh unpadded bf16/fp16 prefill goes through the kernel in multiples of
-    128 rows, the remaining tail rows, decode steps and padded batches through the framework's dense attention."""
+    128 rows, the remaining tail rows, decode steps and padded batches through :func:`_dense`."""
     B, Hq, N, D = query.shape
     n_kv = key.shape[2]
     out = torch.empty(B, N, Hq, D, dtype=query.dtype, device=query.device)

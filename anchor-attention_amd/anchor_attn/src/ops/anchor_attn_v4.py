@@ -187,80 +187,92 @@ def _no_backend_chosen() -> bool:
     return torch.backends.cuda.flash_sdp_enabled() and torch.backends.cuda.mem_efficient_sdp_enabled() and torch.backends.cuda.math_sdp_enabled()
 
 
-def _rows_kernels_take(Q, K, V, mask=None, out=None) -> bool:
-    """The kernels' types, head dimensions, alignment, sizes of one launch and 32-bit addressing of one head; all of them hold
-    for ``out`` too, whose strides can be wider than ``Q``'s."""
-    if not (Q.is_cuda and Q.dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == Q.dtype and K.device == V.device == Q.device):
-        return False
-    if not Q.dim() == K.dim() == V.dim() == 4:
-        return False
-    B, H, N, D = Q.shape
-    if D not in (64, 128) or K.shape != V.shape or K.shape[3] != D or K.shape[0] != B or not B or not K.shape[1] or H % K.shape[1] or not H:
-        return False
+def _rows_tensors(Q, K, V, mask=None, out=None):
+    """``data_ptr, stride_b, stride_h, stride_n`` of ``Q``, ``K``, ``V`` and ``out`` (not given: ``Q``'s) for the launch; None
+    where the kernels do not take them: their types, head dimensions, alignment, sizes of one launch and 32-bit addressing
+    of one head.  All of them hold for ``out`` too, whose strides can be wider than ``Q``'s."""
+    dtype, device, q_shape, kv_shape = Q.dtype, Q.device, Q.shape, K.shape
+    if not (Q.is_cuda and dtype in (torch.bfloat16, torch.float16) and K.dtype == V.dtype == dtype and K.device == V.device == device):
+        return None
+    if not (len(q_shape) == len(kv_shape) == 4 and V.shape == kv_shape):
+        return None
+    B, H, N, D = q_shape
+    kv_batch, kv_heads, n_keys, kv_dim = kv_shape
+    if D not in (64, 128) or kv_dim != D or kv_batch != B or not B or not kv_heads or H % kv_heads or not H:
+        return None
     if out is None:
         out = Q
-    elif out.shape != Q.shape or out.dtype != Q.dtype or out.device != Q.device:
-        return False
-    n_keys = K.shape[2]
+    elif out.shape != q_shape or out.dtype != dtype or out.device != device:
+        return None
+    tensors = []
     for t, rows in ((Q, N), (K, n_keys), (V, n_keys), (out, N)):
-        sb, sh, sn, sd = t.stride()
-        if sd != 1 or (sb | sh | sn) & 7 or t.data_ptr() & 15 or not D <= sn <= 1 << 14 or not 0 < rows <= 1 << 20 or rows * sn * 2 >= 1 << 32:
-            return False
-    col_blocks = (N * (H // K.shape[1]) + 127) // 128
+        ptr, (sb, sh, sn, sd) = t.data_ptr(), t.stride()
+        if sd != 1 or (sb | sh | sn) & 7 or ptr & 15 or not D <= sn <= 1 << 14 or not 0 < rows <= 1 << 20 or rows * sn * 2 >= 1 << 32:
+            return None
+        tensors += (ptr, sb, sh, sn)
+    col_blocks = (N * (H // kv_heads) + 127) // 128
     # (that many column blocks are one chunk each; but a decode step's chunk holds 2^13 keys, a masked one 2^16)
-    if B * K.shape[1] * col_blocks * (1 if col_blocks > 1 and mask is None else (n_keys >> 13) + 1) >= 1 << 24:
-        return False
+    if B * kv_heads * col_blocks * (1 if col_blocks > 1 and mask is None else (n_keys >> 13) + 1) >= 1 << 24:
+        return None
     if mask is not None:
-        if type(mask) is not torch.Tensor or mask.device != Q.device or mask.dtype != torch.bool or mask.dim() != 4:
-            return False
+        if type(mask) is not torch.Tensor or mask.device != device or mask.dtype != torch.bool or mask.dim() != 4:
+            return None
         if mask.shape[0] not in (1, B) or tuple(mask.shape[1:]) != (1, N, n_keys):
-            return False
+            return None
         if B >= 1 << 16 or col_blocks >= 1 << 16 or N * ((n_keys + 63) // 64) * 8 >= 1 << 32:
-            return False
-    return True
+            return None
+    return tensors
 
 
-def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
-    """Whether the attention of these tensors is to be computed by :func:`dense_rows_attention`: its kernels take them, and
-    nothing about the call asks for the framework's own operations."""
+def _rows_dispatch(Q, K, V, mask=None, out=None):
+    """:func:`_rows_tensors` where the attention of these tensors is to be computed by the own kernels: they take them, and
+    nothing about the call asks for the framework's own operations; otherwise None."""
     if not (type(Q) is type(K) is type(V) is torch.Tensor and _called_plainly() and _no_backend_chosen()):
-        return False
+        return None
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != Q.dtype:  # (attention is computed in that type)
-        return False
+        return None
     # Thousands of padded prompts of a few tokens: a work-group per (prompt, KV head) has one tile to do, and library attention, where it
     # need not repeat heads, is faster: 128 prompts of 16 tokens, 32 heads of 128, 37 us against 64 (32 tokens 68 against 71; 16 prompts 36
     # against 28; 32/8 heads 241 against 30).
     if mask is not None and 1 < Q.shape[2] and K.shape[2] < 32 and Q.shape[1] == K.shape[1] and Q.shape[0] * Q.shape[1] > 2048:
-        return False
-    return _rows_kernels_take(Q, K, V, mask, out)
+        return None
+    return _rows_tensors(Q, K, V, mask, out)
+
+
+def dense_rows_supported(Q, K, V, mask=None, out=None) -> bool:
+    """Whether the attention of these tensors is to be computed by :func:`dense_rows_attention`."""
+    return _rows_dispatch(Q, K, V, mask, out) is not None
 
 
 def dense_rows_attention(Q, K, V, causal_offset: int = 0, sm_scale: float = None, out: torch.Tensor = None, mask: torch.Tensor = None):
     """Attention of ``Q`` ``[B,H,n_rows,D]`` over ``K``/``V`` ``[B,H_kv,n_keys,D]`` on the same MFMA core: query row ``i``
     sees keys ``0 .. causal_offset + i``, or, with a boolean ``mask`` ``[B or 1, 1, n_rows, n_keys]``, the keys it is True for.
-    Any row and key count (:func:`_rows_kernels_take` names the rest)."""
-    if not _rows_kernels_take(Q, K, V, mask, out):
+    Any row and key count (:func:`_rows_tensors` names the rest)."""
+    tensors = _rows_tensors(Q, K, V, mask, out)
+    if tensors is None:
         raise _hip.AnchorAttnHipError("dense_rows_attention: unsupported tensors (bf16 or fp16 on one GPU, head dimension 64 or 128, rows of at "
                                       "most 16384 elements on 16-byte boundaries, a boolean mask [B or 1, 1, n_rows, n_keys], out like Q)")
-    return _dense_rows(Q, K, V, causal_offset, sm_scale, out, mask)
+    return _dense_rows(tensors, Q, K, causal_offset, sm_scale, out, mask)
 
 
-def _dense_rows(Q, K, V, causal_offset, sm_scale, out, mask):
-    # (the tensors have been looked at: the launch trusts their shapes)
+def _dense_rows(tensors, Q, K, causal_offset, sm_scale, out, mask):
+    # (`tensors` comes from _rows_tensors for this very call, which has looked at them: the launch trusts their shapes)
     B, H, N, D = Q.shape
-    n_keys = K.shape[2]
+    _, kv_heads, n_keys, _ = K.shape
     sm_scale = sm_scale if sm_scale else 1.0 / (D ** 0.5)
-    output = torch.empty_like(Q) if out is None else out
+    output = out
+    if out is None:
+        output = torch.empty_like(Q)
+        tensors[12:] = _hip.t3(output)
     mask_args = (None, 0, 0)
     if mask is not None:
         mask = mask if mask.stride(3) == 1 else mask.contiguous()
         mask_args = (mask.data_ptr(), mask.stride(0) if mask.shape[0] > 1 else 0, mask.stride(2))
     lib = _hip.lib()
-    sizes = (B, H, K.shape[1], N, n_keys, D, int(causal_offset))
+    sizes = (B, H, kv_heads, N, n_keys, D, int(causal_offset))
     nbytes = lib.aa_dense_rows_workspace_bytes(*sizes, mask is not None)
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=Q.device) if nbytes else None
-    args = (*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output), *mask_args, ws.data_ptr() if nbytes else None, nbytes, *sizes,
-            float(sm_scale), _hip.dtype_code(Q))
+    args = (*tensors, *mask_args, ws.data_ptr() if nbytes else None, nbytes, *sizes, float(sm_scale), _hip.dtype_code(Q))
     if Q.device.index == torch.cuda.current_device():
         _hip.check(lib.aa_dense_rows_fwd(*args, _stream()))
     else:  # (a pipeline's later layers lie on other GPUs than the current one)
