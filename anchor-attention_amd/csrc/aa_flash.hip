@@ -1,4 +1,4 @@
-// MFMA flash-attention core for gfx950, used four ways:
+// MFMA flash-attention core for gfx950, used five ways:
 //   kAnchor : stage 1 - windowed causal attention over [0,S) U [bb*S, r]; emits M, L, Acc
 //   kSparse : stage 3 - resumes from (M, L, Acc) over K/V rows gathered at selected indices
 //   kDense  : plain causal attention (baseline)
@@ -159,8 +159,8 @@ __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, cons
 // dimension (kKS per 32 keys of Q.K^T) and of 32-column output blocks (kDB).
 //
 // Work-groups per CU: with 128 two (248 registers, 64 KB of LDS).  With 64 a tile has half the MFMAs but the same soft-max,
-// so the vector ALU bounds it, and a third wave per SIMD (168 registers; 2 and 8 of them spill around the tile loop in anchor
-// and sparse mode) keeps that busy: 69 % of the cycles, matrix pipe 49 %.  16384 tokens, 32/8 heads of 64: stage 1 470 -> 413 us
+// so the vector ALU bounds it, and a third wave per SIMD (168 registers; 2, 8 and 2 of them spill around the tile loop in
+// anchor, sparse and bf16 rows mode) keeps that busy: 69 % of the cycles, matrix pipe 49 %.  16384 tokens, 32/8 heads of 64: stage 1 470 -> 413 us
 // against two work-groups per CU and 256-byte LDS rows of which half was filled.
 template <int MODE, typename T, int D>
 __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const FlashArgs p) {

@@ -94,8 +94,8 @@ hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream) {
 
 // Masked mode: packs the byte mask of one column block's rows, 64 keys to a word, and notes for each 64-key tile whether any
 // and whether every one of the rows sees it.  A work-group takes 1024 keys of the block's rows, a lane 16 of them; the four
-// waves share the rows, eight loads in flight each.  Bound by the latency of two or three rounds of loads: a mask is read
-// once (rows that two column blocks share are packed twice, to the same words).  A row's last keys are read as its last 16
+// waves share the rows, eight loads in flight each.  Bound by the latency of its rounds of loads (32 rows each: one or two with heads
+// in groups of four at most, four without groups): a mask is read once (rows that two column blocks share are packed twice, to the same words).  A row's last keys are read as its last 16
 // and shifted, not byte by byte.  3 x 2500 x 2500: 32.1 us with a wave to a block's rows and a byte loop, 7.3 us now.
 constexpr int kPackKeys = 1024;
 __global__ void __launch_bounds__(256) mask_pack_kernel(const FlashArgs p, const uint8_t* mask, const int64_t mask_sb, const int64_t mask_sn) {
