@@ -19,11 +19,21 @@
 // at one head-dim column is fetched with the transposing LDS read ds_read_b64_tr_b16 (within a group
 // of 16 lanes, lane i receives column i of the 4x16 block whose rows the group's lanes point at).
 //
-// The running row max m is subtracted inside the first product: the score accumulators start from
-// -m (a per-lane constant, kept replicated in a 16-register tuple) instead of zero, so the tile
-// arrives as S - m and p = exp2(S - m) needs no subtraction.  Only when some row's max grows (rare
-// after the first tiles) does the wave take a slow path that shifts the tile, re-bases the tuple and
-// rescales the accumulators - which is exact for the lanes whose max did not move (shift 0, factor 1).
+// A reference m is subtracted inside the first product: the score accumulators start from -m (a per-lane
+// constant, kept replicated in a 16-register tuple) instead of zero, so the tile arrives as S - m and
+// p = exp2(S - m) needs no subtraction.  m is the running row max: with a probability in one 16-bit number the key that
+// weighs most then has p = 1, which is exact (kept at the max of a row's first keys, the error of P.V grows by up to a factor of
+// three where few keys weigh much).  Whether a lane's max grew is a comparison of S - m with zero, before the two lanes of
+// a row have exchanged anything; only when one did (rare after the first tiles) does the wave take a slow path that completes
+// the max, shifts the tile, re-bases the tuple and rescales the accumulators - exact for the lanes whose
+// max did not move (shift 0, factor 1).  (The exchange on every half-tile instead: 16384 tokens dense, 32/8 heads of 128, 1830 us
+// against 1796.)
+//
+// bf16 rows and masked modes, which keep a probability as two numbers, need no max at all (kLazyRef): m is the row max of the
+// first 32 keys and stays, and a larger score gives a p above 1, which is held as precisely as one below.  When the
+// sum of a half-tile's p exceeds kRebaseSum - an overflowing exp2 included - the wave forms that half's scores again,
+// moves m to the row's max and rescales, before these p are used.  (fp16 forms 2^15 p, which has no room above p = 1.)
+// 777 rows over 777 keys, 32/8 heads of 128: 23.0 -> 21.1 us; a padded batch of 3 x 2500: 203 -> 193.
 //
 // Inside a 64-key tile the two 32-key halves are staggered so that matrix and vector work overlap
 // within a wave: S0 | S1 with soft-max(S0) | P0.V0 with soft-max(S1) | P1.V1.  The online soft-max
@@ -49,6 +59,8 @@ namespace aa {
 constexpr int kBN = 64;        // keys per LDS tile
 constexpr int kLoadBytes = 4096; // what one LDS-DMA instruction of the work-group brings (256 threads x 16 bytes)
 constexpr int kDist = 4;         // MFMA operands are fetched from LDS this many MFMAs ahead of their use
+constexpr float kRebaseSum = 16384.f;  // (kLazyRef) largest sum of 16 probabilities that is used as it is
+constexpr float kNoRef = -8.5e37f;     // (kLazyRef) reference of a row that has seen no key: what it sees first overflows exp2
 constexpr int kIdxWin = 1024;    // selected-key indices held in LDS at a time (16 tiles)
 constexpr int32_t kMixedTile = 1 << 30;  // (masked) flag of a listed tile of which some pairs are masked
 
@@ -169,6 +181,12 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   __shared__ __attribute__((aligned(16))) FlashSmem<MODE, D> sm;
   constexpr int BM = 128;
   constexpr bool kAnyRows = MODE == kRows || MODE == kMasked;
+  constexpr bool kLazyRef = kAnyRows && T::kProbLog2 == 0.f;  // the reference does not follow the row max (see the top of the file)
+  // Whether the rounded probabilities are named where they are formed: otherwise the compiler moves half of the exponentials and
+  // conversions to the block of their use, where no MFMAs run beside them (131072 tokens, 32/8 heads of 128, all stages: 7.60 ms
+  // against 7.53).  Head dimension 64 spills registers for it (anchor, sparse, fp16 rows).
+  constexpr bool kPinned = D == 128 || kLazyRef || MODE == kDense;
+  constexpr bool kChecksSums = kLazyRef && AA_ABLATE != 1 && AA_ABLATE != 2;
   static_assert(D == 128 || D == 64, "head dimension");
   constexpr int kKS = D / 16;       // MFMAs per 32-key block of S^T = K Q^T
   constexpr int kDB = D / 32;       // 32-column blocks of the head dimension: accumulators of O^T
@@ -457,9 +475,10 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     l_run = l_in;
   }
 
-  // m_ref is what the score accumulators are pre-loaded with (negated); it equals m_run except before
-  // the first tile of a fresh row (m_run = -inf, m_ref = 0)
-  float m_ref = (MODE == kSparse) ? m_run : 0.f;
+  // m_ref is what the score accumulators are pre-loaded with (negated).  Where it follows the running max it equals m_run
+  // except before the first key of a fresh row (m_run = -inf, m_ref = 0); m_over is what S - m_ref has to exceed for a new max
+  float m_ref = MODE == kSparse ? m_run : kLazyRef ? kNoRef : 0.f;
+  float m_over = MODE == kSparse ? 0.f : -INFINITY;
   floatx16 negm;
 #pragma unroll
   for (int r = 0; r < 16; ++r) negm[r] = -m_ref;
@@ -524,16 +543,15 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     _Pragma("unroll") for (int r = 0; r < 16; ++r)                                   \
       if (AA_KEY_OF(kb, r) >= cnt) sx[r] = -INFINITY;                                \
   }
-  // row max of one half (both halves of the wave hold the same query), relative to m_ref
-#define AA_ROWMAX(sx, mx)                                                            \
+  // this lane's max of one half (the lane 32 positions away holds the other keys of the same query)
+#define AA_LANEMAX(sx, mx)                                                           \
   {                                                                                  \
     float t0 = fmaxf(fmaxf(sx[0], sx[1]), sx[2]), t1 = fmaxf(fmaxf(sx[3], sx[4]), sx[5]);      \
     float t2 = fmaxf(fmaxf(sx[6], sx[7]), sx[8]), t3 = fmaxf(fmaxf(sx[9], sx[10]), sx[11]);    \
     float t4 = fmaxf(fmaxf(sx[12], sx[13]), sx[14]);                                 \
     t0 = fmaxf(fmaxf(t0, t1), t2);                                                   \
     t3 = fmaxf(fmaxf(t3, t4), sx[15]);                                               \
-    t0 = fmaxf(t0, t3);                                                              \
-    mx = max_with_other_half(t0);                                                     \
+    mx = fmaxf(t0, t3);                                                              \
   }
   // (rows: maxima and scores are kept as raw dot products; the scale is applied to the difference, in float32)
 #define AA_EXP2(x) ((AA_ABLATE == 1 || AA_ABLATE == 2) ? (x) : fast_exp2(kAnyRows ? (x) * score_scale : (x)))
@@ -546,6 +564,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     if (AA_ABLATE != 2) { sum += e0; sum += e1; sum += e2; sum += e3; }              \
     pw[(c) >> 1][2 * ((c) & 1) + 0] = T::pack(e0, e1);                                 \
     pw[(c) >> 1][2 * ((c) & 1) + 1] = T::pack(e2, e3);                                 \
+    if (kPinned) asm volatile("" : "+v"(pw[(c) >> 1][2 * ((c) & 1) + 0]), "+v"(pw[(c) >> 1][2 * ((c) & 1) + 1]));   \
     if (kAnyRows) { /* what the rounding left, as a second 16-bit number */            \
       pw##_rest[(c) >> 1][2 * ((c) & 1) + 0] = T::pack_rest(e0, e1, pw[(c) >> 1][2 * ((c) & 1) + 0]);  \
       pw##_rest[(c) >> 1][2 * ((c) & 1) + 1] = T::pack_rest(e2, e3, pw[(c) >> 1][2 * ((c) & 1) + 1]);  \
@@ -568,6 +587,26 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
                                            *reinterpret_cast<const vec8*>(&pw##_rest[((i) / kDB) & 1]), acc[(i) % kDB]); \
   }
 #define AA_FENCE __builtin_amdgcn_sched_barrier(0)
+  // scores of 32-key half kb of the tile whose K rows lie at immediate offset rd, from c_init on
+#define AA_SCORES(sx, kb, rd, c_init)                                                                                   \
+  _Pragma("unroll") for (int ks = 0; ks < kKS; ++ks)                                                                    \
+    sx = T::mfma(*(const lds_vec8*)(uintptr_t)(k_rd[ks] + (uint32_t)((rd) + 32 * (kb) * kRowBytes)), qreg[ks], ks == 0 ? c_init : sx);
+  const floatx16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+  if (kLazyRef && n_tiles > 0) {  // the reference: the row max of the first 32 keys
+    const int key0 = AA_TILE_KEY0(0);
+    const bool mixed = MODE == kMasked && (entry_next & kMixedTile);
+    const u32x2 mask_word = {mask_word_next[0] >> (4 * half), mask_word_next[1] >> (4 * half)};
+    floatx16 sx;
+    float mx;
+    AA_SCORES(sx, 0, 0, zero16)
+    AA_MASK(sx, 0)
+    AA_LANEMAX(sx, mx)
+    mx = max_with_other_half(mx);
+    m_ref = mx == -INFINITY ? kNoRef : mx;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) negm[r] = -m_ref;
+  }
 
   // One tile.  The LDS buffer it reads (BUF) is a compile-time constant - the loop below is unrolled by two - so that
   // the buffer's offset is part of every LDS instruction's immediate offset and the read addresses are loop-invariant.
@@ -628,7 +667,34 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
       shortx4 vlo[kNV], vhi[kNV];  // V operand of slot kNS + i, i = (kb*2 + st)*kDB + db
       u32x4 pw0[2], pw1[2];        // P^T fragments (bf16 pairs) of the two halves
       u32x4 pw0_rest[2], pw1_rest[2];  // (rows) and of what their rounding left
-      float mx0, mx1, sum0 = 0.f, sum1 = 0.f, shift0 = 0.f, alpha1 = 1.f;
+      float sum0 = 0.f, sum1 = 0.f;
+      float mx0, mx1, shift0 = 0.f, alpha1 = 1.f;  // (where the reference follows the running max)
+      bool moved0 = false, moved1 = false;
+      // The half whose probabilities sum to more than kRebaseSum once more, from a reference that is the row's max.  (Its
+      // scores start from zero: those of a row that had no reference hold nothing but kNoRef.)
+      auto rebase = [&](auto kb_const, floatx16& sx, u32x4 (&pw)[2], u32x4 (&pw_rest)[2], float& sum) __attribute__((always_inline)) {
+        constexpr int kb = decltype(kb_const)::value;
+        float mx;
+        AA_SCORES(sx, kb, rd_off, zero16)
+        AA_MASK(sx, kb)
+        AA_LANEMAX(sx, mx)
+        const float m_new = fmaxf(m_ref, max_with_other_half(mx));
+        const float alpha = AA_EXP2(m_ref - m_new);
+        m_ref = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sx[r] -= m_new;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) negm[r] = -m_new;
+#pragma unroll
+        for (int db = 0; db < kDB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+        sum = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { AA_EXP_CHUNK(sx, pw, sum, c) }
+      };
+      (void)rebase;
 #define AA_K_FETCH(t) ka[t] = *(const lds_vec8*)(uintptr_t)(k_rd[(t) % kKS] + (uint32_t)(rd_off + 32 * ((t) / kKS) * kRowBytes))
 
       // The MFMAs of a tile are slots 0 .. kNS + kNV - 1 (head dimension 128: 16 for S^T, then 16 for O^T); the operand of
@@ -669,32 +735,31 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
         AA_S_MFMA(s1, n);
         AA_FENCE;
       }
-      if (AA_ABLATE != 2) {
-        AA_MASK(s0, 0)
-        AA_ROWMAX(s0, mx0)
-      } else {
-        mx0 = -INFINITY;
-      }
-      const bool moved0 = __any(m_ref + mx0 > m_run);
-      if (moved0) {
-        // slow path: some row's max grew.  Lanes whose max did not move get shift 0 and alpha 1 (exact).
-        // S1 is being accumulated on top of the old -m_ref and is shifted once it is complete.
-        // (rows: a chunk may hold no key of a row's so far - its max stays -inf and its reference 0)
-        const float m_new = fmaxf(m_run, m_ref + mx0);
-        const float m_base = kAnyRows && m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = AA_EXP2(m_run - m_base);
-        shift0 = m_base - m_ref;
-        m_run = m_new;
-        m_ref = m_base;
-        l_run *= alpha;
+      if (AA_ABLATE != 2) { AA_MASK(s0, 0) }
+      if (!kLazyRef && AA_ABLATE != 2) {
+        AA_LANEMAX(s0, mx0)
+        moved0 = __any(mx0 > m_over);
+        if (moved0) {
+          // some row's max grew.  Lanes whose max did not move get shift 0 and alpha 1 (exact).
+          // S1 is being accumulated on top of the old -m_ref and is shifted once it is complete.
+          // (a chunk may hold no key of a row's so far - its max stays -inf and its reference 0)
+          const float m_new = fmaxf(m_run, m_ref + max_with_other_half(mx0));
+          const float m_base = m_new == -INFINITY ? 0.f : m_new;
+          m_over = m_new - m_base;
+          const float alpha = AA_EXP2(m_run - m_base);
+          shift0 = m_base - m_ref;
+          m_run = m_new;
+          m_ref = m_base;
+          l_run *= alpha;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s0[r] -= shift0;
+          for (int r = 0; r < 16; ++r) s0[r] -= shift0;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) negm[r] = -m_base;
+          for (int r = 0; r < 16; ++r) negm[r] = -m_base;
 #pragma unroll
-        for (int db = 0; db < kDB; ++db)
+          for (int db = 0; db < kDB; ++db)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+            for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+        }
       }
       AA_FENCE;
 #pragma unroll
@@ -705,13 +770,17 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
         for (int u = 0; u < 4 / kSMid; ++u) { AA_EXP_CHUNK(s0, pw0, sum0, (n - kKS - kSPre) * (4 / kSMid) + u) }
         AA_FENCE;
       }
-      l_run += sum0;
 #pragma unroll
       for (int n = kKS + kSPre + kSMid; n < kNS; ++n) {
         AA_OPERAND_FETCH(n + kDist)
         AA_S_MFMA(s1, n);
         AA_FENCE;
       }
+      if (kChecksSums && __builtin_expect(__any(sum0 > kRebaseSum), 0)) {
+        rebase(std::integral_constant<int, 0>{}, s0, pw0, pw0_rest, sum0);
+        AA_SCORES(s1, 1, rd_off, negm)
+      }
+      l_run += sum0;
 
       // ---- phase C: O^T += V0^T P0^T, with the soft-max of S1 between the MFMAs --------------------
 #pragma unroll
@@ -720,30 +789,29 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
         AA_PV_MFMA(n - kNS, pw0)
         AA_FENCE;
       }
-      if (moved0) {
+      if (!kLazyRef && moved0) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) s1[r] -= shift0;
       }
-      if (AA_ABLATE != 2) {
-        AA_MASK(s1, 1)
-        AA_ROWMAX(s1, mx1)
-      } else {
-        mx1 = -INFINITY;
-      }
-      const bool moved1 = __any(m_ref + mx1 > m_run);
-      if (moved1) {
-        // as above, except that O^T is rescaled only after the P0 V0 products in flight have been added
-        const float m_new = fmaxf(m_run, m_ref + mx1);
-        const float m_base = kAnyRows && m_new == -INFINITY ? 0.f : m_new;
-        alpha1 = AA_EXP2(m_run - m_base);
-        const float shift = m_base - m_ref;
-        m_run = m_new;
-        m_ref = m_base;
-        l_run *= alpha1;
+      if (AA_ABLATE != 2) { AA_MASK(s1, 1) }
+      if (!kLazyRef && AA_ABLATE != 2) {
+        AA_LANEMAX(s1, mx1)
+        moved1 = __any(mx1 > m_over);
+        if (moved1) {
+          // as above, except that O^T is rescaled only after the P0 V0 products in flight have been added
+          const float m_new = fmaxf(m_run, m_ref + max_with_other_half(mx1));
+          const float m_base = m_new == -INFINITY ? 0.f : m_new;
+          m_over = m_new - m_base;
+          alpha1 = AA_EXP2(m_run - m_base);
+          const float shift = m_base - m_ref;
+          m_run = m_new;
+          m_ref = m_base;
+          l_run *= alpha1;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s1[r] -= shift;
+          for (int r = 0; r < 16; ++r) s1[r] -= shift;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) negm[r] = -m_base;
+          for (int r = 0; r < 16; ++r) negm[r] = -m_base;
+        }
       }
       AA_FENCE;
 #pragma unroll
@@ -754,19 +822,20 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
         for (int u = 0; u < 4 / kVMid; ++u) { AA_EXP_CHUNK(s1, pw1, sum1, (n - kNS - kVPre) * (4 / kVMid) + u) }
         AA_FENCE;
       }
-      l_run += sum1;
 #pragma unroll
       for (int n = kNS + kVPre + kVMid; n < kNS + 2 * kDB; ++n) {
         AA_OPERAND_FETCH(n + kDist)
         AA_PV_MFMA(n - kNS, pw0)
         AA_FENCE;
       }
-      if (moved1) {
+      if (!kLazyRef && moved1) {
 #pragma unroll
         for (int db = 0; db < kDB; ++db)
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[db][r] *= alpha1;
       }
+      if (kChecksSums && __builtin_expect(__any(sum1 > kRebaseSum), 0)) rebase(std::integral_constant<int, 1>{}, s1, pw1, pw1_rest, sum1);
+      l_run += sum1;
 
       // ---- phase D: O^T += V1^T P1^T ---------------------------------------------------------------
 #pragma unroll
@@ -810,7 +879,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 #undef AA_TILE_KEY0
 #undef AA_KEY_OF
 #undef AA_MASK
-#undef AA_ROWMAX
+#undef AA_LANEMAX
 #undef AA_EXP2
 #undef AA_PROB
 #undef AA_EXP_CHUNK
@@ -818,10 +887,12 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 #undef AA_V_FETCH
 #undef AA_PV_MFMA
 #undef AA_FENCE
+#undef AA_SCORES
 
   if (kAnyRows && __builtin_expect(__any(holds_nan(acc) && !is_nan(l_run)), 0)) {
     // V holds infinities or NaN: the wave's sums once more (see aa_nonfinite.h)
-    const float m_base = m_run == -INFINITY ? 0.f : m_run;
+    const float m_last = kLazyRef ? m_ref : m_run;
+    const float m_base = m_last == -INFINITY || m_last == kNoRef ? 0.f : m_last;
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -908,7 +979,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // rows_combine_kernel merges the chunks
     const int64_t slot = ((((int64_t)b * p.n_kv_heads + kvh) * p.n_col_blocks + qunit) * p.n_chunks + chunk) * 4 + wave;
     if (half == 0) {
-      p.M_out[slot * 32 + c32] = m_run;
+      p.M_out[slot * 32 + c32] = !kLazyRef ? m_run : m_ref == kNoRef ? -INFINITY : m_ref;
       p.L_out[slot * 32 + c32] = l_tot;
     }
     float* af = p.acc_out + slot * (kDB * 4 * 256) + lane * 4;
