@@ -38,8 +38,17 @@ struct Bf16 {
     bf16x2 h = __builtin_convertvector(f, bf16x2);
     return *reinterpret_cast<uint32_t*>(&h);
   }
-  // the pair that rounding to `packed` took from a and b
-  static __device__ __forceinline__ uint32_t pack_rest(float a, float b, uint32_t packed) { return pack(a - lo(packed), b - hi(packed)); }
+  // the pair that rounding to `packed` took from a and b: a - lo and b - hi, exact, one instruction each as dot products of the pair
+  // with (-1, 0) and (0, -1).  (The pairs are hidden from the compiler, which encodes constants of this instruction wrongly.)
+  // Unpacked and subtracted: 777 rows over 777 keys, 32/8 heads of 128, 20.9 us against 20.5; padded 3 x 2500 194.8 against 191.7.
+  static __device__ __forceinline__ uint32_t pack_rest(float a, float b, uint32_t packed) {
+    uint32_t minus_lo = 0x0000bf80u, minus_hi = 0xbf800000u;
+    asm("" : "+s"(minus_lo));
+    asm("" : "+s"(minus_hi));
+    const bf16x2 p = *reinterpret_cast<const bf16x2*>(&packed);
+    return pack(__builtin_amdgcn_fdot2_f32_bf16(p, *reinterpret_cast<const bf16x2*>(&minus_lo), a, false),
+                __builtin_amdgcn_fdot2_f32_bf16(p, *reinterpret_cast<const bf16x2*>(&minus_hi), b, false));
+  }
   static __device__ __forceinline__ float round(float a) { return lo(pack(a, 0.f)); }  // float -> nearest bf16 -> float
   // (a * b).to(bf16) as the operator's definition compiles: a float32 product, then the rounding
   static __device__ __forceinline__ float round_product(float a, float b) { return round(a * b); }
@@ -61,7 +70,13 @@ struct F16 {
     f16x2 h = __builtin_convertvector(f, f16x2);
     return *reinterpret_cast<uint32_t*>(&h);
   }
-  static __device__ __forceinline__ uint32_t pack_rest(float a, float b, uint32_t packed) { return pack(a - lo(packed), b - hi(packed)); }
+  // (as fused operations, which take 16-bit operands as they are; the factor is hidden from the compiler, which makes a conversion
+  // and a subtraction of it)
+  static __device__ __forceinline__ uint32_t pack_rest(float a, float b, uint32_t packed) {
+    float minus_one = -1.f;
+    asm("" : "+s"(minus_one));
+    return pack(__builtin_fmaf(lo(packed), minus_one, a), __builtin_fmaf(hi(packed), minus_one, b));
+  }
   static __device__ __forceinline__ float round(float a) { return lo(pack(a, 0.f)); }
   // (a * b).to(fp16) as the operator's definition compiles: ONE rounding of the exact product (the multiply and the
   // cast become a single mixed-precision instruction).  Written out so that it does not depend on what this compiler

@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   // They depend on nothing, whereas the first K/V tile needs the index list, which needs its own round trip to
   // memory.  The 64 KB of accumulator state follow the first tile's loads (further down) and are not waited for
   // before the first scores are computed.
-  float m_run, l_run;
+  float l_run;
   const uint16_t* qrow = qp + (int64_t)my_row * p.q_sn + 8 * half + (kAnyRows ? (my_col - my_row * group) * p.q_sh : 0);
   if (MODE == kSparse && !have_queries) request_queries(my_row);
   const bool feeds_next = list_chains && qb + 1 < nq;  // the next block takes its first tile from this one
@@ -464,20 +464,18 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 
   // ---- running state (sparse mode loaded it at the top) -----------------------------------------
   if (MODE != kSparse) {
-    m_run = -INFINITY;
     l_run = 0.f;
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
   } else {
-    m_run = m_in;
     l_run = l_in;
   }
 
-  // m_ref is what the score accumulators are pre-loaded with (negated).  Where it follows the running max it equals m_run
-  // except before the first key of a fresh row (m_run = -inf, m_ref = 0); m_over is what S - m_ref has to exceed for a new max
-  float m_ref = MODE == kSparse ? m_run : kLazyRef ? kNoRef : 0.f;
+  // m_ref is what the score accumulators are pre-loaded with (negated).  Where it follows the running max, m_over is what S - m_ref
+  // has to exceed for a new max: 0, and before the first key of a row (m_ref = 0) -inf.  So m_ref + m_over is the running max
+  float m_ref = MODE == kSparse ? m_in : kLazyRef ? kNoRef : 0.f;
   float m_over = MODE == kSparse ? 0.f : -INFINITY;
   floatx16 negm;
 #pragma unroll
@@ -743,13 +741,12 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
           // some row's max grew.  Lanes whose max did not move get shift 0 and alpha 1 (exact).
           // S1 is being accumulated on top of the old -m_ref and is shifted once it is complete.
           // (a chunk may hold no key of a row's so far - its max stays -inf and its reference 0)
-          const float m_new = fmaxf(m_run, m_ref + max_with_other_half(mx0));
+          const float m_new = fmaxf(m_ref + m_over, m_ref + max_with_other_half(mx0));
           const float m_base = m_new == -INFINITY ? 0.f : m_new;
-          m_over = m_new - m_base;
-          const float alpha = AA_EXP2(m_run - m_base);
+          const float alpha = AA_EXP2(m_ref + m_over - m_base);
           shift0 = m_base - m_ref;
-          m_run = m_new;
           m_ref = m_base;
+          if (MODE != kSparse) m_over = m_new == -INFINITY ? -INFINITY : 0.f;
           l_run *= alpha;
 #pragma unroll
           for (int r = 0; r < 16; ++r) s0[r] -= shift0;
@@ -799,13 +796,12 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
         moved1 = __any(mx1 > m_over);
         if (moved1) {
           // as above, except that O^T is rescaled only after the P0 V0 products in flight have been added
-          const float m_new = fmaxf(m_run, m_ref + max_with_other_half(mx1));
+          const float m_new = fmaxf(m_ref + m_over, m_ref + max_with_other_half(mx1));
           const float m_base = m_new == -INFINITY ? 0.f : m_new;
-          m_over = m_new - m_base;
-          alpha1 = AA_EXP2(m_run - m_base);
+          alpha1 = AA_EXP2(m_ref + m_over - m_base);
           const float shift = m_base - m_ref;
-          m_run = m_new;
           m_ref = m_base;
+          if (MODE != kSparse) m_over = m_new == -INFINITY ? -INFINITY : 0.f;
           l_run *= alpha1;
 #pragma unroll
           for (int r = 0; r < 16; ++r) s1[r] -= shift;
@@ -891,8 +887,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 
   if (kAnyRows && __builtin_expect(__any(holds_nan(acc) && !is_nan(l_run)), 0)) {
     // V holds infinities or NaN: the wave's sums once more (see aa_nonfinite.h)
-    const float m_last = kLazyRef ? m_ref : m_run;
-    const float m_base = m_last == -INFINITY || m_last == kNoRef ? 0.f : m_last;
+    const float m_base = m_ref == kNoRef ? 0.f : m_ref;
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -919,6 +914,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 
   // ---- epilogue --------------------------------------------------------------------------------
   const float l_tot = l_run + xor32(l_run);
+  const float m_run = !kLazyRef ? m_ref + m_over : m_ref == kNoRef ? -INFINITY : m_ref;
   if (MODE == kAnchor && !finishes) {
     if (half == 0) {
       p.M_out[bh * p.n_ctx + my_row] = m_run;
@@ -979,7 +975,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // rows_combine_kernel merges the chunks
     const int64_t slot = ((((int64_t)b * p.n_kv_heads + kvh) * p.n_col_blocks + qunit) * p.n_chunks + chunk) * 4 + wave;
     if (half == 0) {
-      p.M_out[slot * 32 + c32] = !kLazyRef ? m_run : m_ref == kNoRef ? -INFINITY : m_ref;
+      p.M_out[slot * 32 + c32] = m_run;
       p.L_out[slot * 32 + c32] = l_tot;
     }
     float* af = p.acc_out + slot * (kDB * 4 * 256) + lane * 4;
