@@ -22,9 +22,13 @@ from .anchor_step_1_2_v2 import (_check_inputs, _row_major, _stream, anchor_attn
 LOG2E = 1.44269504
 
 
+def _ratio_denominator(B, H, N, block_size, step):
+    return B * H * N * N / (block_size * step) // 2
+
+
 def _ratio(true_counts, B, H, N, block_size, step):
     # same expression as the reference (anchor_attn_v4.py:271); stays a 0-dim device tensor
-    denominator = B * H * N * N / (block_size * step) // 2
+    denominator = _ratio_denominator(B, H, N, block_size, step)
     if torch.get_default_dtype() != torch.float32 or not true_counts.is_contiguous():
         return true_counts.sum() / denominator  # (the quotient of whole numbers has the default type)
     ratio = torch.empty((), dtype=torch.float32, device=true_counts.device)
@@ -59,16 +63,19 @@ def _anchor_attn(Q, K, V, sm_scale=None, block_size=64, step=16, difference=100,
     output = torch.empty_like(Q) if out is None else out
     assert output.shape == Q.shape and output.dtype == Q.dtype and output.stride(-1) == 1
     ws = _workspace(B, H, N, D, block_size, step, Q.device)
-    n_bb = N // (block_size * step)
-    counts = torch.empty((B, H, n_bb, 1), dtype=torch.int32, device=Q.device) if return_sparsity_ratio else None
-    _hip.check(_hip.lib().aa_anchor_attn_fwd(
-        *_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output),
-        ws.data_ptr(), ws.numel(), counts.data_ptr() if counts is not None else None,
-        B, H, K.shape[1], N, D, block_size, step, float(sm_scale), float(difference), scale_mode, int(geometry),
-        _hip.dtype_code(Q), _stream()))
-    if return_sparsity_ratio:
-        return output, _ratio(counts, B, H, N, block_size, step)
-    return output, 1.0
+    tensors = (*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output), ws.data_ptr(), ws.numel())
+    sizes = (B, H, K.shape[1], N, D, block_size, step, float(sm_scale), float(difference), scale_mode, int(geometry),
+             _hip.dtype_code(Q), _stream())
+    if not return_sparsity_ratio:
+        _hip.check(_hip.lib().aa_anchor_attn_fwd(*tensors, None, *sizes))
+        return output, 1.0
+    if torch.get_default_dtype() == torch.float32:
+        ratio = torch.empty((), dtype=torch.float32, device=Q.device)
+        _hip.check(_hip.lib().aa_anchor_attn_ratio_fwd(*tensors, ratio.data_ptr(), _ratio_denominator(B, H, N, block_size, step), *sizes))
+        return output, ratio
+    counts = torch.empty((B, H, N // (block_size * step), 1), dtype=torch.int32, device=Q.device)
+    _hip.check(_hip.lib().aa_anchor_attn_fwd(*tensors, counts.data_ptr(), *sizes))
+    return output, _ratio(counts, B, H, N, block_size, step)
 
 
 def _stage3(Q, K, V, coords, counts, L, M, Acc, sm_scale, block_size, step, out=None):

@@ -238,14 +238,19 @@ size_t aa_workspace_bytes(int batch, int n_q_heads, int n_ctx, int head_dim, int
   return carve(batch, n_q_heads, n_ctx, head_dim, block_size, step).total;
 }
 
-// Stage 1; with qbar/abar non-null (block_size <= 128) the kernel also emits the pooled queries and anchors, with `out`
-// non-null the output of big block 0, whose rows select no keys, in the place of their state and pooled rows.
+// What stage 1 does for the stages after it in the whole operator.
+struct Stage1Extras {
+  void* qbar; void* abar;  // pooled queries and anchors (block_size <= 128)
+  float* thr; float scale2, theta_log2;  // and the thresholds of the pooled rows
+  // the output of big block 0, whose rows select no keys, in the place of their state and pooled rows
+  void* out; int64_t o_sb, o_sh, o_sn;
+  int32_t* zero_counts; float* zero_ratio;  // a single big block: what the later stages would say
+};
+
 static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                        const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
-                       float* M, float* L, float* acc_frag, void* qbar, void* abar,
-                       void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
-                       int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                       float* M, float* L, float* acc_frag, const Stage1Extras& x, int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                        int block_size, int step, float sm_scale, int scale_mode, int dtype, void* stream) {
   int rc;
   if ((rc = check_dims({batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step}, who))) return rc;
@@ -263,8 +268,10 @@ static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_s
   a.k = (const uint16_t*)k; a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
   a.v = (const uint16_t*)v; a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn;
   a.M_out = M; a.L_out = L; a.acc_out = acc_frag;
-  a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
-  a.qbar_out = (uint16_t*)qbar; a.abar_out = (uint16_t*)abar;
+  a.out = (uint16_t*)x.out; a.o_sb = x.o_sb; a.o_sh = x.o_sh; a.o_sn = x.o_sn;
+  a.qbar_out = (uint16_t*)x.qbar; a.abar_out = (uint16_t*)x.abar;
+  a.thr_out = reinterpret_cast<uint32_t*>(x.thr); a.scale2 = x.scale2; a.theta_log2 = x.theta_log2;
+  a.zero_counts = x.zero_counts; a.ratio = x.zero_ratio;
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size;
   a.sm_scale = sm_scale; a.scale_mode = scale_mode; a.dtype = dtype;
@@ -277,8 +284,8 @@ int aa_stage1_anchor_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
                          float* M, float* L, float* acc_frag,
                          int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                          int block_size, int step, float sm_scale, int scale_mode, int dtype, void* stream) {
-  return stage1_impl("aa_stage1_anchor_fwd", q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc_frag, nullptr,
-                     nullptr, nullptr, 0, 0, 0, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, scale_mode, dtype, stream);
+  return stage1_impl("aa_stage1_anchor_fwd", q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc_frag, Stage1Extras{},
+                     batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, scale_mode, dtype, stream);
 }
 
 int aa_pool_q_anchor(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn, const float* M,
@@ -297,12 +304,14 @@ int aa_pool_q_anchor(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn, co
   return check_launch(launch_pool(a, (hipStream_t)stream), who);
 }
 
-int aa_stage2_select(const void* qbar, const void* abar,
+static float select_scale2(double sm_scale) { return (float)(sm_scale * 1.44269504); }  // double product, then float32, as the definition does
+
+// Stage 2; have_thresholds: stage 1 has formed them.
+static int stage2_impl(const char* who, bool have_thresholds, const void* qbar, const void* abar,
                      const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                      uint32_t* mask_ws, int32_t* coords, int32_t* counts,
                      int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                      int block_size, int step, double sm_scale, float theta_log2, int geometry, int dtype, void* stream) {
-  const char* who = "aa_stage2_select";
   int rc;
   if ((rc = check_dtype(dtype, who))) return rc;
   const Dims dims = {batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step};
@@ -319,16 +328,25 @@ int aa_stage2_select(const void* qbar, const void* abar,
   a.coords_per_head = aa_coords_entries_per_head(n_ctx, block_size, step);
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size;
-  a.scale2 = (float)(sm_scale * 1.44269504);  // double product, then float32, as the definition does
+  a.scale2 = select_scale2(sm_scale);
   a.theta_log2 = theta_log2;
   a.dtype = dtype;
   a.key_lo = geometry == AA_GEOMETRY_AS_RUN ? block_size : block_size * step;
   a.key_slack = geometry == AA_GEOMETRY_AS_RUN ? block_size : 0;
   if (n_ctx > block_size * step) {  // (a single big block has no candidates: its counts are 0)
-    if ((rc = check_launch(launch_select_thresholds(a, (hipStream_t)stream), who))) return rc;
+    if (!have_thresholds && (rc = check_launch(launch_select_thresholds(a, (hipStream_t)stream), who))) return rc;
     if ((rc = check_launch(launch_select_scores(a, (hipStream_t)stream), who))) return rc;
   }
   return check_launch(launch_select_compact(a, (hipStream_t)stream), who);
+}
+
+int aa_stage2_select(const void* qbar, const void* abar,
+                     const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                     uint32_t* mask_ws, int32_t* coords, int32_t* counts,
+                     int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                     int block_size, int step, double sm_scale, float theta_log2, int geometry, int dtype, void* stream) {
+  return stage2_impl("aa_stage2_select", false, qbar, abar, k, k_sb, k_sh, k_sn, mask_ws, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
+                     head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream);
 }
 
 int aa_stage2_select_static(const void* qbar, const void* abar,
@@ -352,8 +370,8 @@ int aa_stage2_select_static(const void* qbar, const void* abar,
                           n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream);
 }
 
-// Stage 3 for the rows from big block `first_big_block` (0 or 1) on.
-static int stage3_impl(const char* who, int first_big_block,
+// Stage 3 for the rows from big block `first_big_block` (0 or 1) on; with `ratio`, also the sum of all counts over `denominator`.
+static int stage3_impl(const char* who, int first_big_block, float* ratio, double denominator,
                        const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                          const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                          const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
@@ -383,6 +401,7 @@ static int stage3_impl(const char* who, int first_big_block,
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size; a.first_big_block = first_big_block;
   a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
+  a.ratio = ratio; a.n_ratio_counts = (int64_t)batch * n_q_heads * (n_ctx / a.big_block); a.ratio_inverse = 1.f / (float)denominator;
   return check_launch(run_flash(a, 1, (hipStream_t)stream), who);
 }
 
@@ -394,19 +413,19 @@ int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
                          void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
                          int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                          int block_size, int step, float sm_scale, int dtype, void* stream) {
-  return stage3_impl("aa_stage3_sparse_fwd", 0, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc_frag,
+  return stage3_impl("aa_stage3_sparse_fwd", 0, nullptr, 1.0, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc_frag,
                      out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, dtype, stream);
 }
 
-int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+// The whole operator; with `ratio` the counts are kept in the workspace and their sum over `denominator` is formed.
+static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                        const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                        void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
-                       void* workspace, size_t workspace_bytes, int32_t* counts_out,
+                       void* workspace, size_t workspace_bytes, int32_t* counts_out, float* ratio, double denominator,
                        int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                        int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
                        int dtype, void* stream) {
-  const char* who = "aa_anchor_attn_fwd";
   int rc;
   // (all that a later stage could refuse is looked at first: stage 1 already writes the first big block's output)
   const Dims dims = {batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step};
@@ -430,30 +449,70 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   int32_t* counts = counts_direct ? counts_out : (int32_t*)(ws + w.counts);
   if ((rc = check_tensor(out, o_sb, o_sh, o_sn, n_ctx, head_dim, who, "out"))) return rc;
   // A stage-1 work-group holds 128 query rows: whole pooled rows when block_size <= 128, and then it pools them itself
-  // (same arithmetic as aa_pool_q_anchor, bit for bit) instead of a separate pass over the queries.
+  // (same arithmetic as aa_pool_q_anchor, bit for bit) and finds their thresholds instead of a pass over the queries and a launch.
   const bool fused_pool = block_size <= 128;
-  if ((rc = stage1_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc, fused_pool ? qbar : nullptr,
-                        fused_pool ? abar : nullptr, out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step,
-                        (float)sm_scale, scale_mode, dtype, stream)))
-    return rc;
-  // Big block 0 selects nothing and is finished by now; stages 2 and 3 are for the others.
+  // Big block 0 selects nothing and is finished by stage 1; stages 2 and 3 are for the others.
   const bool selects = n_ctx > block_size * step;
-  if (!fused_pool && selects &&
-      (rc = aa_pool_q_anchor(q, q_sb, q_sh, q_sn, M, qbar, abar, batch, n_q_heads, n_ctx, head_dim, block_size, dtype, stream)))
+  Stage1Extras x = {};
+  if (fused_pool) {
+    x.qbar = qbar; x.abar = abar;
+    x.thr = reinterpret_cast<float*>(mask + mask_bit_words(batch, n_q_heads, n_ctx, block_size, step));
+    x.scale2 = select_scale2(sm_scale); x.theta_log2 = theta_log2;
+  }
+  x.out = out; x.o_sb = o_sb; x.o_sh = o_sh; x.o_sn = o_sn;
+  if (!selects) { x.zero_counts = counts; x.zero_ratio = ratio; }
+  if ((rc = stage1_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc, x, batch, n_q_heads, n_kv_heads,
+                        n_ctx, head_dim, block_size, step, (float)sm_scale, scale_mode, dtype, stream)))
     return rc;
-  if ((rc = aa_stage2_select(qbar, abar, k, k_sb, k_sh, k_sn, mask, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
-                             head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream)))
-    return rc;
-  if ((rc = stage3_impl(who, 1, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc, out,
-                                 o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, (float)sm_scale,
-                                 dtype, stream)))
-    return rc;
+  if (selects) {
+    if (!fused_pool &&
+        (rc = aa_pool_q_anchor(q, q_sb, q_sh, q_sn, M, qbar, abar, batch, n_q_heads, n_ctx, head_dim, block_size, dtype, stream)))
+      return rc;
+    if ((rc = stage2_impl(who, fused_pool, qbar, abar, k, k_sb, k_sh, k_sn, mask, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
+                          head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream)))
+      return rc;
+    if ((rc = stage3_impl(who, 1, ratio, denominator, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc,
+                          out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, (float)sm_scale, dtype,
+                          stream)))
+      return rc;
+  }
   if (counts_out != nullptr && !counts_direct) {
     const size_t bytes = (size_t)batch * n_q_heads * (n_ctx / (block_size * step)) * 4;
     hipError_t e = hipMemcpyAsync(counts_out, counts, bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream);
     if ((rc = check_launch(e, who))) return rc;
   }
   return AA_OK;
+}
+
+int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                       const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                       const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                       void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                       void* workspace, size_t workspace_bytes, int32_t* counts_out,
+                       int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                       int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
+                       int dtype, void* stream) {
+  return anchor_attn_impl("aa_anchor_attn_fwd", q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, out, o_sb, o_sh, o_sn,
+                          workspace, workspace_bytes, counts_out, nullptr, 1.0, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size,
+                          step, sm_scale, theta_log2, scale_mode, geometry, dtype, stream);
+}
+
+int aa_anchor_attn_ratio_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                             const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                             const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                             void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                             void* workspace, size_t workspace_bytes, float* ratio, double denominator,
+                             int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                             int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
+                             int dtype, void* stream) {
+  const char* who = "aa_anchor_attn_ratio_fwd";
+  if (ratio == nullptr || !(denominator > 0.0)) {
+    set_error("%s: ratio must not be NULL and denominator (%g) must be positive", who, denominator);
+    return AA_EBADARG;
+  }
+  return anchor_attn_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, out, o_sb, o_sh, o_sn, workspace, workspace_bytes,
+                          nullptr, ratio, denominator, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, theta_log2,
+                          scale_mode, geometry, dtype, stream);
 }
 
 int aa_sparsity_ratio(const int32_t* counts, int64_t n, double denominator, float* ratio, void* stream) {

@@ -53,6 +53,7 @@
 #include "aa_common.h"
 #include "aa_kernels.h"
 #include "aa_nonfinite.h"
+#include "aa_threshold.h"
 
 namespace aa {
 
@@ -211,6 +212,11 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   // list's round trip to memory and the wait for its stores.
   const int group = p.n_q_heads / p.n_kv_heads;
   const int nq = MODE == kSparse ? p.q_blocks_per_wg : 1;
+  // (sparse) one work-group more than the query blocks need sums the counts to the ratio, beside the others
+  if (MODE == kSparse && p.ratio != nullptr && blockIdx.x + 1 == gridDim.x) {
+    sum_counts(p.counts, p.n_ratio_counts, p.ratio_inverse, p.ratio, reinterpret_cast<int64_t*>(sm.idx));
+    return;
+  }
   const int S = p.big_block;
   // (sparse mode may leave out the first big block, whose rows select nothing)
   const int n_qunit = kAnyRows ? 1 : (p.n_ctx - (MODE == kSparse ? p.first_big_block * S : 0)) / (BM * nq);
@@ -956,9 +962,9 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
           }
           reinterpret_cast<uint16_t*>(p.qbar_out)[((bh * n_pr) + R0 / bs + pp) * D + tid] = (uint16_t)(T::pack(a0 / d, 0.f) & 0xffffu);
         }
-      } else if (tid >= 128 && tid - 128 < n_pooled) {
-        // meanwhile, in wave 2: one thread per pooled anchor
-        const int pp = tid - 128;
+      } else if (wave == 2) {
+        // meanwhile, in wave 2: the pooled anchors, with all 64 lanes shared among them, and their thresholds
+        const int lanes = 64 / n_pooled, pp = lane / lanes;
         float am = 0.f;
         for (int r0 = pp * bs; r0 < (pp + 1) * bs; r0 += 16) {
           float w[16];
@@ -967,7 +973,13 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 #pragma unroll
           for (int t = 0; t < 16; ++t) am += w[t];
         }
-        reinterpret_cast<uint16_t*>(p.abar_out)[bh * n_pr + R0 / bs + pp] = (uint16_t)(T::pack(am / d, 0.f) & 0xffffu);
+        const uint32_t a16 = T::pack(am / d, 0.f) & 0xffffu;
+        const int64_t row = bh * n_pr + R0 / bs + pp;
+        if (lane % lanes == 0) reinterpret_cast<uint16_t*>(p.abar_out)[row] = (uint16_t)a16;
+        if (p.thr_out != nullptr) {
+          const uint32_t x = select_threshold<T>(T::from16((uint16_t)a16), p.scale2, p.theta_log2, lane, lanes);
+          if (lane % lanes == 0) p.thr_out[row] = x;
+        }
       }
     }
   } else if (kAnyRows && p.n_chunks > 1) {
@@ -1032,6 +1044,10 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     }
     chained = more && list_chains;
     have_queries = more;
+    if (MODE == kAnchor && R0 == 0 && tid == 0) {  // (a single big block: nothing is selected, and no later stage says so)
+      if (p.zero_counts != nullptr) p.zero_counts[bh] = 0;
+      if (p.ratio != nullptr && bh == 0) *p.ratio = 0.f;
+    }
   }
   }  // query blocks of the work-group
 }
@@ -1059,7 +1075,7 @@ static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
     a.q_blocks_per_wg = nq;
   }
   const dim3 grid(MODE == kRows || MODE == kMasked ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
-                                : (uint32_t)(blocks / a.q_blocks_per_wg)), block(256);
+                                : (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0)), block(256);
   if (a.head_dim == 128) {
     if (a.dtype == 0) hipLaunchKernelGGL((flash_kernel<MODE, Bf16, 128>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((flash_kernel<MODE, F16, 128>), grid, block, 0, stream, a);

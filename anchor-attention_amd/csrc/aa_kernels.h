@@ -13,6 +13,12 @@ struct FlashArgs {
   // anchor mode, optional (both or neither; block_size <= 128): the work-group also mean-pools its 128 raw query rows
   // and anchors into qbar [B,Hq,N/block_size,head_dim] and abar [B,Hq,N/block_size], bit for bit what pool_kernel computes
   uint16_t* qbar_out; uint16_t* abar_out;
+  // ... and, where it pools, the selection thresholds of its pooled rows (aa_threshold.h) into thr_out [B,Hq,N/block_size]
+  uint32_t* thr_out; float scale2, theta_log2;
+  // anchor mode, optional: [B,Hq], set to 0 where big block 0 is finished (the only one: nobody else writes its counts)
+  int32_t* zero_counts;
+  // anchor and sparse mode, optional: the ratio of selected keys, sum(counts[0 .. n_ratio_counts)) * ratio_inverse (anchor: 0)
+  float* ratio; int64_t n_ratio_counts; float ratio_inverse;
   const float* M; const float* L; const float* acc_frag;  // sparse mode (resume state)
   const int32_t* coords; const int32_t* counts; int64_t coords_per_head;  // sparse mode
   int batch, n_q_heads, n_kv_heads, n_ctx;

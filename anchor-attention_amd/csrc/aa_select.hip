@@ -10,15 +10,13 @@
 //           In the 32x32 accumulator a lane holds one key column; OR-ing its registers over the pooled
 //           rows of a big block and a wave ballot give a 32-bit key mask per (q head, big block, key
 //           block) with no LDS and no atomics.
-//  thresholds  the as-specified test "float(bf16(raw * scale)) + theta >= anchor" is monotone in the raw
-//           float32 dot product, so for every pooled row there is one float32 number x* with
-//           "test passes  <=>  raw >= x*".  A tiny kernel finds x* per pooled row by bisection over
-//           the ordered float32 bit patterns, evaluating the test exactly as written; the score
-//           kernel's epilogue is then a single compare per element.
+//  thresholds  the selection test as a threshold on the raw dot product (aa_threshold.h), so that the score
+//           kernel's epilogue is a single compare per element; stage 1 forms them where it pools.
 //  compact  one wave per (batch, q head, big block) turns that big block's mask row into an ascending
 //           index list with popcounts and a wave prefix sum.
 #include "aa_common.h"
 #include "aa_kernels.h"
+#include "aa_threshold.h"
 
 namespace aa {
 
@@ -76,42 +74,22 @@ hipError_t launch_pool(const PoolArgs& a, hipStream_t stream) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Smallest float32 x with  float(round16(x * scale2)) + theta >= anchor  (NaN if there is none); round16 rounds to the
-// tensors' 16-bit type.
+// Thresholds of given anchors: eight lanes to a row, eleven rounds.
+constexpr int kThrLanes = 8;
 template <typename T>
-__device__ __forceinline__ bool select_test(const float x, const float scale2, const float theta, const float anchor) {
-  const float sc = T::round_product(x, scale2);  // the score as (dot * scale).to(dtype) evaluates it for this type
-  return (sc + theta) >= anchor;      // float32 add and compare, non-strict
-}
-__device__ __forceinline__ float ordered_to_float(const uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k ^ 0x80000000u) : ~k);  // monotone bijection uint32 -> float32
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) select_threshold_kernel(const uint16_t* __restrict__ abar, float* __restrict__ thr, const int n,
+__global__ void __launch_bounds__(256) select_threshold_kernel(const uint16_t* __restrict__ abar, uint32_t* __restrict__ thr, const int n,
                                                                 const float scale2, const float theta) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const float anchor = T::from16(abar[i]);
-  // ordered keys: 0x007fffff <-> -inf, 0xff800000 <-> +inf (NaNs lie outside that range)
-  uint32_t lo = 0x007fffffu, hi = 0xff800000u;
-  float out;
-  if (!select_test<T>(ordered_to_float(hi), scale2, theta, anchor)) {
-    out = __uint_as_float(0x7fc00000u);  // no float passes: NaN compares false with everything
-  } else {
-    while (lo < hi) {  // invariant: test(hi) is true
-      const uint32_t mid = lo + ((hi - lo) >> 1);
-      if (select_test<T>(ordered_to_float(mid), scale2, theta, anchor)) hi = mid; else lo = mid + 1;
-    }
-    out = ordered_to_float(hi);
-  }
-  thr[i] = out;
+  const int i = min((int)(blockIdx.x * (256 / kThrLanes) + threadIdx.x / kThrLanes), n - 1);  // (past the end: the last row again, all lanes active)
+  const uint32_t x = select_threshold<T>(T::from16(abar[i]), scale2, theta, threadIdx.x & 63, kThrLanes);
+  if (threadIdx.x % kThrLanes == 0) thr[i] = x;
 }
 
 hipError_t launch_select_thresholds(const SelectArgs& a, hipStream_t stream) {
   const int n = a.batch * a.n_q_heads * (a.n_ctx / a.block_size);
-  if (a.dtype == 0) hipLaunchKernelGGL(select_threshold_kernel<Bf16>, dim3((n + 255) / 256), dim3(256), 0, stream, a.abar, a.thr, n, a.scale2, a.theta_log2);
-  else hipLaunchKernelGGL(select_threshold_kernel<F16>, dim3((n + 255) / 256), dim3(256), 0, stream, a.abar, a.thr, n, a.scale2, a.theta_log2);
+  const dim3 grid((n + 256 / kThrLanes - 1) / (256 / kThrLanes));
+  uint32_t* thr = reinterpret_cast<uint32_t*>(a.thr);
+  if (a.dtype == 0) hipLaunchKernelGGL(select_threshold_kernel<Bf16>, grid, dim3(256), 0, stream, a.abar, thr, n, a.scale2, a.theta_log2);
+  else hipLaunchKernelGGL(select_threshold_kernel<F16>, grid, dim3(256), 0, stream, a.abar, thr, n, a.scale2, a.theta_log2);
   return hipGetLastError();
 }
 
@@ -381,18 +359,10 @@ hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The share of selected keys: a few KB of counts summed by one work-group, bound by its launch.  The framework's sum and
-// division of the same counts were four launches (conversion, sum, a scalar's copy, division), 14 us of the 207 us that the
-// operator took on 4096 tokens with 32/8 heads of 128.
+// The share of selected keys where the operator's last launch has not formed it.
 __global__ void __launch_bounds__(256) ratio_kernel(const int32_t* counts, const int64_t n, const float inverse, float* ratio) {
-  __shared__ long long part[4];
-  long long sum = 0;
-  for (int64_t i = threadIdx.x; i < n; i += 256) sum += counts[i];
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, 64);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
-  __syncthreads();
-  if (threadIdx.x == 0) *ratio = (float)(part[0] + part[1] + part[2] + part[3]) * inverse;
+  __shared__ int64_t part[4];
+  sum_counts(counts, n, inverse, ratio, part);
 }
 
 hipError_t launch_ratio(const int32_t* counts, int64_t n, float inverse, float* ratio, hipStream_t stream) {

@@ -170,6 +170,17 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
                        int dtype, void* stream);
 
+/* The same with the sparsity ratio in the place of the counts: *ratio is what aa_sparsity_ratio() forms of all counts and
+ * `denominator` (which must be positive), by the operator's own launches. */
+int aa_anchor_attn_ratio_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                             const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                             const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                             void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                             void* workspace, size_t workspace_bytes, float* ratio, double denominator,
+                             int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                             int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
+                             int dtype, void* stream);
+
 /* sum(counts[0 .. n)) / denominator as one float32 on the device: the sparsity ratio of anchor_attn_v4.py:270-272, with the
  * sum in 64-bit integers, rounded to float32 and multiplied by float32(1 / denominator). */
 int aa_sparsity_ratio(const int32_t* counts, int64_t n, double denominator, float* ratio, void* stream);
