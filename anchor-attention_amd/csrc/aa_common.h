@@ -165,9 +165,18 @@ __host__ __device__ inline int64_t coords_tri(int64_t bb, int64_t S, int64_t bs)
 //   8 % n_units == 0 : s = 8 / n_units XCDs share a unit and take its rows alternately (row = idx / inner, the
 //                      `inner` work-groups of a row stay together), so that each gets the same mix of heavy and light;
 //   otherwise        : the hardware order is kept.
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uint32_t per_unit, uint32_t inner) {
+// `abreast`: an XCD takes its units (in the last case: all XCDs all units) side by side, the heaviest of each first, instead of one
+// after the other, so that the launch does not end with the heaviest work-groups of its last unit.
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uint32_t per_unit, uint32_t inner, bool abreast) {
   const uint32_t total = n_units * per_unit;
   const uint32_t xcd = wg % 8u, k = wg / 8u;
+  if (abreast) {
+    if (total % 8u != 0u || n_units % 8u != 0u) return wg % n_units * per_unit + wg / n_units;
+    // (the XCD's 32 CUs are filled in turn: without the rotation a number of units that divides 32 ties a CU to a unit, and
+    // units differ in weight: two prompts of 3900, one padded, 239 us one after the other, 280 without it and 239 with it)
+    const uint32_t own = n_units / 8u, turn = 32u % own == 0u ? k / 32u : 0u;
+    return ((k + turn) % own * 8u + xcd) * per_unit + k / own;
+  }
   if (total % 8u != 0u) return wg;
   if (n_units % 8u == 0u) return (k / per_unit * 8u + xcd) * per_unit + k % per_unit;
   if (8u % n_units == 0u) {

@@ -244,14 +244,14 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // A work-group owns 128 columns of one KV head - a column is one (query row, head of the group) pair, heads running
     // fastest, so all heads of a group use the same K/V tile - and one chunk of the keys.  Work-groups of one chunk are
     // neighbours on one XCD (they read the same K/V rows), latest columns, which see the most keys, first.
-    uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, p.n_col_blocks * p.n_chunks, 1);
+    uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, p.n_col_blocks * p.n_chunks, 1, p.abreast);
     qunit = p.n_col_blocks - 1 - (int)(vid % p.n_col_blocks);  vid /= p.n_col_blocks;
     chunk = vid % p.n_chunks;  vid /= p.n_chunks;
     kvh = vid % p.n_kv_heads;
     b = vid / p.n_kv_heads;
     g = 0;
   } else {
-    uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, group * n_qunit, group);
+    uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, group * n_qunit, group, p.abreast);
     g = vid % group;  vid /= group;
     qunit = vid % n_qunit;  vid /= n_qunit;
     kvh = vid % p.n_kv_heads;
@@ -1076,6 +1076,11 @@ static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
   }
   const dim3 grid(MODE == kRows || MODE == kMasked ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
                                 : (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0)), block(256);
+  // More units (KV heads of all batch elements) than XCDs: side by side as long as the K and V that an XCD then works on fit its L2
+  // of 4 MB.  Left-padded batches: 3 x 2500 with 32/8 heads of 128 194 -> 184 us, 28/4 184 -> 162, 3 x 1000 with 32/8 heads of 64 39.9 -> 30.0, 4 x 2900
+  // 162 -> 150; the operator on 2 x 4096 tokens with those heads 181 -> 172.  Larger contexts, where the order hardly matters: within 1 %.
+  const int units = a.batch * a.n_kv_heads;
+  a.abreast = MODE != kSparse && 8 % units != 0 && (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20;
   if (a.head_dim == 128) {
     if (a.dtype == 0) hipLaunchKernelGGL((flash_kernel<MODE, Bf16, 128>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((flash_kernel<MODE, F16, 128>), grid, block, 0, stream, a);

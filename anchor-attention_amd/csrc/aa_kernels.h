@@ -27,6 +27,7 @@ struct FlashArgs {
   int first_big_block;  // sparse mode: 1 leaves out the rows of big block 0 (anchor mode has finished them), 0 takes all rows
   float sm_scale; int scale_mode;
   int q_blocks_per_wg;  // set by the launcher
+  bool abreast;         // set by the launcher: see xcd_remap
   // rows mode: n_rows query rows over n_ctx keys, row i sees keys 0 .. causal_offset + i.  The (row, head) columns of a
   // KV head come in blocks of 128, the keys in chunks of chunk_tiles 64-key tiles; with more than one chunk the work-groups
   // write M_out, L_out, acc_out [batch, n_kv_heads, n_col_blocks, n_chunks, 128 columns] for rows_combine_kernel
