@@ -45,7 +45,8 @@ _SIGNATURES = {
     "aa_stage2_select_static": (c_int, [c_void_p, c_void_p] + _T3 + [c_void_p] * 2 + _DIMS5 + [c_int, c_int, c_double, c_float, c_int, c_int, c_void_p]),
     "aa_stage3_sparse_fwd": (c_int, _T3 * 3 + [c_void_p] * 5 + _T3 + _DIMS5 + [c_int, c_int, c_float, c_int, c_void_p]),
     "aa_anchor_attn_fwd": (c_int, _T3 * 4 + [c_void_p, c_size_t, c_void_p] + _DIMS5 + [c_int, c_int, c_double, c_float, c_int, c_int, c_int, c_void_p]),
-    "aa_anchor_attn_ratio_fwd": (c_int, _T3 * 4 + [c_void_p, c_size_t, c_void_p, c_double] + _DIMS5 + [c_int, c_int, c_double, c_float, c_int, c_int, c_int, c_void_p]),
+    "aa_anchor_attn_ratio_fwd": (c_int, _T3 * 4 + [c_void_p, c_size_t, c_void_p, c_void_p, c_double] + _DIMS5 + [c_int, c_int, c_double, c_float, c_int, c_int, c_int, c_void_p]),
+    "aa_wait_ratio": (c_int, [c_void_p, c_float, c_int]),
     "aa_sparsity_ratio": (c_int, [c_void_p, c_int64, c_double, c_void_p, c_void_p]),
     "aa_dense_causal_fwd": (c_int, _T3 * 4 + _DIMS5 + [c_float, c_int, c_void_p]),
     # batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset (, masked)
@@ -104,6 +105,6 @@ def dtype_code(t) -> int:
 
 def t3(t):
     """(data_ptr, stride_b, stride_h, stride_n) of a [B,H,N,D] tensor whose last stride is 1."""
-    assert t.dim() == 4 and t.stride(3) == 1
-    sb, sh, sn, _ = t.stride()
-    return (t.data_ptr(), sb, sh, sn)
+    strides = t.stride()
+    assert len(strides) == 4 and strides[3] == 1
+    return (t.data_ptr(), *strides[:3])

@@ -1,5 +1,6 @@
 // C ABI of the AnchorAttention gfx950 kernels: argument validation, scratch carving, launches.
 // Declarations and their reference counterparts: include/anchor_attn_hip.h.
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -244,7 +245,7 @@ struct Stage1Extras {
   float* thr; float scale2, theta_log2;  // and the thresholds of the pooled rows
   // the output of big block 0, whose rows select no keys, in the place of their state and pooled rows
   void* out; int64_t o_sb, o_sh, o_sn;
-  int32_t* zero_counts; float* zero_ratio;  // a single big block: what the later stages would say
+  int32_t* zero_counts; float* zero_ratio; float* zero_ratio_host;  // a single big block: what the later stages would say
 };
 
 static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
@@ -271,7 +272,7 @@ static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_s
   a.out = (uint16_t*)x.out; a.o_sb = x.o_sb; a.o_sh = x.o_sh; a.o_sn = x.o_sn;
   a.qbar_out = (uint16_t*)x.qbar; a.abar_out = (uint16_t*)x.abar;
   a.thr_out = reinterpret_cast<uint32_t*>(x.thr); a.scale2 = x.scale2; a.theta_log2 = x.theta_log2;
-  a.zero_counts = x.zero_counts; a.ratio = x.zero_ratio;
+  a.zero_counts = x.zero_counts; a.ratio = x.zero_ratio; a.ratio_host = x.zero_ratio_host;
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size;
   a.sm_scale = sm_scale; a.scale_mode = scale_mode; a.dtype = dtype;
@@ -371,7 +372,7 @@ int aa_stage2_select_static(const void* qbar, const void* abar,
 }
 
 // Stage 3 for the rows from big block `first_big_block` (0 or 1) on; with `ratio`, also the sum of all counts over `denominator`.
-static int stage3_impl(const char* who, int first_big_block, float* ratio, double denominator,
+static int stage3_impl(const char* who, int first_big_block, float* ratio, float* ratio_host, double denominator,
                        const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                          const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                          const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
@@ -401,7 +402,7 @@ static int stage3_impl(const char* who, int first_big_block, float* ratio, doubl
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size; a.first_big_block = first_big_block;
   a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
-  a.ratio = ratio; a.n_ratio_counts = (int64_t)batch * n_q_heads * (n_ctx / a.big_block); a.ratio_inverse = 1.f / (float)denominator;
+  a.ratio = ratio; a.ratio_host = ratio_host; a.n_ratio_counts = (int64_t)batch * n_q_heads * (n_ctx / a.big_block); a.ratio_inverse = 1.f / (float)denominator;
   return check_launch(run_flash(a, 1, (hipStream_t)stream), who);
 }
 
@@ -413,7 +414,7 @@ int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
                          void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
                          int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                          int block_size, int step, float sm_scale, int dtype, void* stream) {
-  return stage3_impl("aa_stage3_sparse_fwd", 0, nullptr, 1.0, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc_frag,
+  return stage3_impl("aa_stage3_sparse_fwd", 0, nullptr, nullptr, 1.0, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc_frag,
                      out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, dtype, stream);
 }
 
@@ -422,7 +423,7 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
                        const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                        const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                        void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
-                       void* workspace, size_t workspace_bytes, int32_t* counts_out, float* ratio, double denominator,
+                       void* workspace, size_t workspace_bytes, int32_t* counts_out, float* ratio, float* ratio_host, double denominator,
                        int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                        int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
                        int dtype, void* stream) {
@@ -460,7 +461,7 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
     x.scale2 = select_scale2(sm_scale); x.theta_log2 = theta_log2;
   }
   x.out = out; x.o_sb = o_sb; x.o_sh = o_sh; x.o_sn = o_sn;
-  if (!selects) { x.zero_counts = counts; x.zero_ratio = ratio; }
+  if (!selects) { x.zero_counts = counts; x.zero_ratio = ratio; x.zero_ratio_host = ratio_host; }
   if ((rc = stage1_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc, x, batch, n_q_heads, n_kv_heads,
                         n_ctx, head_dim, block_size, step, (float)sm_scale, scale_mode, dtype, stream)))
     return rc;
@@ -471,7 +472,7 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
     if ((rc = stage2_impl(who, fused_pool, qbar, abar, k, k_sb, k_sh, k_sn, mask, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
                           head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream)))
       return rc;
-    if ((rc = stage3_impl(who, 1, ratio, denominator, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc,
+    if ((rc = stage3_impl(who, 1, ratio, ratio_host, denominator, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc,
                           out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, (float)sm_scale, dtype,
                           stream)))
       return rc;
@@ -493,7 +494,7 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
                        int dtype, void* stream) {
   return anchor_attn_impl("aa_anchor_attn_fwd", q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, out, o_sb, o_sh, o_sn,
-                          workspace, workspace_bytes, counts_out, nullptr, 1.0, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size,
+                          workspace, workspace_bytes, counts_out, nullptr, nullptr, 1.0, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size,
                           step, sm_scale, theta_log2, scale_mode, geometry, dtype, stream);
 }
 
@@ -501,7 +502,7 @@ int aa_anchor_attn_ratio_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t 
                              const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                              const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                              void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
-                             void* workspace, size_t workspace_bytes, float* ratio, double denominator,
+                             void* workspace, size_t workspace_bytes, float* ratio, float* ratio_host, double denominator,
                              int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                              int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
                              int dtype, void* stream) {
@@ -511,8 +512,20 @@ int aa_anchor_attn_ratio_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t 
     return AA_EBADARG;
   }
   return anchor_attn_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, out, o_sb, o_sh, o_sn, workspace, workspace_bytes,
-                          nullptr, ratio, denominator, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, theta_log2,
+                          nullptr, ratio, ratio_host, denominator, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, theta_log2,
                           scale_mode, geometry, dtype, stream);
+}
+
+int aa_wait_ratio(const float* ratio_host, float unset, int timeout_us) {
+  const volatile float* word = ratio_host;
+  const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(timeout_us);
+  for (;;) {
+    for (int i = 0; i < 32; ++i) {
+      if (*word != unset) return 1;
+      __builtin_ia32_pause();
+    }
+    if (std::chrono::steady_clock::now() >= end) return *word != unset;
+  }
 }
 
 int aa_sparsity_ratio(const int32_t* counts, int64_t n, double denominator, float* ratio, void* stream) {

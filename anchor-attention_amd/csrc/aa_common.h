@@ -138,14 +138,19 @@ __device__ __forceinline__ float max_with_other_half(float v) {
 // The share of selected keys, sum(counts[0 .. n)) * inverse, by one work-group of 256 threads: a few KB, bound by the latency of
 // a round trip or two.  `part`: four words of LDS.  (As a launch of its own 5.8 us of the 198 us of the operator on 4096 tokens with
 // 32/8 heads of 128, and the framework's sum and division, four launches, 14 us.)
-__device__ __forceinline__ void sum_counts(const int32_t* counts, const int64_t n, const float inverse, float* ratio, int64_t* part) {
+__device__ __forceinline__ void store_ratio(const float x, float* ratio, float* ratio_host) {
+  *ratio = x;
+  if (ratio_host != nullptr) __hip_atomic_store(ratio_host, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void sum_counts(const int32_t* counts, const int64_t n, const float inverse, float* ratio, float* ratio_host,
+                                           int64_t* part) {
   int64_t sum = 0;
   for (int64_t i = threadIdx.x; i < n; i += 256) sum += counts[i];
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor((long long)sum, d, 64);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
   __syncthreads();
-  if (threadIdx.x == 0) *ratio = (float)(part[0] + part[1] + part[2] + part[3]) * inverse;
+  if (threadIdx.x == 0) store_ratio((float)(part[0] + part[1] + part[2] + part[3]) * inverse, ratio, ratio_host);
 }
 
 // ---- geometry --------------------------------------------------------------------------------

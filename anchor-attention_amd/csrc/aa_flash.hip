@@ -212,11 +212,13 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   // list's round trip to memory and the wait for its stores.
   const int group = p.n_q_heads / p.n_kv_heads;
   const int nq = MODE == kSparse ? p.q_blocks_per_wg : 1;
-  // (sparse) one work-group more than the query blocks need sums the counts to the ratio, beside the others
-  if (MODE == kSparse && p.ratio != nullptr && blockIdx.x + 1 == gridDim.x) {
-    sum_counts(p.counts, p.n_ratio_counts, p.ratio_inverse, p.ratio, reinterpret_cast<int64_t*>(sm.idx));
+  // (sparse) one work-group more than the query blocks need, the first, sums the counts to the ratio beside the others
+  const bool sums = MODE == kSparse && p.ratio != nullptr;
+  if (sums && blockIdx.x == 0) {
+    sum_counts(p.counts, p.n_ratio_counts, p.ratio_inverse, p.ratio, p.ratio_host, reinterpret_cast<int64_t*>(sm.idx));
     return;
   }
+  const uint32_t wg = blockIdx.x - (sums ? 1u : 0u);
   const int S = p.big_block;
   // (sparse mode may leave out the first big block, whose rows select nothing)
   const int n_qunit = kAnyRows ? 1 : (p.n_ctx - (MODE == kSparse ? p.first_big_block * S : 0)) / (BM * nq);
@@ -231,7 +233,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // first, go round-robin over the XCDs with a rotation, so that every XCD sees every head and every depth.
     const uint32_t per_pair = (uint32_t)group * (uint32_t)(S / (BM * nq));  // work-groups of a pair
     const uint32_t n_units = (uint32_t)(p.batch * p.n_kv_heads);
-    const uint32_t xcd = blockIdx.x % 8u, k = blockIdx.x / 8u;
+    const uint32_t xcd = wg % 8u, k = wg / 8u;
     const uint32_t kp = k / per_pair, within = k % per_pair;
     const uint32_t pair = kp * 8u + (xcd + kp) % 8u;
     const int bb_ = p.n_ctx / S - 1 - (int)(pair / n_units);
@@ -244,14 +246,14 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // A work-group owns 128 columns of one KV head - a column is one (query row, head of the group) pair, heads running
     // fastest, so all heads of a group use the same K/V tile - and one chunk of the keys.  Work-groups of one chunk are
     // neighbours on one XCD (they read the same K/V rows), latest columns, which see the most keys, first.
-    uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, p.n_col_blocks * p.n_chunks, 1, p.abreast);
+    uint32_t vid = xcd_remap(wg, p.batch * p.n_kv_heads, p.n_col_blocks * p.n_chunks, 1, p.abreast);
     qunit = p.n_col_blocks - 1 - (int)(vid % p.n_col_blocks);  vid /= p.n_col_blocks;
     chunk = vid % p.n_chunks;  vid /= p.n_chunks;
     kvh = vid % p.n_kv_heads;
     b = vid / p.n_kv_heads;
     g = 0;
   } else {
-    uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, group * n_qunit, group, p.abreast);
+    uint32_t vid = xcd_remap(wg, p.batch * p.n_kv_heads, group * n_qunit, group, p.abreast);
     g = vid % group;  vid /= group;
     qunit = vid % n_qunit;  vid /= n_qunit;
     kvh = vid % p.n_kv_heads;
@@ -1046,7 +1048,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     have_queries = more;
     if (MODE == kAnchor && R0 == 0 && tid == 0) {  // (a single big block: nothing is selected, and no later stage says so)
       if (p.zero_counts != nullptr) p.zero_counts[bh] = 0;
-      if (p.ratio != nullptr && bh == 0) *p.ratio = 0.f;
+      if (p.ratio != nullptr && bh == 0) store_ratio(0.f, p.ratio, p.ratio_host);
     }
   }
   }  // query blocks of the work-group

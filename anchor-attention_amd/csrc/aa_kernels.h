@@ -19,6 +19,7 @@ struct FlashArgs {
   int32_t* zero_counts;
   // anchor and sparse mode, optional: the ratio of selected keys, sum(counts[0 .. n_ratio_counts)) * ratio_inverse (anchor: 0)
   float* ratio; int64_t n_ratio_counts; float ratio_inverse;
+  float* ratio_host;  // the same number in host memory, for a caller that waits for it and not for the launch to end
   const float* M; const float* L; const float* acc_frag;  // sparse mode (resume state)
   const int32_t* coords; const int32_t* counts; int64_t coords_per_head;  // sparse mode
   int batch, n_q_heads, n_kv_heads, n_ctx;

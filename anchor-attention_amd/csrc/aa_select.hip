@@ -362,7 +362,7 @@ hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream) {
 // The share of selected keys where the operator's last launch has not formed it.
 __global__ void __launch_bounds__(256) ratio_kernel(const int32_t* counts, const int64_t n, const float inverse, float* ratio) {
   __shared__ int64_t part[4];
-  sum_counts(counts, n, inverse, ratio, part);
+  sum_counts(counts, n, inverse, ratio, nullptr, part);
 }
 
 hipError_t launch_ratio(const int32_t* counts, int64_t n, float inverse, float* ratio, hipStream_t stream) {

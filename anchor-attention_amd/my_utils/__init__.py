@@ -15,15 +15,19 @@ class Logger:
         cls.log_file_path = os.path.join("log", path or str(time.time()))
 
     @classmethod
-    def log(cls, message: str):
+    def log(cls, message):
+        """``message``: a string, or a function that returns it - called with the file open, so that a message which has to be
+        fetched from the GPU is waited for last."""
         if not cls.enabled:
             return
         try:
             directory = os.path.dirname(cls.log_file_path)
             if directory:
                 os.makedirs(directory, exist_ok=True)
-            stamp = datetime.datetime.now().strftime("%Y-%m-%d %H:%M:%S.%f")[:-3]
             with open(cls.log_file_path, "a") as f:
+                if callable(message):
+                    message = message()
+                stamp = datetime.datetime.now().isoformat(" ", "milliseconds")
                 f.write(f"{stamp} - {message}\n")
         except OSError as e:
             print(f"Unable to write to log file: {e}")

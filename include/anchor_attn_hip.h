@@ -171,15 +171,20 @@ int aa_anchor_attn_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        int dtype, void* stream);
 
 /* The same with the sparsity ratio in the place of the counts: *ratio is what aa_sparsity_ratio() forms of all counts and
- * `denominator` (which must be positive), by the operator's own launches. */
+ * `denominator` (which must be positive), by the operator's own launches.  ratio_host (optional, may be NULL): a word of pinned host
+ * memory that the GPU can write; it receives the same number as soon as that is known, while stage 3 is still at work. */
 int aa_anchor_attn_ratio_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                              const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                              const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                              void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
-                             void* workspace, size_t workspace_bytes, float* ratio, double denominator,
+                             void* workspace, size_t workspace_bytes, float* ratio, float* ratio_host, double denominator,
                              int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                              int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
                              int dtype, void* stream);
+
+/* Host side: waits until *ratio_host differs from `unset`, which the caller has stored there before the launch (a ratio is never
+ * negative), for at most timeout_us microseconds.  Returns 1 if it does, 0 if the time is over. */
+int aa_wait_ratio(const float* ratio_host, float unset, int timeout_us);
 
 /* sum(counts[0 .. n)) / denominator as one float32 on the device: the sparsity ratio of anchor_attn_v4.py:270-272, with the
  * sum in 64-bit integers, rounded to float32 and multiplied by float32(1 / denominator). */
