@@ -10,6 +10,8 @@
 // factor that keeps small ones off the subnormals' grid, see kProbLog2).  That costs a second MFMA
 // per V operand (with one: 0.80 ms, 20 us and 0.19 ms) and brings the error against float64 from up to 1.02 times that of
 // library attention to the same (1.460e-3, 1.468e-3 with one, padded 3 x 1000, bf16).
+#include <cmath>
+
 #include "aa_common.h"
 #include "aa_kernels.h"
 
@@ -171,17 +173,20 @@ hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mas
   return hipGetLastError();
 }
 
-// How the keys of a rows-mode problem are cut into chunks.  The chip holds 512 work-groups (two per CU) at head dimension
-// 128 and 768 at 64.  Every number of chunks up to 64 is priced and the cheapest taken: the longest chain of tiles, or all tiles
-// over the chip's places, at a price per tile, and for several chunks one more launch and a write and a read of the state (64 KB per
-// column block and chunk at head dimension 128).
+// How the keys of a rows-mode problem are cut into chunks: every number of chunks up to 64 is priced and the cheapest taken.
 //
-// The prices are not the tile's times (a work-group alone on its CU takes 1.45 us a tile at head dimension 128 and 1.1 at 64, each
-// work-group of a full chip 3.1 and 2.9): the form knows nothing of how uneven column blocks fill the last round, and with these times it
-// takes counts that are 3.9 and 7.2 % slower than the best.  They are those for which it comes closest: with 75 sizes of each head dimension (40 to 5000
-// rows, up to 40000 keys, 1 to 16 KV heads, 1 to 8 heads a group) the count taken is 0.9 % slower than the best of fifteen on
-// average and 6.6 % at worst, 64: 2.7 and 15 %.  (Prices from the kernel with one MFMA per V operand, 1.1 and 1.9, 1.0 and 1.7 us a tile and
-// 6 us + 4 MB/us for the state: 1.8 and 17 %, 5.2 and 29 %: they cut 2047 rows with 32/8 heads of 64, 61.8 us against 48.3 whole.)
+// Work-groups are dealt to the CUs in turn, the ones with the most tiles first, so the CU that gets the longest chain of tiles gets, 256
+// work-groups on, its second one (head dimension 64: and a third) as long as the chip has room: a tile takes 1.1 us while a
+// work-group is alone on its CU and 1.8 beside another (64: 0.8, 1.1 and 1.3 beside two).  A launch takes as long as that CU or
+// as all tiles at the rate of a full chip, 0.9 us a tile and CU (64: 0.45) - the fourth powers are added, which lies between the larger and the sum - and
+// a part of a chain for the uneven end of more than one round.  Several chunks cost one more launch and a write and a read
+// of the state (64 KB per column block and chunk at head dimension 128).
+//
+// The prices are fitted to 192 sizes (20 to 5000 rows over up to 40000 keys, 2 to 32 KV heads in groups of 4 and 7, each with up to twelve
+// numbers of chunks): the number taken is 0.6 % slower than the best of the measured ones on average and 8.6 % at worst, 64: 0.9 and 10.6 %.  The form
+// before, which had the longest chain or the rounds of a full chip at one price, came to 2.4 and 26 %, 64: 3.5 and 23 %: it did not know that a few work-groups
+// more than CUs share them with the lightest ones (1194 rows, 28/4 heads of 128: 36.9 us in three chunks, 30.2 whole).  On 80 sizes that it was not
+// fitted to: 1.3 % on average and 11.6 % at worst, the form before 4.3 and 26 %; one of them in 40 is 6.7 % slower than before.
 //
 // A column block whose rows end later sees no fewer keys, so the blocks that reach a tile are counted in closed form and a plan costs the
 // same whatever the rows: with a loop over the column blocks for every count it took the host 276 us for 32768 rows over 65536 keys
@@ -196,7 +201,12 @@ void plan_rows(FlashArgs& a) {
   const int all_see = min(a.causal_offset / 64 + 1, max_tiles);
   int64_t total = (int64_t)all_see * a.n_col_blocks;  // tiles of one unit
   for (int t = all_see; t < max_tiles; ++t) total += blocks_at(t);
-  const int slots = a.head_dim == 128 ? 512 : 768;
+  const bool wide = a.head_dim == 128;
+  const int slots = wide ? 512 : 768;
+  const double alone = wide ? 1.07 : 0.835, beside_one = wide ? 1.81 : 1.105, beside_two = 1.306;  // us a tile
+  const double full_chip = wide ? 0.912 : 0.448, uneven_end = wide ? 0.616 : 0.098, one_round = wide ? 0.083 : 0.244;
+  const double merge = wide ? 2.65 : 1.57, merge_per_mb = wide ? 0.242 : 0.467;
+  const int64_t second = units <= 256 ? 256 / units : 1;  // the number, among a unit's work-groups, of the one that joins the first on its CU
   double best = 1e30;
   a.n_chunks = 1;
   a.chunk_tiles = max_tiles;
@@ -206,10 +216,18 @@ void plan_rows(FlashArgs& a) {
     int64_t wgs = 0;
     for (int c = 0; c < chunks; ++c) wgs += blocks_at(c * len);
     wgs *= units;
-    const double t_tile = a.head_dim == 128 ? (wgs <= 256 ? 1.5 : 1.8) : (wgs <= 256 ? 1.2 : 1.45);
-    const double rounds = (double)((wgs + slots - 1) / slots) * ((double)total * units / wgs);
-    double us = t_tile * (rounds > len ? rounds : len);
-    if (chunks > 1) us += a.head_dim == 128 ? 4.0 + (double)wgs * 128 * 128 * 8 / 4e6 : 2.0 + (double)wgs * 128 * 64 * 8 / 2e6;
+    // tiles of a unit's k-th work-group: latest column blocks first, chunk by chunk
+    auto tiles_of = [&](const int64_t k) {
+      if (k >= (int64_t)a.n_col_blocks * chunks) return 0;
+      const int block = a.n_col_blocks - 1 - (int)(k % a.n_col_blocks), last_row = (int)(min(128 * (int64_t)block + 128, (int64_t)a.n_rows * group) - 1) / group;
+      const int seen = min(a.causal_offset + last_row, a.n_ctx - 1) / 64 + 1;
+      return max(0, min(seen - (int)(k / a.n_col_blocks) * len, len));
+    };
+    const int t0 = tiles_of(0), t1 = min(tiles_of(second), t0), t2 = wide ? 0 : min(tiles_of(2 * second), t1);
+    const double chain = alone * (t0 - t1) + beside_one * (t1 - t2) + beside_two * t2, all = full_chip * (double)total * units / 256;
+    const double c2 = chain * chain, a2 = all * all;
+    double us = std::sqrt(std::sqrt(c2 * c2 + a2 * a2)) + (wgs > slots ? uneven_end * len : 0.0) + one_round * (double)wgs / slots;
+    if (chunks > 1) us += merge + merge_per_mb * (double)wgs * 128 * a.head_dim * 8 / 1e6;
     if (us < best) {
       best = us;
       a.n_chunks = chunks;
