@@ -8,10 +8,18 @@ transformers 4.45 sources (modules/llama/causal_model_forward.py:100-126, module
 Here both are thin wrappers around whatever forward the installed transformers has, so nothing is tied to one
 release: the causal-LM wrapper asks the model's own ``logits_to_keep`` mechanism for one position, the MLP wrapper
 calls the module's own forward on slices.
+
+``fuse_between_products`` changes no value either: the norms and the MLPs' activation and product, single operations of the
+framework with a pass over memory each, run as one kernel where nothing watches the single operations.
 """
 import functools
+import types
 
 import torch
+
+from anchor_attn.src.ops import _hip
+from anchor_attn.src.ops.anchor_attn_v4 import _called_plainly
+from anchor_attn.src.ops.anchor_step_1_2_v2 import _stream
 
 MLP_CHUNK_TOKENS = 32768  # the reference's chunk (llama_mlp_forward.py:52)
 
@@ -66,4 +74,93 @@ def chunk_mlp_over_tokens(model, chunk_tokens: int = MLP_CHUNK_TOKENS) -> int:
 
         forward._chunks_tokens = True
         m.forward = forward
+    return n
+
+
+def _kernel_takes(*tensors) -> bool:
+    """Plain 16-bit tensors on one GPU, contiguous on 16-byte boundaries, in an eager call that nothing differentiates or watches."""
+    first = tensors[0]
+    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda") or not _called_plainly():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != first.dtype or t.device != first.device or not t.is_contiguous():
+            return False
+        if (grad and t.requires_grad) or not 0 < t.numel() < 1 << 35 or t.data_ptr() & 15:
+            return False
+    return True
+
+
+def _launch(fn, device, *args) -> None:
+    if device.index == torch.cuda.current_device():
+        _hip.check(fn(*args, _stream()))
+    else:
+        with torch.cuda.device(device):
+            _hip.check(fn(*args, _stream()))
+
+
+def _rms_norm_forward(self, hidden_states):
+    weight = self.weight
+    n = hidden_states.shape[-1] if hidden_states.dim() else 0
+    if not (weight.shape == (n,) and n % 8 == 0 and 0 < n <= 16384 and hidden_states.numel() // n < 1 << 24
+            and _kernel_takes(hidden_states, weight)):
+        return type(self).forward(self, hidden_states)
+    out = torch.empty_like(hidden_states)
+    _launch(_hip.lib().aa_rms_norm, out.device, hidden_states.data_ptr(), weight.data_ptr(), out.data_ptr(), out.numel() // n, n,
+            float(self.variance_epsilon), _hip.dtype_code(out))
+    return out
+
+
+def _is_silu(act) -> bool:
+    """The framework's or transformers' SiLU module, and no hook that would see it called."""
+    return (type(act).__name__ in ("SiLU", "SiLUActivation") and not (act._forward_hooks or act._forward_pre_hooks)
+            and not (torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks))
+
+
+def _gated_mlp_forward(self, x):
+    if not (_kernel_takes(x) and _is_silu(self.act_fn)):
+        return type(self).forward(self, x)
+    gate, up = self.gate_proj(x), self.up_proj(x)
+    if gate.shape == up.shape and gate.numel() % 8 == 0 and _kernel_takes(gate, up):
+        h = torch.empty_like(gate)
+        _launch(_hip.lib().aa_silu_mul, h.device, gate.data_ptr(), up.data_ptr(), h.data_ptr(), h.numel(), _hip.dtype_code(h))
+    else:
+        h = self.act_fn(gate) * up
+    return self.down_proj(h)
+
+
+# (bound methods of these are copied with their module and pickled as its ``forward``, the class's own)
+_rms_norm_forward.__name__ = _gated_mlp_forward.__name__ = "forward"
+
+
+def _computes(cls, stub, x, want) -> bool:
+    """Whether the class's own forward does what the kernel would take over, bit for bit on a few numbers."""
+    try:
+        return torch.equal(cls.forward(stub, x), want)
+    except Exception:  # noqa: BLE001 - a class that works otherwise
+        return False
+
+
+def fuse_between_products(model) -> int:
+    """RMS norms and gated MLPs of the model's family whose classes compute what the kernels do, and whose instances have no
+    ``forward`` of their own, get one that uses the kernels.  Returns how many; calling it again changes nothing."""
+    x = torch.linspace(-3.0, 3.0, 32, dtype=torch.float32, device="cpu").reshape(2, 16).bfloat16()
+    norm = types.SimpleNamespace(weight=x[0] + 1.0, variance_epsilon=1e-3)
+    scaled = x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-3)
+    normed = norm.weight * scaled.to(x.dtype)
+    mlp = types.SimpleNamespace(gate_proj=lambda t: t * 3, up_proj=lambda t: t + 1, down_proj=lambda t: t * 0.5, act_fn=torch.nn.functional.silu)
+    gated = torch.nn.functional.silu(x * 3) * (x + 1) * 0.5
+    n = 0
+    with torch.no_grad():
+        for m in model.modules():
+            name, fused = type(m).__name__, None
+            if "forward" in m.__dict__:
+                continue
+            if name in ("LlamaRMSNorm", "Qwen2RMSNorm") and _computes(type(m), norm, x, normed):
+                fused = _rms_norm_forward
+            elif name in ("LlamaMLP", "Qwen2MLP") and _is_silu(getattr(m, "act_fn", None)) and _computes(type(m), mlp, x, gated):
+                fused = _gated_mlp_forward
+            if fused is not None:
+                m.forward = types.MethodType(fused, m)
+                n += 1
     return n

@@ -16,7 +16,7 @@ import json
 
 from my_utils import Logger
 
-from anchor_attn.src.modules.model_forward import MLP_CHUNK_TOKENS, chunk_mlp_over_tokens, keep_last_token_logits
+from anchor_attn.src.modules.model_forward import MLP_CHUNK_TOKENS, chunk_mlp_over_tokens, fuse_between_products, keep_last_token_logits
 
 ATTENTION_CONFIG_EXAMPLE = {
     "default": {},
@@ -101,6 +101,7 @@ def patch_model(model, pattern: str, config=None):
             setattr(model.config, k, v)
     if last_token_logits:
         keep_last_token_logits(model)
+    fuse_between_products(model)
     chunk_mlp_over_tokens(model, mlp_chunk_tokens)
     Logger.log(f"replace attention with {pattern}: {cfg}")
     return model

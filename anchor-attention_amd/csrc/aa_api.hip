@@ -681,4 +681,26 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   return a.n_chunks > 1 ? check_launch(launch_rows_combine(a, (hipStream_t)stream), who) : AA_OK;
 }
 
+int aa_rms_norm(const void* x, const void* weight, void* out, int64_t rows, int hidden, float eps, int dtype, void* stream) {
+  const char* who = "aa_rms_norm";
+  int rc;
+  if ((rc = check_dtype(dtype, who)) || (rc = check_ptr(x, who, "x")) || (rc = check_ptr(weight, who, "weight")) || (rc = check_ptr(out, who, "out"))) return rc;
+  if (rows <= 0 || rows > 0xffffff || hidden <= 0 || hidden > 16384 || hidden % 8 != 0) {  // (a launch takes less than 2^32 threads, 256 a row)
+    set_error("%s: %lld rows of %d elements are not supported (at most 2^24 - 1 rows of at most 16384, a multiple of 8)", who, (long long)rows, hidden);
+    return AA_EUNSUPPORTED;
+  }
+  return check_launch(launch_rms_norm((const uint16_t*)x, (const uint16_t*)weight, (uint16_t*)out, rows, hidden, eps, dtype, (hipStream_t)stream), who);
+}
+
+int aa_silu_mul(const void* gate, const void* up, void* out, int64_t n, int dtype, void* stream) {
+  const char* who = "aa_silu_mul";
+  int rc;
+  if ((rc = check_dtype(dtype, who)) || (rc = check_ptr(gate, who, "gate")) || (rc = check_ptr(up, who, "up")) || (rc = check_ptr(out, who, "out"))) return rc;
+  if (n <= 0 || n % 8 != 0 || n / 8 > 0xffffff00LL) {
+    set_error("%s: %lld elements are not supported (a multiple of 8, at most 2^35)", who, (long long)n);
+    return AA_EUNSUPPORTED;
+  }
+  return check_launch(launch_silu_mul((const uint16_t*)gate, (const uint16_t*)up, (uint16_t*)out, n, dtype, (hipStream_t)stream), who);
+}
+
 }  // extern "C"

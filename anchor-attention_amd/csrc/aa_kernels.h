@@ -61,6 +61,11 @@ bool decode_takes(int n_rows, int group, bool masked);
 void plan_decode(FlashArgs& a);
 hipError_t launch_decode(const FlashArgs& a, hipStream_t stream);
 
+// x, out [rows, hidden], weight [hidden], contiguous; hidden a multiple of 8 and at most 16384
+hipError_t launch_rms_norm(const uint16_t* x, const uint16_t* weight, uint16_t* out, int64_t rows, int hidden, float eps, int dtype, hipStream_t stream);
+// n elements, a multiple of 8
+hipError_t launch_silu_mul(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t n, int dtype, hipStream_t stream);
+
 struct PoolArgs {
   const uint16_t* q; int64_t q_sb, q_sh, q_sn;
   const float* M;

@@ -221,6 +221,14 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                       int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
                       float sm_scale, int dtype, void* stream);
 
+/* ---- between a patched model's matrix products ------------------------------------------------
+ * What the models that the attention plug is used in compute around it, one pass each, with the 16-bit roundings of the framework's
+ * single operations (all tensors 16-byte aligned and contiguous):
+ * aa_rms_norm: out[r, :] = weight * round16(x[r, :] * rsqrt(mean(x[r, :]^2) + eps)), float32 inside;
+ * aa_silu_mul: out = round16(silu(gate)) * up over n elements. */
+int aa_rms_norm(const void* x, const void* weight, void* out, int64_t rows, int hidden, float eps, int dtype, void* stream);
+int aa_silu_mul(const void* gate, const void* up, void* out, int64_t n, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

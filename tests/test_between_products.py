@@ -1,0 +1,137 @@
+"""The norms and gated activations of patched models as single kernels, against the framework's single operations.
+
+Bound: both round to the 16-bit type twice (unit roundoff u), from float32 numbers that differ in their last bits (order of the sum of
+squares, exponential), so a result may differ by one unit for either rounding: 4 u |want|."""
+import copy
+import pickle
+import types
+
+import pytest
+import torch
+
+
+def _close(got, want):
+    u = 2.0 ** -8 if want.dtype == torch.bfloat16 else 2.0 ** -11
+    assert got.dtype == want.dtype and got.shape == want.shape
+    assert bool(((got.double() - want.double()).abs() <= 4 * u * want.double().abs() + 2.0 ** -23).all())
+
+
+def _tiny(family="Llama", **kw):
+    import transformers
+    torch.manual_seed(0)
+    cfg = getattr(transformers, f"{family}Config")(hidden_size=256, intermediate_size=512, num_hidden_layers=2, num_attention_heads=4,
+                                                   num_key_value_heads=2, vocab_size=100, max_position_embeddings=512, **kw)
+    return getattr(transformers, f"{family}ForCausalLM")(cfg).eval()
+
+
+@pytest.mark.parametrize("family", ["Llama", "Qwen2"])
+def test_which_modules_are_fused_and_that_copies_keep_their_own(family):
+    from anchor_attn import patch_model
+    m = patch_model(_tiny(family), "flash")
+    fused = [x for x in m.modules() if isinstance(x.__dict__.get("forward"), types.MethodType)]
+    assert sorted({type(x).__name__ for x in fused}) == [f"{family}RMSNorm"] and len(fused) == 5  # (MLPs: the chunking wrapper is outside)
+    assert all(x.forward.__self__ is x for x in fused)
+    norm = copy.deepcopy(m.model.norm)
+    assert norm.forward.__self__ is norm
+    with torch.no_grad():
+        norm.weight.fill_(2.0)
+        x = torch.randn(3, 256)
+        assert torch.equal(norm(x), 2.0 * m.model.norm(x))  # (on the CPU: the class's own)
+    again = pickle.loads(pickle.dumps(m.model.norm))
+    assert torch.equal(again(x), m.model.norm(x))
+    before = [x.forward for x in fused]
+    assert [x.forward for x in fused if patch_model(m, "dense")] == before
+    other = patch_model(_tiny(family, hidden_act="gelu"), "flash")  # another activation stays with its own forward
+    assert "fused" not in repr(other.model.layers[0].mlp.act_fn)
+    y = torch.randn(1, 5, 256)
+    assert torch.equal(other.model.layers[0].mlp(y), type(other.model.layers[0].mlp).forward(other.model.layers[0].mlp, y))
+
+
+def test_classes_that_compute_something_else_are_left_alone():
+    from anchor_attn.src.modules.model_forward import fuse_between_products
+
+    class LlamaRMSNorm(torch.nn.Module):  # a norm whose weight is an offset from one
+        def __init__(self):
+            super().__init__()
+            self.weight, self.variance_epsilon = torch.nn.Parameter(torch.zeros(16)), 1e-3
+
+        def forward(self, x):
+            y = x.float()
+            return ((1.0 + self.weight.float()) * y * torch.rsqrt(y.pow(2).mean(-1, keepdim=True) + self.variance_epsilon)).to(x.dtype)
+    m = torch.nn.Sequential(LlamaRMSNorm())
+    assert fuse_between_products(m) == 0 and "forward" not in m[0].__dict__
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (3, 64), (257, 896), (5, 2048), (2, 2056), (66, 4096), (3, 8192), (2, 16384), (1, 16376)])
+def test_norm_against_the_single_operations(rows, hidden, dtype):
+    from transformers.models.llama.modeling_llama import LlamaRMSNorm
+
+    from anchor_attn.src.modules.model_forward import fuse_between_products
+    g = torch.Generator(device="cuda").manual_seed(hidden)
+    m = LlamaRMSNorm(hidden, 1e-5).to("cuda", dtype)
+    with torch.no_grad():
+        m.weight.copy_(1.0 + 0.2 * torch.randn(hidden, generator=g, device="cuda"))
+        x = (torch.randn(1, rows, hidden, generator=g, device="cuda") * torch.linspace(0.01, 30.0, rows, device="cuda")[None, :, None]).to(dtype)
+        assert fuse_between_products(m) == 1
+        _close(m(x), LlamaRMSNorm.forward(m, x))
+        x[0, 0, 0] = float("inf")
+        assert torch.equal(m(x).isnan(), LlamaRMSNorm.forward(m, x).isnan())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 1, 8), (1, 3, 24), (2, 77, 512), (1, 300, 1000)])
+def test_gated_activation_against_the_single_operations(shape, dtype):
+    from transformers import LlamaConfig
+    from transformers.models.llama.modeling_llama import LlamaMLP
+
+    from anchor_attn.src.modules.model_forward import fuse_between_products
+    g = torch.Generator(device="cuda").manual_seed(shape[1])
+    m = LlamaMLP(LlamaConfig(hidden_size=shape[2], intermediate_size=shape[2], num_attention_heads=1)).to("cuda", dtype)
+    for name in ("gate_proj", "up_proj", "down_proj"):
+        setattr(m, name, torch.nn.Identity())
+    x = (8.0 * torch.randn(shape, generator=g, device="cuda")).to(dtype)
+    assert fuse_between_products(m) == 1
+    with torch.no_grad():
+        _close(m(x), LlamaMLP.forward(m, x))
+
+
+@pytest.mark.gpu
+def test_calls_that_stay_with_the_single_operations(monkeypatch):
+    from transformers.models.llama.modeling_llama import LlamaRMSNorm
+
+    from anchor_attn.src.modules.model_forward import fuse_between_products
+    from anchor_attn.src.ops import _hip
+    m = LlamaRMSNorm(64).to("cuda", torch.bfloat16)
+    fuse_between_products(m)
+    monkeypatch.setattr(_hip.lib(), "aa_rms_norm", lambda *a: pytest.fail("the kernel"))
+    x = torch.randn(4, 64, device="cuda", dtype=torch.bfloat16)
+    y = m(x)  # gradients are enabled and the weight wants one
+    y.sum().backward()
+    assert m.weight.grad is not None
+    with torch.no_grad():
+        wide = torch.randn(4, 128, device="cuda", dtype=torch.bfloat16)
+        for t in (x.float(), wide[:, ::2], wide[:, :64], torch.randn(4 * 64 + 1, device="cuda").bfloat16()[1:].view(4, 64), x[:0], x.cpu().cuda().requires_grad_(False).double()):
+            assert torch.equal(m(t), LlamaRMSNorm.forward(m, t))
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert torch.equal(m(x), LlamaRMSNorm.forward(m, x))
+        assert torch.equal(torch.func.vmap(m)(x[None]), LlamaRMSNorm.forward(m, x[None]))
+    monkeypatch.undo()
+
+
+@pytest.mark.gpu
+def test_patched_model_gives_the_logits_of_the_unfused_one():
+    from anchor_attn import patch_model
+    m = patch_model(_tiny().to("cuda", torch.bfloat16), "flash")
+    tokens = torch.randint(0, 100, (2, 33), device="cuda")
+    with torch.no_grad():
+        got = m(tokens).logits
+        for x in m.modules():
+            if isinstance(x.__dict__.get("forward"), types.MethodType):
+                del x.__dict__["forward"]
+        for layer in m.model.layers:
+            del layer.mlp.__dict__["forward"]
+        want = m(tokens).logits
+    assert float((got - want).norm() / want.norm()) < 1e-2
