@@ -95,12 +95,13 @@ __device__ __forceinline__ int k_swizzle(const int r) { return D == 128 ? r & 15
 template <int D>
 __device__ __forceinline__ int v_swizzle(const int r) { return D == 128 ? (r & 7) << 1 : (r & 3) << 1; }
 
-template <int MODE, int D>
+template <int MODE, int D, int TEAMS>
 struct FlashSmem {
   struct {
     char k[2][kBN * 2 * D];
     char v[2][kBN * 2 * D];
-  } t;  // (the epilogue stages the output in the tile space)
+  } t[TEAMS];  // (the epilogue stages the output in the tile space)
+  floatx2 stats[TEAMS > 1 ? 256 : 1];  // the second team's reference and sum, lane by lane
   // sparse mode: window of the big block's index list; masked mode: the chunk's tiles that hold a visible key, and their number
   int32_t idx[MODE == kSparse ? kIdxWin : MODE == kMasked ? kMaskedTiles + 4 : 4];
 };
@@ -175,11 +176,18 @@ __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, cons
 // so the vector ALU bounds it, and a third wave per SIMD (168 registers; 2, 8 and 2 of them spill around the tile loop in
 // anchor, sparse and bf16 rows mode) keeps that busy: 69 % of the cycles, matrix pipe 49 %.  16384 tokens, 32/8 heads of 64: stage 1 470 -> 413 us
 // against two work-groups per CU and 256-byte LDS rows of which half was filled.
-template <int MODE, typename T, int D>
-__global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const FlashArgs p) {
+//
+// TEAMS: the waves that own the 128 rows, four to a team.  Two teams take the tiles alternately, each with LDS tiles and accumulators
+// of its own, and are merged through LDS at the end, like two chunks of the keys without a launch between them.  This is for
+// launches that leave CUs with a single work-group, i.e. one wave to a SIMD, in which the chain scores -> soft-max -> P.V
+// of every tile is exposed.  At head dimension 64 a tile of each team takes 2250 to 3000 clocks, two tiles of one team 3100; at 128, where
+// the operand reads and tile loads of one team fill more of the LDS's time, 4400 against 3900, so 128 has one team.
+template <int MODE, typename T, int D, int TEAMS>
+__global__ void __launch_bounds__(256 * TEAMS, TEAMS > 1 ? 1 : D == 128 ? 2 : 3) flash_kernel(const FlashArgs p) {
   typedef typename T::vec8 vec8;
   typedef __attribute__((address_space(3))) vec8 lds_vec8;
-  __shared__ __attribute__((aligned(16))) FlashSmem<MODE, D> sm;
+  static_assert(TEAMS == 1 || (TEAMS == 2 && MODE != kSparse && D == 64), "teams");
+  __shared__ __attribute__((aligned(16))) FlashSmem<MODE, D, TEAMS> sm;
   constexpr int BM = 128;
   constexpr bool kAnyRows = MODE == kRows || MODE == kMasked;
   constexpr bool kLazyRef = kAnyRows && T::kProbLog2 == 0.f;  // the reference does not follow the row max (see the top of the file)
@@ -199,7 +207,9 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   constexpr int kLoadRows = 256 / kSlots;    // rows that one load instruction of the work-group fills
   constexpr int kHalfLoads = kBN / kLoadRows;  // load instructions of a K (or V) tile
 
-  const int tid = threadIdx.x;
+  const int tid = TEAMS > 1 ? threadIdx.x & 255 : threadIdx.x;  // (within the team)
+  const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  auto& tiles = sm.t[team];
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
@@ -341,7 +351,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   // ---- tile schedule -------------------------------------------------------------------------
   // (anchor) the first big block's rows select no keys further on: where the caller gives the output, they are done here
   const bool finishes = MODE == kAnchor && p.out != nullptr && bb == 0;
-  const bool pool = MODE == kAnchor && p.qbar_out != nullptr && !finishes;
+  const bool pool = MODE == kAnchor && TEAMS == 1 && p.qbar_out != nullptr && !finishes;  // (two teams: a single big block only)
   int n_tiles, n_init = 0;
   int key_base = 0;  // (rows) first key of the chunk
   int entry_next = 0;  // (masked) list entry of the tile to be fetched next
@@ -367,7 +377,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     if (n_tiles <= 0) return;  // (never chunk 0: every row sees at least one key)
     if (MODE == kMasked) {
       // list the chunk's tiles in which any row of the work-group sees a key
-      if (wave == 0) {
+      if (wave == 0 && team == 0) {
         const uint8_t* flags = p.tile_flags + ((int64_t)b * p.n_col_blocks + qunit) * p.mask_words_per_row + chunk * p.chunk_tiles;
         int listed = 0;
         for (int t = 0; t < n_tiles; t += 64) {
@@ -380,8 +390,8 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
       }
       __syncthreads();
       n_tiles = __builtin_amdgcn_readfirstlane(sm.idx[kMaskedTiles]);
-      entry_next = n_tiles > 0 ? __builtin_amdgcn_readfirstlane(sm.idx[0]) : 0;
-      entry_after = sm.idx[n_tiles > 1 ? 1 : 0];
+      entry_next = n_tiles > team ? __builtin_amdgcn_readfirstlane(sm.idx[team]) : 0;
+      entry_after = sm.idx[max(min(team + TEAMS, n_tiles - 1), 0)];
     }
   } else {
     n_tiles = sparse_tiles;
@@ -419,7 +429,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   // this thread's chunk of a row (swizzled: see the top of the file) and the wave's slice of the LDS tiles
   const uint32_t k_col = (uint32_t)((tid % kSlots) ^ k_swizzle<D>(tid / kSlots)) * 16u;
   const uint32_t v_col = (uint32_t)((tid % kSlots) ^ v_swizzle<D>(tid / kSlots)) * 16u;
-  const uint32_t lds_k0 = lds_addr(sm.t.k[0]) + wave * 1024, lds_v0 = lds_addr(sm.t.v[0]) + wave * 1024;
+  const uint32_t lds_k0 = lds_addr(tiles.k[0]) + wave * 1024, lds_v0 = lds_addr(tiles.v[0]) + wave * 1024;
   // byte offset of this thread's chunk of row tid / kSlots of a block of kLoadRows tile rows from the block's first row
   const uint32_t k_voff = (tid / kSlots) * k_row_bytes + k_col, v_voff = (tid / kSlots) * v_row_bytes + v_col;
   // (anchor mode with pooling) the work-group's raw query rows, fetched like a tile by the last tile's load slots
@@ -443,15 +453,15 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
       row_offs[kHalfLoads + j] = __umul24(r, v_row_bytes) + vc;
     }
   };
-  if (kAnyRows) set_row_offs(p.n_ctx - AA_TILE_KEY0(0));
+  if (kAnyRows) set_row_offs(p.n_ctx - AA_TILE_KEY0(min(team, n_tiles - 1)));
   request_mask_word();
-  if (n_tiles > 0 && !chained) {
+  if (n_tiles > team && !chained) {
     const uint32_t first = MODE == kSparse ? (uint32_t)cur * kTileBytes : 0u;
     uint32_t keys0[kHalfLoads] = {};
     if (MODE == kSparse) tile_gather_keys<D>(keys0, sm.idx, 0, tid);
 #pragma unroll
     for (int j = 0; j < 2 * kHalfLoads; ++j)
-      tile_fetch_one<MODE, D>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(0), kAnyRows ? row_offs : keys0,
+      tile_fetch_one<MODE, D>(j, kbase, vbase, k_row_bytes, v_row_bytes, k_col, v_col, AA_TILE_KEY0(team), kAnyRows ? row_offs : keys0,
                            lds_k0 + first, lds_v0 + first, k_voff, v_voff);
   }
   // the accumulator state: the youngest loads in flight, first needed by the first P.V product
@@ -516,7 +526,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
   const int c32_t = lane_t & 31, half_t = lane_t >> 5;
   uint32_t k_rd[kKS];
 #pragma unroll
-  for (int ks = 0; ks < kKS; ++ks) k_rd[ks] = lds_addr(sm.t.k[0]) + first_buf + c32_t * kRowBytes + (((2 * ks + half_t) ^ k_swizzle<D>(c32_t)) << 4);
+  for (int ks = 0; ks < kKS; ++ks) k_rd[ks] = lds_addr(tiles.k[0]) + first_buf + c32_t * kRowBytes + (((2 * ks + half_t) ^ k_swizzle<D>(c32_t)) << 4);
   // transposing V read i: a group of 16 lanes covers 16 head-dim columns; lane points at row r0 = 4*half + (lane%16)/4
   // (+ multiples of 8, which the swizzle does not see), bf16 columns 32*(i&3) + 16*((lane>>4)&1) + 4*(lane&3): chunk
   // 4*(i&3) + y0 with y0 < 4, swizzled -> one offset per value of i & 3
@@ -525,7 +535,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     const int r0 = 4 * half_t + ((lane_t & 15) >> 2);
     const int y0 = 2 * ((lane_t >> 4) & 1) + ((lane_t & 3) >> 1);
 #pragma unroll
-    for (int m = 0; m < kDB; ++m) v_rd[m] = lds_addr(sm.t.v[0]) + first_buf + r0 * kRowBytes + (((4 * m + y0) ^ v_swizzle<D>(r0)) << 4) + 8 * (lane_t & 1);
+    for (int m = 0; m < kDB; ++m) v_rd[m] = lds_addr(tiles.v[0]) + first_buf + r0 * kRowBytes + (((4 * m + y0) ^ v_swizzle<D>(r0)) << 4) + 8 * (lane_t & 1);
   }
 
 
@@ -599,8 +609,8 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     sx = T::mfma(*(const lds_vec8*)(uintptr_t)(k_rd[ks] + (uint32_t)((rd) + 32 * (kb) * kRowBytes)), qreg[ks], ks == 0 ? c_init : sx);
   const floatx16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-  if (kLazyRef && n_tiles > 0) {  // the reference: the row max of the first 32 keys
-    const int key0 = AA_TILE_KEY0(0);
+  if (kLazyRef && n_tiles > team) {  // the reference: the row max of the first 32 keys
+    const int key0 = AA_TILE_KEY0(team);
     const bool mixed = MODE == kMasked && (entry_next & kMixedTile);
     const u32x2 mask_word = {mask_word_next[0] >> (4 * half), mask_word_next[1] >> (4 * half)};
     floatx16 sx;
@@ -639,11 +649,11 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // 128 raw query rows into the idle buffer instead, rows 0..63 where K tiles go and rows 64..127 where V tiles go,
     // chunks in place)
     // (sparse, chained: the last tile of a block fetches the list's first tile, for the next block)
-    const int i_next = i + 1 < n_tiles ? i + 1 : (feeds_next ? 0 : i);
+    const int i_next = i + TEAMS < n_tiles ? i + TEAMS : (feeds_next ? 0 : i);
     if (MODE == kMasked) {
       entry_next = __builtin_amdgcn_readfirstlane(entry_after);
       request_mask_word();
-      entry_after = sm.idx[min(i + 2, n_tiles - 1)];
+      entry_after = sm.idx[min(i + 2 * TEAMS, n_tiles - 1)];
     }
     const int key0_next = AA_TILE_KEY0(i_next);
     const bool fetch_queries = MODE == kAnchor && pool && i + 1 == n_tiles;  // wave-uniform
@@ -871,20 +881,20 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     if (AA_ABLATE != 8 && AA_ABLATE != 9) __syncthreads();
   };
   if (MODE == kSparse || MODE == kMasked) {
-    for (int i = 0; i < n_tiles; ++i) run_tile(std::integral_constant<int, -1>{}, i);
+    for (int i = team; i < n_tiles; i += TEAMS) run_tile(std::integral_constant<int, -1>{}, i);
   } else {
     // (anchor, dense: 128 query rows and 64-key tiles, so the window of a query block holds an even number of tiles)
-    for (int i = 0; i < n_tiles; i += 2) {
+    for (int i = team; i < n_tiles; i += 2 * TEAMS) {
       run_tile(std::integral_constant<int, 0>{}, i);
-      if (kAnyRows && i + 1 == n_tiles) break;
-      run_tile(std::integral_constant<int, 1>{}, i + 1);
+      if ((kAnyRows || TEAMS > 1) && i + TEAMS >= n_tiles) break;
+      run_tile(std::integral_constant<int, 1>{}, i + TEAMS);
     }
   }
+  if (TEAMS > 1 && team == 1 && n_tiles % TEAMS != 0) __syncthreads();  // (the barrier of the first team's last tile)
 #undef AA_TILE_KEY0
 #undef AA_KEY_OF
 #undef AA_MASK
 #undef AA_LANEMAX
-#undef AA_EXP2
 #undef AA_PROB
 #undef AA_EXP_CHUNK
 #undef AA_V_SRC
@@ -901,6 +911,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
     for (int i = 0; i < 2 * n_tiles; ++i) {  // 32 keys at a time
+      if (TEAMS > 1 && (i >> 1) % TEAMS != team) continue;
       int key0 = key_base + 32 * i;
       uint32_t seen;
       if (MODE == kMasked) {
@@ -919,6 +930,42 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
       exact_pv_tile<T, D>(acc, qreg, kbase, vbase, k_row_bytes, v_row_bytes, key0, p.n_ctx, seen, m_base, score_scale, lane);
     }
   }
+
+  if (TEAMS > 1) {
+    // ---- the second team's state -> the first ----------------------------------------------------
+    char* state = sm.t[1].k[0];  // (its tiles: as many bytes as its accumulators)
+    static_assert(sizeof(sm.t[0]) == 256 * D / 2 * sizeof(float), "a team's accumulators fill its tile space");
+    const float m_own = !kLazyRef ? m_ref + m_over : m_ref == kNoRef ? -INFINITY : m_ref;
+    if (team == 1) {
+#pragma unroll
+      for (int db = 0; db < kDB; ++db)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          floatx4 t;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) t[c] = acc[db][rg * 4 + c];
+          *reinterpret_cast<floatx4*>(state + (db * 4 + rg) * 4096 + tid * 16) = t;
+        }
+      sm.stats[tid] = floatx2{m_own, l_run};
+    }
+    __syncthreads();
+    if (team == 1) return;  // (barriers further down count the waves that are left)
+    const floatx2 other = sm.stats[tid];
+    const float m_new = fmaxf(m_own, other[0]), m_base = m_new == -INFINITY ? 0.f : m_new;
+    const float w_own = AA_EXP2(m_own - m_base), w_other = AA_EXP2(other[0] - m_base);
+    l_run = l_run * w_own + other[1] * w_other;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        const floatx4 t = *reinterpret_cast<const floatx4*>(state + (db * 4 + rg) * 4096 + tid * 16);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[db][rg * 4 + c] = acc[db][rg * 4 + c] * w_own + t[c] * w_other;
+      }
+    m_ref = kLazyRef && m_new == -INFINITY ? kNoRef : m_base;
+    if (m_new != -INFINITY) m_over = 0.f;
+  }
+#undef AA_EXP2
 
   // ---- epilogue --------------------------------------------------------------------------------
   const float l_tot = l_run + xor32(l_run);
@@ -943,7 +990,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
       // of its anchors: float32 sums over block_size rows in ascending row order, divided by block_size, rounded to
       // bf16 - the same operations in the same order as pool_kernel, so the results are the same bit for bit.
       const int pbuf = n_tiles & 1;  // where the queries went
-      float* mlds = reinterpret_cast<float*>(sm.t.k[pbuf ^ 1]);
+      float* mlds = reinterpret_cast<float*>(tiles.k[pbuf ^ 1]);
       if (half == 0) mlds[wave * 32 + c32] = m_run;
       __syncthreads();
       const int bs = p.block_size, n_pooled = BM / bs;  // pooled rows of this work-group (1 for block_size 128)
@@ -955,7 +1002,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
         for (int pp = 0; pp < n_pooled; ++pp) {
           float a0 = 0.f;
           for (int r0 = pp * bs; r0 < (pp + 1) * bs; r0 += 16) {  // 16 rows at a time (never across the K/V halves): reads first, then the ordered sums
-            const char* rowp = (r0 < 64 ? sm.t.k[pbuf] : sm.t.v[pbuf]) + (r0 & 63) * kRowBytes + 2 * tid;
+            const char* rowp = (r0 < 64 ? tiles.k[pbuf] : tiles.v[pbuf]) + (r0 & 63) * kRowBytes + 2 * tid;
             uint16_t w[16];
 #pragma unroll
             for (int t = 0; t < 16; ++t) w[t] = *reinterpret_cast<const uint16_t*>(rowp + t * kRowBytes);
@@ -1010,8 +1057,8 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
     // the other buffer may already hold the next block's first tile.
     const bool more = MODE == kSparse && qb + 1 < nq;
     if (more) request_queries(my_row + BM);  // (the registers of this block's raw queries are long free)
-    char* ob = (MODE == kSparse ? (wave < 2 ? sm.t.k[cur ^ 1] : sm.t.v[cur ^ 1]) + (wave & 1) * 32 * kRowBytes
-                                : sm.t.k[0] + wave * 32 * kRowBytes);
+    char* ob = (MODE == kSparse ? (wave < 2 ? tiles.k[cur ^ 1] : tiles.v[cur ^ 1]) + (wave & 1) * 32 * kRowBytes
+                                : tiles.k[0] + wave * 32 * kRowBytes);
     constexpr int kChunkMask = D / 8 - 1;
     // (the staging offsets are the same for every block of the work-group; computed from an opaque copy of the lane
     // number they are formed here, a few instructions per block, instead of occupying registers throughout the tile loop)
@@ -1058,8 +1105,20 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) flash_kernel(const Flas
 #define AA_SPARSE_QBLOCKS 4  // most 128-row query blocks a stage-3 work-group handles one after the other
 #endif
 
+template <int MODE, typename T, int D>
+static void launch_for(const FlashArgs& a, const dim3 grid, const int teams, hipStream_t stream) {
+  if constexpr (MODE != kSparse && D == 64) {
+    if (teams == 2) {
+      hipLaunchKernelGGL((flash_kernel<MODE, T, D, 2>), grid, dim3(512), 0, stream, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((flash_kernel<MODE, T, D, 1>), grid, dim3(256), 0, stream, a);
+}
+
 template <int MODE>
 static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
+  constexpr bool kAnyRowsMode = MODE == kRows || MODE == kMasked;
   FlashArgs a = args;
   a.q_blocks_per_wg = 1;
   int64_t blocks = (int64_t)a.batch * a.n_q_heads * (a.n_ctx / 128);
@@ -1077,18 +1136,24 @@ static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
     a.q_blocks_per_wg = nq;
   }
   const dim3 grid(MODE == kRows || MODE == kMasked ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
-                                : (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0)), block(256);
+                                : (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0));
   // More units (KV heads of all batch elements) than XCDs: side by side as long as the K and V that an XCD then works on fit its L2
   // of 4 MB.  Left-padded batches: 3 x 2500 with 32/8 heads of 128 194 -> 184 us, 28/4 184 -> 162, 3 x 1000 with 32/8 heads of 64 39.9 -> 30.0, 4 x 2900
   // 162 -> 150; the operator on 2 x 4096 tokens with those heads 181 -> 172.  Larger contexts, where the order hardly matters: within 1 %.
   const int units = a.batch * a.n_kv_heads;
   a.abreast = MODE != kSparse && 8 % units != 0 && (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20;
+  // Two teams where a work-group is alone on its CU and its tiles pay for the merge (1.5 us).  Head dimension 64: 2048 tokens with 14/2
+  // heads, one launch, 26.4 -> 22.9 us, dense 25.9 -> 22.3, 1024 tokens dense 15.0 -> 14.1, a prompt of 2348 44.3 -> 40.4, padded 2 x 1000 25.7 -> 23.3;
+  // 512 tokens dense (8 tiles) 9.6 -> 10.2, and 512 work-groups (32 heads, 2048 tokens) 27.6 -> 29.5.
+  // (anchor: a single big block only, whose rows are finished or leave their state; larger contexts give the same bits in any batch)
+  const bool fits = MODE != kAnchor || (a.n_ctx == a.big_block && (a.qbar_out == nullptr || a.out != nullptr));
+  const int teams = fits && grid.x <= 256 && (kAnyRowsMode ? a.chunk_tiles : a.n_ctx / kBN) >= 12 ? 2 : 1;
   if (a.head_dim == 128) {
-    if (a.dtype == 0) hipLaunchKernelGGL((flash_kernel<MODE, Bf16, 128>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((flash_kernel<MODE, F16, 128>), grid, block, 0, stream, a);
+    if (a.dtype == 0) launch_for<MODE, Bf16, 128>(a, grid, teams, stream);
+    else launch_for<MODE, F16, 128>(a, grid, teams, stream);
   } else {  // 64: the C-ABI layer admits nothing else
-    if (a.dtype == 0) hipLaunchKernelGGL((flash_kernel<MODE, Bf16, 64>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((flash_kernel<MODE, F16, 64>), grid, block, 0, stream, a);
+    if (a.dtype == 0) launch_for<MODE, Bf16, 64>(a, grid, teams, stream);
+    else launch_for<MODE, F16, 64>(a, grid, teams, stream);
   }
   return hipGetLastError();
 }
