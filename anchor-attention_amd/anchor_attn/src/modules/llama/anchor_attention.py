@@ -20,7 +20,7 @@ import torch
 import torch.nn.functional as F
 
 from anchor_attn.src.ops.anchor_attn_v4 import (LOG2E, _anchor_attn, _dense_rows, _rows_dispatch, anchor_attn,
-                                                dense_causal_attention)
+                                                dense_causal_attention, rows_beside)
 
 ATTN_NAME = "anchor_attn"
 DENSE_ATTN_NAME = "anchor_attn_dense"
@@ -34,10 +34,11 @@ record_ratio: bool = False
 last_ratio: Optional[torch.Tensor] = None
 
 
-def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[int], out=None):
+def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[int], out=None, beside: Optional[list] = None):
     """Dense attention for the parts the sparse operator does not cover (tail rows, decode, padded batches).
     ``causal_offset``: query row i may see keys ``<= causal_offset + i`` (None: use ``attention_mask`` as is).  Writes into
     ``out`` where it is given and the own kernel runs, otherwise returns a new tensor; either way the result is returned.
+    With a list ``beside`` the own kernel is not launched: what it is to do is left there for the operator's launch.
     The own kernel takes bf16/fp16 inference on the GPU; the framework's attention does everything else (other types and
     head dimensions, gradients and tangents, vmap, tracing, the CPU)."""
     groups = query.shape[1] // key.shape[1]
@@ -47,6 +48,9 @@ def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[i
     # (the own kernel scales raw scores in float32: by a positive number whose product with them neither vanishes nor overflows)
     if (by_mask or by_offset) and not wants_grad and (scaling is None or 1e-30 < scaling < 1e30):
         tensors = _rows_dispatch(query, key, value, attention_mask, out)
+        if tensors is not None and beside is not None and query.device.index == torch.cuda.current_device():
+            beside.append(rows_beside(tensors, query, key, causal_offset, scaling))
+            return out
         if tensors is not None:
             return _dense_rows(tensors, query, key, causal_offset or 0, scaling, out, attention_mask)
     mask = attention_mask
@@ -56,8 +60,8 @@ def _dense(query, key, value, attention_mask, scaling, causal_offset: Optional[i
     return F.scaled_dot_product_attention(query, key, value, attn_mask=mask, scale=scaling, enable_gqa=groups > 1)
 
 
-def _dense_into(out, query, key, value, attention_mask, scaling, causal_offset):
-    got = _dense(query, key, value, attention_mask, scaling, causal_offset, out)
+def _dense_into(out, query, key, value, attention_mask, scaling, causal_offset, beside=None):
+    got = _dense(query, key, value, attention_mask, scaling, causal_offset, out, beside)
     if got is not out:
         out.copy_(got)
 
@@ -80,16 +84,18 @@ def anchor_attention_forward(module, query: torch.Tensor, key: torch.Tensor, val
         return out, None
     pad = N % big
     main = N - pad
+    rows = []
+    if pad:
+        _dense_into(out_bhnd[:, :, main:], query[:, :, main:], key, value, None, scaling, main, rows)
+    beside = {"rows": rows[0]} if rows else {}
     if record_ratio:
         sm_scale = scaling if scaling else 1.0 / (D ** 0.5)
         _, last_ratio = _anchor_attn(query[:, :, :main], key[:, :, :main], value[:, :, :main], sm_scale, block_size, step,
-                                     theta * LOG2E, True, out=out_bhnd[:, :, :main])
+                                     theta * LOG2E, True, out=out_bhnd[:, :, :main], **beside)
     else:
         anchor_attn(query[:, :, :main], key[:, :, :main], value[:, :, :main], sm_scale=scaling,
                     block_size=block_size, step=step, difference=theta,
-                    return_computational_ratio=False, out=out_bhnd[:, :, :main])
-    if pad:
-        _dense_into(out_bhnd[:, :, main:], query[:, :, main:], key, value, None, scaling, main)
+                    return_computational_ratio=False, out=out_bhnd[:, :, :main], **beside)
     return out, None
 
 

@@ -54,6 +54,10 @@ _SIGNATURES = {
     "aa_rms_norm": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_float, c_int, c_void_p]),
     "aa_silu_mul": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_void_p]),
     "aa_dense_rows_fwd": (c_int, _T3 * 4 + [c_void_p, c_int64, c_int64] + [c_void_p, c_size_t] + [c_int] * 7 + [c_float, c_int, c_void_p]),
+    # the operator's sizes, then n_rows, n_keys, causal_offset
+    "aa_anchor_attn_rows_workspace_bytes": (c_size_t, [c_int] * 10),
+    "aa_anchor_attn_rows_fwd": (c_int, _T3 * 8 + [c_int] * 3 + [c_float] + [c_void_p, c_size_t, c_void_p, c_void_p, c_void_p, c_double] + _DIMS5
+                                + [c_int, c_int, c_double, c_float, c_int, c_int, c_int, c_void_p]),
 }
 
 EXPORTS = tuple(_SIGNATURES)

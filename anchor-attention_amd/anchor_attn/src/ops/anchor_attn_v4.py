@@ -84,7 +84,7 @@ def _workspace(B, H, N, D, block_size, step, device):
 
 def _anchor_attn(Q, K, V, sm_scale=None, block_size=64, step=16, difference=100, return_sparsity_ratio=False,
                  BLOCK_SIZE_M=128, BLOCK_SIZE_N=128, out=None, scale_mode=_hip.AA_SCALE_BF16_CHAIN,
-                 geometry=_hip.AA_GEOMETRY_AS_RUN, host_ratio=None):
+                 geometry=_hip.AA_GEOMETRY_AS_RUN, host_ratio=None, rows=None):
     """All three stages on the current stream, one C call (``difference`` is in the log2 domain
     here, as in the reference's private function, anchor_attn_v4.py:226-273)."""
     B, H, N, D = Q.shape
@@ -93,21 +93,34 @@ def _anchor_attn(Q, K, V, sm_scale=None, block_size=64, step=16, difference=100,
     _check_inputs(Q, K, V)
     output = torch.empty_like(Q) if out is None else out
     assert output.shape == Q.shape and output.dtype == Q.dtype and output.stride(-1) == 1
-    ws = _workspace(B, H, N, D, block_size, step, Q.device)
-    tensors = (*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output), ws.data_ptr(), ws.numel())
-    sizes = (B, H, K.shape[1], N, D, block_size, step, float(sm_scale), float(difference), scale_mode, int(geometry),
-             _hip.dtype_code(Q), _stream())
-    if not return_sparsity_ratio:
-        _hip.check(_hip.lib().aa_anchor_attn_fwd(*tensors, None, *sizes))
-        return output, 1.0
-    if torch.get_default_dtype() == torch.float32:
+    sizes = (B, H, K.shape[1], N, D, block_size, step)
+    if rows is None:
+        ws, beside = _workspace(B, H, N, D, block_size, step, Q.device), ()
+    else:
+        problem, row_tensors, row_sizes, row_scale = rows
+        assert problem == (B, H, K.shape[1], D, Q.dtype), "rows beside the operator have its batch, heads, head dimension and type"
+        nbytes = _hip.lib().aa_anchor_attn_rows_workspace_bytes(*sizes, *row_sizes)
+        ws, beside = torch.empty((nbytes,), dtype=torch.uint8, device=Q.device), (*row_tensors, *row_sizes, row_scale)
+    tensors = (*_hip.t3(Q), *_hip.t3(K), *_hip.t3(V), *_hip.t3(output), *beside, ws.data_ptr(), ws.numel())
+    options = (*sizes, float(sm_scale), float(difference), scale_mode, int(geometry), _hip.dtype_code(Q), _stream())
+    counts = ratio = None
+    if return_sparsity_ratio and torch.get_default_dtype() == torch.float32:
         ratio = torch.empty((), dtype=torch.float32, device=Q.device)
-        _hip.check(_hip.lib().aa_anchor_attn_ratio_fwd(*tensors, ratio.data_ptr(), ctypes.addressof(host_ratio) if host_ratio is not None else None,
-                                                        _ratio_denominator(B, H, N, block_size, step), *sizes))
-        return output, ratio
-    counts = torch.empty((B, H, N // (block_size * step), 1), dtype=torch.int32, device=Q.device)
-    _hip.check(_hip.lib().aa_anchor_attn_fwd(*tensors, counts.data_ptr(), *sizes))
-    return output, _ratio(counts, B, H, N, block_size, step)
+    elif return_sparsity_ratio:
+        counts = torch.empty((B, H, N // (block_size * step), 1), dtype=torch.int32, device=Q.device)
+    counts_ptr = counts.data_ptr() if counts is not None else None
+    ratio_args = (None, None, 1.0)
+    if ratio is not None:
+        ratio_args = (ratio.data_ptr(), ctypes.addressof(host_ratio) if host_ratio is not None else None, _ratio_denominator(B, H, N, block_size, step))
+    if rows is not None:
+        _hip.check(_hip.lib().aa_anchor_attn_rows_fwd(*tensors, counts_ptr, *ratio_args, *options))
+    elif ratio is not None:
+        _hip.check(_hip.lib().aa_anchor_attn_ratio_fwd(*tensors, *ratio_args, *options))
+    else:
+        _hip.check(_hip.lib().aa_anchor_attn_fwd(*tensors, counts_ptr, *options))
+    if counts is not None:
+        ratio = _ratio(counts, B, H, N, block_size, step)
+    return output, ratio if return_sparsity_ratio else 1.0
 
 
 def _stage3(Q, K, V, coords, counts, L, M, Acc, sm_scale, block_size, step, out=None):
@@ -156,13 +169,15 @@ def anchor_attn_without_anchor(Q, K, V, sm_scale: float = None, block_size: int 
 
 
 def anchor_attn(Q, K, V, sm_scale: float = None, block_size: int = 128, step: int = 16, difference: float = 12,
-                return_computational_ratio: bool = True, out: torch.Tensor = None, strict_reference: bool = True):
+                return_computational_ratio: bool = True, out: torch.Tensor = None, strict_reference: bool = True, rows=None):
     """Sparse prefill attention.  ``Q`` ``[B,H,N,D]`` bf16 or fp16; ``K``/``V`` ``[B,H or H_kv,N,D]`` of the same type;
     returns ``out`` or ``(out, ratio)`` exactly like the reference.
 
     ``strict_reference=False`` (analysis only, never the default) lets stage 2 choose from ``[S, bb*S)``
     - the range of the reference's fused variant, anchor_fuse_step_1_2_v2.py:152 - instead of the as-run
-    ``[block_size, bb*S - block_size)``: no key is attended twice and none is left out."""
+    ``[block_size, bb*S - block_size)``: no key is attended twice and none is left out.
+
+    ``rows``: dense attention of other rows that is computed with the operator's first launch (:func:`rows_beside`)."""
     difference *= LOG2E
     Q, K, V = _prepare(Q, K, V)
     assert Q.stride(-1) == 1 and K.stride(-1) == 1 and V.stride(-1) == 1, \
@@ -178,7 +193,7 @@ def anchor_attn(Q, K, V, sm_scale: float = None, block_size: int = 128, step: in
     sm_scale = sm_scale if sm_scale else 1.0 / (D ** 0.5)
     host_ratio = _host_ratio(Q.device) if return_computational_ratio else None
     sparse_output, sparse_ratio = _anchor_attn(Q, K, V, sm_scale, block_size, step, difference,
-                                               return_computational_ratio, out=out, host_ratio=host_ratio,
+                                               return_computational_ratio, out=out, host_ratio=host_ratio, rows=rows,
                                                geometry=_hip.AA_GEOMETRY_AS_RUN if strict_reference else _hip.AA_GEOMETRY_INTENDED)
     if return_computational_ratio:
         _log_ratio(sparse_ratio, host_ratio)
@@ -293,6 +308,12 @@ def dense_rows_attention(Q, K, V, causal_offset: int = 0, sm_scale: float = None
         raise _hip.AnchorAttnHipError("dense_rows_attention: unsupported tensors (bf16 or fp16 on one GPU, head dimension 64 or 128, rows of at "
                                       "most 16384 elements on 16-byte boundaries, a boolean mask [B or 1, 1, n_rows, n_keys], out like Q)")
     return _dense_rows(tensors, Q, K, causal_offset, sm_scale, out, mask)
+
+
+def rows_beside(tensors, Q, K, causal_offset, sm_scale):
+    """``rows`` of :func:`anchor_attn` for the attention that ``_dense_rows`` computes of the same arguments (``tensors`` with ``out``)."""
+    B, H, N, D = Q.shape
+    return (B, H, K.shape[1], D, Q.dtype), tensors, (N, K.shape[2], int(causal_offset)), float(sm_scale if sm_scale else 1.0 / (D ** 0.5))
 
 
 def _dense_rows(tensors, Q, K, causal_offset, sm_scale, out, mask):

@@ -246,6 +246,7 @@ struct Stage1Extras {
   // the output of big block 0, whose rows select no keys, in the place of their state and pooled rows
   void* out; int64_t o_sb, o_sh, o_sn;
   int32_t* zero_counts; float* zero_ratio; float* zero_ratio_host;  // a single big block: what the later stages would say
+  const FlashArgs* rows;  // a rows-mode problem that shares the launch
 };
 
 static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
@@ -276,6 +277,7 @@ static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_s
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size;
   a.sm_scale = sm_scale; a.scale_mode = scale_mode; a.dtype = dtype;
+  if (x.rows != nullptr) return check_launch(launch_anchor_and_rows(a, *x.rows, (hipStream_t)stream), who);
   return check_launch(run_flash(a, 0, (hipStream_t)stream), who);
 }
 
@@ -418,7 +420,8 @@ int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
                      out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, dtype, stream);
 }
 
-// The whole operator; with `ratio` the counts are kept in the workspace and their sum over `denominator` is formed.
+// The whole operator; with `ratio` the counts are kept in the workspace and their sum over `denominator` is formed.  `rows`: a rows-mode
+// problem, checked and planned, that shares stage 1's launch.
 static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                        const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                        const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
@@ -426,7 +429,7 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
                        void* workspace, size_t workspace_bytes, int32_t* counts_out, float* ratio, float* ratio_host, double denominator,
                        int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                        int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
-                       int dtype, void* stream) {
+                       int dtype, void* stream, const FlashArgs* rows = nullptr) {
   int rc;
   // (all that a later stage could refuse is looked at first: stage 1 already writes the first big block's output)
   const Dims dims = {batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step};
@@ -461,10 +464,12 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
     x.scale2 = select_scale2(sm_scale); x.theta_log2 = theta_log2;
   }
   x.out = out; x.o_sb = o_sb; x.o_sh = o_sh; x.o_sn = o_sn;
+  x.rows = rows;
   if (!selects) { x.zero_counts = counts; x.zero_ratio = ratio; x.zero_ratio_host = ratio_host; }
   if ((rc = stage1_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc, x, batch, n_q_heads, n_kv_heads,
                         n_ctx, head_dim, block_size, step, (float)sm_scale, scale_mode, dtype, stream)))
     return rc;
+  if (rows != nullptr && rows->n_chunks > 1 && (rc = check_launch(launch_rows_combine(*rows, (hipStream_t)stream), who))) return rc;
   if (selects) {
     if (!fused_pool &&
         (rc = aa_pool_q_anchor(q, q_sb, q_sh, q_sn, M, qbar, abar, batch, n_q_heads, n_ctx, head_dim, block_size, dtype, stream)))
@@ -630,6 +635,36 @@ size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, i
   return carve_rows(a, decode_takes(n_rows, n_q_heads / n_kv_heads, masked != 0)).total;
 }
 
+// Tensors and scratch of a planned rows-mode problem, checked and put into `a`.
+static int rows_args(const char* who, FlashArgs& a, const RowsScratch& r, const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                     const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                     void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn, void* workspace, size_t workspace_bytes, float sm_scale, int dtype) {
+  int rc;
+  if ((rc = check_tensor(q, q_sb, q_sh, q_sn, a.n_rows, a.head_dim, who, "q"))) return rc;
+  if ((rc = check_tensor(k, k_sb, k_sh, k_sn, a.n_ctx, a.head_dim, who, "k"))) return rc;
+  if ((rc = check_tensor(v, v_sb, v_sh, v_sn, a.n_ctx, a.head_dim, who, "v"))) return rc;
+  if ((rc = check_tensor(out, o_sb, o_sh, o_sn, a.n_rows, a.head_dim, who, "out"))) return rc;
+  if (!(sm_scale > 0.f)) {  // the running maxima are those of the raw dot products
+    set_error("%s: sm_scale %g must be positive", who, (double)sm_scale);
+    return AA_EUNSUPPORTED;
+  }
+  if (r.total > 0) {
+    if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
+    if (workspace_bytes < r.total) {
+      set_error("%s: workspace has %zu bytes, %zu needed", who, workspace_bytes, r.total);
+      return AA_EBADARG;
+    }
+  }
+  a.q = (const uint16_t*)q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_sn = q_sn;
+  a.k = (const uint16_t*)k; a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
+  a.v = (const uint16_t*)v; a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn;
+  a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
+  a.acc_out = (float*)workspace; a.M_out = a.acc_out + r.state_columns * a.head_dim; a.L_out = a.M_out + r.state_columns;
+  a.acc_frag = a.acc_out; a.M = a.M_out; a.L = a.L_out;
+  a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
+  return AA_OK;
+}
+
 int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                       const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                       const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
@@ -643,42 +678,99 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   int rc;
   if ((rc = check_dtype(dtype, who))) return rc;
   if ((rc = plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, mask != nullptr))) return rc;
-  if ((rc = check_tensor(q, q_sb, q_sh, q_sn, n_rows, head_dim, who, "q"))) return rc;
-  if ((rc = check_tensor(k, k_sb, k_sh, k_sn, n_keys, head_dim, who, "k"))) return rc;
-  if ((rc = check_tensor(v, v_sb, v_sh, v_sn, n_keys, head_dim, who, "v"))) return rc;
-  if ((rc = check_tensor(out, o_sb, o_sh, o_sn, n_rows, head_dim, who, "out"))) return rc;
-  if (!(sm_scale > 0.f)) {  // the running maxima are those of the raw dot products
-    set_error("%s: sm_scale %g must be positive", who, (double)sm_scale);
-    return AA_EUNSUPPORTED;
-  }
   const bool decode = decode_takes(n_rows, n_q_heads / n_kv_heads, mask != nullptr);
   const RowsScratch r = carve_rows(a, decode);
-  if (r.total > 0) {
-    if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
-    if (workspace_bytes < r.total) {
-      set_error("%s: workspace has %zu bytes, %zu needed", who, workspace_bytes, r.total);
-      return AA_EBADARG;
-    }
-  }
-  a.q = (const uint16_t*)q; a.q_sb = q_sb; a.q_sh = q_sh; a.q_sn = q_sn;
-  a.k = (const uint16_t*)k; a.k_sb = k_sb; a.k_sh = k_sh; a.k_sn = k_sn;
-  a.v = (const uint16_t*)v; a.v_sb = v_sb; a.v_sh = v_sh; a.v_sn = v_sn;
-  a.out = (uint16_t*)out; a.o_sb = o_sb; a.o_sh = o_sh; a.o_sn = o_sn;
-  char* ws = static_cast<char*>(workspace);
-  a.acc_out = (float*)ws; a.M_out = a.acc_out + r.state_columns * head_dim; a.L_out = a.M_out + r.state_columns;
-  a.acc_frag = a.acc_out; a.M = a.M_out; a.L = a.L_out;
-  a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
+  if ((rc = rows_args(who, a, r, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, out, o_sb, o_sh, o_sn, workspace, workspace_bytes,
+                      sm_scale, dtype)))
+    return rc;
   if (decode) {
     a.mask_bytes = mask; a.mask_sb = mask_sb;
     return check_launch(launch_decode(a, (hipStream_t)stream), who);
   }
   if (mask != nullptr) {
+    char* ws = static_cast<char*>(workspace);
     a.mask_words = (const uint64_t*)(ws + r.words);
     a.tile_flags = (const uint8_t*)(ws + r.flags);
     if ((rc = check_launch(launch_mask_pack(a, mask, mask_sb, mask_sn, (hipStream_t)stream), who))) return rc;
   }
   if ((rc = check_launch(run_flash(a, mask != nullptr ? 4 : 3, (hipStream_t)stream), who))) return rc;
   return a.n_chunks > 1 ? check_launch(launch_rows_combine(a, (hipStream_t)stream), who) : AA_OK;
+}
+
+// A rows-mode problem beside the operator, planned.
+struct RowsBeside {
+  bool shares;  // stage 1's launch (else it has its own after the operator: a few rows are the decode kernel's)
+  FlashArgs args;
+  RowsScratch scratch;
+  size_t operator_bytes;  // the operator's scratch; the rows' follows it
+};
+static int plan_beside(const char* who, RowsBeside& r, int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim, int block_size, int step,
+                       int n_rows, int n_keys, int causal_offset) {
+  const Dims dims = {batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step};
+  int rc;
+  r.args = FlashArgs{};
+  if ((rc = check_dims(dims, who)) || (rc = plan_dense_rows(who, r.args, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, false)))
+    return rc;
+  const bool decode = decode_takes(n_rows, n_q_heads / n_kv_heads, false);
+  r.shares = false;
+  if (!decode) {
+    FlashArgs beside = r.args, anchor = {};
+    anchor.batch = batch; anchor.n_q_heads = n_q_heads; anchor.n_ctx = n_ctx; anchor.head_dim = head_dim; anchor.big_block = block_size * step;
+    plan_rows_beside(beside, anchor);
+    // (a launch takes less than 2^32 threads, 256 to a work-group)
+    r.shares = (int64_t)batch * n_q_heads * (n_ctx / 128) + (int64_t)batch * n_kv_heads * beside.n_col_blocks * beside.n_chunks + 8 <= 0xffffff;
+    if (r.shares) r.args = beside;
+  }
+  r.scratch = carve_rows(r.args, decode);
+  r.operator_bytes = carve(batch, n_q_heads, n_ctx, head_dim, block_size, step).total;
+  return AA_OK;
+}
+
+size_t aa_anchor_attn_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim, int block_size, int step,
+                                           int n_rows, int n_keys, int causal_offset) {
+  RowsBeside r;
+  if (plan_beside("aa_anchor_attn_rows_workspace_bytes", r, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, n_rows, n_keys, causal_offset))
+    return 0;
+  return r.operator_bytes + r.scratch.total;
+}
+
+int aa_anchor_attn_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                            const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                            const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                            void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                            const void* rq, int64_t rq_sb, int64_t rq_sh, int64_t rq_sn,
+                            const void* rk, int64_t rk_sb, int64_t rk_sh, int64_t rk_sn,
+                            const void* rv, int64_t rv_sb, int64_t rv_sh, int64_t rv_sn,
+                            void* rout, int64_t ro_sb, int64_t ro_sh, int64_t ro_sn, int n_rows, int n_keys, int causal_offset, float rows_scale,
+                            void* workspace, size_t workspace_bytes, int32_t* counts_out, float* ratio, float* ratio_host, double denominator,
+                            int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                            int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
+                            int dtype, void* stream) {
+  const char* who = "aa_anchor_attn_rows_fwd";
+  RowsBeside r;
+  int rc;
+  if ((rc = check_dtype(dtype, who))) return rc;
+  if ((rc = plan_beside(who, r, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, n_rows, n_keys, causal_offset))) return rc;
+  if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
+  if (workspace_bytes < r.operator_bytes + r.scratch.total) {
+    set_error("%s: workspace has %zu bytes, %zu needed", who, workspace_bytes, r.operator_bytes + r.scratch.total);
+    return AA_EBADARG;
+  }
+  if (ratio != nullptr && !(denominator > 0.0)) {
+    set_error("%s: denominator (%g) must be positive", who, denominator);
+    return AA_EBADARG;
+  }
+  char* rows_ws = static_cast<char*>(workspace) + r.operator_bytes;
+  if ((rc = rows_args(who, r.args, r.scratch, rq, rq_sb, rq_sh, rq_sn, rk, rk_sb, rk_sh, rk_sn, rv, rv_sb, rv_sh, rv_sn, rout, ro_sb, ro_sh, ro_sn,
+                      rows_ws, r.scratch.total, rows_scale, dtype)))
+    return rc;
+  if ((rc = anchor_attn_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, out, o_sb, o_sh, o_sn, workspace, r.operator_bytes,
+                             counts_out, ratio, ratio_host, denominator, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale,
+                             theta_log2, scale_mode, geometry, dtype, stream, r.shares ? &r.args : nullptr)))
+    return rc;
+  if (r.shares) return AA_OK;
+  return aa_dense_rows_fwd(rq, rq_sb, rq_sh, rq_sn, rk, rk_sb, rk_sh, rk_sn, rv, rv_sb, rv_sh, rv_sn, rout, ro_sb, ro_sh, ro_sn, nullptr, 0, 0, rows_ws,
+                           r.scratch.total, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, rows_scale, dtype, stream);
 }
 
 int aa_rms_norm(const void* x, const void* weight, void* out, int64_t rows, int hidden, float eps, int dtype, void* stream) {

@@ -183,11 +183,10 @@ __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, cons
 // of every tile is exposed.  At head dimension 64 a tile of each team takes 2250 to 3000 clocks, two tiles of one team 3100; at 128, where
 // the operand reads and tile loads of one team fill more of the LDS's time, 4400 against 3900, so 128 has one team.
 template <int MODE, typename T, int D, int TEAMS>
-__global__ void __launch_bounds__(256 * TEAMS, TEAMS > 1 ? 1 : D == 128 ? 2 : 3) flash_kernel(const FlashArgs p) {
+__device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t block, FlashSmem<MODE, D, TEAMS>& sm) {
   typedef typename T::vec8 vec8;
   typedef __attribute__((address_space(3))) vec8 lds_vec8;
   static_assert(TEAMS == 1 || (TEAMS == 2 && MODE != kSparse && D == 64), "teams");
-  __shared__ __attribute__((aligned(16))) FlashSmem<MODE, D, TEAMS> sm;
   constexpr int BM = 128;
   constexpr bool kAnyRows = MODE == kRows || MODE == kMasked;
   constexpr bool kLazyRef = kAnyRows && T::kProbLog2 == 0.f;  // the reference does not follow the row max (see the top of the file)
@@ -224,11 +223,11 @@ __global__ void __launch_bounds__(256 * TEAMS, TEAMS > 1 ? 1 : D == 128 ? 2 : 3)
   const int nq = MODE == kSparse ? p.q_blocks_per_wg : 1;
   // (sparse) one work-group more than the query blocks need, the first, sums the counts to the ratio beside the others
   const bool sums = MODE == kSparse && p.ratio != nullptr;
-  if (sums && blockIdx.x == 0) {
+  if (sums && block == 0) {
     sum_counts(p.counts, p.n_ratio_counts, p.ratio_inverse, p.ratio, p.ratio_host, reinterpret_cast<int64_t*>(sm.idx));
     return;
   }
-  const uint32_t wg = blockIdx.x - (sums ? 1u : 0u);
+  const uint32_t wg = block - (sums ? 1u : 0u);
   const int S = p.big_block;
   // (sparse mode may leave out the first big block, whose rows select nothing)
   const int n_qunit = kAnyRows ? 1 : (p.n_ctx - (MODE == kSparse ? p.first_big_block * S : 0)) / (BM * nq);
@@ -1101,31 +1100,43 @@ __global__ void __launch_bounds__(256 * TEAMS, TEAMS > 1 ? 1 : D == 128 ? 2 : 3)
   }  // query blocks of the work-group
 }
 
+template <int MODE, typename T, int D, int TEAMS>
+__global__ void __launch_bounds__(256 * TEAMS, TEAMS > 1 ? 1 : D == 128 ? 2 : 3) flash_kernel(const FlashArgs p) {
+  __shared__ __attribute__((aligned(16))) FlashSmem<MODE, D, TEAMS> sm;
+  flash_body<MODE, T, D, TEAMS>(p, blockIdx.x, sm);
+}
+
+// Anchor mode and rows mode in one launch, for a prompt that ends in part of a big block: the rows of that part depend on no other
+// stage.  The rows' work-groups come first; anchor work-groups, longest first, fill the CUs beside and after them, so that the
+// uneven end of one launch is the other's work and the rows need fewer key chunks to fill the chip - often none, and then no merge.
+// The first anchor work-group's number is a multiple of 8: both bodies' maps from work-groups to XCDs hold.
+// One launch against two, whole prompts: 32/8 heads of 128, 2200 tokens 68.5 -> 55.0 us, 3148 138 -> 109, 6001 375 -> 353, 40001 2955 -> 2878; 32/8
+// heads of 64, 6001 230 -> 207; 14/2 heads of 64, 2600 44.3 -> 31.9, 7500 165 -> 142, 30000 630 -> 600.
+template <typename T, int D, int TEAMS>
+__global__ void __launch_bounds__(256 * TEAMS, TEAMS > 1 ? 1 : D == 128 ? 2 : 3)
+flash_pair_kernel(const FlashArgs anchor, const FlashArgs rows, const uint32_t n_rows_wgs) {
+  __shared__ __attribute__((aligned(16))) union {
+    FlashSmem<kAnchor, D, TEAMS> anchor;
+    FlashSmem<kRows, D, TEAMS> rows;
+  } sm;
+  const uint32_t n_first = (n_rows_wgs + 7u) & ~7u;
+  if (blockIdx.x >= n_first) flash_body<kAnchor, T, D, TEAMS>(anchor, blockIdx.x - n_first, sm.anchor);
+  else if (blockIdx.x < n_rows_wgs) flash_body<kRows, T, D, TEAMS>(rows, blockIdx.x, sm.rows);
+}
+
 #ifndef AA_SPARSE_QBLOCKS
 #define AA_SPARSE_QBLOCKS 4  // most 128-row query blocks a stage-3 work-group handles one after the other
 #endif
 
-template <int MODE, typename T, int D>
-static void launch_for(const FlashArgs& a, const dim3 grid, const int teams, hipStream_t stream) {
-  if constexpr (MODE != kSparse && D == 64) {
-    if (teams == 2) {
-      hipLaunchKernelGGL((flash_kernel<MODE, T, D, 2>), grid, dim3(512), 0, stream, a);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((flash_kernel<MODE, T, D, 1>), grid, dim3(256), 0, stream, a);
-}
-
+// Sets what the launcher decides for a launch of one mode; the number of work-groups.
 template <int MODE>
-static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
-  constexpr bool kAnyRowsMode = MODE == kRows || MODE == kMasked;
-  FlashArgs a = args;
+static uint32_t place(FlashArgs& a) {
   a.q_blocks_per_wg = 1;
   int64_t blocks = (int64_t)a.batch * a.n_q_heads * (a.n_ctx / 128);
   if (MODE == kSparse) {
     const int per_big_block = a.big_block / 128;
     blocks -= (int64_t)a.batch * a.n_q_heads * a.first_big_block * per_big_block;
-    if (blocks == 0) return hipSuccess;
+    if (blocks == 0) return 0;
     // Chained blocks save a work-group's start and the list's round trip, but few work-groups leave CUs idle: as many as
     // still fill the chip twice (two work-groups per CU at head dimension 128, three at 64).  Four at any size against this
     // rule, operator: 14/2 heads of 64, 8192 tokens, every key selected 491 -> 288 us; 32/8 heads of 128, 4096 tokens
@@ -1135,26 +1146,56 @@ static hipError_t launch(const FlashArgs& args, hipStream_t stream) {
     while (nq > 1 && (per_big_block % nq != 0 || blocks / nq < fills_twice)) nq /= 2;
     a.q_blocks_per_wg = nq;
   }
-  const dim3 grid(MODE == kRows || MODE == kMasked ? (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks
-                                : (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0));
   // More units (KV heads of all batch elements) than XCDs: side by side as long as the K and V that an XCD then works on fit its L2
   // of 4 MB.  Left-padded batches: 3 x 2500 with 32/8 heads of 128 194 -> 184 us, 28/4 184 -> 162, 3 x 1000 with 32/8 heads of 64 39.9 -> 30.0, 4 x 2900
   // 162 -> 150; the operator on 2 x 4096 tokens with those heads 181 -> 172.  Larger contexts, where the order hardly matters: within 1 %.
   const int units = a.batch * a.n_kv_heads;
   a.abreast = MODE != kSparse && 8 % units != 0 && (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20;
+  if (MODE == kRows || MODE == kMasked) return (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks;
+  return (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0);
+}
+
+template <int MODE>
+static int teams_of(const FlashArgs& a, const uint32_t work_groups) {
   // Two teams where a work-group is alone on its CU and its tiles pay for the merge (1.5 us).  Head dimension 64: 2048 tokens with 14/2
   // heads, one launch, 26.4 -> 22.9 us, dense 25.9 -> 22.3, 1024 tokens dense 15.0 -> 14.1, a prompt of 2348 44.3 -> 40.4, padded 2 x 1000 25.7 -> 23.3;
   // 512 tokens dense (8 tiles) 9.6 -> 10.2, and 512 work-groups (32 heads, 2048 tokens) 27.6 -> 29.5.
   // (anchor: a single big block only, whose rows are finished or leave their state; larger contexts give the same bits in any batch)
-  const bool fits = MODE != kAnchor || (a.n_ctx == a.big_block && (a.qbar_out == nullptr || a.out != nullptr));
-  const int teams = fits && grid.x <= 256 && (kAnyRowsMode ? a.chunk_tiles : a.n_ctx / kBN) >= 12 ? 2 : 1;
-  if (a.head_dim == 128) {
-    if (a.dtype == 0) launch_for<MODE, Bf16, 128>(a, grid, teams, stream);
-    else launch_for<MODE, F16, 128>(a, grid, teams, stream);
-  } else {  // 64: the C-ABI layer admits nothing else
-    if (a.dtype == 0) launch_for<MODE, Bf16, 64>(a, grid, teams, stream);
-    else launch_for<MODE, F16, 64>(a, grid, teams, stream);
-  }
+  const bool fits = MODE == kAnchor ? a.n_ctx == a.big_block && (a.qbar_out == nullptr || a.out != nullptr) : MODE != kSparse;
+  return a.head_dim == 64 && fits && work_groups <= 256 && (MODE == kRows || MODE == kMasked ? a.chunk_tiles : a.n_ctx / kBN) >= 12 ? 2 : 1;
+}
+
+template <int MODE, typename T>
+static void launch_for(const FlashArgs& a, const uint32_t work_groups, hipStream_t stream) {
+  const dim3 grid(work_groups);
+  if (a.head_dim == 128) hipLaunchKernelGGL((flash_kernel<MODE, T, 128, 1>), grid, dim3(256), 0, stream, a);
+  else if (teams_of<MODE>(a, work_groups) == 1) hipLaunchKernelGGL((flash_kernel<MODE, T, 64, 1>), grid, dim3(256), 0, stream, a);
+  else if constexpr (MODE != kSparse) hipLaunchKernelGGL((flash_kernel<MODE, T, 64, 2>), grid, dim3(512), 0, stream, a);
+}
+
+template <int MODE>
+static hipError_t launch(FlashArgs a, hipStream_t stream) {
+  const uint32_t work_groups = place<MODE>(a);
+  if (work_groups == 0) return hipSuccess;
+  if (a.dtype == 0) launch_for<MODE, Bf16>(a, work_groups, stream);
+  else launch_for<MODE, F16>(a, work_groups, stream);
+  return hipGetLastError();
+}
+
+template <typename T>
+static void launch_pair_for(const FlashArgs& a, const FlashArgs& r, const uint32_t n_anchor, const uint32_t n_rows, hipStream_t stream) {
+  const uint32_t both = ((n_rows + 7u) & ~7u) + n_anchor;
+  const dim3 grid(both);
+  if (a.head_dim == 128) hipLaunchKernelGGL((flash_pair_kernel<T, 128, 1>), grid, dim3(256), 0, stream, a, r, n_rows);
+  else if (teams_of<kAnchor>(a, both) == 1 || teams_of<kRows>(r, both) == 1)
+    hipLaunchKernelGGL((flash_pair_kernel<T, 64, 1>), grid, dim3(256), 0, stream, a, r, n_rows);
+  else hipLaunchKernelGGL((flash_pair_kernel<T, 64, 2>), grid, dim3(512), 0, stream, a, r, n_rows);
+}
+
+hipError_t launch_anchor_and_rows(FlashArgs anchor, FlashArgs rows, hipStream_t stream) {
+  const uint32_t n_anchor = place<kAnchor>(anchor), n_rows = place<kRows>(rows);
+  if (anchor.dtype == 0) launch_pair_for<Bf16>(anchor, rows, n_anchor, n_rows, stream);
+  else launch_pair_for<F16>(anchor, rows, n_anchor, n_rows, stream);
   return hipGetLastError();
 }
 

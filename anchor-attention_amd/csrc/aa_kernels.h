@@ -45,11 +45,15 @@ struct FlashArgs {
 
 // mode: 0 anchor (stage 1), 1 sparse (stage 3), 2 dense causal, 3 rows, 4 masked
 hipError_t launch_flash(const FlashArgs& a, int mode, hipStream_t stream);
+// anchor mode and rows mode (same types and head dimension) in one launch
+hipError_t launch_anchor_and_rows(FlashArgs anchor, FlashArgs rows, hipStream_t stream);
 
 // rows mode with several chunks: merges the chunks of `a` (the arguments of the launch that wrote them) into a.out
 hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream);
 // rows mode: sets n_col_blocks, n_chunks and chunk_tiles from the sizes
 void plan_rows(FlashArgs& a);
+// ... for a launch that anchor work-groups of `anchor` share (launch_anchor_and_rows)
+void plan_rows_beside(FlashArgs& a, const FlashArgs& anchor);
 constexpr int kMaskedTiles = 1024;  // most tiles in a chunk of masked mode (the list of a chunk's visible tiles lives in LDS)
 // masked mode: fills mask_words and tile_flags of `a` from a byte mask [batch, n_rows, n_ctx] with strides (mask_sb, mask_sn, 1)
 hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mask_sb, int64_t mask_sn, hipStream_t stream);

@@ -221,6 +221,24 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                       int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
                       float sm_scale, int dtype, void* stream);
 
+/* The operator and, beside it, dense attention of other rows (r*, n_rows, n_keys, causal_offset, rows_scale: as in aa_dense_rows_fwd
+ * without a mask; same batch, heads, head_dim and type): what a prompt that ends in part of a big block needs.  The rows depend on no stage and
+ * share stage 1's launch.  counts_out and ratio (with ratio_host and denominator) may be NULL.  The outputs must not overlap. */
+size_t aa_anchor_attn_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim, int block_size, int step,
+                                           int n_rows, int n_keys, int causal_offset);
+int aa_anchor_attn_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
+                            const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+                            const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
+                            void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
+                            const void* rq, int64_t rq_sb, int64_t rq_sh, int64_t rq_sn,
+                            const void* rk, int64_t rk_sb, int64_t rk_sh, int64_t rk_sn,
+                            const void* rv, int64_t rv_sb, int64_t rv_sh, int64_t rv_sn,
+                            void* rout, int64_t ro_sb, int64_t ro_sh, int64_t ro_sn, int n_rows, int n_keys, int causal_offset, float rows_scale,
+                            void* workspace, size_t workspace_bytes, int32_t* counts_out, float* ratio, float* ratio_host, double denominator,
+                            int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
+                            int block_size, int step, double sm_scale, float theta_log2, int scale_mode, int geometry,
+                            int dtype, void* stream);
+
 /* ---- between a patched model's matrix products ------------------------------------------------
  * What the models that the attention plug is used in compute around it, one pass each, with the 16-bit roundings of the framework's
  * single operations (all tensors 16-byte aligned and contiguous):
