@@ -15,8 +15,8 @@ import ctypes
 import threading
 import time
 
+import my_utils
 import torch
-from my_utils import Logger
 
 from . import _hip
 from .anchor_step_1_2_v2 import (_check_inputs, _row_major, _stream, anchor_attn_step_1,
@@ -46,7 +46,7 @@ _host_ratios = threading.local()
 def _host_ratio(device):
     """This thread's word of pinned host memory for ratios of calls on ``device``, unset; None if the ratio of a call cannot be
     waited for.  One word is enough: a call that uses it returns when the GPU has written it."""
-    if not (Logger.enabled and device.type == "cuda" and torch.get_default_dtype() == torch.float32) or torch.cuda.is_current_stream_capturing():
+    if not (my_utils.Logger.enabled and device.type == "cuda" and torch.get_default_dtype() == torch.float32) or torch.cuda.is_current_stream_capturing():
         return None
     words = _host_ratios.__dict__
     word = words.get(str(device))
@@ -69,9 +69,13 @@ def _log_ratio(sparse_ratio, host_ratio=None):
         there = host_ratio is not None and _hip.lib().aa_wait_ratio(ctypes.addressof(host_ratio), _UNSET, 100000)
         text = f"anchor sparse_ratio:{host_ratio.value if there else sparse_ratio}"
         return text
-    if Logger.enabled or host_ratio is not None:
-        Logger.log(message)  # (which opens its file first, while the GPU works)
-        if text is None:  # (it could not: the GPU still has to have written the word before the next call uses it)
+    log = my_utils.Logger.log
+    try:
+        if my_utils.Logger.enabled:
+            # (the own logger opens its file first, while the GPU works; one that a program put in its place is given the line)
+            log(message if getattr(log, "takes_function", False) else message())
+    finally:
+        if text is None and host_ratio is not None:  # (not written: the GPU still has to have stored the word before the next call uses it)
             message()
 
 

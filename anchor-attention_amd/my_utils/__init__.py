@@ -32,6 +32,8 @@ class Logger:
         except OSError as e:
             print(f"Unable to write to log file: {e}")
 
+    log.__func__.takes_function = True  # (a function in this one's place may know strings only)
+
     @classmethod
     def log_error(cls, m: str):
         cls.log(f"ERROR: {m}")

@@ -76,3 +76,28 @@ def test_threads_and_streams_log_their_own(log_file):
         t.join()
     assert not failures, failures
     assert sorted(_logged(log_file)) == sorted(str(r) for r in ratios) and len(set(ratios)) == 3
+
+
+@pytest.mark.parametrize("raises", [False, True])
+def test_a_logger_in_the_place_of_the_own_one_gets_the_line(monkeypatch, log_file, raises):
+    import my_utils
+    from anchor_attn.src.ops.anchor_attn_v4 import anchor_attn
+    lines = []
+
+    class Other:
+        enabled = True
+
+        @staticmethod
+        def log(message):
+            lines.append(message)
+            if raises:
+                raise RuntimeError("no room")
+    monkeypatch.setattr(my_utils, "Logger", Other)
+    q, k, v = _inputs(1536, 3)
+    if raises:
+        with pytest.raises(RuntimeError, match="no room"):
+            anchor_attn(q, k, v, block_size=32)
+    else:
+        lines.append(f"anchor sparse_ratio:{float(anchor_attn(q, k, v, block_size=32)[1])}")
+        assert lines[0] == lines[1]
+    assert isinstance(lines[0], str) and lines[0].startswith("anchor sparse_ratio:0.")
