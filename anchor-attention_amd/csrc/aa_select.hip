@@ -315,47 +315,103 @@ hipError_t launch_select_scores(const SelectArgs& a, hipStream_t stream) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// One wave per (batch, query head, big block): the candidate keys [key_lo, bb*S - key_slack) of the big block's mask row
-// become an ascending index list (popcount per 32-key word, wave prefix sum, each lane writes its word's set bits).
-__global__ void __launch_bounds__(64) select_compact_kernel(const SelectArgs p) {
+// One work-group per (batch, query head, big block): the candidate keys [key_lo, key_hi = bb*S - key_slack) of the big block's mask row
+// become an ascending index list.
+// What bounds it is the longest row: its chain of loads, prefix sums and stores (one wave with 64 words at a time: 63 links at 131072
+// tokens, 37 us), and where many keys are selected its stores, a lane's own run of places each.  So eight waves take 4096 words
+// at a time, eight to a lane, all loaded at once; their 64 (turn, wave) totals are summed by one more scan, with one barrier.  A wave
+// whose words hold more than COMPACT_DENSE keys on average writes 64 keys at a time to neighbouring places.  32 heads, one
+// wave -> eight: 131072 tokens with 0.6 % of the keys 37 -> 15 us, 50 % 439 -> 97, all 938 -> 131; 40960 tokens 12.6 -> 5.8, all 81 -> 17.
+// (COMPACT_DENSE: 40960 tokens with 25 % of the keys, 8 to a word, take 16 us each lane for itself and 20 together, with 50 % 40 and 17.)
+constexpr int COMPACT_WAVES = 8, COMPACT_TURNS = 8, COMPACT_WORDS = 64 * COMPACT_WAVES;
+constexpr int COMPACT_DENSE = 12;
+
+__device__ __forceinline__ int wave_scan(int x, const int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(x, d, 64);
+    if (lane >= d) x += up;
+  }
+  return x;
+}
+
+__global__ void __launch_bounds__(COMPACT_WORDS) select_compact_kernel(const SelectArgs p) {
+  static_assert(COMPACT_WAVES * COMPACT_TURNS == 64 && COMPACT_TURNS % 2 == 0, "a lane for each total, two turns to a scan");
+  __shared__ int part[2][64];
   const int bb = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n_bb = p.n_ctx / p.big_block;
   const int n_t = p.n_ctx / 128;
   const int64_t bh = (int64_t)b * p.n_q_heads + h;
-  const int key_lo = p.key_lo, key_hi = bb * p.big_block - p.key_slack;  // candidate keys [key_lo, key_hi)
+  const int key_lo = p.key_lo, key_hi = bb * p.big_block - p.key_slack;
+  const int w_lo = key_lo / 32, w_hi = (key_hi + 31) / 32;  // mask words [w_lo, w_hi) of the row
+  const uint32_t* mw = p.mask + (bh * n_bb + bb) * n_t * 4;
+  int32_t* out = p.coords + bh * p.coords_per_head + coords_tri(bb, p.big_block, p.block_size);
+  const auto load = [&](const int wi) {
+    const int k0 = wi * 32;
+    uint32_t word = wi < w_hi ? mw[wi] : 0u;
+    // the first and the last word may reach outside the candidate range (block sizes below 32 keys)
+    if (k0 < key_lo) word &= key_lo - k0 >= 32 ? 0u : ~0u << (key_lo - k0);
+    if (k0 + 32 > key_hi) word &= key_hi <= k0 ? 0u : ~0u >> (k0 + 32 - key_hi);
+    return word;
+  };
   int base = 0;
-  if (key_hi > key_lo) {
-    const int w_lo = key_lo / 32, w_hi = (key_hi + 31) / 32;  // mask words [w_lo, w_hi) of the row
-    const uint32_t* mw = p.mask + (bh * n_bb + bb) * n_t * 4;
-    int32_t* out = p.coords + bh * p.coords_per_head + coords_tri(bb, p.big_block, p.block_size);
-    for (int w0 = w_lo; w0 < w_hi; w0 += 64) {
-      const int wi = w0 + lane;
-      uint32_t word = wi < w_hi ? mw[wi] : 0u;
-      // the first and the last word may reach outside the candidate range (block sizes below 32 keys)
-      const int k0 = wi * 32;
-      if (k0 < key_lo) word &= key_lo - k0 >= 32 ? 0u : ~0u << (key_lo - k0);
-      if (k0 + 32 > key_hi) word &= key_hi <= k0 ? 0u : ~0u >> (k0 + 32 - key_hi);
-      const int pc = __popc(word);
-      int incl = pc;
+  if (key_hi > key_lo && w_hi - w_lo <= 64) {  // a single wave's words: no barrier, and no stores of other waves to wait behind
+    if (wave != 0) return;
+    uint32_t word = load(w_lo + lane);
+    const int incl = wave_scan(__popc(word), lane);
+    int pos = incl - __popc(word);
+    for (; word != 0u; word &= word - 1u) out[pos++] = (w_lo + lane) * 32 + (__ffs(word) - 1);
+    base = __builtin_amdgcn_readlane(incl, 63);
+  } else if (key_hi > key_lo) {
+    for (int w0 = w_lo, set = 0; w0 < w_hi; w0 += COMPACT_TURNS * COMPACT_WORDS, set ^= 1) {
+      uint32_t words[COMPACT_TURNS];
+      int incl[COMPACT_TURNS];
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += up;
+      for (int i = 0; i < COMPACT_TURNS; ++i) words[i] = load(w0 + i * COMPACT_WORDS + (int)threadIdx.x);
+#pragma unroll
+      for (int i = 0; i < COMPACT_TURNS; i += 2) {
+        int both = 0;  // (two sums of at most 2048 in one scan)
+        if (w0 + i * COMPACT_WORDS < w_hi) both = wave_scan(__popc(words[i]) | __popc(words[i + 1]) << 16, lane);
+        incl[i] = both & 0xffff;
+        incl[i + 1] = both >> 16;
+        if (lane == 63) {
+          part[set][i * COMPACT_WAVES + wave] = incl[i];
+          part[set][(i + 1) * COMPACT_WAVES + wave] = incl[i + 1];
+        }
       }
-      int pos = base + incl - pc;
-      while (word) {
-        out[pos++] = k0 + (__ffs(word) - 1);
-        word &= word - 1;
+      // (two sets of totals: a wave writes a set again only after the barrier between, which all reach after reading it)
+      __syncthreads();
+      const int totals = part[set][lane];
+      const int before = base + wave_scan(totals, lane) - totals;
+      base = __builtin_amdgcn_readlane(before + totals, 63);
+#pragma unroll
+      for (int i = 0; i < COMPACT_TURNS; ++i) {
+        if (w0 + i * COMPACT_WORDS >= w_hi) break;
+        uint32_t word = words[i];
+        int pos = __builtin_amdgcn_readlane(before, i * COMPACT_WAVES + wave);
+        const int key = (w0 + i * COMPACT_WORDS + wave * 64) * 32;  // of the wave's first word
+        if (__builtin_amdgcn_readlane(incl[i], 63) > COMPACT_DENSE * __popcll(__ballot(word != 0u))) {
+#pragma unroll 8
+          for (int src = 0; src < 64; src += 2) {
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)word, src), hi = (uint32_t)__builtin_amdgcn_readlane((int)word, src + 1);
+            const int below = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+            if (((lane < 32 ? lo : hi) >> (lane & 31)) & 1u) out[pos + below] = key + src * 32 + lane;
+            pos += __popc(lo) + __popc(hi);
+          }
+        } else {
+          pos += incl[i] - __popc(word);
+          for (; word != 0u; word &= word - 1u) out[pos++] = key + lane * 32 + (__ffs(word) - 1);
+        }
       }
-      base += __shfl(incl, 63, 64);
     }
   }
-  if (lane == 0) p.counts[bh * n_bb + bb] = base;
+  if (threadIdx.x == 0) p.counts[bh * n_bb + bb] = base;
 }
 
 hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL(select_compact_kernel, dim3(a.n_ctx / a.big_block, a.n_q_heads, a.batch), dim3(64), 0, stream, a);
+  const bool short_rows = a.n_ctx - a.big_block <= 64 * 32;  // (then no row has more words)
+  hipLaunchKernelGGL(select_compact_kernel, dim3(a.n_ctx / a.big_block, a.n_q_heads, a.batch), dim3(short_rows ? 64 : COMPACT_WORDS), 0, stream, a);
   return hipGetLastError();
 }
 
