@@ -112,8 +112,10 @@ def _rms_norm_forward(self, hidden_states):
 
 
 def _is_silu(act) -> bool:
-    """The framework's or transformers' SiLU module, and no hook that would see it called."""
-    return (type(act).__name__ in ("SiLU", "SiLUActivation") and not (act._forward_hooks or act._forward_pre_hooks)
+    """The framework's or transformers' SiLU module (another class of that name may compute something else), and nothing that sees it called."""
+    kind = type(act)
+    return ((kind is torch.nn.SiLU or (kind.__module__, kind.__name__) == ("transformers.activations", "SiLUActivation"))
+            and not (act._forward_hooks or act._forward_pre_hooks or "forward" in act.__dict__)
             and not (torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks))
 
 

@@ -62,6 +62,25 @@ def test_classes_that_compute_something_else_are_left_alone():
     assert fuse_between_products(m) == 0 and "forward" not in m[0].__dict__
 
 
+def test_other_activations_of_that_name_are_left_alone():
+    from transformers import LlamaConfig
+    from transformers.models.llama.modeling_llama import LlamaMLP
+
+    from anchor_attn.src.modules.model_forward import _is_silu, fuse_between_products
+
+    class SiLU(torch.nn.Module):  # a cheaper curve
+        def forward(self, x):
+            return x * torch.nn.functional.hardsigmoid(x)
+    m = LlamaMLP(LlamaConfig(hidden_size=16, intermediate_size=16, num_attention_heads=1))
+    m.act_fn = SiLU()
+    assert fuse_between_products(m) == 0
+    for act in (torch.nn.SiLU(), LlamaMLP(LlamaConfig(hidden_size=16, intermediate_size=16, num_attention_heads=1)).act_fn):
+        assert _is_silu(act)
+        act.forward = lambda x: x  # (a forward of the instance's own)
+        assert not _is_silu(act)
+    assert fuse_between_products(torch.nn.Sequential(LlamaMLP(LlamaConfig(hidden_size=16, intermediate_size=16, num_attention_heads=1)))) == 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,hidden", [(1, 8), (3, 64), (257, 896), (5, 2048), (2, 2056), (66, 4096), (3, 8192), (2, 16384), (1, 16376)])
