@@ -78,13 +78,16 @@ def chunk_mlp_over_tokens(model, chunk_tokens: int = MLP_CHUNK_TOKENS) -> int:
 
 
 def _kernel_takes(*tensors) -> bool:
-    """Plain 16-bit tensors on one GPU, contiguous on 16-byte boundaries, in an eager call that nothing differentiates or watches."""
+    """Plain 16-bit tensors on one GPU, contiguous on 16-byte boundaries, in an eager call that nothing differentiates or watches.
+    (What a tracer puts in the place of a tensor is not asked for its sizes: the answer would end the trace or tie it to them.)"""
+    if not (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors) and _called_plainly()):
+        return False
     first = tensors[0]
-    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda") or not _called_plainly():
+    if not first.is_cuda or first.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda"):
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
-        if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != first.dtype or t.device != first.device or not t.is_contiguous():
+        if t.dtype != first.dtype or t.device != first.device or not t.is_contiguous():
             return False
         if (grad and t.requires_grad) or not 0 < t.numel() < 1 << 35 or t.data_ptr() & 15:
             return False
@@ -101,9 +104,10 @@ def _launch(fn, device, *args) -> None:
 
 def _rms_norm_forward(self, hidden_states):
     weight = self.weight
-    n = hidden_states.shape[-1] if hidden_states.dim() else 0
-    if not (weight.shape == (n,) and n % 8 == 0 and 0 < n <= 16384 and hidden_states.numel() // n < 1 << 24
-            and _kernel_takes(hidden_states, weight)):
+    if not _kernel_takes(hidden_states, weight):
+        return type(self).forward(self, hidden_states)
+    n = weight.numel()
+    if not (hidden_states.shape[-1:] == weight.shape and n % 8 == 0 and n <= 16384 and hidden_states.numel() // n < 1 << 24):
         return type(self).forward(self, hidden_states)
     out = torch.empty_like(hidden_states)
     _launch(_hip.lib().aa_rms_norm, out.device, hidden_states.data_ptr(), weight.data_ptr(), out.data_ptr(), out.numel() // n, n,

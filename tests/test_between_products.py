@@ -62,6 +62,24 @@ def test_classes_that_compute_something_else_are_left_alone():
     assert fuse_between_products(m) == 0 and "forward" not in m[0].__dict__
 
 
+@pytest.mark.parametrize("kind", ["norm", "mlp"])
+def test_tracers_see_the_single_operations(kind):
+    """Symbolic tracing, and export with a size that stays open, meet the class's own forward: no branch on a size or a device."""
+    from transformers import LlamaConfig
+    from transformers.models.llama.modeling_llama import LlamaMLP, LlamaRMSNorm
+
+    from anchor_attn.src.modules.model_forward import fuse_between_products
+    m = LlamaRMSNorm(16) if kind == "norm" else LlamaMLP(LlamaConfig(hidden_size=16, intermediate_size=16, num_attention_heads=1))
+    outer, x, longer = torch.nn.Sequential(m), torch.randn(2, 3, 16), torch.randn(2, 5, 16)
+    assert fuse_between_products(outer) == 1
+    with torch.no_grad():
+        want = type(m).forward(m, longer)
+        assert torch.equal(torch.fx.symbolic_trace(outer)(longer), want)
+        for strict in (False, True):
+            exported = torch.export.export(outer, (x,), dynamic_shapes=({1: torch.export.Dim("tokens")},), strict=strict)
+            assert torch.equal(exported.module()(longer), want)
+
+
 def test_other_activations_of_that_name_are_left_alone():
     from transformers import LlamaConfig
     from transformers.models.llama.modeling_llama import LlamaMLP
