@@ -102,17 +102,21 @@ def _launch(fn, device, *args) -> None:
             _hip.check(fn(*args, _stream()))
 
 
-def _rms_norm_forward(self, hidden_states):
-    weight = self.weight
-    if not _kernel_takes(hidden_states, weight):
-        return type(self).forward(self, hidden_states)
-    n = weight.numel()
-    if not (hidden_states.shape[-1:] == weight.shape and n % 8 == 0 and n <= 16384 and hidden_states.numel() // n < 1 << 24):
-        return type(self).forward(self, hidden_states)
-    out = torch.empty_like(hidden_states)
-    _launch(_hip.lib().aa_rms_norm, out.device, hidden_states.data_ptr(), weight.data_ptr(), out.data_ptr(), out.numel() // n, n,
-            float(self.variance_epsilon), _hip.dtype_code(out))
-    return out
+def _rms_norm_forward(own):
+    """A norm's forward in the place of its class's, ``own``.  (One that a program gives the class later is used instead; and by its
+    name the bound method is pickled as the class's.)"""
+    def forward(self, hidden_states):
+        if type(self).forward is not own or not _kernel_takes(hidden_states, self.weight):
+            return type(self).forward(self, hidden_states)
+        weight, n = self.weight, self.weight.numel()
+        if not (hidden_states.shape[-1:] == weight.shape and n % 8 == 0 and n <= 16384 and hidden_states.numel() // n < 1 << 24):
+            return own(self, hidden_states)
+        out = torch.empty_like(hidden_states)
+        _launch(_hip.lib().aa_rms_norm, out.device, hidden_states.data_ptr(), weight.data_ptr(), out.data_ptr(), out.numel() // n, n,
+                float(self.variance_epsilon), _hip.dtype_code(out))
+        return out
+
+    return forward
 
 
 def _is_silu(act) -> bool:
@@ -123,26 +127,27 @@ def _is_silu(act) -> bool:
             and not (torch.nn.modules.module._global_forward_hooks or torch.nn.modules.module._global_forward_pre_hooks))
 
 
-def _gated_mlp_forward(self, x):
-    if not (_kernel_takes(x) and _is_silu(self.act_fn)):
-        return type(self).forward(self, x)
-    gate, up = self.gate_proj(x), self.up_proj(x)
-    if gate.shape == up.shape and gate.numel() % 8 == 0 and _kernel_takes(gate, up):
-        h = torch.empty_like(gate)
-        _launch(_hip.lib().aa_silu_mul, h.device, gate.data_ptr(), up.data_ptr(), h.data_ptr(), h.numel(), _hip.dtype_code(h))
-    else:
-        h = self.act_fn(gate) * up
-    return self.down_proj(h)
+def _gated_mlp_forward(own, own_act):
+    """An MLP's forward in the place of its class's, ``own``, with an activation whose class has the forward ``own_act``."""
+    def forward(self, x):
+        act = self.act_fn
+        if not (type(self).forward is own and _kernel_takes(x) and _is_silu(act) and type(act).forward is own_act):
+            return type(self).forward(self, x)
+        gate, up = self.gate_proj(x), self.up_proj(x)
+        if gate.shape == up.shape and gate.numel() % 8 == 0 and _kernel_takes(gate, up):
+            h = torch.empty_like(gate)
+            _launch(_hip.lib().aa_silu_mul, h.device, gate.data_ptr(), up.data_ptr(), h.data_ptr(), h.numel(), _hip.dtype_code(h))
+        else:
+            h = act(gate) * up
+        return self.down_proj(h)
 
-
-# (bound methods of these are copied with their module and pickled as its ``forward``, the class's own)
-_rms_norm_forward.__name__ = _gated_mlp_forward.__name__ = "forward"
+    return forward
 
 
 def _computes(cls, stub, x, want) -> bool:
     """Whether the class's own forward does what the kernel would take over, bit for bit on a few numbers."""
     try:
-        return torch.equal(cls.forward(stub, x), want)
+        return torch.equal(cls.forward(stub, x.clone()), want)  # (an activation may work in place)
     except Exception:  # noqa: BLE001 - a class that works otherwise
         return False
 
@@ -155,17 +160,19 @@ def fuse_between_products(model) -> int:
     scaled = x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-3)
     normed = norm.weight * scaled.to(x.dtype)
     mlp = types.SimpleNamespace(gate_proj=lambda t: t * 3, up_proj=lambda t: t + 1, down_proj=lambda t: t * 0.5, act_fn=torch.nn.functional.silu)
+    silu = torch.nn.functional.silu(x)
     gated = torch.nn.functional.silu(x * 3) * (x + 1) * 0.5
     n = 0
     with torch.no_grad():
         for m in model.modules():
-            name, fused = type(m).__name__, None
+            name, fused, act = type(m).__name__, None, getattr(m, "act_fn", None)
             if "forward" in m.__dict__:
                 continue
             if name in ("LlamaRMSNorm", "Qwen2RMSNorm") and _computes(type(m), norm, x, normed):
-                fused = _rms_norm_forward
-            elif name in ("LlamaMLP", "Qwen2MLP") and _is_silu(getattr(m, "act_fn", None)) and _computes(type(m), mlp, x, gated):
-                fused = _gated_mlp_forward
+                fused = _rms_norm_forward(type(m).forward)
+            elif (name in ("LlamaMLP", "Qwen2MLP") and _is_silu(act) and _computes(type(act), act, x, silu)
+                  and _computes(type(m), mlp, x, gated)):
+                fused = _gated_mlp_forward(type(m).forward, type(act).forward)
             if fused is not None:
                 m.forward = types.MethodType(fused, m)
                 n += 1

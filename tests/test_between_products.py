@@ -62,6 +62,28 @@ def test_classes_that_compute_something_else_are_left_alone():
     assert fuse_between_products(m) == 0 and "forward" not in m[0].__dict__
 
 
+def test_a_forward_that_a_class_is_given_later_is_used(monkeypatch):
+    from transformers import LlamaConfig
+    from transformers.models.llama.modeling_llama import LlamaMLP, LlamaRMSNorm
+
+    from anchor_attn.src.modules import model_forward
+    norm, mlp = LlamaRMSNorm(16), LlamaMLP(LlamaConfig(hidden_size=16, intermediate_size=16, num_attention_heads=1))
+    x = torch.randn(2, 16).bfloat16()
+    assert model_forward.fuse_between_products(torch.nn.Sequential(norm, mlp).bfloat16()) == 2
+    monkeypatch.setattr(model_forward, "_kernel_takes", lambda *tensors: True)
+    monkeypatch.setattr(model_forward, "_launch", lambda *args: pytest.fail("the kernel"))
+    with pytest.raises(pytest.fail.Exception):
+        norm(x)
+    with monkeypatch.context() as m:
+        m.setattr(LlamaRMSNorm, "forward", lambda self, t: t + 1)
+        m.setattr(LlamaMLP, "forward", lambda self, t: t + 2)
+        assert torch.equal(norm(x), x + 1) and torch.equal(mlp(x), x + 2)
+    with monkeypatch.context() as m:
+        m.setattr(type(mlp.act_fn), "forward", lambda self, t: t * 3)
+        assert torch.equal(mlp(x), mlp.down_proj(mlp.gate_proj(x) * 3 * mlp.up_proj(x)))
+        assert model_forward.fuse_between_products(torch.nn.Sequential(LlamaMLP(LlamaConfig(hidden_size=16, intermediate_size=16, num_attention_heads=1)))) == 0
+
+
 @pytest.mark.parametrize("kind", ["norm", "mlp"])
 def test_tracers_see_the_single_operations(kind):
     """Symbolic tracing, and export with a size that stays open, meet the class's own forward: no branch on a size or a device."""
