@@ -9,7 +9,8 @@ patch.py:36-45,142-144); the competitor patterns of the reference are not part o
 name through ``AttentionInterface``, so patching is: register the plug once, point the model's config at it,
 and copy the pattern's parameters onto the config (patch.py:106-109 does the same ``setattr`` loop).  Like the
 reference (patch.py:146-157), every pattern but "default" also makes the model return logits for the last position
-only and evaluates the MLPs in chunks of 32768 positions (``model_forward.py``).
+only and evaluates the MLPs in chunks of 32768 positions; the norms and the MLPs' activations run as one kernel each
+(``model_forward.py``).
 """
 import copy
 import json
@@ -73,7 +74,10 @@ def patch_model(model, pattern: str, config=None):
     config : None, a dict or a JSON string; for the anchor patterns ``{"block_size_M": 128, "theta": 12, "step": 16}``
              (the defaults; keys left out keep them).  Two optional keys with no counterpart in the reference steer
              the model-level patches the reference applies unconditionally: ``"last_token_logits"`` (default True) and
-             ``"mlp_chunk_tokens"`` (default 32768; 0 leaves the MLPs alone).
+             ``"mlp_chunk_tokens"`` (default 32768; 0 leaves the MLPs alone).  A third, ``"fuse_between_products"`` (default
+             True), steers one that the reference does not have: in eager 16-bit inference norms and gated activations are
+             single kernels, whose results may differ from the single operations' in the last 16-bit unit; False leaves
+             them alone (a model patched before keeps what it has).
     """
     from transformers import PreTrainedModel
     if not isinstance(model, PreTrainedModel):
@@ -89,6 +93,7 @@ def patch_model(model, pattern: str, config=None):
     cfg.update(_config_dict(config))
     last_token_logits = bool(cfg.pop("last_token_logits", True))
     mlp_chunk_tokens = int(cfg.pop("mlp_chunk_tokens", MLP_CHUNK_TOKENS))
+    fuse = bool(cfg.pop("fuse_between_products", True))
     if pattern == "flash":
         model.set_attn_implementation("sdpa")
     elif pattern == "dense":
@@ -101,7 +106,8 @@ def patch_model(model, pattern: str, config=None):
             setattr(model.config, k, v)
     if last_token_logits:
         keep_last_token_logits(model)
-    fuse_between_products(model)
+    if fuse:
+        fuse_between_products(model)
     chunk_mlp_over_tokens(model, mlp_chunk_tokens)
     Logger.log(f"replace attention with {pattern}: {cfg}")
     return model

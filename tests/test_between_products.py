@@ -47,6 +47,14 @@ def test_which_modules_are_fused_and_that_copies_keep_their_own(family):
     assert torch.equal(other.model.layers[0].mlp(y), type(other.model.layers[0].mlp).forward(other.model.layers[0].mlp, y))
 
 
+@pytest.mark.parametrize("pattern", ["flash", "dense", "anchor_attn"])
+def test_the_config_declines_the_fusion(pattern):
+    from anchor_attn import patch_model
+    m = patch_model(_tiny(), pattern, {"fuse_between_products": False})
+    assert not any(isinstance(x.__dict__.get("forward"), types.MethodType) for x in m.modules()) and not hasattr(m.config, "fuse_between_products")
+    assert sum(isinstance(x.__dict__.get("forward"), types.MethodType) for x in patch_model(m, pattern).modules()) == 5
+
+
 def test_classes_that_compute_something_else_are_left_alone():
     from anchor_attn.src.modules.model_forward import fuse_between_products
 
