@@ -48,6 +48,7 @@
 //   K row r, chunk c  ->  slot c ^ (r & 15)          c ^ ((r & 7) ^ (r >> 3 & 1))   (row-per-lane 16-byte reads)
 //   V row r, chunk c  ->  slot c ^ ((r & 7) << 1)    c ^ ((r & 3) << 1)             (transposing 8-byte reads)
 // These choices measure conflict-free for their read pattern (and each is 2-way conflicted for the other's).
+#include <cstddef>
 #include <type_traits>
 
 #include "aa_common.h"
@@ -103,7 +104,7 @@ struct FlashSmem {
   } t[TEAMS];  // (the epilogue stages the output in the tile space)
   floatx2 stats[TEAMS > 1 ? 256 : 1];  // the second team's reference and sum, lane by lane
   // sparse mode: window of the big block's index list; masked mode: the chunk's tiles that hold a visible key, and their number
-  int32_t idx[MODE == kSparse ? kIdxWin : MODE == kMasked ? kMaskedTiles + 4 : 4];
+  alignas(16) int32_t idx[MODE == kSparse ? kIdxWin : MODE == kMasked ? kMaskedTiles + 4 : 4];
 };
 
 // Query pre-scaling into the exp2 domain, eight elements at a time.  `chain`: both constants and both products rounded
@@ -190,6 +191,8 @@ template <int MODE, typename T, int D, int TEAMS>
 __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t block, FlashSmem<MODE, D, TEAMS>& sm) {
   typedef typename T::vec8 vec8;
   typedef __attribute__((address_space(3))) vec8 lds_vec8;
+  typedef FlashSmem<MODE, D, TEAMS> Smem;
+  static_assert(offsetof(Smem, idx) % 16 == 0, "the index window is written 16 bytes at a time");
   static_assert(TEAMS == 1 || (TEAMS == 2 && MODE != kSparse && D == 64), "teams");
   constexpr int BM = 128;
   constexpr bool kAnyRows = MODE == kRows || MODE == kMasked;
