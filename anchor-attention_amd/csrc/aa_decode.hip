@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(64 * WAVES) decode_kernel(const FlashArgs p) {
     slot ^= 1;
   }
 
-  if (__builtin_expect(__any(holds_nan(acc) && !is_nan(l_run)), 0)) {
+  if (__builtin_expect(__any(is_nan(sum_of_all(acc)) && !is_nan(l_run)), 0)) {
     // V holds infinities or NaN: the wave's sums once more (see aa_nonfinite.h)
     const float m_base = m_run == -INFINITY ? 0.f : m_run;
 #pragma unroll

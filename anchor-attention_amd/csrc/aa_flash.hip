@@ -32,7 +32,8 @@
 // bf16 rows and masked modes, which keep a probability as two numbers, need no max at all (kLazyRef): m is the row max of the
 // first 32 keys and stays, and a larger score gives a p above 1, which is held as precisely as one below.  When the
 // sum of a half-tile's p exceeds kRebaseSum - an overflowing exp2 included - the wave forms that half's scores again,
-// moves m to the row's max and rescales, before these p are used.  (fp16 forms 2^15 p, which has no room above p = 1.)
+// moves m to the row's max and rescales, before these p are used.  (fp16 forms 2^15 p, which has no room above p = 1.)  What the
+// larger p take from the range of V is given back at the end, where sums that overflowed are formed again (aa_nonfinite.h).
 // 777 rows over 777 keys, 32/8 heads of 128: 23.0 -> 21.1 us; a padded batch of 3 x 2500: 203 -> 193.
 //
 // Inside a 64-key tile the two 32-key halves are staggered so that matrix and vector work overlap
@@ -909,34 +910,6 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
 #undef AA_FENCE
 #undef AA_SCORES
 
-  if (kAnyRows && __builtin_expect(__any(holds_nan(acc) && !is_nan(l_run)), 0)) {
-    // V holds infinities or NaN: the wave's sums once more (see aa_nonfinite.h)
-    const float m_base = m_ref == kNoRef ? 0.f : m_ref;
-#pragma unroll
-    for (int db = 0; db < kDB; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
-    for (int i = 0; i < 2 * n_tiles; ++i) {  // 32 keys at a time
-      if (TEAMS > 1 && (i >> 1) % TEAMS != team) continue;
-      int key0 = key_base + 32 * i;
-      uint32_t seen;
-      if (MODE == kMasked) {
-        const int32_t entry = __builtin_amdgcn_readfirstlane(sm.idx[i >> 1]);
-        const int tile = entry & (kMixedTile - 1);
-        key0 = tile * kBN + 32 * (i & 1);
-        seen = ~0u;
-        if (entry & kMixedTile) {
-          const char* w = reinterpret_cast<const char*>(p.mask_words + ((int64_t)b * p.n_rows * p.mask_words_per_row + tile));
-          seen = *reinterpret_cast<const uint32_t*>(w + mask_row_off + 4 * (i & 1));
-        }
-      } else {
-        const int count = my_last_key + 1 - key0;
-        seen = count >= 32 ? ~0u : count <= 0 ? 0u : (1u << count) - 1u;
-      }
-      exact_pv_tile<T, D>(acc, qreg, kbase, vbase, k_row_bytes, v_row_bytes, key0, p.n_ctx, seen, m_base, score_scale, lane);
-    }
-  }
-
   if (TEAMS > 1) {
     // ---- the second team's state -> the first ----------------------------------------------------
     char* state = sm.t[1].k[0];  // (its tiles: as many bytes as its accumulators)
@@ -970,6 +943,50 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       }
     m_ref = kLazyRef && m_new == -INFINITY ? kNoRef : m_base;
     if (m_new != -INFINITY) m_over = 0.f;
+  }
+
+  const float acc_sum = kAnyRows ? sum_of_all(acc) : 0.f;
+  if (kAnyRows && __builtin_expect(__any((kLazyRef ? !is_finite(acc_sum) : is_nan(acc_sum)) && !is_nan(l_run)), 0)) {
+    // V holds infinities or NaN, or is too large for probabilities above 1: the wave's sums once more (see aa_nonfinite.h)
+    auto each_half = [&](auto&& visit) __attribute__((always_inline)) {
+      for (int i = 0; i < 2 * n_tiles; ++i) {  // 32 keys at a time
+        int key0 = key_base + 32 * i;
+        uint32_t seen;
+        if (MODE == kMasked) {
+          const int32_t entry = __builtin_amdgcn_readfirstlane(sm.idx[i >> 1]);
+          const int tile = entry & (kMixedTile - 1);
+          key0 = tile * kBN + 32 * (i & 1);
+          seen = ~0u;
+          if (entry & kMixedTile) {
+            const char* w = reinterpret_cast<const char*>(p.mask_words + ((int64_t)b * p.n_rows * p.mask_words_per_row + tile));
+            seen = *reinterpret_cast<const uint32_t*>(w + mask_row_off + 4 * (i & 1));
+          }
+        } else {
+          const int count = my_last_key + 1 - key0;
+          seen = count >= 32 ? ~0u : count <= 0 ? 0u : (1u << count) - 1u;
+        }
+        visit(key0, seen);
+      }
+    };
+    if (kLazyRef) {
+      float mx = -INFINITY;
+      each_half([&](const int key0, const uint32_t seen) __attribute__((always_inline)) {
+        mx = exact_max(exact_scores<T, D>(qreg, kbase, k_row_bytes, key0, p.n_ctx, lane), seen, lane, mx);
+      });
+      mx = max_with_other_half(mx);
+      if (m_ref != kNoRef) {
+        l_run *= AA_EXP2(m_ref - mx);
+        m_ref = mx;
+      }
+    }
+    const float m_base = m_ref == kNoRef ? 0.f : m_ref;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+    each_half([&](const int key0, const uint32_t seen) __attribute__((always_inline)) {
+      exact_pv_tile<T, D>(acc, qreg, kbase, vbase, k_row_bytes, v_row_bytes, key0, p.n_ctx, seen, m_base, score_scale, lane);
+    });
   }
 #undef AA_EXP2
 

@@ -1,10 +1,14 @@
-// P.V where V is not finite, for the kernels that keep a probability as two 16-bit numbers (rows, masked and decode).
+// P.V where its sums are not finite, for the kernels that keep a probability as two 16-bit numbers (rows, masked and decode).
 //
 // With one product per key an infinite V gives an infinity.  With two it gives NaN: the rest of a probability may be 0 or
 // negative, and so are the keys past the last one, which repeat its row.  A wave that finds NaN among its sums therefore forms them once
 // more here: the rest meets V with its infinities and NaN left out, keys past the end count as 0 and a positive probability
 // does not round to 0.  What is NaN after that is NaN in float32 as well: a V that is, infinities of both signs, and an infinity at
 // a key of probability 0 (a masked key whose tile other rows of the work-group see).
+//
+// The bf16 rows and masked modes' probabilities are relative to a score that may lie up to 14 bits below the row's max (aa_flash.hip): 32 keys
+// sum to as much as 2^15, and P.V overflows float32 from |V| = 3.4e38 / (1024 n) on for n keys.  There a wave that finds infinities
+// among its sums comes here too and takes the row's max first, so that V may be as large as with probabilities up to 1, 3.4e38 / n.
 //
 // The operands come straight from memory, V two bytes at a time: some tens of times slower than the kernels' own tiles, and
 // reached by such V only.  The others pay one addition per accumulator register: 777 rows over 777 keys 22.40 -> 22.49 us, a
@@ -14,20 +18,46 @@
 
 namespace aa {
 
-__device__ __forceinline__ bool is_nan(float x) {
-  asm volatile("" : "+v"(x));  // (also where the compiler is told that there is none)
-  return (__float_as_uint(x) & 0x7fffffffu) > 0x7f800000u;
+// The bits of a float without its sign, hidden from the compiler: where it is told that there is no NaN, it would make of a comparison
+// of them one of floats, which NaN does not pass.
+__device__ __forceinline__ uint32_t magnitude_bits(const float x) {
+  uint32_t bits = __float_as_uint(x) & 0x7fffffffu;
+  asm volatile("" : "+v"(bits));
+  return bits;
 }
+__device__ __forceinline__ bool is_nan(const float x) { return magnitude_bits(x) > 0x7f800000u; }
+__device__ __forceinline__ bool is_finite(const float x) { return magnitude_bits(x) < 0x7f800000u; }
 
-// whether an accumulator of this lane is NaN (infinities of both signs count too)
+// NaN if an accumulator of this lane is NaN or infinities of both signs are among them, infinite or NaN if one of them is infinite
 template <int N>
-__device__ __forceinline__ bool holds_nan(const floatx16 (&acc)[N]) {
+__device__ __forceinline__ float sum_of_all(const floatx16 (&acc)[N]) {
   float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int db = 0; db < N; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) sum[r & 3] += acc[db][r];
-  return is_nan((sum[0] + sum[1]) + (sum[2] + sum[3]));
+  return (sum[0] + sum[1]) + (sum[2] + sum[3]);
+}
+
+// Raw scores of the 32 keys from key0 on (S^T, layout of the kernels).
+template <typename T, int D>
+__device__ __forceinline__ floatx16 exact_scores(const typename T::vec8 (&qreg)[D / 16], const char* kbase, const uint32_t k_row_bytes, const int key0,
+                                                 const int n_keys, const int lane) {
+  const char* kp = kbase + (uint64_t)(uint32_t)min(key0 + (lane & 31), n_keys - 1) * k_row_bytes + 16 * (lane >> 5);
+  floatx16 s;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) s = T::mfma(*reinterpret_cast<const typename T::vec8*>(kp + 32 * ks), qreg[ks], s);
+  return s;
+}
+
+// The largest of them that this lane holds and its column sees (`seen`: as below), or `mx`.
+__device__ __forceinline__ float exact_max(const floatx16& s, const uint32_t seen, const int lane, float mx) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    if ((seen >> (8 * (r >> 2) + 4 * (lane >> 5) + (r & 3))) & 1u) mx = fmaxf(mx, s[r]);
+  return mx;
 }
 
 // Adds the 32 keys from key0 on to acc (O^T, layout of the kernels).  `seen`: bit j says whether this lane's column sees
@@ -40,12 +70,7 @@ __device__ __forceinline__ void exact_pv_tile(floatx16 (&acc)[D / 32], const typ
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
   const int half = lane >> 5, c32 = lane & 31;
-  const char* kp = kbase + (uint64_t)(uint32_t)min(key0 + c32, n_keys - 1) * k_row_bytes + 16 * half;
-  floatx16 s;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) s[r] = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) s = T::mfma(*reinterpret_cast<const vec8*>(kp + 32 * ks), qreg[ks], s);
+  const floatx16 s = exact_scores<T, D>(qreg, kbase, k_row_bytes, key0, n_keys, lane);
   u32x4 pw[2], pw_rest[2];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {  // accumulator registers 2i, 2i+1

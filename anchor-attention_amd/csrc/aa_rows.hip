@@ -14,6 +14,7 @@
 
 #include "aa_common.h"
 #include "aa_kernels.h"
+#include "aa_nonfinite.h"
 
 namespace aa {
 
@@ -42,22 +43,35 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
 #pragma unroll 4
   for (int c = 0; c < n_chunks; ++c) m_all = fmaxf(m_all, p.M[(slot0 + 4 * c) * 32 + c32]);
   floatx4 acc[4];
-  float l_all = 0.f;
+  float l_all;
+  auto merge = [&](const float factor) __attribute__((always_inline)) {
+    l_all = 0.f;
 #pragma unroll
-  for (int rg = 0; rg < 4; ++rg) acc[rg] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int rg = 0; rg < 4; ++rg) acc[rg] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 2
-  for (int c = 0; c < n_chunks; ++c) {
-    const int64_t slot = slot0 + 4 * c;
-    const float m = p.M[slot * 32 + c32];
-    const float w = m == -INFINITY ? 0.f : fast_exp2((m - m_all) * scale);  // (a chunk without a key of this row's)
-    l_all += w * p.L[slot * 32 + c32];
-    const float* af = p.acc_frag + (slot * kDB + db) * (4 * 256) + lane * 4;
+    for (int c = 0; c < n_chunks; ++c) {
+      const int64_t slot = slot0 + 4 * c;
+      const float m = p.M[slot * 32 + c32];
+      const float w = m == -INFINITY ? 0.f : fast_exp2((m - m_all) * scale) * factor;  // (a chunk without a key of this row's)
+      l_all += w * p.L[slot * 32 + c32];
+      const float* af = p.acc_frag + (slot * kDB + db) * (4 * 256) + lane * 4;
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      const floatx4 t = *reinterpret_cast<const floatx4*>(af + rg * 256);
+      for (int rg = 0; rg < 4; ++rg) {
+        const floatx4 t = *reinterpret_cast<const floatx4*>(af + rg * 256);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[rg][e] += w * t[e];
+        for (int e = 0; e < 4; ++e) acc[rg][e] += w * t[e];
+      }
     }
+  };
+  merge(1.f);
+  if (T::kProbLog2 == 0.f) {
+    // bf16 chunks' sums are finite but may have probabilities above 1 in them (aa_nonfinite.h), and V so large that together they are not.
+    // Then once more, divided by the power of two that the sum of the probabilities holds: exact, and no larger than V.
+    float sum = 0.f;
+#pragma unroll
+    for (int rg = 0; rg < 4; ++rg) sum += (acc[rg][0] + acc[rg][1]) + (acc[rg][2] + acc[rg][3]);
+    if (__builtin_expect(__any(!is_finite(sum) && l_all > 1.f && is_finite(l_all)), 0))
+      merge(l_all > 1.f && is_finite(l_all) ? __uint_as_float((254u << 23) - (__float_as_uint(l_all) & 0x7f800000u)) : 1.f);
   }
   const float inv = l_all == 0.f ? 0.f : 1.f / l_all;  // (masked mode: a row that sees no key gives 0)
   uint32_t w[4][2];

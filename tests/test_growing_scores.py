@@ -68,3 +68,26 @@ def test_dense_rows_masked_and_operator(d, dtype):
     k[:, :, 1024:2048, 0] += 112.0
     got = anchor_attn(q, k, v, sm_scale=0.125, block_size=64, difference=1e4, strict_reference=False)[0]
     _check(got, _reference(q, k, v, scaled, _causal(3072)), v)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n,rows", [(900, 900), (6000, 77)])  # (teams of waves at head dimension 64; chunks that are merged)
+def test_values_that_sums_of_larger_probabilities_would_overflow_with(n, rows, d):
+    """Every second 32 keys score 6.75 nats above the others, so that probabilities relative to a part's first 32 keys are up to 2^9.7 and
+    none is redone for it; values from what n probabilities of 1 hold without overflow downwards, past 1024 times smaller."""
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_rows_attention
+    g = torch.Generator().manual_seed(n + d)
+    q, k = torch.zeros(1, 4, rows, d, dtype=torch.bfloat16), torch.zeros(1, 2, n, d, dtype=torch.bfloat16)
+    q[..., 0] = 8.0
+    k[..., 0] = (torch.arange(n) // 32 % 2) * 6.75
+    unit = torch.rand(1, 2, n, d, generator=g) * 0.5 + 0.5
+    unit[..., 1::2] *= -1.0
+    q, k, keep = q.cuda(), k.cuda(), _causal(n, rows)
+    for power in range(0, 20, 2):
+        v = (unit * (3.4e38 / n / 2.0 ** power)).bfloat16().cuda()
+        want = _reference(q, k, v, 0.125, keep)
+        _check(dense_rows_attention(q, k, v, n - rows, sm_scale=0.125), want, v)
+        _check(dense_rows_attention(q, k, v, sm_scale=0.125, mask=keep[None, None]), want, v)
+    v[:, :, 5, 0] = float("inf")  # (and infinities stay what they are)
+    got = dense_rows_attention(q, k, v, n - rows, sm_scale=0.125)
+    assert bool((got[:, :, 5:, 0] == float("inf")).all()) and bool(torch.isfinite(got[..., 1:]).all())
