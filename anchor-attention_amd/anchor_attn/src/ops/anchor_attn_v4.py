@@ -41,11 +41,12 @@ def _ratio(true_counts, B, H, N, block_size, step):
 
 _UNSET = -1.0
 _host_ratios = threading.local()
+_left_words, _left_lock = [], threading.Lock()
 
 
 def _host_ratio(device):
     """This thread's word of pinned host memory for ratios of calls on ``device``, unset; None if the ratio of a call cannot be
-    waited for.  One word is enough: a call that uses it returns when the GPU has written it."""
+    waited for.  One word is enough: a call that uses it returns when the GPU has written it, or leaves it (:func:`_leave_host_ratio`)."""
     if not (my_utils.Logger.enabled and device.type == "cuda" and torch.get_default_dtype() == torch.float32) or torch.cuda.is_current_stream_capturing():
         return None
     words = _host_ratios.__dict__
@@ -55,6 +56,15 @@ def _host_ratio(device):
         word = words[str(device)] = (tensor, ctypes.c_float.from_address(tensor.data_ptr()))
     word[1].value = _UNSET
     return word[1]
+
+
+def _leave_host_ratio(device):
+    """After a call that ended early, with its launch perhaps on the way: what that still stores is not the next call's, which gets
+    another word.  This one is kept until the stream has come to here."""
+    word, done = _host_ratios.__dict__.pop(str(device)), torch.cuda.Event()
+    with _left_lock:
+        done.record(torch.cuda.current_stream(device))
+        _left_words[:] = [left for left in _left_words if not left[1].query()] + [(word, done)]
 
 
 def _log_ratio(sparse_ratio, host_ratio=None):
@@ -196,13 +206,18 @@ def anchor_attn(Q, K, V, sm_scale: float = None, block_size: int = 128, step: in
     B, H, N, D = Q.shape
     sm_scale = sm_scale if sm_scale else 1.0 / (D ** 0.5)
     host_ratio = _host_ratio(Q.device) if return_computational_ratio else None
-    sparse_output, sparse_ratio = _anchor_attn(Q, K, V, sm_scale, block_size, step, difference,
-                                               return_computational_ratio, out=out, host_ratio=host_ratio, rows=rows,
-                                               geometry=_hip.AA_GEOMETRY_AS_RUN if strict_reference else _hip.AA_GEOMETRY_INTENDED)
-    if return_computational_ratio:
-        _log_ratio(sparse_ratio, host_ratio)
-        return sparse_output, sparse_ratio
-    return sparse_output
+    try:
+        sparse_output, sparse_ratio = _anchor_attn(Q, K, V, sm_scale, block_size, step, difference,
+                                                   return_computational_ratio, out=out, host_ratio=host_ratio, rows=rows,
+                                                   geometry=_hip.AA_GEOMETRY_AS_RUN if strict_reference else _hip.AA_GEOMETRY_INTENDED)
+        if return_computational_ratio:
+            _log_ratio(sparse_ratio, host_ratio)
+            return sparse_output, sparse_ratio
+        return sparse_output
+    except BaseException:  # (an interrupt among them)
+        if host_ratio is not None:
+            _leave_host_ratio(Q.device)
+        raise
 
 
 def anchor_attn_test_time(Q, K, V, sm_scale: float = None, block_size: int = 128, step: int = 16,

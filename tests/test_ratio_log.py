@@ -78,6 +78,35 @@ def test_threads_and_streams_log_their_own(log_file):
     assert sorted(_logged(log_file)) == sorted(str(r) for r in ratios) and len(set(ratios)) == 3
 
 
+def test_a_call_that_is_left_early_does_not_reach_the_next_ones_line(monkeypatch, log_file):
+    from anchor_attn.src.ops import anchor_attn_v4 as v4
+    first, second = _inputs(1536, 1), _inputs(1536, 5)
+    want = [float(v4.anchor_attn(*x, block_size=32)[1]) for x in (first, second)]
+    assert want[0] != want[1]
+    a = torch.randn(8192, 8192, device="cuda").bfloat16()
+    b = torch.empty_like(a)
+
+    def interrupted(*args):
+        raise KeyboardInterrupt
+    for _ in range(3):
+        for _ in range(40):  # (keeps the stream busy until the second call waits)
+            torch.mm(a, a, out=b)
+        with monkeypatch.context() as m:
+            m.setattr(v4, "_log_ratio", interrupted)
+            with pytest.raises(KeyboardInterrupt):
+                v4.anchor_attn(*first, block_size=32)
+        assert float(v4.anchor_attn(*second, block_size=32)[1]) == want[1]
+        assert _logged(log_file)[-1] == str(want[1])
+    with pytest.raises(Exception, match="workspace|unsupported|head"):
+        v4.anchor_attn(*[x[..., :32].contiguous() for x in first], block_size=32)  # (refused before any launch)
+    torch.cuda.synchronize()
+    with pytest.raises(Exception):
+        v4.anchor_attn(*[x[..., :32].contiguous() for x in first], block_size=32)
+    assert len(v4._left_words) <= 1  # (what is done is given back)
+    v4.anchor_attn(*first, block_size=32)
+    assert _logged(log_file)[-1] == str(want[0])
+
+
 @pytest.mark.parametrize("raises", [False, True])
 def test_a_logger_in_the_place_of_the_own_one_gets_the_line(monkeypatch, log_file, raises):
     import my_utils
