@@ -41,10 +41,19 @@ def test_which_modules_are_fused_and_that_copies_keep_their_own(family):
     assert torch.equal(again(x), m.model.norm(x))
     before = [x.forward for x in fused]
     assert [x.forward for x in fused if patch_model(m, "dense")] == before
-    other = patch_model(_tiny(family, hidden_act="gelu"), "flash")  # another activation stays with its own forward
-    assert "fused" not in repr(other.model.layers[0].mlp.act_fn)
-    y = torch.randn(1, 5, 256)
-    assert torch.equal(other.model.layers[0].mlp(y), type(other.model.layers[0].mlp).forward(other.model.layers[0].mlp, y))
+
+
+def test_other_activations_keep_their_own_forward(monkeypatch):
+    from anchor_attn.src.modules import model_forward
+    gelu, silu = _tiny(hidden_act="gelu").model.layers[0].mlp.bfloat16(), _tiny().model.layers[0].mlp.bfloat16()
+    assert model_forward.fuse_between_products(gelu) == 0 and "forward" not in gelu.__dict__
+    # an MLP that is given another activation after it was fused
+    assert model_forward.fuse_between_products(silu) == 1
+    x = torch.randn(1, 5, 256).bfloat16()
+    monkeypatch.setattr(model_forward, "_kernel_takes", lambda *tensors: True)
+    monkeypatch.setattr(model_forward, "_launch", lambda *args: pytest.fail("the kernel"))
+    silu.act_fn = gelu.act_fn
+    assert torch.equal(silu(x), type(silu).forward(silu, x))
 
 
 @pytest.mark.parametrize("pattern", ["flash", "dense", "anchor_attn"])
@@ -189,12 +198,20 @@ def test_calls_that_stay_with_the_single_operations(monkeypatch):
 
 
 @pytest.mark.gpu
-def test_patched_model_gives_the_logits_of_the_unfused_one():
+@pytest.mark.parametrize("act,mlps", [("silu", 2), ("gelu", 0)])
+def test_patched_model_gives_the_logits_of_the_unfused_one(monkeypatch, act, mlps):
     from anchor_attn import patch_model
-    m = patch_model(_tiny().to("cuda", torch.bfloat16), "flash")
+    from anchor_attn.src.ops import _hip
+    m = patch_model(_tiny(hidden_act=act).to("cuda", torch.bfloat16), "flash")
     tokens = torch.randint(0, 100, (2, 33), device="cuda")
+    calls = []
     with torch.no_grad():
-        got = m(tokens).logits
+        with monkeypatch.context() as watched:
+            for name in ("aa_rms_norm", "aa_silu_mul"):
+                inner = getattr(_hip.lib(), name)
+                watched.setattr(_hip.lib(), name, lambda *a, inner=inner, name=name: (calls.append(name), inner(*a))[1])
+            got = m(tokens).logits
+        assert calls.count("aa_rms_norm") == 5 and calls.count("aa_silu_mul") == mlps
         for x in m.modules():
             if isinstance(x.__dict__.get("forward"), types.MethodType):
                 del x.__dict__["forward"]
