@@ -70,8 +70,9 @@ def _leave_host_ratio(device):
 def _log_ratio(sparse_ratio, host_ratio=None):
     """The reference logs the ratio on every call (anchor_attn_v4.py:321-323).  Formatting the 0-dim device tensor
     copies it to the host, i.e. waits for the whole operator; a ``host_ratio`` that the operator was given is there as soon as
-    stage 2 is done, and the call returns while stage 3 runs.  One launch of 2048 tokens, 14/2 heads of 64: 63 us a call against 28; 4096
-    tokens, 32/8 heads of 128: 190 against 165."""
+    stage 2 is done (a single big block: when its first rows are), and the call returns while the GPU is at work.  Calls in a row: 2048 tokens, 14/2
+    heads of 64 63 us each against 28; 4096 tokens, 32/8 heads of 128 190 against 165.  (One call until its output is complete gains less
+    from it: with all the steps that this was one of 81 -> 50 and 218 -> 187.)"""
     text = None
 
     def message():
@@ -190,6 +191,9 @@ def anchor_attn(Q, K, V, sm_scale: float = None, block_size: int = 128, step: in
     ``strict_reference=False`` (analysis only, never the default) lets stage 2 choose from ``[S, bb*S)``
     - the range of the reference's fused variant, anchor_fuse_step_1_2_v2.py:152 - instead of the as-run
     ``[block_size, bb*S - block_size)``: no key is attended twice and none is left out.
+
+    With the ratio, a call waits for that number where the logger is on, and not for the output, which is ordered by the stream like any
+    GPU result.
 
     ``rows``: dense attention of other rows that is computed with the operator's first launch (:func:`rows_beside`)."""
     difference *= LOG2E
