@@ -178,10 +178,10 @@ __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, cons
 // D is the head dimension, 128 or 64: it sets the LDS row pitch, the number of tile loads, of MFMA steps over the head
 // dimension (kKS per 32 keys of Q.K^T) and of 32-column output blocks (kDB).
 //
-// Work-groups per CU: with 128 two (248 registers, 64 KB of LDS).  With 64 a tile has half the MFMAs but the same soft-max,
-// so the vector ALU bounds it, and a third wave per SIMD (168 registers; 2, 8 and 2 of them spill around the tile loop in
-// anchor, sparse and bf16 rows mode) keeps that busy: 69 % of the cycles, matrix pipe 49 %.  16384 tokens, 32/8 heads of 64: stage 1 470 -> 413 us
-// against two work-groups per CU and 256-byte LDS rows of which half was filled.
+// Work-groups per CU: with 128 two (up to 253 registers, 64 KB of LDS).  With 64 a tile has half the MFMAs but the same soft-max,
+// so the vector ALU bounds it, and a third wave per SIMD (168 registers; around the tile loop 2 of them spill in anchor mode, 9 in sparse,
+// 1 in fp16 rows mode, 2 and in fp16 5 in the launch of both) keeps that busy: 75 % of the cycles, matrix pipe 56 % (16384 tokens, 32/8
+// heads of 64, fp16).  Stage 1 there 470 -> 413 us against two work-groups per CU and 256-byte LDS rows of which half was filled.
 //
 // TEAMS: the waves that own the 128 rows, four to a team.  Two teams take the tiles alternately, each with LDS tiles and accumulators
 // of its own, and are merged through LDS at the end, like two chunks of the keys without a launch between them.  This is for

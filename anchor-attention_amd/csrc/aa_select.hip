@@ -12,8 +12,8 @@
 //           block) with no LDS and no atomics.
 //  thresholds  the selection test as a threshold on the raw dot product (aa_threshold.h), so that the score
 //           kernel's epilogue is a single compare per element; stage 1 forms them where it pools.
-//  compact  one wave per (batch, q head, big block) turns that big block's mask row into an ascending
-//           index list with popcounts and a wave prefix sum.
+//  compact  one work-group per (batch, q head, big block) turns that big block's mask row into an ascending
+//           index list with popcounts and prefix sums: eight waves, or one where a row has at most 64 words.
 #include "aa_common.h"
 #include "aa_kernels.h"
 #include "aa_threshold.h"
