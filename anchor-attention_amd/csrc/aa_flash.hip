@@ -910,46 +910,12 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
 #undef AA_FENCE
 #undef AA_SCORES
 
-  if (TEAMS > 1) {
-    // ---- the second team's state -> the first ----------------------------------------------------
-    char* state = sm.t[1].k[0];  // (its tiles: as many bytes as its accumulators)
-    static_assert(sizeof(sm.t[0]) == 256 * D / 2 * sizeof(float), "a team's accumulators fill its tile space");
-    const float m_own = !kLazyRef ? m_ref + m_over : m_ref == kNoRef ? -INFINITY : m_ref;
-    if (team == 1) {
-#pragma unroll
-      for (int db = 0; db < kDB; ++db)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          floatx4 t;
-#pragma unroll
-          for (int c = 0; c < 4; ++c) t[c] = acc[db][rg * 4 + c];
-          *reinterpret_cast<floatx4*>(state + (db * 4 + rg) * 4096 + tid * 16) = t;
-        }
-      sm.stats[tid] = floatx2{m_own, l_run};
-    }
-    __syncthreads();
-    if (team == 1) return;  // (barriers further down count the waves that are left)
-    const floatx2 other = sm.stats[tid];
-    const float m_new = fmaxf(m_own, other[0]), m_base = m_new == -INFINITY ? 0.f : m_new;
-    const float w_own = AA_EXP2(m_own - m_base), w_other = AA_EXP2(other[0] - m_base);
-    l_run = l_run * w_own + other[1] * w_other;
-#pragma unroll
-    for (int db = 0; db < kDB; ++db)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const floatx4 t = *reinterpret_cast<const floatx4*>(state + (db * 4 + rg) * 4096 + tid * 16);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[db][rg * 4 + c] = acc[db][rg * 4 + c] * w_own + t[c] * w_other;
-      }
-    m_ref = kLazyRef && m_new == -INFINITY ? kNoRef : m_base;
-    if (m_new != -INFINITY) m_over = 0.f;
-  }
-
   const float acc_sum = kAnyRows ? sum_of_all(acc) : 0.f;
   if (kAnyRows && __builtin_expect(__any((kLazyRef ? !is_finite(acc_sum) : is_nan(acc_sum)) && !is_nan(l_run)), 0)) {
     // V holds infinities or NaN, or is too large for probabilities above 1: the wave's sums once more (see aa_nonfinite.h)
     auto each_half = [&](auto&& visit) __attribute__((always_inline)) {
       for (int i = 0; i < 2 * n_tiles; ++i) {  // 32 keys at a time
+        if (TEAMS > 1 && (i >> 1) % TEAMS != team) continue;
         int key0 = key_base + 32 * i;
         uint32_t seen;
         if (MODE == kMasked) {
@@ -987,6 +953,43 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     each_half([&](const int key0, const uint32_t seen) __attribute__((always_inline)) {
       exact_pv_tile<T, D>(acc, qreg, kbase, vbase, k_row_bytes, v_row_bytes, key0, p.n_ctx, seen, m_base, score_scale, lane);
     });
+  }
+
+  if (TEAMS > 1) {
+    // ---- the second team's state -> the first ----------------------------------------------------
+    char* state = sm.t[1].k[0];  // (its tiles: as many bytes as its accumulators)
+    static_assert(sizeof(sm.t[0]) == 256 * D / 2 * sizeof(float), "a team's accumulators fill its tile space");
+    const float m_own = !kLazyRef ? m_ref + m_over : m_ref == kNoRef ? -INFINITY : m_ref;
+    if (team == 1) {
+#pragma unroll
+      for (int db = 0; db < kDB; ++db)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          floatx4 t;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) t[c] = acc[db][rg * 4 + c];
+          *reinterpret_cast<floatx4*>(state + (db * 4 + rg) * 4096 + tid * 16) = t;
+        }
+      sm.stats[tid] = floatx2{m_own, l_run};
+    }
+    __syncthreads();
+    if (team == 1) return;  // (barriers further down count the waves that are left)
+    const floatx2 other = sm.stats[tid];
+    const float m_new = fmaxf(m_own, other[0]), m_base = m_new == -INFINITY ? 0.f : m_new;
+    // (bf16 rows: half of both, sums and state alike, so that two finite parts have a finite sum; all chunks have this factor)
+    constexpr float kShare = kLazyRef ? 0.5f : 1.f;
+    const float w_own = AA_EXP2(m_own - m_base) * kShare, w_other = AA_EXP2(other[0] - m_base) * kShare;
+    l_run = l_run * w_own + other[1] * w_other;
+#pragma unroll
+    for (int db = 0; db < kDB; ++db)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        const floatx4 t = *reinterpret_cast<const floatx4*>(state + (db * 4 + rg) * 4096 + tid * 16);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[db][rg * 4 + c] = acc[db][rg * 4 + c] * w_own + t[c] * w_other;
+      }
+    m_ref = kLazyRef && m_new == -INFINITY ? kNoRef : m_base;
+    if (m_new != -INFINITY) m_over = 0.f;
   }
 #undef AA_EXP2
 
