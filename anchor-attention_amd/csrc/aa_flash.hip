@@ -1155,9 +1155,9 @@ flash_pair_kernel(const FlashArgs anchor, const FlashArgs rows, const uint32_t n
 #define AA_SPARSE_QBLOCKS 4  // most 128-row query blocks a stage-3 work-group handles one after the other
 #endif
 
-// Sets what the launcher decides for a launch of one mode; the number of work-groups.
+// Sets what the launcher decides for a launch of one mode, alone or with another; the number of work-groups.
 template <int MODE>
-static uint32_t place(FlashArgs& a) {
+static uint32_t place(FlashArgs& a, const bool alone) {
   a.q_blocks_per_wg = 1;
   int64_t blocks = (int64_t)a.batch * a.n_q_heads * (a.n_ctx / 128);
   if (MODE == kSparse) {
@@ -1176,8 +1176,14 @@ static uint32_t place(FlashArgs& a) {
   // More units (KV heads of all batch elements) than XCDs: side by side as long as the K and V that an XCD then works on fit its L2
   // of 4 MB.  Left-padded batches: 3 x 2500 with 32/8 heads of 128 194 -> 184 us, 28/4 184 -> 162, 3 x 1000 with 32/8 heads of 64 39.9 -> 30.0, 4 x 2900
   // 162 -> 150; the operator on 2 x 4096 tokens with those heads 181 -> 172.  Larger contexts, where the order hardly matters: within 1 %.
+  // So also fewer units than XCDs whose rows a unit's XCDs cannot share evenly (an odd number with 4 units): the hardware order ended with the heaviest
+  // work-groups of the last unit.  1578 rows, 14/2 heads of 64 28.0 -> 23.3 us; padded 2 x 1920 48.5 -> 42.8; dense 4864 tokens 90.1 -> 69.3; with 28/4
+  // heads of 128 1501 rows in one chunk 54.2 -> 41.3, dense 3712 fp16 142.5 -> 120.3.  A launch that anchor and rows work-groups share gains
+  // nothing on average (44 sizes: from 10 % faster to 10 % slower).
   const int units = a.batch * a.n_kv_heads;
-  a.abreast = MODE != kSparse && 8 % units != 0 && (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20;
+  const int rows = MODE == kRows || MODE == kMasked ? a.n_col_blocks * a.n_chunks : a.n_ctx / 128;  // (of a unit: what xcd_remap deals out)
+  a.abreast = MODE != kSparse && (8 % units != 0 ? (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20
+                                                          : alone && rows % (8 / units) != 0);
   if (MODE == kRows || MODE == kMasked) return (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks;
   return (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0);
 }
@@ -1202,7 +1208,7 @@ static void launch_for(const FlashArgs& a, const uint32_t work_groups, hipStream
 
 template <int MODE>
 static hipError_t launch(FlashArgs a, hipStream_t stream) {
-  const uint32_t work_groups = place<MODE>(a);
+  const uint32_t work_groups = place<MODE>(a, true);
   if (work_groups == 0) return hipSuccess;
   if (a.dtype == 0) launch_for<MODE, Bf16>(a, work_groups, stream);
   else launch_for<MODE, F16>(a, work_groups, stream);
@@ -1220,7 +1226,7 @@ static void launch_pair_for(const FlashArgs& a, const FlashArgs& r, const uint32
 }
 
 hipError_t launch_anchor_and_rows(FlashArgs anchor, FlashArgs rows, hipStream_t stream) {
-  const uint32_t n_anchor = place<kAnchor>(anchor), n_rows = place<kRows>(rows);
+  const uint32_t n_anchor = place<kAnchor>(anchor, false), n_rows = place<kRows>(rows, false);
   if (anchor.dtype == 0) launch_pair_for<Bf16>(anchor, rows, n_anchor, n_rows, stream);
   else launch_pair_for<F16>(anchor, rows, n_anchor, n_rows, stream);
   return hipGetLastError();

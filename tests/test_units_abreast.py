@@ -1,4 +1,4 @@
-"""More KV heads (of all batch elements) than XCDs: work-groups take them side by side.  Every row must still be computed, once, at
+"""More KV heads (of all batch elements) than XCDs, or fewer that share them unevenly: work-groups take them side by side.  Every row must still be computed, once, at
 numbers of units that do and do not divide the XCDs and their CUs, against float64 (bound as in test_dense_rows.py)."""
 import pytest
 import torch
@@ -15,6 +15,9 @@ pytestmark = pytest.mark.gpu
     (3, 8, 4, 190, 128),    # twelve units: all XCDs take all units
     (5, 4, 2, 129, 64),     # ten, and a number of work-groups that 8 does not divide
     (9, 8, 8, 257, 64),
+    (1, 28, 4, 333, 128),   # fewer than XCDs, with rows that the XCDs of a unit cannot share evenly
+    (1, 14, 2, 333, 64),
+    (2, 2, 1, 700, 64),
 ])
 def test_rows_masked_dense_and_operator(batch, hq, hkv, n, d):
     from anchor_attn.src.ops.anchor_attn_v4 import anchor_attn, dense_causal_attention, dense_rows_attention
