@@ -51,6 +51,7 @@ _SIGNATURES = {
     "aa_dense_causal_fwd": (c_int, _T3 * 4 + _DIMS5 + [c_float, c_int, c_void_p]),
     # batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset (, masked)
     "aa_dense_rows_workspace_bytes": (c_size_t, [c_int] * 8),
+    "aa_dense_rows_workspace_bytes_of": (c_size_t, [c_int] * 9),
     "aa_rms_norm": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_float, c_int, c_void_p]),
     "aa_silu_mul": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_void_p]),
     "aa_dense_rows_fwd": (c_int, _T3 * 4 + [c_void_p, c_int64, c_int64] + [c_void_p, c_size_t] + [c_int] * 7 + [c_float, c_int, c_void_p]),

@@ -354,9 +354,10 @@ def _dense_rows(tensors, Q, K, causal_offset, sm_scale, out, mask):
         mask_args = (mask.data_ptr(), mask.stride(0) if mask.shape[0] > 1 else 0, mask.stride(2))
     lib = _hip.lib()
     sizes = (B, H, kv_heads, N, n_keys, D, int(causal_offset))
-    nbytes = lib.aa_dense_rows_workspace_bytes(*sizes, mask is not None)
+    dtype = _hip.dtype_code(Q)
+    nbytes = lib.aa_dense_rows_workspace_bytes_of(*sizes, mask is not None, dtype)
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=Q.device) if nbytes else None
-    args = (*tensors, *mask_args, ws.data_ptr() if nbytes else None, nbytes, *sizes, float(sm_scale), _hip.dtype_code(Q))
+    args = (*tensors, *mask_args, ws.data_ptr() if nbytes else None, nbytes, *sizes, float(sm_scale), dtype)
     if Q.device.index == torch.cuda.current_device():
         _hip.check(lib.aa_dense_rows_fwd(*args, _stream()))
     else:  # (a pipeline's later layers lie on other GPUs than the current one)

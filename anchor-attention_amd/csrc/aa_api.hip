@@ -1,5 +1,6 @@
 // C ABI of the AnchorAttention gfx950 kernels: argument validation, scratch carving, launches.
 // Declarations and their reference counterparts: include/anchor_attn_hip.h.
+#include <algorithm>
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
@@ -567,9 +568,9 @@ int aa_dense_causal_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   return check_launch(run_flash(a, 2, (hipStream_t)stream), who);
 }
 
-// Sizes of a rows-mode problem, checked and planned; `masked`: with a boolean mask in the place of the causal rule.
+// Sizes of a rows-mode problem, checked and planned for its type; `masked`: with a boolean mask in the place of the causal rule.
 static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim,
-                           int causal_offset, bool masked) {
+                           int causal_offset, bool masked, int dtype) {
   if (batch <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_rows <= 0 || n_keys <= 0 || causal_offset < 0) {
     set_error("%s: batch, head counts, n_rows and n_keys must be positive and causal_offset not negative (got %d, %d, %d, %d, %d, %d)", who,
               batch, n_q_heads, n_kv_heads, n_rows, n_keys, causal_offset);
@@ -594,7 +595,7 @@ static int plan_dense_rows(const char* who, FlashArgs& a, int batch, int n_q_hea
     set_error("%s: problem too large for one launch", who);
     return AA_EUNSUPPORTED;
   }
-  a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_rows = n_rows; a.n_ctx = n_keys; a.head_dim = head_dim;
+  a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_rows = n_rows; a.n_ctx = n_keys; a.head_dim = head_dim; a.dtype = dtype;
   a.causal_offset = masked ? n_keys : causal_offset;
   a.mask_words_per_row = masked ? (n_keys + 63) / 64 : 0;
   a.big_block = n_keys; a.block_size = 128;  // (unused in this mode; not zero)
@@ -627,12 +628,26 @@ static RowsScratch carve_rows(const FlashArgs& a, bool decode) {
   return r;
 }
 
-size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
-                                     int masked) {
+size_t aa_dense_rows_workspace_bytes_of(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
+                                        int masked, int dtype) {
+  const char* who = "aa_dense_rows_workspace_bytes_of";
   FlashArgs a = {};
-  if (plan_dense_rows("aa_dense_rows_workspace_bytes", a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, masked != 0))
+  if (check_dtype(dtype, who) ||
+      plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, masked != 0, dtype))
     return 0;
   return carve_rows(a, decode_takes(n_rows, n_q_heads / n_kv_heads, masked != 0)).total;
+}
+
+size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
+                                     int masked) {
+  const char* who = "aa_dense_rows_workspace_bytes";
+  size_t most = 0;
+  for (const int dtype : {AA_DTYPE_BF16, AA_DTYPE_F16}) {
+    FlashArgs a = {};
+    if (plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, masked != 0, dtype)) return 0;
+    most = std::max(most, carve_rows(a, decode_takes(n_rows, n_q_heads / n_kv_heads, masked != 0)).total);
+  }
+  return most;
 }
 
 // Tensors and scratch of a planned rows-mode problem, checked and put into `a`.
@@ -677,7 +692,8 @@ int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
   FlashArgs a = {};
   int rc;
   if ((rc = check_dtype(dtype, who))) return rc;
-  if ((rc = plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, mask != nullptr))) return rc;
+  if ((rc = plan_dense_rows(who, a, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, mask != nullptr, dtype)))
+    return rc;
   const bool decode = decode_takes(n_rows, n_q_heads / n_kv_heads, mask != nullptr);
   const RowsScratch r = carve_rows(a, decode);
   if ((rc = rows_args(who, a, r, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, out, o_sb, o_sh, o_sn, workspace, workspace_bytes,
@@ -705,11 +721,12 @@ struct RowsBeside {
   size_t operator_bytes;  // the operator's scratch; the rows' follows it
 };
 static int plan_beside(const char* who, RowsBeside& r, int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim, int block_size, int step,
-                       int n_rows, int n_keys, int causal_offset) {
+                       int n_rows, int n_keys, int causal_offset, int dtype) {
   const Dims dims = {batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step};
   int rc;
   r.args = FlashArgs{};
-  if ((rc = check_dims(dims, who)) || (rc = plan_dense_rows(who, r.args, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, false)))
+  if ((rc = check_dims(dims, who)) || 
+      (rc = plan_dense_rows(who, r.args, batch, n_q_heads, n_kv_heads, n_rows, n_keys, head_dim, causal_offset, false, dtype)))
     return rc;
   const bool decode = decode_takes(n_rows, n_q_heads / n_kv_heads, false);
   r.shares = false;
@@ -728,10 +745,15 @@ static int plan_beside(const char* who, RowsBeside& r, int batch, int n_q_heads,
 
 size_t aa_anchor_attn_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim, int block_size, int step,
                                            int n_rows, int n_keys, int causal_offset) {
-  RowsBeside r;
-  if (plan_beside("aa_anchor_attn_rows_workspace_bytes", r, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, n_rows, n_keys, causal_offset))
-    return 0;
-  return r.operator_bytes + r.scratch.total;
+  const char* who = "aa_anchor_attn_rows_workspace_bytes";
+  size_t most = 0;
+  for (const int dtype : {AA_DTYPE_BF16, AA_DTYPE_F16}) {
+    RowsBeside r;
+    if (plan_beside(who, r, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, n_rows, n_keys, causal_offset, dtype)) return 0;
+    most = std::max(most, r.operator_bytes + r.scratch.total);
+    if (r.shares) break;  // (then the type does not matter)
+  }
+  return most;
 }
 
 int aa_anchor_attn_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
@@ -750,7 +772,7 @@ int aa_anchor_attn_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q
   RowsBeside r;
   int rc;
   if ((rc = check_dtype(dtype, who))) return rc;
-  if ((rc = plan_beside(who, r, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, n_rows, n_keys, causal_offset))) return rc;
+  if ((rc = plan_beside(who, r, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, n_rows, n_keys, causal_offset, dtype))) return rc;
   if ((rc = check_ptr(workspace, who, "workspace"))) return rc;
   if (workspace_bytes < r.operator_bytes + r.scratch.total) {
     set_error("%s: workspace has %zu bytes, %zu needed", who, workspace_bytes, r.operator_bytes + r.scratch.total);

@@ -50,7 +50,7 @@ hipError_t launch_anchor_and_rows(FlashArgs anchor, FlashArgs rows, hipStream_t 
 
 // rows mode with several chunks: merges the chunks of `a` (the arguments of the launch that wrote them) into a.out
 hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream);
-// rows mode: sets n_col_blocks, n_chunks and chunk_tiles from the sizes
+// rows mode: sets n_col_blocks, n_chunks and chunk_tiles from the sizes and the type
 void plan_rows(FlashArgs& a);
 // ... for a launch that anchor work-groups of `anchor` share (launch_anchor_and_rows)
 void plan_rows_beside(FlashArgs& a, const FlashArgs& anchor);

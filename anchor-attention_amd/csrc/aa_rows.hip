@@ -208,17 +208,20 @@ constexpr int kMaxChunks = 64;
 // How the keys of a rows-mode problem are cut into chunks: every number of chunks up to 64 is priced and the cheapest taken.
 //
 // Work-groups are dealt to the CUs in turn, the ones with the most tiles first, so the CU that gets the longest chain of tiles gets, 256
-// work-groups on, its second one (head dimension 64: and a third) as long as the chip has room: a tile takes 1.1 us while a
+// work-groups on, its second one (head dimension 64: and a third) as long as the chip has room: a bf16 tile takes 1.1 us while a
 // work-group is alone on its CU and 1.8 beside another (64: 0.8, 1.1 and 1.3 beside two).  A launch takes as long as that CU or
 // as all tiles at the rate of a full chip, 0.9 us a tile and CU (64: 0.45) - the fourth powers are added, which lies between the larger and the sum - and
 // a part of a chain for the uneven end of more than one round.  Several chunks cost one more launch and a write and a read
-// of the state (64 KB per column block and chunk at head dimension 128).
+// of the state (64 KB per column block and chunk at head dimension 128).  fp16 has prices of its own: its probabilities need the running max, so that
+// a tile of a work-group alone takes 1.2 us at head dimension 128.
 //
-// The prices are fitted to 192 sizes (20 to 5000 rows over up to 40000 keys, 2 to 32 KV heads in groups of 4 and 7, each with up to twelve
-// numbers of chunks): the number taken is 0.6 % slower than the best of the measured ones on average and 8.6 % at worst, 64: 0.9 and 10.6 %.  The form
-// before, which had the longest chain or the rounds of a full chip at one price, came to 2.4 and 26 %, 64: 3.5 and 23 %: it did not know that a few work-groups
-// more than CUs share them with the lightest ones (1194 rows, 28/4 heads of 128: 36.9 us in three chunks, 30.2 whole).  On 80 sizes that it was not
-// fitted to: 1.3 % on average and 11.6 % at worst, the form before 4.3 and 26 %; one of them in 40 is 6.7 % slower than before.
+// The bf16 prices were fitted to 192 sizes (20 to 5000 rows over up to 40000 keys, 2 to 32 KV heads in groups of 4 and 7, each with up to twelve
+// numbers of chunks), the fp16 ones to the 2042 of 5 to 3000 rows and 1 to 4 prompts on which both are compared here.  The number taken is slower than the
+// best of about ten measured ones by 1.0 % on average (98 of 100 within 11 %), fp16 0.7 (8) %, at 64 2.3 (27) and 1.4 (15) %, most of it where a
+// call is so short that a second launch costs the host more than it gives the GPU.  The form before, which had the longest chain or the rounds of a full chip at
+// one price, came to 2.4, 1.2, 4.3 and 2.5 %: it did not know that a few work-groups more than CUs share them with the lightest ones (1194 rows,
+// 28/4 heads of 128: 36.9 us in three chunks, 30.2 whole); 30 of the 4084 are more than 5 % slower than with it, by 14 % at most.  With the bf16 prices for
+// fp16 those were 92 (22 %): 649 rows over 2890 keys, 32/8 heads of 128, 82.2 us in one chunk, 68.6 in three.
 //
 // A column block whose rows end later sees no fewer keys, so the blocks that reach a tile are counted in closed form and a plan costs the
 // same whatever the rows: with a loop over the column blocks for every count it took the host 276 us for 32768 rows over 65536 keys
@@ -228,9 +231,11 @@ void plan_rows(FlashArgs& a) {
   const int64_t units = (int64_t)a.batch * a.n_kv_heads, total = unit_tiles(a, max_tiles);
   const bool wide = a.head_dim == 128;
   const int slots = wide ? 512 : 768;
-  const double alone = wide ? 1.07 : 0.835, beside_one = wide ? 1.81 : 1.105, beside_two = 1.306;  // us a tile
-  const double full_chip = wide ? 0.912 : 0.448, uneven_end = wide ? 0.616 : 0.098, one_round = wide ? 0.083 : 0.244;
-  const double merge = wide ? 2.65 : 1.57, merge_per_mb = wide ? 0.242 : 0.467;
+  // us a tile; us a tile of the longest chain, a full chip's round, a merge and a MB of state
+  struct Prices { double alone, beside_one, beside_two, full_chip, uneven_end, one_round, merge, merge_per_mb; };
+  static const Prices kPrices[2][2] = {{{0.835, 1.105, 1.306, 0.448, 0.098, 0.244, 1.57, 0.467}, {1.07, 1.81, 0.0, 0.912, 0.616, 0.083, 2.65, 0.242}},
+                                           {{0.87, 1.16, 1.27, 0.46, 0.10, 0.26, 2.5, 0.365}, {1.21, 1.61, 0.0, 0.88, 0.45, 0.083, 2.15, 0.23}}};
+  const Prices& price = kPrices[a.dtype != 0][wide];
   const int64_t second = units <= 256 ? 256 / units : 1;  // the number, among a unit's work-groups, of the one that joins the first on its CU
   double best = 1e30;
   a.n_chunks = 1;
@@ -249,10 +254,11 @@ void plan_rows(FlashArgs& a) {
       return max(0, min(seen - (int)(k / a.n_col_blocks) * len, len));
     };
     const int t0 = tiles_of(0), t1 = min(tiles_of(second), t0), t2 = wide ? 0 : min(tiles_of(2 * second), t1);
-    const double chain = alone * (t0 - t1) + beside_one * (t1 - t2) + beside_two * t2, all = full_chip * (double)total * units / 256;
+    const double chain = price.alone * (t0 - t1) + price.beside_one * (t1 - t2) + price.beside_two * t2;
+    const double all = price.full_chip * (double)total * units / 256;
     const double c2 = chain * chain, a2 = all * all;
-    double us = std::sqrt(std::sqrt(c2 * c2 + a2 * a2)) + (wgs > slots ? uneven_end * len : 0.0) + one_round * (double)wgs / slots;
-    if (chunks > 1) us += merge + merge_per_mb * (double)wgs * 128 * a.head_dim * 8 / 1e6;
+    double us = std::sqrt(std::sqrt(c2 * c2 + a2 * a2)) + (wgs > slots ? price.uneven_end * len : 0.0) + price.one_round * (double)wgs / slots;
+    if (chunks > 1) us += price.merge + price.merge_per_mb * (double)wgs * 128 * a.head_dim * 8 / 1e6;
     if (us < best) {
       best = us;
       a.n_chunks = chunks;

@@ -209,9 +209,12 @@ int aa_dense_causal_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
  * mask, if not NULL, takes the place of the causal rule: byte [b, i, j] of [batch, n_rows, n_keys] with element strides
  * (mask_sb, mask_sn, 1), which may be 0, says whether row i sees key j (0: no), for every head; a row that sees no key
  * gives 0.  (Padded batches and sliding windows; the reference unpads with flash_attn_varlen_func.)
- * workspace: aa_dense_rows_workspace_bytes() bytes of device scratch, which may be none (contents undefined afterwards). */
+ * workspace: aa_dense_rows_workspace_bytes() bytes of device scratch, which may be none (contents undefined afterwards);
+ * that is enough for either type, aa_dense_rows_workspace_bytes_of() what one of them needs. */
 size_t aa_dense_rows_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
                                      int masked);
+size_t aa_dense_rows_workspace_bytes_of(int batch, int n_q_heads, int n_kv_heads, int n_rows, int n_keys, int head_dim, int causal_offset,
+                                        int masked, int dtype);
 int aa_dense_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                       const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                       const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,

@@ -111,6 +111,19 @@ def test_dense_rows_refuse_more_work_groups_than_a_launch_takes():
     assert lib.aa_dense_rows_workspace_bytes(1 << 20, 1, 1, 1, 9000, 64, 0, 0) > 0  # (two chunks)
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (28, 4, 128), (14, 2, 64)])
+def test_rows_workspace_is_enough_for_either_type(hq, hkv, d):
+    """The chunks of the keys, and so their state, depend on the type; a caller that does not say which gets the larger."""
+    lib, differ = _hip.lib(), 0
+    for rows, keys in [(1, 40000), (300, 300), (649, 2890), (1089, 40001), (1400, 9000), (3000, 30000)]:
+        for masked in (0, 1):
+            args = (1, hq, hkv, rows, keys, d, keys - rows, masked)
+            of = [lib.aa_dense_rows_workspace_bytes_of(*args, t) for t in (_hip.AA_DTYPE_BF16, _hip.AA_DTYPE_F16)]
+            assert lib.aa_dense_rows_workspace_bytes(*args) == max(of)
+            differ += of[0] != of[1]
+    assert differ > 0 and lib.aa_dense_rows_workspace_bytes_of(1, hq, hkv, 8, 8, d, 0, 0, 7) == 0
+
+
 @pytest.mark.parametrize("n_rows,n_keys,masked", [(32768, 65536, 0), (131072, 131072, 1)])
 def test_planning_dense_rows_costs_the_host_the_same_for_large_calls(n_rows, n_keys, masked):
     """Done twice a call: 276 us and 1.1 ms when every count of chunks was tried on every column block, 4 us in closed form."""
