@@ -26,7 +26,7 @@
 // three where few keys weigh much).  Whether a lane's max grew is a comparison of S - m with zero, before the two lanes of
 // a row have exchanged anything; only when one did (rare after the first tiles) does the wave take a slow path that completes
 // the max, shifts the tile, re-bases the tuple and rescales the accumulators - exact for the lanes whose
-// max did not move (shift 0, factor 1).  (The exchange on every half-tile instead: 16384 tokens dense, 32/8 heads of 128, 1830 us
+// max did not move (shift 0, factor 1).  Where one key outweighs the rest by far, not even the lane's own max is formed (kBySum).  (The exchange on every half-tile instead: 16384 tokens dense, 32/8 heads of 128, 1830 us
 // against 1796.)
 //
 // bf16 rows and masked modes, which keep a probability as two numbers, need no max at all (kLazyRef): m is the row max of the
@@ -551,18 +551,18 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // causal / list-end mask of one 32-key half (only tiles on the diagonal or at the end of a list need it)
 #define AA_MASK(sx, kb)                                                              \
   if (MODE == kMasked) {                                                             \
-    if (mixed) {                                                                     \
+    if (__builtin_expect(mixed, 0)) {                                                \
       uint32_t seen_ = mask_word[kb];                                                \
       asm volatile("" : "+v"(seen_)); /* (the bits are taken apart here, not earlier) */ \
       _Pragma("unroll") for (int r = 0; r < 16; ++r)                                 \
         if (!((seen_ >> (8 * (r >> 2) + (r & 3))) & 1u)) sx[r] = -INFINITY;          \
     }                                                                                \
-  } else if (MODE != kSparse) {                                                             \
-    if (key0 + 32 * (kb) + 31 > wave_last_key) {                                     \
+  } else if (MODE != kSparse) {                                                      \
+    if (__builtin_expect(key0 + 32 * (kb) + 31 > wave_last_key, 0)) {                \
       _Pragma("unroll") for (int r = 0; r < 16; ++r)                                 \
         if (AA_KEY_OF(kb, r) > my_last_key) sx[r] = -INFINITY;                       \
     }                                                                                \
-  } else if (key0 + 32 * (kb) + 32 > cnt) {                                          \
+  } else if (__builtin_expect(key0 + 32 * (kb) + 32 > cnt, 0)) {                     \
     _Pragma("unroll") for (int r = 0; r < 16; ++r)                                   \
       if (AA_KEY_OF(kb, r) >= cnt) sx[r] = -INFINITY;                                \
   }
@@ -631,13 +631,24 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     for (int r = 0; r < 16; ++r) negm[r] = -m_ref;
   }
 
-  // One tile.  The LDS buffer it reads (BUF) is a compile-time constant - the loop below is unrolled by two - so that
+  // Where the reference follows the running max, a key above it has a probability of 1 or more, so a lane whose 16 probabilities of a
+  // half-tile sum to less has none: once a wave's sums have been low (an attention sink: the rest of the keys weigh little), tiles
+  // without masked pairs are run without forming maxima (kFew) until a sum says otherwise.  (Compared as bits: a NaN counts as large.)
+  // These tiles have loops of their own: a choice inside a tile costs the branches and register copies that it saves maxima.  131072 tokens,
+  // 32/8 heads of 128, few keys selected 7.71 -> 7.44 ms; 16384 dense 1875 -> 1810 us; 16384 fp16, heads of 64, 472 -> 451; scores without a
+  // sink, 32768 tokens with nearly every key selected: 9.11 -> 9.08 ms.
+  constexpr bool kBySum = !kAnyRows && AA_ABLATE != 1 && AA_ABLATE != 2;
+  const uint32_t kSumLimit = __float_as_uint(0.999f), kSumLow = __float_as_uint(0.5f);
+  bool few = false;
+
+  // One tile.  The LDS buffer it reads (BUF) is a compile-time constant - the loops below are unrolled by two - so that
   // the buffer's offset is part of every LDS instruction's immediate offset and the read addresses are loop-invariant.
-  // Sparse mode, whose tile counts can be odd, keeps one copy of the tile (BUF = -1): the buffer is i & 1 and the read
+  // Sparse mode, whose tile counts can be odd, keeps one copy of each kind of tile (BUF = -1): the buffer is i & 1 and the read
   // addresses step back and forth between the two buffers.  So does masked mode, for which two copies spill 25 registers.
   int32_t buf_step = (MODE == kSparse && cur) ? -kTileBytes : kTileBytes;
-  auto run_tile = [&](auto buf_const, const int i) __attribute__((always_inline)) {
+  auto tile = [&](auto buf_const, auto few_const, const int i) __attribute__((always_inline)) {
     constexpr int kBuf = decltype(buf_const)::value;
+    constexpr bool kFew = decltype(few_const)::value;
     constexpr uint32_t rd_off = kBuf > 0 ? kBuf * kTileBytes : 0;  // immediate part of the LDS read addresses
     const int buf = kBuf >= 0 ? kBuf : cur;
     const int key0 = AA_TILE_KEY0(i);  // (masked: entry_next is still this tile's)
@@ -663,7 +674,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       entry_after = sm.idx[min(i + 2 * TEAMS, n_tiles - 1)];
     }
     const int key0_next = AA_TILE_KEY0(i_next);
-    const bool fetch_queries = MODE == kAnchor && pool && i + 1 == n_tiles;  // wave-uniform
+    const bool fetch_queries = MODE == kAnchor && !kFew && pool && i + 1 == n_tiles;  // wave-uniform (a window's last tile has masked pairs)
     // (selects, not branches: the eight slots stay straight-line code; the base address is scalar, and the vector offset
     // is chosen once per tile and operand kind)
     const uint32_t k_voff_sel = fetch_queries ? q_voff : k_voff, v_voff_sel = fetch_queries ? q_voff : v_voff;
@@ -718,6 +729,37 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         for (int c = 0; c < 4; ++c) { AA_EXP_CHUNK(sx, pw, sum, c) }
       };
       (void)rebase;
+      // (kFew) A half whose probabilities do not sum to less than 1 once more, the row's max looked at, as a tile without kFew does: the same bits.
+      auto look_again = [&](auto kb_const, floatx16& sx, u32x4 (&pw)[2], u32x4 (&pw_rest)[2], float& sum) __attribute__((always_inline)) {
+        constexpr int kb = decltype(kb_const)::value;
+        float mx;
+        AA_SCORES(sx, kb, rd_off, negm)
+        AA_LANEMAX(sx, mx)
+        if (__any(mx > m_over)) {
+          const float m_new = fmaxf(m_ref + m_over, m_ref + max_with_other_half(mx));
+          const float m_base = m_new == -INFINITY ? 0.f : m_new;
+          const float alpha = AA_EXP2(m_ref + m_over - m_base), shift = m_base - m_ref;
+          m_ref = m_base;
+          l_run *= alpha;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sx[r] -= shift;
+          if (kb == 0) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s1[r] -= shift;
+          }
+#pragma unroll
+          for (int r = 0; r < 16; ++r) negm[r] = -m_base;
+#pragma unroll
+          for (int db = 0; db < kDB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+        }
+        sum = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { AA_EXP_CHUNK(sx, pw, sum, c) }
+        few = false;
+      };
+      (void)look_again;
 #define AA_K_FETCH(t) ka[t] = *(const lds_vec8*)(uintptr_t)(k_rd[(t) % kKS] + (uint32_t)(rd_off + 32 * ((t) / kKS) * kRowBytes))
 
       // The MFMAs of a tile are slots 0 .. kNS + kNV - 1 (head dimension 128: 16 for S^T, then 16 for O^T); the operand of
@@ -758,11 +800,11 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         AA_S_MFMA(s1, n);
         AA_FENCE;
       }
-      if (AA_ABLATE != 2) { AA_MASK(s0, 0) }
-      if (!kLazyRef && AA_ABLATE != 2) {
+      if (AA_ABLATE != 2 && !kFew) { AA_MASK(s0, 0) }
+      if (!kLazyRef && AA_ABLATE != 2 && !kFew) {
         AA_LANEMAX(s0, mx0)
         moved0 = __any(mx0 > m_over);
-        if (moved0) {
+        if (__builtin_expect(moved0, 0)) {
           // some row's max grew.  Lanes whose max did not move get shift 0 and alpha 1 (exact).
           // S1 is being accumulated on top of the old -m_ref and is shifted once it is complete.
           // (a chunk may hold no key of a row's so far - its max stays -inf and its reference 0)
@@ -802,6 +844,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         rebase(std::integral_constant<int, 0>{}, s0, pw0, pw0_rest, sum0);
         AA_SCORES(s1, 1, rd_off, negm)
       }
+      if (kFew && __builtin_expect(__any(__float_as_uint(sum0) >= kSumLimit), 0)) look_again(std::integral_constant<int, 0>{}, s0, pw0, pw0_rest, sum0);
       l_run += sum0;
 
       // ---- phase C: O^T += V0^T P0^T, with the soft-max of S1 between the MFMAs --------------------
@@ -811,15 +854,15 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         AA_PV_MFMA(n - kNS, pw0)
         AA_FENCE;
       }
-      if (!kLazyRef && moved0) {
+      if (!kLazyRef && !kFew && __builtin_expect(moved0, 0)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) s1[r] -= shift0;
       }
-      if (AA_ABLATE != 2) { AA_MASK(s1, 1) }
-      if (!kLazyRef && AA_ABLATE != 2) {
+      if (AA_ABLATE != 2 && !kFew) { AA_MASK(s1, 1) }
+      if (!kLazyRef && AA_ABLATE != 2 && !kFew) {
         AA_LANEMAX(s1, mx1)
         moved1 = __any(mx1 > m_over);
-        if (moved1) {
+        if (__builtin_expect(moved1, 0)) {
           // as above, except that O^T is rescaled only after the P0 V0 products in flight have been added
           const float m_new = fmaxf(m_ref + m_over, m_ref + max_with_other_half(mx1));
           const float m_base = m_new == -INFINITY ? 0.f : m_new;
@@ -849,13 +892,18 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         AA_PV_MFMA(n - kNS, pw0)
         AA_FENCE;
       }
-      if (!kLazyRef && moved1) {
+      if (!kLazyRef && !kFew && __builtin_expect(moved1, 0)) {
 #pragma unroll
         for (int db = 0; db < kDB; ++db)
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[db][r] *= alpha1;
       }
       if (kChecksSums && __builtin_expect(__any(sum1 > kRebaseSum), 0)) rebase(std::integral_constant<int, 1>{}, s1, pw1, pw1_rest, sum1);
+      if (kFew) {
+        if (__builtin_expect(__any(__float_as_uint(sum1) >= kSumLimit), 0)) look_again(std::integral_constant<int, 1>{}, s1, pw1, pw1_rest, sum1);
+      } else if (kBySum) {
+        few = !__any(max(max(__float_as_uint(sum0), __float_as_uint(sum1)), __float_as_uint(m_over)) >= kSumLow);
+      }
       l_run += sum1;
 
       // ---- phase D: O^T += V1^T P1^T ---------------------------------------------------------------
@@ -887,14 +935,42 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     if (MODE == kMasked) asm volatile("" : "+v"(mask_word_next[0]), "+v"(mask_word_next[1]));
     if (AA_ABLATE != 8 && AA_ABLATE != 9) __syncthreads();
   };
-  if (MODE == kSparse || MODE == kMasked) {
-    for (int i = team; i < n_tiles; i += TEAMS) run_tile(std::integral_constant<int, -1>{}, i);
-  } else {
-    // (anchor, dense: 128 query rows and 64-key tiles, so the window of a query block holds an even number of tiles)
-    for (int i = team; i < n_tiles; i += 2 * TEAMS) {
-      run_tile(std::integral_constant<int, 0>{}, i);
-      if ((kAnyRows || TEAMS > 1) && i + TEAMS >= n_tiles) break;
-      run_tile(std::integral_constant<int, 1>{}, i + TEAMS);
+  // (a tile without masked pairs, by its number)
+  auto whole = [&](const int i) __attribute__((always_inline)) {
+    const int key0 = AA_TILE_KEY0(i);
+    return MODE == kSparse ? key0 + kBN <= cnt : key0 + kBN - 1 <= wave_last_key;
+  };
+  typedef std::integral_constant<int, 0> Buf0;
+  typedef std::integral_constant<int, 1> Buf1;
+  typedef std::integral_constant<int, -1> BufCur;
+  int i = team;
+  while (i < n_tiles) {
+    if (MODE == kSparse || MODE == kMasked) {
+      do {
+        tile(BufCur{}, std::false_type{}, i);
+        i += TEAMS;
+      } while (i < n_tiles && !(kBySum && few && whole(i)));
+      if constexpr (kBySum) {
+        while (i < n_tiles && few && whole(i)) {
+          tile(BufCur{}, std::true_type{}, i);
+          i += TEAMS;
+        }
+      }
+    } else {
+      // (anchor, dense: 128 query rows and 64-key tiles, so the window of a query block holds an even number of tiles)
+      do {
+        tile(Buf0{}, std::false_type{}, i);
+        if ((kAnyRows || TEAMS > 1) && i + TEAMS >= n_tiles) { i += TEAMS; break; }
+        tile(Buf1{}, std::false_type{}, i + TEAMS);
+        i += 2 * TEAMS;
+      } while (i < n_tiles && !(kBySum && few && i + TEAMS < n_tiles && whole(i + TEAMS)));
+      if constexpr (kBySum) {
+        while (i + TEAMS < n_tiles && few && whole(i + TEAMS)) {
+          tile(Buf0{}, std::true_type{}, i);
+          tile(Buf1{}, std::true_type{}, i + TEAMS);
+          i += 2 * TEAMS;
+        }
+      }
     }
   }
   if (TEAMS > 1 && team == 1 && n_tiles % TEAMS != 0) __syncthreads();  // (the barrier of the first team's last tile)
