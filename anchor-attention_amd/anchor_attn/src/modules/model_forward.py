@@ -9,11 +9,13 @@ Here both are thin wrappers around whatever forward the installed transformers h
 release: the causal-LM wrapper asks the model's own ``logits_to_keep`` mechanism for one position, the MLP wrapper
 calls the module's own forward on slices.
 
-``fuse_between_products`` runs the norms and the MLPs' activation and product, single operations of the framework with a pass over
-memory each, as one kernel where nothing watches the single operations.  The 16-bit roundings are theirs, but the sum of squares has
-another order, so a norm may differ in the last 16-bit unit (of 6001 x 2048 random elements, 4 in a million in bf16, 27 in fp16; the
-activation and product in none), and what a model computes from it by as much as its own roundings make out.
+``fuse_between_products`` runs the norms, the MLPs' activation and product and the rotary embedding of queries and keys, single operations of
+the framework with a pass over memory each, as one kernel where nothing watches the single operations.  The 16-bit roundings are
+theirs, but the sum of squares has another order, so a norm may differ in the last 16-bit unit (of 6001 x 2048 random elements, 4 in a
+million in bf16, 27 in fp16; the activation and product and the embedding in none), and what a model computes from it by as much as
+its own roundings make out.
 """
+import copy
 import functools
 import types
 
@@ -146,6 +148,102 @@ def _gated_mlp_forward(own, own_act):
     return forward
 
 
+_ROPE = "apply_rotary_pos_emb"
+
+
+def _rope_tensors(q, k, cos, sin):
+    """What the kernel is given of these tensors, with new ones for its results (the keys' contiguous, as a cache lays them out); None where
+    it does not take them."""
+    tensors = (q, k, cos, sin)
+    if not (all(type(t) is torch.Tensor for t in tensors) and _called_plainly()):
+        return None
+    if not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda"):
+        return None
+    if not (q.dim() == k.dim() == 4 and cos.dim() == sin.dim() == 3 and cos.shape == sin.shape):
+        return None
+    (B, H, N, D), kv_heads = q.shape, k.shape[1]
+    if not (k.shape == (B, kv_heads, N, D) and cos.shape in ((B, N, D), (1, N, D)) and D % 16 == 0 and D <= 256 and 0 < q.numel() < 1 << 35 and 0 < k.numel() < 1 << 35):
+        return None
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return None
+    if any(t.dtype != q.dtype or t.device != q.device or t.data_ptr() & 15 for t in tensors) or not (cos.is_contiguous() and sin.is_contiguous()):
+        return None
+    outs = torch.empty_like(q), torch.empty(k.shape, dtype=k.dtype, device=k.device)
+    for t in (q, k, *outs):
+        sb, sh, sn, sd = t.stride()
+        if sd != 1 or (sb | sh | sn) & 7 or not D <= sn <= 1 << 14 or N > 1 << 20 or N * sn * 2 >= 1 << 32:
+            return None
+    return outs, (*_hip.t3(q), *_hip.t3(k), *_hip.t3(outs[0]), *_hip.t3(outs[1]), cos.data_ptr(), sin.data_ptr(), N * D if cos.shape[0] > 1 else 0,
+                  B, H, kv_heads, N, D, _hip.dtype_code(q))
+
+
+class _Names(dict):
+    """The global names of a function, as they are at any time, but for one."""
+
+    def __init__(self, names, rope):
+        super().__init__({_ROPE: rope, "__builtins__": names["__builtins__"]})
+        self.names = names
+
+    def __missing__(self, name):
+        return self.names[name]
+
+
+class _Bound:
+    """A forward bound to its module, which copies and pickles as a bound method does: the copy's, and by its name."""
+
+    def __init__(self, module, forward):
+        self.module, self.forward = module, forward
+        functools.update_wrapper(self, types.MethodType(type(module).forward, module))
+
+    def __call__(self, *args, **kwargs):
+        return self.forward(self.module, *args, **kwargs)
+
+    def __deepcopy__(self, memo):
+        return _Bound(copy.deepcopy(self.module, memo), self.forward)
+
+    def __reduce__(self):
+        return getattr, (self.module, "forward")
+
+
+def _attention_forward(own):
+    """An attention's forward in the place of its class's, ``own``: the same code, in which one name, the rotary embedding of its
+    queries and keys, means the kernel where that takes the tensors.  (Of a forward or an embedding that a program puts in their
+    places later, that is used.)"""
+    single_operations = own.__globals__[_ROPE]
+
+    def rope(*args, **kwargs):
+        taken = _rope_tensors(*args) if len(args) == 4 and not kwargs else None
+        if taken is None:
+            return single_operations(*args, **kwargs)
+        outs, numbers = taken
+        _launch(_hip.lib().aa_rope, outs[0].device, *numbers)
+        return outs
+
+    fused = types.FunctionType(own.__code__, _Names(own.__globals__, rope), own.__name__, own.__defaults__, own.__closure__)
+    fused.__kwdefaults__ = own.__kwdefaults__
+
+    def forward(self, *args, **kwargs):
+        if not _called_plainly() or type(self).forward is not own or own.__globals__.get(_ROPE) is not single_operations:
+            return type(self).forward(self, *args, **kwargs)
+        return fused(self, *args, **kwargs)
+
+    return forward
+
+
+def _rotates(own) -> bool:
+    """Whether an attention's forward is a plain function that embeds by that name, bit for bit as the kernel does on a few numbers."""
+    if type(own) is not types.FunctionType or _ROPE not in own.__code__.co_names or type(own.__globals__.get(_ROPE)) is not types.FunctionType:
+        return False
+    x = torch.linspace(-3.0, 3.0, 2 * 3 * 2 * 16, dtype=torch.float32, device="cpu").reshape(2, 3, 2, 16).bfloat16()
+    cos, sin = (x[:, 0] * 0.3).cos(), (x[:, 1] * 0.7).sin()  # (halves that differ)
+    want = [t * cos[:, None] + torch.cat((-t[..., 8:], t[..., :8]), -1) * sin[:, None] for t in (x, x[:, :1] + 1)]
+    try:
+        got = own.__globals__[_ROPE](x, x[:, :1] + 1, cos, sin)
+        return len(got) == 2 and all(torch.equal(a, b) for a, b in zip(got, want))
+    except Exception:  # noqa: BLE001 - one that works otherwise
+        return False
+
+
 def _computes(cls, stub, x, want) -> bool:
     """Whether the class's own forward does what the kernel would take over, bit for bit on a few numbers."""
     try:
@@ -155,7 +253,7 @@ def _computes(cls, stub, x, want) -> bool:
 
 
 def fuse_between_products(model) -> int:
-    """RMS norms and gated MLPs of the model's family whose classes compute what the kernels do, and whose instances have no
+    """RMS norms, gated MLPs and attentions of the model's family whose classes compute what the kernels do, and whose instances have no
     ``forward`` of their own, get one that uses the kernels.  Returns how many; calling it again changes nothing."""
     x = torch.linspace(-3.0, 3.0, 32, dtype=torch.float32, device="cpu").reshape(2, 16).bfloat16()
     norm = types.SimpleNamespace(weight=x[0] + 1.0, variance_epsilon=1e-3)
@@ -175,6 +273,9 @@ def fuse_between_products(model) -> int:
             elif (name in ("LlamaMLP", "Qwen2MLP") and _is_silu(act) and _computes(type(act), act, x, silu)
                   and _computes(type(m), mlp, x, gated)):
                 fused = _gated_mlp_forward(type(m).forward, type(act).forward)
+            elif name in ("LlamaAttention", "Qwen2Attention") and _rotates(type(m).forward):
+                m.forward = _Bound(m, _attention_forward(type(m).forward))
+                n += 1
             if fused is not None:
                 m.forward = types.MethodType(fused, m)
                 n += 1

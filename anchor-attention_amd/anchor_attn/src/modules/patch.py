@@ -9,8 +9,8 @@ patch.py:36-45,142-144); the competitor patterns of the reference are not part o
 name through ``AttentionInterface``, so patching is: register the plug once, point the model's config at it,
 and copy the pattern's parameters onto the config (patch.py:106-109 does the same ``setattr`` loop).  Like the
 reference (patch.py:146-157), every pattern but "default" also makes the model return logits for the last position
-only and evaluates the MLPs in chunks of 32768 positions; the norms and the MLPs' activations run as one kernel each
-(``model_forward.py``).
+only and evaluates the MLPs in chunks of 32768 positions; the norms, the MLPs' activations and the rotary embeddings run as one kernel
+each (``model_forward.py``).
 """
 import copy
 import json
@@ -75,8 +75,8 @@ def patch_model(model, pattern: str, config=None):
              (the defaults; keys left out keep them).  Two optional keys with no counterpart in the reference steer
              the model-level patches the reference applies unconditionally: ``"last_token_logits"`` (default True) and
              ``"mlp_chunk_tokens"`` (default 32768; 0 leaves the MLPs alone).  A third, ``"fuse_between_products"`` (default
-             True), steers one that the reference does not have: in eager 16-bit inference norms and gated activations are
-             single kernels, whose results may differ from the single operations' in the last 16-bit unit; False leaves
+             True), steers one that the reference does not have: in eager 16-bit inference norms, gated activations and rotary
+             embeddings are single kernels, whose results may differ from the single operations' in the last 16-bit unit; False leaves
              them alone (a model patched before keeps what it has).
     """
     from transformers import PreTrainedModel

@@ -53,6 +53,7 @@ _SIGNATURES = {
     "aa_dense_rows_workspace_bytes": (c_size_t, [c_int] * 8),
     "aa_dense_rows_workspace_bytes_of": (c_size_t, [c_int] * 9),
     "aa_rms_norm": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_float, c_int, c_void_p]),
+    "aa_rope": (c_int, _T3 * 4 + [c_void_p, c_void_p, c_int64] + _DIMS5 + [c_int, c_void_p]),
     "aa_silu_mul": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_void_p]),
     "aa_dense_rows_fwd": (c_int, _T3 * 4 + [c_void_p, c_int64, c_int64] + [c_void_p, c_size_t] + [c_int] * 7 + [c_float, c_int, c_void_p]),
     # the operator's sizes, then n_rows, n_keys, causal_offset

@@ -817,4 +817,33 @@ int aa_silu_mul(const void* gate, const void* up, void* out, int64_t n, int dtyp
   return check_launch(launch_silu_mul((const uint16_t*)gate, (const uint16_t*)up, (uint16_t*)out, n, dtype, (hipStream_t)stream), who);
 }
 
+int aa_rope(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn, const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+            void* q_out, int64_t qo_sb, int64_t qo_sh, int64_t qo_sn, void* k_out, int64_t ko_sb, int64_t ko_sh, int64_t ko_sn,
+            const void* cos, const void* sin, int64_t cs_sb, int batch, int n_q_heads, int n_kv_heads, int n_tokens, int head_dim,
+            int dtype, void* stream) {
+  const char* who = "aa_rope";
+  int rc;
+  if (batch <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_tokens <= 0) {
+    set_error("%s: batch, head counts and n_tokens must be positive (got %d, %d, %d, %d)", who, batch, n_q_heads, n_kv_heads, n_tokens);
+    return AA_EBADARG;
+  }
+  if (head_dim <= 0 || head_dim > 1024 || head_dim % 16 != 0 ||
+      ((int64_t)n_q_heads + n_kv_heads + 3) / 4 * (head_dim / 16) >= 0xffffff00LL / batch / n_tokens) {
+    set_error("%s: %d x %d tokens of %d + %d heads of %d are not supported (a multiple of 16 up to 1024, fewer than 2^32 pieces of 64 elements)", who,
+              batch, n_tokens, n_q_heads, n_kv_heads, head_dim);
+    return AA_EUNSUPPORTED;
+  }
+  if ((rc = check_dtype(dtype, who)) || (rc = check_tensor(q, q_sb, q_sh, q_sn, n_tokens, head_dim, who, "q")) ||
+      (rc = check_tensor(k, k_sb, k_sh, k_sn, n_tokens, head_dim, who, "k")) || (rc = check_tensor(q_out, qo_sb, qo_sh, qo_sn, n_tokens, head_dim, who, "q_out")) ||
+      (rc = check_tensor(k_out, ko_sb, ko_sh, ko_sn, n_tokens, head_dim, who, "k_out")) || (rc = check_ptr(cos, who, "cos")) || (rc = check_ptr(sin, who, "sin")))
+    return rc;
+  if (cs_sb % 8 != 0) {
+    set_error("%s: cos and sin must have a batch stride that is a multiple of 8 elements (got %lld)", who, (long long)cs_sb);
+    return AA_EMISALIGNED;
+  }
+  RopeArgs a = {(const uint16_t*)q, q_sb, q_sh, q_sn, (const uint16_t*)k, k_sb, k_sh, k_sn, (uint16_t*)q_out, qo_sb, qo_sh, qo_sn,
+                (uint16_t*)k_out, ko_sb, ko_sh, ko_sn, (const uint16_t*)cos, (const uint16_t*)sin, cs_sb, batch, n_q_heads, n_kv_heads, n_tokens, head_dim};
+  return check_launch(launch_rope(a, dtype, (hipStream_t)stream), who);
+}
+
 }  // extern "C"

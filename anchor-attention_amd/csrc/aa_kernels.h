@@ -70,6 +70,17 @@ hipError_t launch_rms_norm(const uint16_t* x, const uint16_t* weight, uint16_t* 
 // n elements, a multiple of 8
 hipError_t launch_silu_mul(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t n, int dtype, hipStream_t stream);
 
+// queries [batch, n_q_heads, n_tokens, head_dim] and keys with n_kv_heads, rotated into q_out and k_out; cos, sin [batch or 1 (cs_sb 0), n_tokens, head_dim]
+struct RopeArgs {
+  const uint16_t* q; int64_t q_sb, q_sh, q_sn;
+  const uint16_t* k; int64_t k_sb, k_sh, k_sn;
+  uint16_t* q_out; int64_t qo_sb, qo_sh, qo_sn;
+  uint16_t* k_out; int64_t ko_sb, ko_sh, ko_sn;
+  const uint16_t* cos; const uint16_t* sin; int64_t cs_sb;
+  int batch, n_q_heads, n_kv_heads, n_tokens, head_dim;  // a multiple of 16; fewer than 2^32 threads
+};
+hipError_t launch_rope(const RopeArgs& a, int dtype, hipStream_t stream);
+
 struct PoolArgs {
   const uint16_t* q; int64_t q_sb, q_sh, q_sn;
   const float* M;

@@ -246,9 +246,15 @@ int aa_anchor_attn_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q
  * What the models that the attention plug is used in compute around it, one pass each, with the 16-bit roundings of the framework's
  * single operations (all tensors 16-byte aligned and contiguous):
  * aa_rms_norm: out[r, :] = weight * round16(x[r, :] * rsqrt(mean(x[r, :]^2) + eps)), float32 inside;
- * aa_silu_mul: out = round16(silu(gate)) * up over n elements. */
+ * aa_silu_mul: out = round16(silu(gate)) * up over n elements;
+ * aa_rope: x * cos + rotate(x) * sin of queries and keys (element strides as everywhere, rows of head_dim consecutive elements), rotate: (first, second
+ * half) -> (-second, first); cos, sin [batch, n_tokens, head_dim] with cs_sb elements from one batch element to the next (0: the same for all). */
 int aa_rms_norm(const void* x, const void* weight, void* out, int64_t rows, int hidden, float eps, int dtype, void* stream);
 int aa_silu_mul(const void* gate, const void* up, void* out, int64_t n, int dtype, void* stream);
+int aa_rope(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn, const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
+            void* q_out, int64_t qo_sb, int64_t qo_sh, int64_t qo_sn, void* k_out, int64_t ko_sb, int64_t ko_sh, int64_t ko_sn,
+            const void* cos, const void* sin, int64_t cs_sb, int batch, int n_q_heads, int n_kv_heads, int n_tokens, int head_dim,
+            int dtype, void* stream);
 
 #ifdef __cplusplus
 }
