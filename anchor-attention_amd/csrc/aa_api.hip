@@ -240,12 +240,18 @@ size_t aa_workspace_bytes(int batch, int n_q_heads, int n_ctx, int head_dim, int
   return carve(batch, n_q_heads, n_ctx, head_dim, block_size, step).total;
 }
 
+// The share of selected keys, their number times `inverse`, where it is wanted; `selected`: a word that is 0, where stage 2 is to form it.
+struct Ratio {
+  float* ratio; float* host; float inverse; uint64_t* selected;
+};
+
 // What stage 1 does for the stages after it in the whole operator.
 struct Stage1Extras {
   void* qbar; void* abar;  // pooled queries and anchors (block_size <= 128)
   float* thr; float scale2, theta_log2;  // and the thresholds of the pooled rows
   // the output of big block 0, whose rows select no keys, in the place of their state and pooled rows
   void* out; int64_t o_sb, o_sh, o_sn;
+  uint64_t* clear;  // Ratio::selected
   int32_t* zero_counts; float* zero_ratio; float* zero_ratio_host;  // a single big block: what the later stages would say
   const FlashArgs* rows;  // a rows-mode problem that shares the launch
 };
@@ -274,7 +280,7 @@ static int stage1_impl(const char* who, const void* q, int64_t q_sb, int64_t q_s
   a.out = (uint16_t*)x.out; a.o_sb = x.o_sb; a.o_sh = x.o_sh; a.o_sn = x.o_sn;
   a.qbar_out = (uint16_t*)x.qbar; a.abar_out = (uint16_t*)x.abar;
   a.thr_out = reinterpret_cast<uint32_t*>(x.thr); a.scale2 = x.scale2; a.theta_log2 = x.theta_log2;
-  a.zero_counts = x.zero_counts; a.ratio = x.zero_ratio; a.ratio_host = x.zero_ratio_host;
+  a.clear = x.clear; a.zero_counts = x.zero_counts; a.ratio = x.zero_ratio; a.ratio_host = x.zero_ratio_host;
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size;
   a.sm_scale = sm_scale; a.scale_mode = scale_mode; a.dtype = dtype;
@@ -311,7 +317,7 @@ int aa_pool_q_anchor(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn, co
 static float select_scale2(double sm_scale) { return (float)(sm_scale * 1.44269504); }  // double product, then float32, as the definition does
 
 // Stage 2; have_thresholds: stage 1 has formed them.
-static int stage2_impl(const char* who, bool have_thresholds, const void* qbar, const void* abar,
+static int stage2_impl(const char* who, bool have_thresholds, const Ratio& r, const void* qbar, const void* abar,
                      const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                      uint32_t* mask_ws, int32_t* coords, int32_t* counts,
                      int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
@@ -335,6 +341,7 @@ static int stage2_impl(const char* who, bool have_thresholds, const void* qbar, 
   a.scale2 = select_scale2(sm_scale);
   a.theta_log2 = theta_log2;
   a.dtype = dtype;
+  if (r.selected != nullptr) { a.selected = r.selected; a.ratio = r.ratio; a.ratio_host = r.host; a.ratio_inverse = r.inverse; }
   a.key_lo = geometry == AA_GEOMETRY_AS_RUN ? block_size : block_size * step;
   a.key_slack = geometry == AA_GEOMETRY_AS_RUN ? block_size : 0;
   if (n_ctx > block_size * step) {  // (a single big block has no candidates: its counts are 0)
@@ -349,7 +356,7 @@ int aa_stage2_select(const void* qbar, const void* abar,
                      uint32_t* mask_ws, int32_t* coords, int32_t* counts,
                      int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                      int block_size, int step, double sm_scale, float theta_log2, int geometry, int dtype, void* stream) {
-  return stage2_impl("aa_stage2_select", false, qbar, abar, k, k_sb, k_sh, k_sn, mask_ws, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
+  return stage2_impl("aa_stage2_select", false, Ratio{}, qbar, abar, k, k_sb, k_sh, k_sn, mask_ws, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
                      head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream);
 }
 
@@ -374,8 +381,8 @@ int aa_stage2_select_static(const void* qbar, const void* abar,
                           n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream);
 }
 
-// Stage 3 for the rows from big block `first_big_block` (0 or 1) on; with `ratio`, also the sum of all counts over `denominator`.
-static int stage3_impl(const char* who, int first_big_block, float* ratio, float* ratio_host, double denominator,
+// Stage 3 for the rows from big block `first_big_block` (0 or 1) on; also the ratio where stage 2 has not formed it.
+static int stage3_impl(const char* who, int first_big_block, const Ratio& r,
                        const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn,
                          const void* k, int64_t k_sb, int64_t k_sh, int64_t k_sn,
                          const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sn,
@@ -405,7 +412,8 @@ static int stage3_impl(const char* who, int first_big_block, float* ratio, float
   a.batch = batch; a.n_q_heads = n_q_heads; a.n_kv_heads = n_kv_heads; a.n_ctx = n_ctx; a.head_dim = head_dim;
   a.big_block = block_size * step; a.block_size = block_size; a.first_big_block = first_big_block;
   a.sm_scale = sm_scale; a.scale_mode = AA_SCALE_FP32; a.dtype = dtype;
-  a.ratio = ratio; a.ratio_host = ratio_host; a.n_ratio_counts = (int64_t)batch * n_q_heads * (n_ctx / a.big_block); a.ratio_inverse = 1.f / (float)denominator;
+  if (r.selected == nullptr) { a.ratio = r.ratio; a.ratio_host = r.host; a.ratio_inverse = r.inverse; }
+  a.n_ratio_counts = (int64_t)batch * n_q_heads * (n_ctx / a.big_block);
   return check_launch(run_flash(a, 1, (hipStream_t)stream), who);
 }
 
@@ -417,7 +425,7 @@ int aa_stage3_sparse_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_sn
                          void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn,
                          int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim,
                          int block_size, int step, float sm_scale, int dtype, void* stream) {
-  return stage3_impl("aa_stage3_sparse_fwd", 0, nullptr, nullptr, 1.0, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc_frag,
+  return stage3_impl("aa_stage3_sparse_fwd", 0, Ratio{}, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc_frag,
                      out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, sm_scale, dtype, stream);
 }
 
@@ -466,6 +474,10 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
   }
   x.out = out; x.o_sb = o_sb; x.o_sh = o_sh; x.o_sn = o_sn;
   x.rows = rows;
+  // (the word for the sum lies where the lists will)
+  const bool sums = selects && ratio != nullptr && select_scores_sums(batch, n_kv_heads, n_ctx);
+  const Ratio r = {ratio, ratio_host, 1.f / (float)denominator, sums ? reinterpret_cast<uint64_t*>(coords) : nullptr};
+  x.clear = r.selected;
   if (!selects) { x.zero_counts = counts; x.zero_ratio = ratio; x.zero_ratio_host = ratio_host; }
   if ((rc = stage1_impl(who, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, M, L, acc, x, batch, n_q_heads, n_kv_heads,
                         n_ctx, head_dim, block_size, step, (float)sm_scale, scale_mode, dtype, stream)))
@@ -475,10 +487,10 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
     if (!fused_pool &&
         (rc = aa_pool_q_anchor(q, q_sb, q_sh, q_sn, M, qbar, abar, batch, n_q_heads, n_ctx, head_dim, block_size, dtype, stream)))
       return rc;
-    if ((rc = stage2_impl(who, fused_pool, qbar, abar, k, k_sb, k_sh, k_sn, mask, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
+    if ((rc = stage2_impl(who, fused_pool, r, qbar, abar, k, k_sb, k_sh, k_sn, mask, coords, counts, batch, n_q_heads, n_kv_heads, n_ctx,
                           head_dim, block_size, step, sm_scale, theta_log2, geometry, dtype, stream)))
       return rc;
-    if ((rc = stage3_impl(who, 1, ratio, ratio_host, denominator, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc,
+    if ((rc = stage3_impl(who, 1, r, q, q_sb, q_sh, q_sn, k, k_sb, k_sh, k_sn, v, v_sb, v_sh, v_sn, coords, counts, M, L, acc,
                           out, o_sb, o_sh, o_sn, batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size, step, (float)sm_scale, dtype,
                           stream)))
       return rc;

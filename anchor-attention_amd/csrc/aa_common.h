@@ -142,6 +142,14 @@ __device__ __forceinline__ void store_ratio(const float x, float* ratio, float* 
   *ratio = x;
   if (ratio_host != nullptr) __hip_atomic_store(ratio_host, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+// The same by all work-groups of a launch, each with the keys that it has selected (`mine`, of its first thread): one 64-bit atomic each, work-groups that
+// have come in the upper bits and keys in the lower 44.  The last one stores the ratio.  The number is the atomic's own, so nothing else has to be ordered.
+__device__ __forceinline__ void add_selected(const uint32_t mine, uint64_t* selected, const float inverse, float* ratio, float* ratio_host) {
+  constexpr uint64_t kOne = 1ull << 44;
+  const uint64_t sum = __hip_atomic_fetch_add(selected, kOne + mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + (kOne + mine);
+  if (sum >> 44 == gridDim.x) store_ratio((float)(int64_t)(sum & (kOne - 1)) * inverse, ratio, ratio_host);
+}
+
 __device__ __forceinline__ void sum_counts(const int32_t* counts, const int64_t n, const float inverse, float* ratio, float* ratio_host,
                                            int64_t* part) {
   int64_t sum = 0;

@@ -232,6 +232,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // (anchor, a single big block) The ratio, which a logged call waits for, is known at once.  From the work-group of the first rows, which is dealt out
   // last, it came 5 us later: calls in a row, 2048 tokens, 14/2 heads of 64 28.3 us -> 23.8, 32/8 heads of 64 29.4 -> 27.4.
   if (MODE == kAnchor && p.ratio != nullptr && block == 0 && threadIdx.x == 0) store_ratio(0.f, p.ratio, p.ratio_host);
+  // (the sum that stage 2 makes)
+  if (MODE == kAnchor && p.clear != nullptr && block == 0 && threadIdx.x == 0) *p.clear = 0;
   // (sparse) one work-group more than the query blocks need, the first, sums the counts to the ratio beside the others
   const bool sums = MODE == kSparse && p.ratio != nullptr;
   if (sums && block == 0) {

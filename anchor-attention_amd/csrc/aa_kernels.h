@@ -17,6 +17,7 @@ struct FlashArgs {
   uint32_t* thr_out; float scale2, theta_log2;
   // anchor mode, optional: [B,Hq], set to 0 where big block 0 is finished (the only one: nobody else writes its counts)
   int32_t* zero_counts;
+  uint64_t* clear;  // anchor mode, optional: a word that is set to 0 (SelectArgs::selected)
   // anchor and sparse mode, optional: the ratio of selected keys, sum(counts[0 .. n_ratio_counts)) * ratio_inverse (anchor: 0)
   float* ratio; int64_t n_ratio_counts; float ratio_inverse;
   float* ratio_host;  // the same number in host memory, for a caller that waits for it and not for the launch to end
@@ -99,6 +100,8 @@ struct SelectArgs {
   int batch, n_q_heads, n_kv_heads, n_ctx;
   int big_block, block_size;
   float scale2, theta_log2;
+  // optional: the share of selected keys, formed by the work-groups of the scores as in FlashArgs; `selected` is 0 before
+  uint64_t* selected; float* ratio; float* ratio_host; float ratio_inverse;
   // candidate keys of big block bb: key_lo <= j < bb*S - key_slack (as run: block_size and block_size; intended: S and 0)
   int key_lo, key_slack;
   int head_dim;  // 128 or 64
@@ -106,6 +109,7 @@ struct SelectArgs {
 };
 hipError_t launch_select_thresholds(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_select_scores(const SelectArgs& a, hipStream_t stream);
+bool select_scores_sums(int batch, int n_kv_heads, int n_ctx);  // whether that is to form the ratio
 hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_ratio(const int32_t* counts, int64_t n, float inverse, float* ratio, hipStream_t stream);
 

@@ -120,6 +120,14 @@ constexpr int kSelRowBytes = 256; // one pooled row in LDS
 #define AA_SEL_WGS 2              // work-groups per CU the kernel is compiled for
 #endif
 
+// Which of the 32 keys from k0 on are candidates, key_lo .. key_hi - 1 (block sizes below 32 keys: the first and the last word of a row reach outside).
+__device__ __forceinline__ uint32_t candidate_bits(const int k0, const int key_lo, const int key_hi) {
+  uint32_t bits = ~0u;
+  if (k0 < key_lo) bits = key_lo - k0 >= 32 ? 0u : ~0u << (key_lo - k0);
+  if (k0 + 32 > key_hi) bits &= key_hi <= k0 ? 0u : ~0u >> (k0 + 32 - key_hi);
+  return bits;
+}
+
 // load16_to_lds for 4 bytes a lane
 __device__ __forceinline__ void sel_load4_to_lds(const char* base, const uint32_t byte_off, const uint32_t lds_dst) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dword %1, %2" : : "{m0}"(lds_dst), "v"(byte_off), "s"(base) : "memory");
@@ -128,7 +136,9 @@ __device__ __forceinline__ void sel_load4_to_lds(const char* base, const uint32_
 // D = head dimension (128 or 64).  With 64 the pooled rows keep their 256-byte pitch in LDS: a row fills eight of its
 // sixteen 16-byte slots (the staging lanes whose slot belongs to no chunk fetch a duplicate that is never read), so
 // the LDS addressing is that of 128 and only the number of MFMA steps over the head dimension changes.
-template <int STEP, int WAVES, int ROWS, typename T, int D>
+//
+// SUMS: the work-groups also form the share of selected keys (add_selected).
+template <int STEP, int WAVES, int ROWS, typename T, int D, bool SUMS>
 __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(const SelectArgs p) {
   constexpr int kKS = D / 16;                    // MFMA steps over the head dimension
   constexpr int kItems = 32 / STEP;              // items per 32-row MFMA group
@@ -146,6 +156,7 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
   static_assert(kBlockItems <= 64, "one lane per item of a block");
   __shared__ __attribute__((aligned(16))) char a_lds[2][ROWS * kSelRowBytes];
   __shared__ __attribute__((aligned(16))) float thr_lds[2][ROWS];
+  __shared__ uint32_t sums[SUMS ? WAVES : 1];
 
   // Work-groups are renumbered so that each XCD owns a contiguous range ordered (batch, KV head, super-tile): the
   // pooled queries a work-group streams are those of its KV head's query heads (1 MiB per KV head at 128k tokens),
@@ -172,7 +183,10 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
   int bb_lo = n_bb;                           // smallest big block any wave of the work-group needs
 #pragma unroll
   for (int i = 0; i < kTilesPerWg; ++i) bb_lo = min(bb_lo, tile_bb_min(kTilesPerWg * ST + i));
-  if (bb_lo >= n_bb) return;
+  if (bb_lo >= n_bb) {
+    if (SUMS && tid == 0) add_selected(0u, p.selected, p.ratio_inverse, p.ratio, p.ratio_host);
+    return;
+  }
   const int group = p.n_q_heads / p.n_kv_heads;
   const int n_items = group * (n_bb - bb_lo);
   const int n_blocks = (n_items * STEP + ROWS - 1) / ROWS;
@@ -232,6 +246,7 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
   typedef __attribute__((address_space(3))) floatx4 lds_floatx4_t;
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+  uint32_t selected = 0u;  // keys of the words that this lane stores
   for (int blk = 0; blk < n_blocks; ++blk) {
     const int buf = blk & 1;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of block blk has landed
@@ -289,18 +304,42 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
       if (item < n_items && bb >= bb_min_w) {
         uint32_t* dst = p.mask + ((((int64_t)b * p.n_q_heads + hq) * n_bb + bb) * n_t + tw) * 4 + kb0;
         *reinterpret_cast<u32x2*>(dst) = u32x2{w_lo, w_hi};
+        if (SUMS) {
+          const int key0 = 128 * tw + 32 * kb0, key_hi = bb * S - p.key_slack;
+          selected += __popc(w_lo & candidate_bits(key0, p.key_lo, key_hi)) + __popc(w_hi & candidate_bits(key0 + 32, p.key_lo, key_hi));
+        }
       }
     }
   }
+  if (SUMS) {
+#pragma unroll
+    for (int d = 1; d < kBlockItems; d <<= 1) selected += __shfl_xor((int)selected, d, 64);
+    if (lane == 0) sums[wave] = selected;
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) selected += sums[w];
+      add_selected(selected, p.selected, p.ratio_inverse, p.ratio, p.ratio_host);
+    }
+  }
 }
+
+static uint32_t scores_work_groups(int batch, int n_kv_heads, int n_ctx) { return (uint32_t)(n_ctx / (64 * AA_SEL_WAVES)) * n_kv_heads * batch; }
+
+// Up to 128 work-groups (8 KV heads: 4096 tokens, 2: 16384) a call is so short that a logged one's wait for the ratio decides when the next can
+// start: with the ratio from here, a list and a launch sooner than from stage 3, calls in a row take 2048 tokens (14/2 heads of 64, blocks of 64) 55.1
+// -> 52.0 us, 4096 (14/2) 76.7 -> 73.2, (32/8 of 64) 102 -> 98.5, (32/8 of 128) 153.7 -> 151.0, 8192 (14/2) 123 -> 120.  Where the GPU has work for that
+// long, the sums and atomics only cost: 256 work-groups 339 -> 341, 512 721 -> 724 and 1343 -> 1348, 1024 1540 -> 1545 us.
+bool select_scores_sums(int batch, int n_kv_heads, int n_ctx) { return scores_work_groups(batch, n_kv_heads, n_ctx) <= 128; }
 
 template <typename T, int D>
 static void launch_select_scores_for(const SelectArgs& a, hipStream_t stream) {
   constexpr int kWaves = AA_SEL_WAVES, kRows = AA_SEL_ROWS;
   const int step = a.big_block / a.block_size;
-  const dim3 grid((uint32_t)(a.n_ctx / (64 * kWaves)) * a.n_kv_heads * a.batch);
-  if (step == 16) hipLaunchKernelGGL((select_scores_kernel<16, kWaves, kRows, T, D>), grid, dim3(64 * kWaves), 0, stream, a);
-  else hipLaunchKernelGGL((select_scores_kernel<32, kWaves, kRows, T, D>), grid, dim3(64 * kWaves), 0, stream, a);
+  const dim3 grid(scores_work_groups(a.batch, a.n_kv_heads, a.n_ctx));
+  const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(64 * kWaves), 0, stream, a); };
+  if (a.selected != nullptr) launch(step == 16 ? select_scores_kernel<16, kWaves, kRows, T, D, true> : select_scores_kernel<32, kWaves, kRows, T, D, true>);
+  else launch(step == 16 ? select_scores_kernel<16, kWaves, kRows, T, D, false> : select_scores_kernel<32, kWaves, kRows, T, D, false>);
 }
 
 hipError_t launch_select_scores(const SelectArgs& a, hipStream_t stream) {
@@ -347,14 +386,7 @@ __global__ void __launch_bounds__(COMPACT_WORDS) select_compact_kernel(const Sel
   const int w_lo = key_lo / 32, w_hi = (key_hi + 31) / 32;  // mask words [w_lo, w_hi) of the row
   const uint32_t* mw = p.mask + (bh * n_bb + bb) * n_t * 4;
   int32_t* out = p.coords + bh * p.coords_per_head + coords_tri(bb, p.big_block, p.block_size);
-  const auto load = [&](const int wi) {
-    const int k0 = wi * 32;
-    uint32_t word = wi < w_hi ? mw[wi] : 0u;
-    // the first and the last word may reach outside the candidate range (block sizes below 32 keys)
-    if (k0 < key_lo) word &= key_lo - k0 >= 32 ? 0u : ~0u << (key_lo - k0);
-    if (k0 + 32 > key_hi) word &= key_hi <= k0 ? 0u : ~0u >> (k0 + 32 - key_hi);
-    return word;
-  };
+  const auto load = [&](const int wi) { return wi < w_hi ? mw[wi] & candidate_bits(wi * 32, key_lo, key_hi) : 0u; };
   int base = 0;
   if (key_hi > key_lo && w_hi - w_lo <= 64) {  // a single wave's words: no barrier, and no stores of other waves to wait behind
     if (wave != 0) return;
