@@ -161,6 +161,31 @@ __device__ __forceinline__ void sum_counts(const int32_t* counts, const int64_t 
   if (threadIdx.x == 0) store_ratio((float)(part[0] + part[1] + part[2] + part[3]) * inverse, ratio, ratio_host);
 }
 
+// ---- division by a number that the host knows --------------------------------------------------
+// Every work-group finds its place by some ten divisions, of 150 to 200 clocks one after the other where the compiler divides by a number it does
+// not know, and those of rows have eight more beside their stores; with the reciprocal from the host a division is a multiplication, two
+// additions and two shifts.  (Granlund and Montgomery, Division by invariant integers using multiplication: exact for all 32-bit numbers.)
+// 32/8 heads of 128: 777 rows 20.1 -> 19.85 us, padded 2 x 1500 63.6 -> 62.3 and 3 x 2500 186 -> 184.4, a decode step over 33001 keys 28.65 -> 28.25;
+// 131072 tokens 7343 -> 7328.
+struct FastDiv {
+  uint32_t mul, shift1, shift2;
+};
+inline FastDiv fast_div(const uint32_t d) {  // d >= 1
+  uint32_t bits = 0;
+  while (bits < 32 && (1ull << bits) < d) ++bits;
+  return {(uint32_t)((((1ull << bits) - d) << 32) / d + 1), bits < 1 ? bits : 1, bits > 0 ? bits - 1 : 0};
+}
+__host__ __device__ __forceinline__ uint32_t quotient(const uint32_t n, const FastDiv& f) {
+  const uint32_t t = (uint32_t)((uint64_t)n * f.mul >> 32);
+  return (t + ((n - t) >> f.shift1)) >> f.shift2;
+}
+// n divided by the divisor of f; n becomes the quotient, the remainder is returned
+__host__ __device__ __forceinline__ uint32_t take_remainder(uint32_t& n, const FastDiv& f, const uint32_t d) {
+  const uint32_t q = quotient(n, f), r = n - q * d;
+  n = q;
+  return r;
+}
+
 // ---- geometry --------------------------------------------------------------------------------
 // Index lists are packed per (batch, query head): big block bb can select at most
 // cap(bb) = bb*S - 2*bs keys (candidates are [bs, bb*S - bs)), and its list starts at
@@ -178,18 +203,9 @@ __host__ __device__ inline int64_t coords_tri(int64_t bb, int64_t S, int64_t bs)
 //   8 % n_units == 0 : s = 8 / n_units XCDs share a unit and take its rows alternately (row = idx / inner, the
 //                      `inner` work-groups of a row stay together), so that each gets the same mix of heavy and light;
 //   otherwise        : the hardware order is kept.
-// `abreast`: an XCD takes its units (in the last case: all XCDs all units) side by side, the heaviest of each first, instead of one
-// after the other, so that the launch does not end with the heaviest work-groups of its last unit.
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uint32_t per_unit, uint32_t inner, bool abreast) {
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uint32_t per_unit, uint32_t inner) {
   const uint32_t total = n_units * per_unit;
   const uint32_t xcd = wg % 8u, k = wg / 8u;
-  if (abreast) {
-    if (total % 8u != 0u || n_units % 8u != 0u) return wg % n_units * per_unit + wg / n_units;
-    // (the XCD's 32 CUs are filled in turn: without the rotation a number of units that divides 32 ties a CU to a unit, and
-    // units differ in weight: two prompts of 3900, one padded, 239 us one after the other, 280 without it and 239 with it)
-    const uint32_t own = n_units / 8u, turn = 32u % own == 0u ? k / 32u : 0u;
-    return ((k + turn) % own * 8u + xcd) * per_unit + k / own;
-  }
   if (total % 8u != 0u) return wg;
   if (n_units % 8u == 0u) return (k / per_unit * 8u + xcd) * per_unit + k % per_unit;
   if (8u % n_units == 0u) {
@@ -197,6 +213,56 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uin
     if ((per_unit / inner) % s == 0u) return (xcd / s) * per_unit + ((k / inner) * s + xcd % s) * inner + k % inner;
   }
   return wg;
+}
+// The same map with the reciprocals and the choice from the host, as (unit, index in the unit).
+// `abreast`: an XCD takes its units (in the last case: all XCDs all units) side by side, the heaviest of each first, instead of one
+// after the other, so that the launch does not end with the heaviest work-groups of its last unit.
+struct Deal {
+  enum Kind : uint32_t { kInTurn, kOwnUnits, kSharedUnits, kAbreast, kAbreastAll } kind;
+  uint32_t n_units, per_unit, inner;
+  uint32_t own;        // (abreast) units of an XCD
+  uint32_t turns;      // (abreast) ... which begin one further on every 32 work-groups
+  uint32_t share_log;  // (shared units) log2 of the XCDs that share one
+  FastDiv by_per_unit, by_inner, by_own, by_units;
+};
+inline Deal make_deal(uint32_t n_units, uint32_t per_unit, uint32_t inner, bool abreast) {
+  Deal d = {Deal::kInTurn, n_units, per_unit, inner, 1, 0, 0, fast_div(per_unit), fast_div(inner), fast_div(1), fast_div(n_units)};
+  const bool even = (uint64_t)n_units * per_unit % 8 == 0;
+  if (abreast) {
+    d.kind = !even || n_units % 8 != 0 ? Deal::kAbreastAll : Deal::kAbreast;
+    d.own = d.kind == Deal::kAbreast ? n_units / 8 : 1;
+    // (the XCD's 32 CUs are filled in turn: without the rotation a number of units that divides 32 ties a CU to a unit, and
+    // units differ in weight: two prompts of 3900, one padded, 239 us one after the other, 280 without it and 239 with it)
+    d.turns = 32 % d.own == 0;
+    d.by_own = fast_div(d.own);
+  } else if (even && n_units % 8 == 0) {
+    d.kind = Deal::kOwnUnits;
+  } else if (even && 8 % n_units == 0 && (per_unit / inner) % (8 / n_units) == 0) {
+    d.kind = Deal::kSharedUnits;
+    for (uint32_t s = 8 / n_units; s > 1; s /= 2) ++d.share_log;
+  }
+  return d;
+}
+__host__ __device__ __forceinline__ void dealt(const Deal& d, const uint32_t wg, uint32_t& unit, uint32_t& index) {
+  const uint32_t xcd = wg % 8u;
+  uint32_t k = wg / 8u;
+  if (d.kind == Deal::kOwnUnits) {
+    index = take_remainder(k, d.by_per_unit, d.per_unit);
+    unit = k * 8u + xcd;
+  } else if (d.kind == Deal::kSharedUnits) {
+    const uint32_t in = take_remainder(k, d.by_inner, d.inner);
+    unit = xcd >> d.share_log;
+    index = ((k << d.share_log) + (xcd & ((1u << d.share_log) - 1u))) * d.inner + in;
+  } else if (d.kind == Deal::kAbreast) {
+    uint32_t turned = k + (d.turns ? k / 32u : 0u);
+    unit = take_remainder(turned, d.by_own, d.own) * 8u + xcd;
+    index = quotient(k, d.by_own);
+  } else {
+    uint32_t n = wg;
+    const uint32_t r = d.kind == Deal::kAbreastAll ? take_remainder(n, d.by_units, d.n_units) : take_remainder(n, d.by_per_unit, d.per_unit);
+    unit = d.kind == Deal::kAbreastAll ? r : n;
+    index = d.kind == Deal::kAbreastAll ? n : r;
+  }
 }
 
 // ---- error plumbing (host) -------------------------------------------------------------------

@@ -51,9 +51,9 @@ __global__ void __launch_bounds__(64 * WAVES) decode_kernel(const FlashArgs p) {
 
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, c32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int chunk = blockIdx.x % p.n_chunks, unit = blockIdx.x / p.n_chunks;
-  const int kvh = unit % p.n_kv_heads, b = unit / p.n_kv_heads;
-  const int group = p.n_q_heads / p.n_kv_heads, n_cols = p.n_rows * group;
+  const int unit = quotient(blockIdx.x, p.by_chunks), chunk = blockIdx.x - unit * p.n_chunks;
+  const int b = quotient(unit, p.by_kv_heads), kvh = unit - b * p.n_kv_heads;
+  const int group = p.group, n_cols = p.n_rows * group;
   const int key_lo = chunk * p.chunk_tiles * kDecTile, key_hi = min(key_lo + p.chunk_tiles * kDecTile, p.n_ctx);
   const int n_tiles = (key_hi - key_lo + kDecTile - 1) / kDecTile;  // at least one: the host cuts the chunks so
 
@@ -106,7 +106,7 @@ __global__ void __launch_bounds__(64 * WAVES) decode_kernel(const FlashArgs p) {
     if (t_next < n_tiles) issue(t_next, 1);
   }
 
-  const int my_col = min(c32, n_cols - 1), my_row = my_col / group;
+  const int my_col = min(c32, n_cols - 1), my_row = quotient(my_col, p.by_group);
   const int my_last_key = MASKED ? p.n_ctx - 1 : min(p.causal_offset + my_row, p.n_ctx - 1);
   const int first_last_key = __builtin_amdgcn_readfirstlane(my_last_key);
   vec8 qreg[kKS];
@@ -263,7 +263,7 @@ __global__ void __launch_bounds__(64 * WAVES) decode_kernel(const FlashArgs p) {
     }
     if (p.n_chunks == 1) {
       const float inv = l == 0.f ? 0.f : 1.f / l;
-      const int row = col / group;
+      const int row = quotient(col, p.by_group);
       uint16_t* op = p.out + b * p.o_sb + (int64_t)(kvh * group + col - row * group) * p.o_sh + (int64_t)row * p.o_sn + d;
       *reinterpret_cast<uint2*>(op) = uint2{T::pack(x[0] * inv, x[1] * inv), T::pack(x[2] * inv, x[3] * inv)};
     } else {
@@ -286,8 +286,8 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const FlashArgs p) 
   __shared__ float red[2][4];
   __shared__ floatx4 part[kParts][kLanes];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int group = p.n_q_heads / p.n_kv_heads, n_cols = p.n_rows * group;
-  const int col = blockIdx.x % n_cols, unit = blockIdx.x / n_cols;
+  const int group = p.group, n_cols = p.n_rows * group;
+  const int unit = quotient(blockIdx.x, p.by_cols), col = blockIdx.x - unit * n_cols;
   const int64_t at0 = (int64_t)unit * p.n_chunks * n_cols + col;
   const float scale = p.sm_scale * kLog2e;
   // (at most 256 chunks: one per thread)
@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(const FlashArgs p) 
       for (int e = 0; e < 4; ++e) sum[e] += part[i][tid][e];
     const float l_all = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     const float inv = l_all == 0.f ? 0.f : 1.f / l_all;
-    const int kvh = unit % p.n_kv_heads, b = unit / p.n_kv_heads, row = col / group;
+    const int b = quotient(unit, p.by_kv_heads), kvh = unit - b * p.n_kv_heads, row = quotient(col, p.by_group);
     uint16_t* op = p.out + b * p.o_sb + (int64_t)(kvh * group + col - row * group) * p.o_sh + (int64_t)row * p.o_sn + 4 * tid;
     *reinterpret_cast<uint2*>(op) = uint2{T::pack(sum[0] * inv, sum[1] * inv), T::pack(sum[2] * inv, sum[3] * inv)};
   }
@@ -375,7 +375,9 @@ static void launch_decode_for(const FlashArgs& a, hipStream_t stream) {
   if (a.n_chunks > 1) hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((uint32_t)units * a.n_rows * group), block, 0, stream, a);
 }
 
-hipError_t launch_decode(const FlashArgs& a, hipStream_t stream) {
+hipError_t launch_decode(FlashArgs a, hipStream_t stream) {
+  set_divisors(a);
+  a.by_cols = fast_div((uint32_t)a.n_rows * a.group);  // (the columns are one block, and each is merged by a work-group)
   if (a.head_dim == 128) {
     if (a.dtype == 0) launch_decode_for<Bf16, 128>(a, stream);
     else launch_decode_for<F16, 128>(a, stream);

@@ -229,7 +229,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // block, one after the other: they share the big block's index list (fetched once), and the output stores of one
   // block drain while the next one is already loading, instead of every 128 rows paying for a work-group launch, the
   // list's round trip to memory and the wait for its stores.
-  const int group = p.n_q_heads / p.n_kv_heads;
+  const int group = p.group;
   const int nq = MODE == kSparse ? p.q_blocks_per_wg : 1;
   // (anchor, a single big block) The ratio, which a logged call waits for, is known at once.  From the work-group of the first rows, which is dealt out
   // last, it came 5 us later: calls in a row, 2048 tokens, 14/2 heads of 64 28.3 us -> 23.8, 32/8 heads of 64 29.4 -> 27.4.
@@ -244,48 +244,38 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   }
   const uint32_t wg = block - (sums ? 1u : 0u);
   const int S = p.big_block;
-  // (sparse mode may leave out the first big block, whose rows select nothing)
-  const int n_qunit = kAnyRows ? 1 : (p.n_ctx - (MODE == kSparse ? p.first_big_block * S : 0)) / (BM * nq);
-  int g, qunit, kvh, b;
+  int g, qunit, bb = 0;
+  uint32_t unit, index;  // the KV head, of all batch elements', and the number of the work-group among its
   int chunk = 0;  // (rows) which chunk of the keys
-  const uint32_t n_pairs = (uint32_t)(p.batch * p.n_kv_heads) * (uint32_t)(p.n_ctx / S - p.first_big_block);
-  if (MODE == kSparse && n_pairs % 8u == 0u) {
+  if (MODE == kSparse && p.pairs) {
     // Stage 3's work per (KV head, big block) pair is the length of the pair's index lists, which depends on the data:
     // a head whose queries select many keys would keep its XCD busy long after the others have finished if whole
     // heads were tied to XCDs.  So the unit that stays on one XCD (and shares its L2) is the pair - the query blocks of
     // a big block and the heads of a KV group gather the same rows - and consecutive pairs, ordered latest big block
     // first, go round-robin over the XCDs with a rotation, so that every XCD sees every head and every depth.
-    const uint32_t per_pair = (uint32_t)group * (uint32_t)(S / (BM * nq));  // work-groups of a pair
-    const uint32_t n_units = (uint32_t)(p.batch * p.n_kv_heads);
-    const uint32_t xcd = wg % 8u, k = wg / 8u;
-    const uint32_t kp = k / per_pair, within = k % per_pair;
-    const uint32_t pair = kp * 8u + (xcd + kp) % 8u;
-    const int bb_ = p.n_ctx / S - 1 - (int)(pair / n_units);
-    const uint32_t unit = pair % n_units;
-    g = within % group;
-    qunit = bb_ * (S / (BM * nq)) + (int)(within / group);
-    kvh = unit % p.n_kv_heads;
-    b = unit / p.n_kv_heads;
+    uint32_t kp = wg / 8u, within = take_remainder(kp, p.by_pair, (uint32_t)(group * p.q_units)), pair = kp * 8u + (wg % 8u + kp) % 8u;
+    unit = take_remainder(pair, p.by_units, (uint32_t)p.units);
+    bb = p.n_big - 1 - (int)pair;
+    g = (int)take_remainder(within, p.by_group, (uint32_t)group);
+    qunit = bb * p.q_units + (int)within;
   } else if (kAnyRows) {
     // A work-group owns 128 columns of one KV head - a column is one (query row, head of the group) pair, heads running
     // fastest, so all heads of a group use the same K/V tile - and one chunk of the keys.  Work-groups of one chunk are
     // neighbours on one XCD (they read the same K/V rows), latest columns, which see the most keys, first.
-    uint32_t vid = xcd_remap(wg, p.batch * p.n_kv_heads, p.n_col_blocks * p.n_chunks, 1, p.abreast);
-    qunit = p.n_col_blocks - 1 - (int)(vid % p.n_col_blocks);  vid /= p.n_col_blocks;
-    chunk = vid % p.n_chunks;  vid /= p.n_chunks;
-    kvh = vid % p.n_kv_heads;
-    b = vid / p.n_kv_heads;
+    dealt(p.deal, wg, unit, index);
+    qunit = p.n_col_blocks - 1 - (int)take_remainder(index, p.by_cols, (uint32_t)p.n_col_blocks);
+    chunk = (int)index;
     g = 0;
   } else {
-    uint32_t vid = xcd_remap(wg, p.batch * p.n_kv_heads, group * n_qunit, group, p.abreast);
-    g = vid % group;  vid /= group;
-    qunit = vid % n_qunit;  vid /= n_qunit;
-    kvh = vid % p.n_kv_heads;
-    b = vid / p.n_kv_heads;
-    qunit = p.n_ctx / (BM * nq) - 1 - qunit;  // longest rows first (later big blocks also carry the longest index lists)
+    dealt(p.deal, wg, unit, index);
+    g = (int)take_remainder(index, p.by_group, (uint32_t)group);
+    // longest rows first (later big blocks also carry the longest index lists; sparse mode may leave out the first, whose rows select nothing)
+    qunit = (MODE == kSparse ? p.n_big * p.q_units : p.n_ctx / BM) - 1 - (int)index;
+    // (all blocks of a work-group lie in one big block: the host picks q_blocks_per_wg so)
+    if (MODE == kAnchor || MODE == kSparse) bb = (int)quotient((uint32_t)qunit, p.by_block);
   }
+  const int b = (int)quotient(unit, p.by_kv_heads), kvh = (int)unit - b * p.n_kv_heads;
   const int hq = kvh * group + g;
-  const int bb = qunit * nq * BM / S;  // (all blocks of a work-group lie in one big block: the host picks q_blocks_per_wg so)
   const int64_t bh = (int64_t)b * p.n_q_heads + hq;
 
   const uint16_t* qp = p.q + b * p.q_sb + hq * p.q_sh;
@@ -305,7 +295,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     cap = max(bb * S - 2 * p.block_size, 0);  // capacity of the big block's list (a multiple of 4)
     // (counts and indices come from device memory the caller filled: a count beyond the capacity or an index beyond
     // the context is clamped rather than followed out of bounds)
-    cnt = max(0, min(p.counts[bh * (p.n_ctx / S) + bb], cap));
+    cnt = max(0, min(p.counts[bh * p.n_big + bb], cap));
     cbase = p.coords + bh * p.coords_per_head + coords_tri(bb, S, p.block_size);
     sparse_tiles = (cnt + kBN - 1) / kBN;
     if (AA_ABLATE == 4 || AA_ABLATE == 7) sparse_tiles = 0;
@@ -348,7 +338,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // (rows) this lane's column, as (row, head of the group): columns past the last one repeat it and are not stored
   const int n_cols = kAnyRows ? p.n_rows * group : 0;
   const int my_col = min(wr0 + c32, n_cols - 1);
-  const int my_row = kAnyRows ? my_col / group : wr0 + c32;
+  const int my_row = kAnyRows ? (int)quotient((uint32_t)my_col, p.by_group) : wr0 + c32;
   // (rows) the last key this lane's row sees, and the smallest such key of the wave (rows ascend with the lane)
   const int my_last_key = kAnyRows ? min(p.causal_offset + my_row, p.n_ctx - 1) : my_row;
   const int wave_last_key = kAnyRows ? __builtin_amdgcn_readfirstlane(my_last_key) : wr0;
@@ -385,7 +375,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     n_tiles = (R0 + BM) / kBN;
   } else if (kAnyRows) {
     const int last_row = min(R0 + BM, n_cols) - 1;
-    const int seen = min(p.causal_offset + last_row / group, p.n_ctx - 1) / kBN + 1;  // tiles up to the last key any column sees
+    const int seen = min(p.causal_offset + (int)quotient((uint32_t)last_row, p.by_group), p.n_ctx - 1) / kBN + 1;  // tiles up to the last key any column sees
     key_base = chunk * p.chunk_tiles * kBN;
     n_tiles = min(seen - chunk * p.chunk_tiles, p.chunk_tiles);
     if (n_tiles <= 0) return;  // (never chunk 0: every row sees at least one key)
@@ -1194,7 +1184,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       const int r = it * kRowsPerStore + lane_e / kLanesPerRow, c = lane_e % kLanesPerRow;
       const u32x4 w = *reinterpret_cast<const u32x4*>(ob + r * kRowBytes + ((c ^ (r & kChunkMask)) << 4));
       if (kAnyRows) {
-        const int col = wr0 + r, row = col / group;
+        const int col = wr0 + r, row = (int)quotient((uint32_t)col, p.by_group);
         if (col < n_cols) *reinterpret_cast<u32x4*>(op + (col - row * group) * p.o_sh + (int64_t)row * p.o_sn + 8 * c) = w;
       } else {
         __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(op + (int64_t)(wr0 + r) * p.o_sn + 8 * c));
@@ -1239,6 +1229,7 @@ flash_pair_kernel(const FlashArgs anchor, const FlashArgs rows, const uint32_t n
 template <int MODE>
 static uint32_t place(FlashArgs& a, const bool alone) {
   a.q_blocks_per_wg = 1;
+  set_divisors(a);
   int64_t blocks = (int64_t)a.batch * a.n_q_heads * (a.n_ctx / 128);
   if (MODE == kSparse) {
     const int per_big_block = a.big_block / 128;
@@ -1252,6 +1243,12 @@ static uint32_t place(FlashArgs& a, const bool alone) {
     int nq = AA_SPARSE_QBLOCKS;
     while (nq > 1 && (per_big_block % nq != 0 || blocks / nq < fills_twice)) nq /= 2;
     a.q_blocks_per_wg = nq;
+    a.q_units = per_big_block / nq;
+    a.by_pair = fast_div(a.group * a.q_units);
+    a.by_block = fast_div(a.q_units);
+    a.pairs = (int64_t)a.units * (a.n_big - a.first_big_block) % 8 == 0;
+  } else if (MODE == kAnchor) {
+    a.by_block = fast_div(a.big_block / 128);
   }
   // More units (KV heads of all batch elements) than XCDs: side by side as long as the K and V that an XCD then works on fit its L2
   // of 4 MB.  Left-padded batches: 3 x 2500 with 32/8 heads of 128 194 -> 184 us, 28/4 184 -> 162, 3 x 1000 with 32/8 heads of 64 39.9 -> 30.0, 4 x 2900
@@ -1260,10 +1257,13 @@ static uint32_t place(FlashArgs& a, const bool alone) {
   // work-groups of the last unit.  1578 rows, 14/2 heads of 64 28.0 -> 23.3 us; padded 2 x 1920 48.5 -> 42.8; dense 4864 tokens 90.1 -> 69.3; with 28/4
   // heads of 128 1501 rows in one chunk 54.2 -> 41.3, dense 3712 fp16 142.5 -> 120.3.  A launch that anchor and rows work-groups share gains
   // nothing on average (44 sizes: from 10 % faster to 10 % slower).
-  const int units = a.batch * a.n_kv_heads;
-  const int rows = MODE == kRows || MODE == kMasked ? a.n_col_blocks * a.n_chunks : a.n_ctx / 128;  // (of a unit: what xcd_remap deals out)
-  a.abreast = MODE != kSparse && (8 % units != 0 ? (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20
+  const int units = a.units;
+  const int rows = MODE == kRows || MODE == kMasked ? a.n_col_blocks * a.n_chunks : a.n_ctx / 128;  // (of a unit: what is dealt out)
+  const bool abreast = MODE != kSparse && (8 % units != 0 ? (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20
                                                           : alone && rows % (8 / units) != 0);
+  if (MODE == kRows || MODE == kMasked) a.deal = make_deal(units, rows, 1, abreast);
+  else if (MODE != kSparse) a.deal = make_deal(units, a.group * rows, a.group, abreast);
+  else a.deal = make_deal(units, a.group * (a.n_big - a.first_big_block) * a.q_units, a.group, false);
   if (MODE == kRows || MODE == kMasked) return (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks;
   return (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0);
 }

@@ -29,13 +29,13 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t id = blockIdx.x;
   const int db = id % kDB;  id /= kDB;
-  const int block = id % p.n_col_blocks;  id /= p.n_col_blocks;
-  const int kvh = id % p.n_kv_heads, b = id / p.n_kv_heads;
-  const int group = p.n_q_heads / p.n_kv_heads, n_cols = p.n_rows * group;
+  const int block = take_remainder(id, p.by_cols, p.n_col_blocks);
+  const int b = quotient(id, p.by_kv_heads), kvh = id - b * p.n_kv_heads;
+  const int group = p.group, n_cols = p.n_rows * group;
   // the chunks that hold keys of this block (the others were not written)
-  const int last_row = (min(128 * block + 128, n_cols) - 1) / group;
+  const int last_row = quotient(min(128 * block + 128, n_cols) - 1, p.by_group);
   const int tiles = min(p.causal_offset + last_row, p.n_ctx - 1) / 64 + 1;
-  const int n_chunks = (tiles + p.chunk_tiles - 1) / p.chunk_tiles;
+  const int n_chunks = quotient(tiles + p.chunk_tiles - 1, p.by_chunk_tiles);
   const int64_t slot0 = ((((int64_t)b * p.n_kv_heads + kvh) * p.n_col_blocks + block) * p.n_chunks) * 4 + wave;
   const float scale = p.sm_scale * kLog2e;
 
@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
   // a lane holds columns 8*rg + 4*half .. +3 of the piece: the two halves of the wave trade register groups, so that each
   // lane stores whole 16-byte chunks (half 0 the even groups, half 1 the odd ones)
   const int col = 128 * block + 32 * wave + c32;
-  const int row = min(col, n_cols - 1) / group;
+  const int row = quotient(min(col, n_cols - 1), p.by_group);
   uint16_t* op = p.out + b * p.o_sb + (int64_t)(kvh * group + min(col, n_cols - 1) - row * group) * p.o_sh + (int64_t)row * p.o_sn + 32 * db;
 #pragma unroll
   for (int pr = 0; pr < 2; ++pr) {
@@ -96,7 +96,8 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
   }
 }
 
-hipError_t launch_rows_combine(const FlashArgs& a, hipStream_t stream) {
+hipError_t launch_rows_combine(FlashArgs a, hipStream_t stream) {
+  set_divisors(a);
   const dim3 grid((uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * (a.head_dim / 32)), block(256);
   if (a.head_dim == 128) {
     if (a.dtype == 0) hipLaunchKernelGGL((rows_combine_kernel<Bf16, 128>), grid, block, 0, stream, a);

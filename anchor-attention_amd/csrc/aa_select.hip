@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
   const int n_bb = p.n_ctx / S;
   const int n_t = p.n_ctx / 128;
   const int n_super = n_t / kTilesPerWg;
-  uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, n_super, 1, false);
+  uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, n_super, 1);
   const int ST = vid % n_super;  // key super-tile (kTilesPerWg * 128 keys); ascending = heaviest first
   vid /= n_super;
   const int kvh = vid % p.n_kv_heads, b = vid / p.n_kv_heads;
