@@ -204,6 +204,11 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // conversions to the block of their use, where no MFMAs run beside them (131072 tokens, 32/8 heads of 128, all stages: 7.60 ms
   // against 7.53).  Head dimension 64 spills registers for it (anchor, sparse, fp16 rows).
   constexpr bool kPinned = D == 128 || kLazyRef || MODE == kDense;
+  // MFMAs of a tile that are issued behind its closing barrier, while the first K operands of the next tile are on their way: with none a wave waits
+  // a whole LDS latency there.  0 against 2: dense 16384 tokens, 32/8 heads of 128, 1692.2 -> 1684.7 us, 131072 7080 -> 7040, 32768 with nearly every key selected
+  // 8508 -> 8472, rows 777 19.9 -> 19.65, 14/2 heads of 64, 2048 tokens dense 22.1 -> 21.7, 1900 rows 25.5 -> 24.75; three of them, with
+  // operands fetched one MFMA before the barrier: 0 to 0.6 % slower than two.  Rows of fp16 at 64 spill for the operands: 1900 26.5 -> 27.1, so none there.
+  constexpr int kTail = MODE == kRows && !kLazyRef && D == 64 ? 0 : 2;
   constexpr bool kChecksSums = kLazyRef && AA_ABLATE != 1 && AA_ABLATE != 2;
   static_assert(D == 128 || D == 64, "head dimension");
   constexpr int kKS = D / 16;       // MFMAs per 32-key block of S^T = K Q^T
@@ -643,6 +648,11 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // Sparse mode, whose tile counts can be odd, keeps one copy of each kind of tile (BUF = -1): the buffer is i & 1 and the read
   // addresses step back and forth between the two buffers.  So does masked mode, for which two copies spill 25 registers.
   int32_t buf_step = (MODE == kSparse && cur) ? -kTileBytes : kTileBytes;
+  vec8 k_first[kDist];  // the K operands of the next tile's first slots
+  if (kTail > 0 && n_tiles > team) {
+#pragma unroll
+    for (int t = 0; t < kDist; ++t) k_first[t] = *(const lds_vec8*)(uintptr_t)(k_rd[t % kKS] + 32 * (t / kKS) * kRowBytes);
+  }
   auto tile = [&](auto buf_const, auto few_const, const int i) __attribute__((always_inline)) {
     constexpr int kBuf = decltype(buf_const)::value;
     constexpr bool kFew = decltype(few_const)::value;
@@ -775,7 +785,10 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       // a quarter of the MFMAs, the row max, half of the MFMAs with the four exp chunks spread over them, the last quarter.
       constexpr int kSPre = kKS / 4, kSMid = kKS / 2, kVPre = kDB / 2, kVMid = kDB;
 #pragma unroll
-      for (int n = 0; n < kDist; ++n) AA_OPERAND_FETCH(n)
+      for (int n = 0; n < kDist; ++n) {
+        if (kTail > 0) ka[n] = k_first[n];
+        else AA_OPERAND_FETCH(n)
+      }
       AA_FENCE;
 
       // ---- phase A: S0^T = K0 Q^T (and the next tile's eight loads) -------------------------------
@@ -903,10 +916,32 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       }
       l_run += sum1;
 
-      // ---- phase D: O^T += V1^T P1^T ---------------------------------------------------------------
+      // ---- phase D: O^T += V1^T P1^T, and the hand-over to the next tile ----------------------------
 #pragma unroll
-      for (int n = kNS + 2 * kDB; n < kNS + kNV; ++n) {
+      for (int n = kNS + 2 * kDB; n < kNS + kNV - kTail; ++n) {
         AA_OPERAND_FETCH(n + kDist)
+        AA_PV_MFMA(n - kNS, pw1)
+        AA_FENCE;
+      }
+      if (kBuf < 0) {  // the read addresses follow the tiles into the other buffer
+#pragma unroll
+        for (int ks = 0; ks < kKS; ++ks) k_rd[ks] += buf_step;
+#pragma unroll
+        for (int m = 0; m < kDB; ++m) v_rd[m] += buf_step;
+        buf_step = -buf_step;
+        cur ^= 1;
+      }
+      if (AA_ABLATE != 9) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile i+1 has landed in LDS
+      // (so has the mask word: named here, or the compiler would wait for it behind the next tile's loads)
+      if (MODE == kMasked) asm volatile("" : "+v"(mask_word_next[0]), "+v"(mask_word_next[1]));
+      if (AA_ABLATE != 8 && AA_ABLATE != 9) __syncthreads();
+      AA_FENCE;
+      constexpr uint32_t rd_next = kBuf == 0 ? kTileBytes : 0;
+#pragma unroll
+      for (int t = 0; t < (kTail > 0 ? kDist : 0); ++t) k_first[t] = *(const lds_vec8*)(uintptr_t)(k_rd[t % kKS] + (uint32_t)(rd_next + 32 * (t / kKS) * kRowBytes));
+      AA_FENCE;
+#pragma unroll
+      for (int n = kNS + kNV - kTail; n < kNS + kNV; ++n) {
         AA_PV_MFMA(n - kNS, pw1)
         AA_FENCE;
       }
@@ -919,18 +954,6 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     }
 #undef AA_FETCH_ONE
 
-    if (kBuf < 0) {  // the read addresses follow the tiles into the other buffer
-#pragma unroll
-      for (int ks = 0; ks < kKS; ++ks) k_rd[ks] += buf_step;
-#pragma unroll
-      for (int m = 0; m < kDB; ++m) v_rd[m] += buf_step;
-      buf_step = -buf_step;
-      cur ^= 1;
-    }
-    if (AA_ABLATE != 9) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile i+1 has landed in LDS
-    // (so has the mask word: named here, or the compiler would wait for it behind the next tile's loads)
-    if (MODE == kMasked) asm volatile("" : "+v"(mask_word_next[0]), "+v"(mask_word_next[1]));
-    if (AA_ABLATE != 8 && AA_ABLATE != 9) __syncthreads();
   };
   // (a tile without masked pairs, by its number)
   auto whole = [&](const int i) __attribute__((always_inline)) {
