@@ -209,11 +209,7 @@ using namespace aa;
 
 extern "C" {
 
-#ifndef AA_ABLATE
-#define AA_ABLATE 0
-#endif
-// (1000 + n marks a timing-only build that leaves part of a kernel out, see aa_flash.hip; never a product)
-int aa_version(void) { return AA_ABLATE ? 1000 + AA_ABLATE : 3; }
+int aa_version(void) { return 3; }
 
 const char* aa_last_error(void) { return g_error; }
 

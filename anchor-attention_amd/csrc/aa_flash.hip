@@ -71,19 +71,6 @@ constexpr int32_t kMixedTile = 1 << 30;  // (masked) flag of a listed tile of wh
 
 enum FlashMode : int { kAnchor = 0, kSparse = 1, kDense = 2, kRows = 3, kMasked = 4 };
 
-// Timing-only ablations.  A build with -DAA_ABLATE=n (`make ablations`) leaves out one ingredient of the kernel so
-// that its cost can be measured (bench_ablations.py); such a build computes WRONG results on purpose, reports
-// aa_version() >= 1000 and is refused by the Python loader.  0, the default, is the product.
-//   1  exp2 of the soft-max replaced by a pass-through        4  (sparse) no tile loop: state in, output out
-//   2  no soft-max arithmetic at all (mask, max, exp, sum)    5  (sparse) accumulator state not loaded
-//   3  no K/V tile loads inside the tile loop                 6  (sparse) at most two tiles per query block
-//                                                             7  (sparse) 4 and 5 together
-//   8  no work-group barrier at the end of a tile             9  neither the barrier nor the wait for the tile's loads
-//  10  the soft-max is computed in full (same instructions, same energy) but the second product takes a loop-invariant
-//      operand instead of P: the dependency scores -> soft-max -> P.V inside a wave is cut, nothing else changes
-#ifndef AA_ABLATE
-#define AA_ABLATE 0
-#endif
 #ifndef AA_SPARSE_CHAIN
 #define AA_SPARSE_CHAIN 1  // 0: every query block of a stage-3 work-group requests its own first tile, queries and state
 #endif
@@ -209,7 +196,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // 8508 -> 8472, rows 777 19.9 -> 19.65, 14/2 heads of 64, 2048 tokens dense 22.1 -> 21.7, 1900 rows 25.5 -> 24.75; three of them, with
   // operands fetched one MFMA before the barrier: 0 to 0.6 % slower than two.  Rows of fp16 at 64 spill for the operands: 1900 26.5 -> 27.1, so none there.
   constexpr int kTail = MODE == kRows && !kLazyRef && D == 64 ? 0 : 2;
-  constexpr bool kChecksSums = kLazyRef && AA_ABLATE != 1 && AA_ABLATE != 2;
+  constexpr bool kChecksSums = kLazyRef;
   static_assert(D == 128 || D == 64, "head dimension");
   constexpr int kKS = D / 16;       // MFMAs per 32-key block of S^T = K Q^T
   constexpr int kDB = D / 32;       // 32-column blocks of the head dimension: accumulators of O^T
@@ -303,8 +290,6 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     cnt = max(0, min(p.counts[bh * p.n_big + bb], cap));
     cbase = p.coords + bh * p.coords_per_head + coords_tri(bb, S, p.block_size);
     sparse_tiles = (cnt + kBN - 1) / kBN;
-    if (AA_ABLATE == 4 || AA_ABLATE == 7) sparse_tiles = 0;
-    if (AA_ABLATE == 6) sparse_tiles = min(sparse_tiles, 2);
   }
   const bool list_chains = MODE == kSparse && AA_SPARSE_CHAIN && sparse_tiles > 0 && sparse_tiles <= kIdxWin / kBN;
   int cur = 0;             // (sparse) LDS buffer of the next tile to be computed
@@ -330,8 +315,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
-        floatx4 t = {0.f, 0.f, 0.f, 0.f};
-        if (AA_ABLATE != 5 && AA_ABLATE != 7) t = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(af + (db * 4 + rg) * 256));
+        const floatx4 t = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(af + (db * 4 + rg) * 256));
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[db][rg * 4 + c] = t[c];
       }
@@ -586,14 +570,14 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     mx = fmaxf(t0, t3);                                                              \
   }
   // (rows: maxima and scores are kept as raw dot products; the scale is applied to the difference, in float32)
-#define AA_EXP2(x) ((AA_ABLATE == 1 || AA_ABLATE == 2) ? (x) : fast_exp2(kAnyRows ? (x) * score_scale : (x)))
-#define AA_PROB(x) (kAnyRows && AA_ABLATE != 1 && AA_ABLATE != 2 ? prob_exp2<T>(x, score_scale) : AA_EXP2(x))
+#define AA_EXP2(x) fast_exp2(kAnyRows ? (x) * score_scale : (x))
+#define AA_PROB(x) (kAnyRows ? prob_exp2<T>(x, score_scale) : AA_EXP2(x))
   // p = exp2(s) (rows: 2^kProbLog2 times that) for accumulator registers 4c .. 4c+3 of one half, summed and rounded into the P^T fragment words
 #define AA_EXP_CHUNK(sx, pw, sum, c)                                                 \
   {                                                                                  \
     const float e0 = AA_PROB(sx[4 * (c) + 0]), e1 = AA_PROB(sx[4 * (c) + 1]);        \
     const float e2 = AA_PROB(sx[4 * (c) + 2]), e3 = AA_PROB(sx[4 * (c) + 3]);        \
-    if (AA_ABLATE != 2) { sum += e0; sum += e1; sum += e2; sum += e3; }              \
+    sum += e0; sum += e1; sum += e2; sum += e3;                                        \
     pw[(c) >> 1][2 * ((c) & 1) + 0] = T::pack(e0, e1);                                 \
     pw[(c) >> 1][2 * ((c) & 1) + 1] = T::pack(e2, e3);                                 \
     if (kPinned) asm volatile("" : "+v"(pw[(c) >> 1][2 * ((c) & 1) + 0]), "+v"(pw[(c) >> 1][2 * ((c) & 1) + 1]));   \
@@ -614,7 +598,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     typedef short shortx8 __attribute__((ext_vector_type(8)));                                         \
     const shortx8 av = __builtin_shufflevector(vlo[i], vhi[i], 0, 1, 2, 3, 4, 5, 6, 7);                \
     acc[(i) % kDB] = T::mfma(*reinterpret_cast<const vec8*>(&av),                                      \
-                             AA_ABLATE == 10 ? qreg[(i) % kKS] : *reinterpret_cast<const vec8*>(&pw[((i) / kDB) & 1]), acc[(i) % kDB]); \
+                             *reinterpret_cast<const vec8*>(&pw[((i) / kDB) & 1]), acc[(i) % kDB]); \
     if (kAnyRows) acc[(i) % kDB] = T::mfma(*reinterpret_cast<const vec8*>(&av),                        \
                                            *reinterpret_cast<const vec8*>(&pw##_rest[((i) / kDB) & 1]), acc[(i) % kDB]); \
   }
@@ -646,7 +630,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // These tiles have loops of their own: a choice inside a tile costs the branches and register copies that it saves maxima.  131072 tokens,
   // 32/8 heads of 128, few keys selected 7.71 -> 7.44 ms; 16384 dense 1875 -> 1810 us; 16384 fp16, heads of 64, 472 -> 451; scores without a
   // sink, 32768 tokens with nearly every key selected: 9.11 -> 9.08 ms.
-  constexpr bool kBySum = !kAnyRows && AA_ABLATE != 1 && AA_ABLATE != 2;
+  constexpr bool kBySum = !kAnyRows;
   const uint32_t kSumLimit = __float_as_uint(0.999f), kSumLow = __float_as_uint(0.5f);
   bool few = false;
 
@@ -803,10 +787,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       for (int n = 0; n < kKS; ++n) {
         AA_OPERAND_FETCH(n + kDist)
         AA_S_MFMA(s0, n);
-        if (AA_ABLATE != 3) {
 #pragma unroll
-          for (int u = 0; u < 2 * kHalfLoads / kKS; ++u) { AA_FETCH_ONE(n * (2 * kHalfLoads / kKS) + u) }
-        }
+        for (int u = 0; u < 2 * kHalfLoads / kKS; ++u) { AA_FETCH_ONE(n * (2 * kHalfLoads / kKS) + u) }
         AA_FENCE;
       }
 
@@ -817,8 +799,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         AA_S_MFMA(s1, n);
         AA_FENCE;
       }
-      if (AA_ABLATE != 2 && !kFew) { AA_MASK(s0, 0) }
-      if (!kLazyRef && AA_ABLATE != 2 && !kFew) {
+      if (!kFew) { AA_MASK(s0, 0) }
+      if (!kLazyRef && !kFew) {
         AA_LANEMAX(s0, mx0)
         moved0 = __any(mx0 > m_over);
         if (__builtin_expect(moved0, 0)) {
@@ -875,8 +857,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
 #pragma unroll
         for (int r = 0; r < 16; ++r) s1[r] -= shift0;
       }
-      if (AA_ABLATE != 2 && !kFew) { AA_MASK(s1, 1) }
-      if (!kLazyRef && AA_ABLATE != 2 && !kFew) {
+      if (!kFew) { AA_MASK(s1, 1) }
+      if (!kLazyRef && !kFew) {
         AA_LANEMAX(s1, mx1)
         moved1 = __any(mx1 > m_over);
         if (__builtin_expect(moved1, 0)) {
@@ -938,10 +920,10 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         buf_step = -buf_step;
         cur ^= 1;
       }
-      if (AA_ABLATE != 9) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile i+1 has landed in LDS
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of tile i+1 has landed in LDS
       // (so has the mask word: named here, or the compiler would wait for it behind the next tile's loads)
       if (MODE == kMasked) asm volatile("" : "+v"(mask_word_next[0]), "+v"(mask_word_next[1]));
-      if (AA_ABLATE != 8 && AA_ABLATE != 9) __syncthreads();
+      __syncthreads();
       AA_FENCE;
       constexpr uint32_t rd_next = kBuf == 0 ? kTileBytes : 0;
 #pragma unroll
@@ -951,9 +933,6 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       for (int n = kNS + kNV - kTail; n < kNS + kNV; ++n) {
         AA_PV_MFMA(n - kNS, pw1)
         AA_FENCE;
-      }
-      if (AA_ABLATE == 10) {  // P is still formed: it only has to exist by the end of the tile
-        asm volatile("" ::"v"(pw0[0]), "v"(pw0[1]), "v"(pw1[0]), "v"(pw1[1]));
       }
 #undef AA_OPERAND_FETCH
 #undef AA_S_MFMA

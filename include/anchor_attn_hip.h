@@ -56,8 +56,7 @@ extern "C" {
 #define AA_GEOMETRY_AS_RUN 0
 #define AA_GEOMETRY_INTENDED 1
 
-/* 2 for this ABI.  1000 + n marks a timing-only build (`make ablations`, AA_ABLATE = n) that leaves part of a kernel out and
- * computes wrong results on purpose; such a build is for bench_ablations.py only and the Python loader refuses it. */
+/* 3 for this ABI.  (1000 and above: a build that leaves part of a kernel out to time the rest; the Python loader refuses it.) */
 int aa_version(void);
 const char* aa_last_error(void);
 
