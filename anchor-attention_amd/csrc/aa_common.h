@@ -167,17 +167,19 @@ __device__ __forceinline__ void sum_counts(const int32_t* counts, const int64_t 
 // additions and two shifts.  (Granlund and Montgomery, Division by invariant integers using multiplication: exact for all 32-bit numbers.)
 // 32/8 heads of 128: 777 rows 20.1 -> 19.85 us, padded 2 x 1500 63.6 -> 62.3 and 3 x 2500 186 -> 184.4, a decode step over 33001 keys 28.65 -> 28.25;
 // 131072 tokens 7343 -> 7328.
+//
+// A reciprocal costs the host a 64-bit division, so a launch forms those that its kernel divides by and no others.  (With thirteen
+// of them for every launch short calls took 0.1 to 0.2 us longer than without any: decode steps over 300 to 9000 keys 15 to 21 us, 0.8 % on average; 0.1 % now.)
 struct FastDiv {
-  uint32_t mul, shift1, shift2;
+  uint32_t mul, shifts;  // two shifts, 0 or 1 in the lower five bits and one in the upper 24
 };
 inline FastDiv fast_div(const uint32_t d) {  // d >= 1
-  uint32_t bits = 0;
-  while (bits < 32 && (1ull << bits) < d) ++bits;
-  return {(uint32_t)((((1ull << bits) - d) << 32) / d + 1), bits < 1 ? bits : 1, bits > 0 ? bits - 1 : 0};
+  const uint32_t bits = d > 1 ? 32 - (uint32_t)__builtin_clz(d - 1) : 0;
+  return {(uint32_t)((((1ull << bits) - d) << 32) / d + 1), bits > 0 ? 1u | (bits - 1) << 8 : 0u};
 }
 __host__ __device__ __forceinline__ uint32_t quotient(const uint32_t n, const FastDiv& f) {
   const uint32_t t = (uint32_t)((uint64_t)n * f.mul >> 32);
-  return (t + ((n - t) >> f.shift1)) >> f.shift2;
+  return (t + ((n - t) >> (f.shifts & 31u))) >> (f.shifts >> 8);
 }
 // n divided by the divisor of f; n becomes the quotient, the remainder is returned
 __host__ __device__ __forceinline__ uint32_t take_remainder(uint32_t& n, const FastDiv& f, const uint32_t d) {
@@ -219,47 +221,44 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uin
 // after the other, so that the launch does not end with the heaviest work-groups of its last unit.
 struct Deal {
   enum Kind : uint32_t { kInTurn, kOwnUnits, kSharedUnits, kAbreast, kAbreastAll } kind;
-  uint32_t n_units, per_unit, inner;
-  uint32_t own;        // (abreast) units of an XCD
-  uint32_t turns;      // (abreast) ... which begin one further on every 32 work-groups
-  uint32_t share_log;  // (shared units) log2 of the XCDs that share one
-  FastDiv by_per_unit, by_inner, by_own, by_units;
+  uint32_t n; FastDiv by_n;  // work-groups of a unit (in turn, own units) or of a row (shared units); units of an XCD or all units (abreast)
+  uint32_t share_log;        // (shared units) log2 of the XCDs that share one
+  uint32_t turns;            // (abreast) an XCD's units begin one further on every 32 work-groups
 };
 inline Deal make_deal(uint32_t n_units, uint32_t per_unit, uint32_t inner, bool abreast) {
-  Deal d = {Deal::kInTurn, n_units, per_unit, inner, 1, 0, 0, fast_div(per_unit), fast_div(inner), fast_div(1), fast_div(n_units)};
+  Deal d = {Deal::kInTurn, per_unit, {}, 0, 0};
   const bool even = (uint64_t)n_units * per_unit % 8 == 0;
   if (abreast) {
     d.kind = !even || n_units % 8 != 0 ? Deal::kAbreastAll : Deal::kAbreast;
-    d.own = d.kind == Deal::kAbreast ? n_units / 8 : 1;
+    d.n = d.kind == Deal::kAbreast ? n_units / 8 : n_units;
     // (the XCD's 32 CUs are filled in turn: without the rotation a number of units that divides 32 ties a CU to a unit, and
     // units differ in weight: two prompts of 3900, one padded, 239 us one after the other, 280 without it and 239 with it)
-    d.turns = 32 % d.own == 0;
-    d.by_own = fast_div(d.own);
+    d.turns = 32 % d.n == 0;
   } else if (even && n_units % 8 == 0) {
     d.kind = Deal::kOwnUnits;
   } else if (even && 8 % n_units == 0 && (per_unit / inner) % (8 / n_units) == 0) {
     d.kind = Deal::kSharedUnits;
+    d.n = inner;
     for (uint32_t s = 8 / n_units; s > 1; s /= 2) ++d.share_log;
   }
+  d.by_n = fast_div(d.n);
   return d;
 }
 __host__ __device__ __forceinline__ void dealt(const Deal& d, const uint32_t wg, uint32_t& unit, uint32_t& index) {
-  const uint32_t xcd = wg % 8u;
-  uint32_t k = wg / 8u;
+  const uint32_t xcd = wg % 8u, k = wg / 8u;
+  uint32_t n = d.kind == Deal::kInTurn || d.kind == Deal::kAbreastAll ? wg : k;
+  if (d.kind == Deal::kAbreast && d.turns) n += k / 32u;
+  const uint32_t r = take_remainder(n, d.by_n, d.n);
   if (d.kind == Deal::kOwnUnits) {
-    index = take_remainder(k, d.by_per_unit, d.per_unit);
-    unit = k * 8u + xcd;
+    unit = n * 8u + xcd;
+    index = r;
   } else if (d.kind == Deal::kSharedUnits) {
-    const uint32_t in = take_remainder(k, d.by_inner, d.inner);
     unit = xcd >> d.share_log;
-    index = ((k << d.share_log) + (xcd & ((1u << d.share_log) - 1u))) * d.inner + in;
+    index = ((n << d.share_log) + (xcd & ((1u << d.share_log) - 1u))) * d.n + r;
   } else if (d.kind == Deal::kAbreast) {
-    uint32_t turned = k + (d.turns ? k / 32u : 0u);
-    unit = take_remainder(turned, d.by_own, d.own) * 8u + xcd;
-    index = quotient(k, d.by_own);
+    unit = r * 8u + xcd;
+    index = quotient(k, d.by_n);
   } else {
-    uint32_t n = wg;
-    const uint32_t r = d.kind == Deal::kAbreastAll ? take_remainder(n, d.by_units, d.n_units) : take_remainder(n, d.by_per_unit, d.per_unit);
     unit = d.kind == Deal::kAbreastAll ? r : n;
     index = d.kind == Deal::kAbreastAll ? n : r;
   }

@@ -375,8 +375,9 @@ static void launch_decode_for(const FlashArgs& a, hipStream_t stream) {
   if (a.n_chunks > 1) hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((uint32_t)units * a.n_rows * group), block, 0, stream, a);
 }
 
-hipError_t launch_decode(FlashArgs a, hipStream_t stream) {
-  set_divisors(a);
+hipError_t launch_decode(FlashArgs& a, hipStream_t stream) {
+  set_heads(a);
+  a.by_chunks = fast_div(a.n_chunks);
   a.by_cols = fast_div((uint32_t)a.n_rows * a.group);  // (the columns are one block, and each is merged by a work-group)
   if (a.head_dim == 128) {
     if (a.dtype == 0) launch_decode_for<Bf16, 128>(a, stream);

@@ -1237,11 +1237,11 @@ flash_pair_kernel(const FlashArgs anchor, const FlashArgs rows, const uint32_t n
 // Sets what the launcher decides for a launch of one mode, alone or with another; the number of work-groups.
 template <int MODE>
 static uint32_t place(FlashArgs& a, const bool alone) {
-  a.q_blocks_per_wg = 1;
-  set_divisors(a);
+  set_heads(a);
   int64_t blocks = (int64_t)a.batch * a.n_q_heads * (a.n_ctx / 128);
   if (MODE == kSparse) {
     const int per_big_block = a.big_block / 128;
+    a.n_big = a.n_ctx / a.big_block;
     blocks -= (int64_t)a.batch * a.n_q_heads * a.first_big_block * per_big_block;
     if (blocks == 0) return 0;
     // Chained blocks save a work-group's start and the list's round trip, but few work-groups leave CUs idle: as many as
@@ -1253,9 +1253,15 @@ static uint32_t place(FlashArgs& a, const bool alone) {
     while (nq > 1 && (per_big_block % nq != 0 || blocks / nq < fills_twice)) nq /= 2;
     a.q_blocks_per_wg = nq;
     a.q_units = per_big_block / nq;
-    a.by_pair = fast_div(a.group * a.q_units);
-    a.by_block = fast_div(a.q_units);
     a.pairs = (int64_t)a.units * (a.n_big - a.first_big_block) % 8 == 0;
+    if (a.pairs) {
+      a.by_pair = fast_div(a.group * a.q_units);
+      a.by_units = fast_div(a.units);
+    } else {
+      a.by_block = fast_div(a.q_units);
+      a.deal = make_deal(a.units, a.group * (a.n_big - a.first_big_block) * a.q_units, a.group, false);
+    }
+    return (uint32_t)(blocks / nq) + (a.ratio != nullptr ? 1 : 0);
   } else if (MODE == kAnchor) {
     a.by_block = fast_div(a.big_block / 128);
   }
@@ -1268,13 +1274,14 @@ static uint32_t place(FlashArgs& a, const bool alone) {
   // nothing on average (44 sizes: from 10 % faster to 10 % slower).
   const int units = a.units;
   const int rows = MODE == kRows || MODE == kMasked ? a.n_col_blocks * a.n_chunks : a.n_ctx / 128;  // (of a unit: what is dealt out)
-  const bool abreast = MODE != kSparse && (8 % units != 0 ? (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20
-                                                          : alone && rows % (8 / units) != 0);
-  if (MODE == kRows || MODE == kMasked) a.deal = make_deal(units, rows, 1, abreast);
-  else if (MODE != kSparse) a.deal = make_deal(units, a.group * rows, a.group, abreast);
-  else a.deal = make_deal(units, a.group * (a.n_big - a.first_big_block) * a.q_units, a.group, false);
-  if (MODE == kRows || MODE == kMasked) return (uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * a.n_chunks;
-  return (uint32_t)(blocks / a.q_blocks_per_wg) + (MODE == kSparse && a.ratio != nullptr ? 1 : 0);
+  const bool abreast = 8 % units != 0 ? (int64_t)((units + 7) / 8) * a.n_ctx * a.head_dim * 4 <= 4 << 20 : alone && rows % (8 / units) != 0;
+  if (MODE == kRows || MODE == kMasked) {
+    a.by_cols = fast_div(a.n_col_blocks);
+    a.deal = make_deal(units, rows, 1, abreast);
+    return (uint32_t)units * rows;
+  }
+  a.deal = make_deal(units, a.group * rows, a.group, abreast);
+  return (uint32_t)blocks;
 }
 
 template <int MODE>

@@ -33,11 +33,14 @@ struct FlashArgs {
   Deal deal;        // which work-group has which rows
   int group;        // query heads of a KV head
   int units;        // KV heads of all batch elements
-  int n_big;        // big blocks
+  int n_big;        // (sparse) big blocks
   int q_units;      // (sparse) work-groups of a big block and query head
   bool pairs;       // (sparse) (KV head, big block) pairs go round-robin
-  FastDiv by_group, by_kv_heads, by_cols, by_chunks, by_chunk_tiles, by_units;
-  FastDiv by_pair, by_block;  // (sparse) work-groups of a (KV head, big block) pair; (sparse, anchor) of a big block and query head
+  FastDiv by_group, by_kv_heads;
+  FastDiv by_cols;    // (rows, masked) column blocks; (merge of a decode step) columns
+  FastDiv by_chunks;  // (decode) chunks; (merge of rows) tiles of a chunk
+  FastDiv by_block;   // (anchor, sparse) work-groups of a big block and query head
+  FastDiv by_pair, by_units;  // (sparse, pairs) work-groups of a (KV head, big block) pair; KV heads of all batch elements
   // rows mode: n_rows query rows over n_ctx keys, row i sees keys 0 .. causal_offset + i.  The (row, head) columns of a
   // KV head come in blocks of 128, the keys in chunks of chunk_tiles 64-key tiles; with more than one chunk the work-groups
   // write M_out, L_out, acc_out [batch, n_kv_heads, n_col_blocks, n_chunks, 128 columns] for rows_combine_kernel
@@ -52,16 +55,12 @@ struct FlashArgs {
   int dtype;            // AA_DTYPE_BF16 / AA_DTYPE_F16: what the 16-bit elements of q, k, v, out, qbar, abar are
 };
 
-inline void set_divisors(FlashArgs& a) {
+// what all kernels find their place by
+inline void set_heads(FlashArgs& a) {
   a.group = a.n_q_heads / a.n_kv_heads;
   a.units = a.batch * a.n_kv_heads;
-  a.n_big = a.big_block > 0 ? a.n_ctx / a.big_block : 1;
   a.by_group = fast_div(a.group);
   a.by_kv_heads = fast_div(a.n_kv_heads);
-  a.by_cols = fast_div(a.n_col_blocks > 0 ? a.n_col_blocks : 1);
-  a.by_chunks = fast_div(a.n_chunks > 0 ? a.n_chunks : 1);
-  a.by_chunk_tiles = fast_div(a.chunk_tiles > 0 ? a.chunk_tiles : 1);
-  a.by_units = fast_div(a.units);
 }
 
 // mode: 0 anchor (stage 1), 1 sparse (stage 3), 2 dense causal, 3 rows, 4 masked
@@ -84,7 +83,7 @@ hipError_t launch_mask_pack(const FlashArgs& a, const uint8_t* mask, int64_t mas
 constexpr int kDecMaxChunks = 256;
 bool decode_takes(int n_rows, int group, bool masked);
 void plan_decode(FlashArgs& a);
-hipError_t launch_decode(FlashArgs a, hipStream_t stream);
+hipError_t launch_decode(FlashArgs& a, hipStream_t stream);
 
 // x, out [rows, hidden], weight [hidden], contiguous; hidden a multiple of 8 and at most 16384
 hipError_t launch_rms_norm(const uint16_t* x, const uint16_t* weight, uint16_t* out, int64_t rows, int hidden, float eps, int dtype, hipStream_t stream);

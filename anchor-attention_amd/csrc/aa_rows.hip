@@ -35,7 +35,7 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
   // the chunks that hold keys of this block (the others were not written)
   const int last_row = quotient(min(128 * block + 128, n_cols) - 1, p.by_group);
   const int tiles = min(p.causal_offset + last_row, p.n_ctx - 1) / 64 + 1;
-  const int n_chunks = quotient(tiles + p.chunk_tiles - 1, p.by_chunk_tiles);
+  const int n_chunks = quotient(tiles + p.chunk_tiles - 1, p.by_chunks);
   const int64_t slot0 = ((((int64_t)b * p.n_kv_heads + kvh) * p.n_col_blocks + block) * p.n_chunks) * 4 + wave;
   const float scale = p.sm_scale * kLog2e;
 
@@ -97,7 +97,9 @@ __global__ void __launch_bounds__(256) rows_combine_kernel(const FlashArgs p) {
 }
 
 hipError_t launch_rows_combine(FlashArgs a, hipStream_t stream) {
-  set_divisors(a);
+  set_heads(a);
+  a.by_cols = fast_div(a.n_col_blocks);
+  a.by_chunks = fast_div(a.chunk_tiles);
   const dim3 grid((uint32_t)a.batch * a.n_kv_heads * a.n_col_blocks * (a.head_dim / 32)), block(256);
   if (a.head_dim == 128) {
     if (a.dtype == 0) hipLaunchKernelGGL((rows_combine_kernel<Bf16, 128>), grid, block, 0, stream, a);
