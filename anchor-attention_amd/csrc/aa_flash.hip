@@ -197,6 +197,10 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // operands fetched one MFMA before the barrier: 0 to 0.6 % slower than two.  Rows of fp16 at 64 spill for the operands: 1900 26.5 -> 27.1, so none there.
   constexpr int kTail = MODE == kRows && !kLazyRef && D == 64 ? 0 : 2;
   constexpr bool kChecksSums = kLazyRef;
+  // What follows a grown max, and the masking of pairs, is laid out of line, except where it is often gone through and spills there: rows of fp16 at 64, whose
+  // maxima grow in the first tiles of every chunk but the first, which holds no sink, and everywhere without one.  In line, out of line and as for one branch
+  // in ten (times): 1493 rows, 14/2 heads, in chunks 26.2, 27.5 and 26.2 us; 1700 rows, 32/8 heads, without a sink 37.6, 41.5 and 37.9, with one 30.5, 30.1 and 29.7.
+  constexpr bool kNotSoRare = MODE == kRows && !kLazyRef && D == 64 && TEAMS == 1;
   static_assert(D == 128 || D == 64, "head dimension");
   constexpr int kKS = D / 16;       // MFMAs per 32-key block of S^T = K Q^T
   constexpr int kDB = D / 32;       // 32-column blocks of the head dimension: accumulators of O^T
@@ -542,6 +546,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // key (or list position) that accumulator register r of 32-key half kb of the tile at key0 stands for
 #define AA_KEY_OF(kb, r) (key0 + 32 * (kb) + 8 * ((r) >> 2) + 4 * half + ((r) & 3))
   // causal / list-end mask of one 32-key half (only tiles on the diagonal or at the end of a list need it)
+#define AA_RARE(x) (kNotSoRare ? __builtin_expect_with_probability((long)(x), 0, 0.9) : __builtin_expect(x, 0))
 #define AA_MASK(sx, kb)                                                              \
   if (MODE == kMasked) {                                                             \
     if (__builtin_expect(mixed, 0)) {                                                \
@@ -551,7 +556,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         if (!((seen_ >> (8 * (r >> 2) + (r & 3))) & 1u)) sx[r] = -INFINITY;          \
     }                                                                                \
   } else if (MODE != kSparse) {                                                      \
-    if (__builtin_expect(key0 + 32 * (kb) + 31 > wave_last_key, 0)) {                \
+    if (AA_RARE(key0 + 32 * (kb) + 31 > wave_last_key)) {                            \
       _Pragma("unroll") for (int r = 0; r < 16; ++r)                                 \
         if (AA_KEY_OF(kb, r) > my_last_key) sx[r] = -INFINITY;                       \
     }                                                                                \
@@ -803,7 +808,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       if (!kLazyRef && !kFew) {
         AA_LANEMAX(s0, mx0)
         moved0 = __any(mx0 > m_over);
-        if (__builtin_expect(moved0, 0)) {
+        if (AA_RARE(moved0)) {
           // some row's max grew.  Lanes whose max did not move get shift 0 and alpha 1 (exact).
           // S1 is being accumulated on top of the old -m_ref and is shifted once it is complete.
           // (a chunk may hold no key of a row's so far - its max stays -inf and its reference 0)
@@ -853,7 +858,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         AA_PV_MFMA(n - kNS, pw0)
         AA_FENCE;
       }
-      if (!kLazyRef && !kFew && __builtin_expect(moved0, 0)) {
+      if (!kLazyRef && !kFew && AA_RARE(moved0)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) s1[r] -= shift0;
       }
@@ -861,7 +866,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       if (!kLazyRef && !kFew) {
         AA_LANEMAX(s1, mx1)
         moved1 = __any(mx1 > m_over);
-        if (__builtin_expect(moved1, 0)) {
+        if (AA_RARE(moved1)) {
           // as above, except that O^T is rescaled only after the P0 V0 products in flight have been added
           const float m_new = fmaxf(m_ref + m_over, m_ref + max_with_other_half(mx1));
           const float m_base = m_new == -INFINITY ? 0.f : m_new;
@@ -891,7 +896,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         AA_PV_MFMA(n - kNS, pw0)
         AA_FENCE;
       }
-      if (!kLazyRef && !kFew && __builtin_expect(moved1, 0)) {
+      if (!kLazyRef && !kFew && AA_RARE(moved1)) {
 #pragma unroll
         for (int db = 0; db < kDB; ++db)
 #pragma unroll
@@ -983,6 +988,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
 #undef AA_TILE_KEY0
 #undef AA_KEY_OF
 #undef AA_MASK
+#undef AA_RARE
 #undef AA_LANEMAX
 #undef AA_PROB
 #undef AA_EXP_CHUNK
