@@ -194,7 +194,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // MFMAs of a tile that are issued behind its closing barrier, while the first K operands of the next tile are on their way: with none a wave waits
   // a whole LDS latency there.  0 against 2: dense 16384 tokens, 32/8 heads of 128, 1692.2 -> 1684.7 us, 131072 7080 -> 7040, 32768 with nearly every key selected
   // 8508 -> 8472, rows 777 19.9 -> 19.65, 14/2 heads of 64, 2048 tokens dense 22.1 -> 21.7, 1900 rows 25.5 -> 24.75; three of them, with
-  // operands fetched one MFMA before the barrier: 0 to 0.6 % slower than two.  Rows of fp16 at 64 spill for the operands: 1900 26.5 -> 27.1, so none there.
+  // operands fetched one MFMA before the barrier: 0 to 0.6 % slower than two.  Rows of fp16 at 64 have no registers for the operands: 1493 of 14/2 heads 26.1 -> 28.2,
+  // 1700 of 32/8 30.3 -> 34.2; with two teams they have, and 850 to 1000 rows of 32/8 heads are from 1 % slower (no sink) to 2 % faster: none either.
   constexpr int kTail = MODE == kRows && !kLazyRef && D == 64 ? 0 : 2;
   constexpr bool kChecksSums = kLazyRef;
   // What follows a grown max, and the masking of pairs, is laid out of line, except where it is often gone through and spills there: rows of fp16 at 64, whose
@@ -350,8 +351,9 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // Before all else, so that their way from memory is not added to that of the mask's tile flags, on which the first tile waits, or of that tile: masked
   // batches of 300 to 4000 tokens 3.5 % on average, up to 24 % (3 x 2500, 32/8 heads of 128, 181.4 -> 175.4 us; 2 x 2000, 14/2 of 64, 46.1 -> 39.4; of 44 sizes
   // four 1 to 3 % slower, where the end of the launch falls otherwise), dense 1024 tokens, 14/2 heads of 64, 14.1 -> 13.85, 777 rows 19.65 -> 19.55, larger
-  // launches +-0.2 %.  fp16 rows at 128, which wait longer for the first tile then, 20.3 -> 21.4: as before.
-  constexpr bool kQueriesFirst = MODE != kSparse && (MODE != kRows || kLazyRef);
+  // launches +-0.2 %.  fp16 rows at 128, which wait longer for the first tile then, 20.3 -> 21.4, and one team's at 64 (1700 of 32/8 heads 30.3 -> 32.1, 1900 of
+  // 14/2 27.4 -> 27.8): after it; two teams' 0.7 % faster (930 of 32/8 16.8 -> 16.6).
+  constexpr bool kQueriesFirst = MODE != kSparse && (MODE != kRows || kLazyRef || TEAMS == 2);
   if (kQueriesFirst) load_queries();
   const bool feeds_next = list_chains && qb + 1 < nq;  // the next block takes its first tile from this one
 
