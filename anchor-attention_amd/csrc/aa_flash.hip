@@ -633,13 +633,23 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
 
   // Where the reference follows the running max, a key above it has a probability of 1 or more, so a lane whose 16 probabilities of a
   // half-tile sum to less has none: once a wave's sums have been low (an attention sink: the rest of the keys weigh little), tiles
-  // without masked pairs are run without forming maxima (kFew) until a sum says otherwise.  (Compared as bits: a NaN counts as large.)
+  // without masked pairs are run without forming maxima (kFew) until a sum says otherwise.  (Compared as bits: a NaN counts as large.  The limit is 1
+  // less what rounding can take from a sum; sums have to be half of it to begin, so that ones about it do not end at once what they began: 0.25 or 0.75
+  // there cost 0.3 to 0.6 % at sinks 6 nats above the rest, and change the others by less than 0.3.)
   // These tiles have loops of their own: a choice inside a tile costs the branches and register copies that it saves maxima.  131072 tokens,
-  // 32/8 heads of 128, few keys selected 7.71 -> 7.44 ms; 16384 dense 1875 -> 1810 us; 16384 fp16, heads of 64, 472 -> 451; scores without a
-  // sink, 32768 tokens with nearly every key selected: 9.11 -> 9.08 ms.
+  // 32/8 heads of 128, few keys selected 7.71 -> 7.44 ms; 16384 dense 1875 -> 1810 us; 16384 fp16, heads of 64, 472 -> 451.  Without a sink nothing is gained.
+  //
+  // A tile in such a loop saves a twentieth of a tile, and leaving it costs a fourth (the half-tile's scores and exponentials once more, and the way into the
+  // other loops).  So a wave leaves twice for nothing, and then once for every kLeaving tiles that it has run.  8192 tokens dense, 32/8 heads of 128, maxima in all
+  // tiles, re-entered at once and with 48 tiles to pay (16, 32): a sink 9 nats above the rest 468 us, 450 and 450; 0.1 % of the keys as strong 478, 475, 474; 0.5 %
+  // 486, 496, 486 (489, 486); 2 % 512, 532, 515 (518, 514); a new maximum every 250 keys 483, 502, 482; every 33 574, 570, 571.  54 such inputs of both head
+  // dimensions: from 4.7 % faster to 0.7 % slower than with all maxima, 0.7 % faster on average; re-entered at once 17 were slower, by up to 5 %.
   constexpr bool kBySum = !kAnyRows;
+  constexpr int kLeaving = 48 * TEAMS;
   const uint32_t kSumLimit = __float_as_uint(0.999f), kSumLow = __float_as_uint(0.5f);
   bool few = false;
+  int paid_until = -kLeaving;    // the tile from which the next leaving is paid for
+  int few_from = 0x7fffffff;     // ... if the last tile's sums were low, the tile from which these loops may be entered
 
   // One tile.  The LDS buffer it reads (BUF) is a compile-time constant - the loops below are unrolled by two - so that
   // the buffer's offset is part of every LDS instruction's immediate offset and the read addresses are loop-invariant.
@@ -763,6 +773,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
 #pragma unroll
         for (int c = 0; c < 4; ++c) { AA_EXP_CHUNK(sx, pw, sum, c) }
         few = false;
+        paid_until += kLeaving;
       };
       (void)look_again;
 #define AA_K_FETCH(t) ka[t] = *(const lds_vec8*)(uintptr_t)(k_rd[(t) % kKS] + (uint32_t)(rd_off + 32 * ((t) / kKS) * kRowBytes))
@@ -908,7 +919,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       if (kFew) {
         if (__builtin_expect(__any(__float_as_uint(sum1) >= kSumLimit), 0)) look_again(std::integral_constant<int, 1>{}, s1, pw1, pw1_rest, sum1);
       } else if (kBySum) {
-        few = !__any(max(max(__float_as_uint(sum0), __float_as_uint(sum1)), __float_as_uint(m_over)) >= kSumLow);
+        few_from = __any(max(max(__float_as_uint(sum0), __float_as_uint(sum1)), __float_as_uint(m_over)) >= kSumLow) ? 0x7fffffff : paid_until;
       }
       l_run += sum1;
 
@@ -962,8 +973,9 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
       do {
         tile(BufCur{}, std::false_type{}, i);
         i += TEAMS;
-      } while (i < n_tiles && !(kBySum && few && whole(i)));
+      } while (i < n_tiles && !(kBySum && i >= few_from && whole(i)));
       if constexpr (kBySum) {
+        few = true;
         while (i < n_tiles && few && whole(i)) {
           tile(BufCur{}, std::true_type{}, i);
           i += TEAMS;
@@ -976,8 +988,9 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         if ((kAnyRows || TEAMS > 1) && i + TEAMS >= n_tiles) { i += TEAMS; break; }
         tile(Buf1{}, std::false_type{}, i + TEAMS);
         i += 2 * TEAMS;
-      } while (i < n_tiles && !(kBySum && few && i + TEAMS < n_tiles && whole(i + TEAMS)));
+      } while (i < n_tiles && !(kBySum && i >= few_from && i + TEAMS < n_tiles && whole(i + TEAMS)));
       if constexpr (kBySum) {
+        few = true;
         while (i + TEAMS < n_tiles && few && whole(i + TEAMS)) {
           tile(Buf0{}, std::true_type{}, i);
           tile(Buf1{}, std::true_type{}, i + TEAMS);

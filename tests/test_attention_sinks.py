@@ -107,3 +107,16 @@ def test_keys_above_the_sink_in_dense_rows(d, dtype, batch):
     q, k, v = _quiet_but(torch.cat((first, first + 101), 2), batch, n, 4, hkv, d, dtype, batch)
     scale = 0.125 * float(torch.tensor(LOG2E).to(dtype)) / LOG2E
     _check(dense_causal_attention(q, k, v, sm_scale=0.125), _weighted(q, k, v, scale, _causal(n).double()[None, None]), v)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_maximum_that_grows_again_and_again(d, dtype):
+    """More leavings of the loops without maxima than rows of 98 tiles pay for, one after the other and again after stretches without."""
+    from anchor_attn.src.ops.anchor_attn_v4 import dense_causal_attention
+    n = 6272
+    at = torch.cat([torch.arange(start, start + 800, 77) for start in (130, 3300, 5400)])
+    q, k, v = _quiet_but(at.expand(1, 2, -1), 1, n, 8, 2, d, dtype, d)
+    k[0, :, at, 0] = (8.0 + 0.25 * torch.arange(1, len(at) + 1)).to(dtype).cuda()
+    scale = 0.125 * float(torch.tensor(LOG2E).to(dtype)) / LOG2E
+    _check(dense_causal_attention(q, k, v, sm_scale=0.125), _weighted(q, k, v, scale, _causal(n).double()[None, None]), v)
