@@ -198,10 +198,14 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // 1700 of 32/8 30.3 -> 34.2; with two teams they have, and 850 to 1000 rows of 32/8 heads are from 1 % slower (no sink) to 2 % faster: none either.
   constexpr int kTail = MODE == kRows && !kLazyRef && D == 64 ? 0 : 2;
   constexpr bool kChecksSums = kLazyRef;
-  // What follows a grown max, and the masking of pairs, is laid out of line, except where it is often gone through and spills there: rows of fp16 at 64, whose
-  // maxima grow in the first tiles of every chunk but the first, which holds no sink, and everywhere without one.  In line, out of line and as for one branch
-  // in ten (times): 1493 rows, 14/2 heads, in chunks 26.2, 27.5 and 26.2 us; 1700 rows, 32/8 heads, without a sink 37.6, 41.5 and 37.9, with one 30.5, 30.1 and 29.7.
-  constexpr bool kNotSoRare = MODE == kRows && !kLazyRef && D == 64 && TEAMS == 1;
+  // What follows a grown max, and the masking of pairs, is laid out of line where it is expected to be rare, which spares what does not follow a jump.  It is
+  // not rare where a call is short and no key outweighs the rest: half of the tiles in anchor and dense mode (one time in two against never: dense 1024
+  // tokens without a sink, 32/8 heads of 128, 25.3 -> 24.4 us, 2048, 14/2 of 64, fp16 27.4 -> 26.7, with a sink 23.6 -> 22.9; an operator call of one big block,
+  // 32/8 of 64, 36.1 -> 35.0; 16384 tokens dense and 131072 of the operator +-0.1 %).  Rows of fp16 at 64 spill out of line, and their maxima grow in the first tiles of
+  // every chunk but the first, which holds no sink, and everywhere without one (one time in two, in ten and never: 1493 rows, 14/2 heads, in chunks
+  // 25.6, 26.2 and 27.5 us; 1700 rows, 32/8 heads, without a sink 37.2, 37.9 and 41.5, with one 30.3, 29.7 and 30.1).  Lists gain 0.8 % from one in two at
+  // 8192 tokens, 14/2 heads of 64, and lose 2 at 4096.
+  constexpr int kGrows = MODE == kAnchor || MODE == kDense ? 2 : MODE == kRows && !kLazyRef && D == 64 && TEAMS == 1 ? 1 : 0;
   static_assert(D == 128 || D == 64, "head dimension");
   constexpr int kKS = D / 16;       // MFMAs per 32-key block of S^T = K Q^T
   constexpr int kDB = D / 32;       // 32-column blocks of the head dimension: accumulators of O^T
@@ -548,7 +552,10 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // key (or list position) that accumulator register r of 32-key half kb of the tile at key0 stands for
 #define AA_KEY_OF(kb, r) (key0 + 32 * (kb) + 8 * ((r) >> 2) + 4 * half + ((r) & 3))
   // causal / list-end mask of one 32-key half (only tiles on the diagonal or at the end of a list need it)
-#define AA_RARE(x) (kNotSoRare ? __builtin_expect_with_probability((long)(x), 0, 0.9) : __builtin_expect(x, 0))
+#define AA_RARE(x)                                                                     \
+  (kGrows == 2   ? __builtin_expect_with_probability((long)(x), 0, 0.55)              \
+   : kGrows == 1 ? __builtin_expect_with_probability((long)(x), 0, 0.9)               \
+                 : __builtin_expect(x, 0))
 #define AA_MASK(sx, kb)                                                              \
   if (MODE == kMasked) {                                                             \
     if (__builtin_expect(mixed, 0)) {                                                \
