@@ -199,25 +199,13 @@ __host__ __device__ inline int64_t coords_tri(int64_t bb, int64_t S, int64_t bs)
 // XCD-aware work-group renumbering.  Consecutive hardware work-group ids go round-robin over the 8 XCDs (each
 // with its own L2).  The work consists of `n_units` units (a KV head of one batch element) of `per_unit`
 // work-groups each, ordered heaviest first inside a unit; work-groups of one unit read the same K/V rows or pooled
-// queries.  Returns the logical index unit * per_unit + idx such that
+// queries.  Gives (unit, idx in the unit) such that
 //   n_units % 8 == 0 : every XCD owns n_units / 8 whole units, every eighth one: the units of one batch element, whose work
 //                      differs from another's where prompts are padded, are spread over the XCDs;
 //   8 % n_units == 0 : s = 8 / n_units XCDs share a unit and take its rows alternately (row = idx / inner, the
 //                      `inner` work-groups of a row stay together), so that each gets the same mix of heavy and light;
 //   otherwise        : the hardware order is kept.
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t n_units, uint32_t per_unit, uint32_t inner) {
-  const uint32_t total = n_units * per_unit;
-  const uint32_t xcd = wg % 8u, k = wg / 8u;
-  if (total % 8u != 0u) return wg;
-  if (n_units % 8u == 0u) return (k / per_unit * 8u + xcd) * per_unit + k % per_unit;
-  if (8u % n_units == 0u) {
-    const uint32_t s = 8u / n_units;
-    if ((per_unit / inner) % s == 0u) return (xcd / s) * per_unit + ((k / inner) * s + xcd % s) * inner + k % inner;
-  }
-  return wg;
-}
-// The same map with the reciprocals and the choice from the host, as (unit, index in the unit).
-// `abreast`: an XCD takes its units (in the last case: all XCDs all units) side by side, the heaviest of each first, instead of one
+// The host makes the choice and the reciprocal.  `abreast`: an XCD takes its units (in the last case: all XCDs all units) side by side, the heaviest of each first, instead of one
 // after the other, so that the launch does not end with the heaviest work-groups of its last unit.
 struct Deal {
   enum Kind : uint32_t { kInTurn, kOwnUnits, kSharedUnits, kAbreast, kAbreastAll } kind;

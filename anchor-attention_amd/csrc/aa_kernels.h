@@ -125,9 +125,11 @@ struct SelectArgs {
   int key_lo, key_slack;
   int head_dim;  // 128 or 64
   int dtype;
+  // set by the launcher of the scores: which work-group has which keys
+  Deal deal; FastDiv by_kv_heads;
 };
 hipError_t launch_select_thresholds(const SelectArgs& a, hipStream_t stream);
-hipError_t launch_select_scores(const SelectArgs& a, hipStream_t stream);
+hipError_t launch_select_scores(SelectArgs a, hipStream_t stream);
 bool select_scores_sums(int batch, int n_kv_heads, int n_ctx);  // whether that is to form the ratio
 hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_ratio(const int32_t* counts, int64_t n, float inverse, float* ratio, hipStream_t stream);

@@ -164,11 +164,10 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
   const int S = p.big_block;
   const int n_bb = p.n_ctx / S;
   const int n_t = p.n_ctx / 128;
-  const int n_super = n_t / kTilesPerWg;
-  uint32_t vid = xcd_remap(blockIdx.x, p.batch * p.n_kv_heads, n_super, 1);
-  const int ST = vid % n_super;  // key super-tile (kTilesPerWg * 128 keys); ascending = heaviest first
-  vid /= n_super;
-  const int kvh = vid % p.n_kv_heads, b = vid / p.n_kv_heads;
+  uint32_t unit, index;
+  dealt(p.deal, blockIdx.x, unit, index);
+  const int ST = index;  // key super-tile (kTilesPerWg * 128 keys); ascending = heaviest first
+  const int b = quotient(unit, p.by_kv_heads), kvh = unit - b * p.n_kv_heads;
   const int n_pr = p.n_ctx / p.block_size;  // pooled rows per head
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -342,7 +341,10 @@ static void launch_select_scores_for(const SelectArgs& a, hipStream_t stream) {
   else launch(step == 16 ? select_scores_kernel<16, kWaves, kRows, T, D, false> : select_scores_kernel<32, kWaves, kRows, T, D, false>);
 }
 
-hipError_t launch_select_scores(const SelectArgs& a, hipStream_t stream) {
+hipError_t launch_select_scores(SelectArgs a, hipStream_t stream) {
+  const uint32_t units = a.batch * a.n_kv_heads;
+  a.deal = make_deal(units, scores_work_groups(a.batch, a.n_kv_heads, a.n_ctx) / units, 1, false);
+  a.by_kv_heads = fast_div(a.n_kv_heads);
   if (a.head_dim == 128) {
     if (a.dtype == 0) launch_select_scores_for<Bf16, 128>(a, stream);
     else launch_select_scores_for<F16, 128>(a, stream);
