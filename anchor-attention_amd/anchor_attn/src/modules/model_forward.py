@@ -189,7 +189,11 @@ class _Names(dict):
 
 
 class _Bound:
-    """A forward bound to its module, which copies and pickles as a bound method does: the copy's, and by its name."""
+    """A forward bound to its module, which copies and pickles as a bound method does, the copy's and by its name, and names its module and
+    function as one.  (It is none: those mark the modules whose kernels take over the whole forward.)"""
+
+    __self__ = property(lambda self: self.module)
+    __func__ = property(lambda self: self.forward)
 
     def __init__(self, module, forward):
         self.module, self.forward = module, forward

@@ -1,6 +1,8 @@
 """The rotary embedding of queries and keys as one kernel, which rounds as the framework's single operations do: the same bits."""
 import copy
+import inspect
 import pickle
+import types
 
 import pytest
 import torch
@@ -48,6 +50,22 @@ def test_attentions_run_their_class_s_code(family, monkeypatch):
             later.setattr(cls, "forward", lambda self, hidden_states, **kwargs: (hidden_states, None))
             assert torch.equal(m(tokens).logits, plain(tokens).logits)
         assert len(taken) == 2
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_a_patched_forward_names_its_module_and_function(family):
+    from anchor_attn import patch_model
+    m = patch_model(_tiny(family), "flash")
+    hidden = torch.randn(1, 5, m.config.hidden_size)
+    embeddings = m.model.rotary_emb(hidden, torch.arange(5)[None])
+    for a in _attentions(m, family):
+        for bound in (a.forward, copy.copy(a.forward), copy.deepcopy(a).forward):
+            assert bound.__name__ == "forward"
+            assert inspect.signature(bound) == inspect.signature(type(a).forward.__get__(a))
+            with torch.no_grad():
+                want = type(a).forward(a, hidden, position_embeddings=embeddings, attention_mask=None)[0]
+                assert torch.equal(types.MethodType(bound.__func__, bound.__self__)(hidden, position_embeddings=embeddings, attention_mask=None)[0], want)
+        assert a.forward.__self__ is a and copy.copy(a.forward).__self__ is a
 
 
 @pytest.mark.gpu
