@@ -243,7 +243,7 @@ int aa_anchor_attn_rows_fwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q
 
 /* ---- between a patched model's matrix products ------------------------------------------------
  * What the models that the attention plug is used in compute around it, one pass each, with the 16-bit roundings of the framework's
- * single operations (all tensors 16-byte aligned and contiguous):
+ * single operations (all tensors 16-byte aligned, those of the first two contiguous):
  * aa_rms_norm: out[r, :] = weight * round16(x[r, :] * rsqrt(mean(x[r, :]^2) + eps)), float32 inside;
  * aa_silu_mul: out = round16(silu(gate)) * up over n elements;
  * aa_rope: x * cos + rotate(x) * sin of queries and keys (element strides as everywhere, rows of head_dim consecutive elements), rotate: (first, second

@@ -68,6 +68,25 @@ def test_a_patched_forward_names_its_module_and_function(family):
         assert a.forward.__self__ is a and copy.copy(a.forward).__self__ is a
 
 
+@pytest.mark.parametrize("change,message", [
+    ({"batch": 0}, "must be positive"), ({"n_kv_heads": -1}, "must be positive"), ({"n_tokens": 0}, "must be positive"),
+    ({"head_dim": 24}, "not supported"), ({"head_dim": 1040}, "not supported"), ({"head_dim": 0}, "not supported"),
+    ({"batch": 1 << 20, "n_tokens": 1 << 12}, "not supported"),  # 2^32 pieces
+    ({"dtype": 2}, "dtype"), ({"q": 0}, "q is NULL"), ({"k_out": 0}, "k_out is NULL"), ({"cos": 0}, "cos is NULL"), ({"sin": 4104}, "sin must be 16-byte aligned"),
+    ({"k": 4104}, "k must be 16-byte aligned"), ({"q_sh": 60}, "q must be 16-byte aligned with strides"), ({"ko_sn": 56}, "smaller than head_dim"),
+    ({"qo_sn": 16392}, "larger than 16384"), ({"n_tokens": 1 << 20, "k_sn": 4096}, "32-bit byte offsets"), ({"cs_sb": 20}, "batch stride"),
+])
+def test_what_the_c_interface_refuses(change, message):
+    """Before anything is launched: the addresses are never read."""
+    from anchor_attn.src.ops import _hip
+    args = {"q": 4096, "q_sb": 2048, "q_sh": 64, "q_sn": 256, "k": 4096, "k_sb": 1024, "k_sh": 64, "k_sn": 128,
+            "q_out": 4096, "qo_sb": 2048, "qo_sh": 64, "qo_sn": 256, "k_out": 4096, "ko_sb": 1024, "ko_sh": 512, "ko_sn": 64,
+            "cos": 4096, "sin": 4096, "cs_sb": 0, "batch": 1, "n_q_heads": 4, "n_kv_heads": 2, "n_tokens": 8, "head_dim": 64, "dtype": 0, "stream": None}
+    assert len(args) == len(_hip.lib().aa_rope.argtypes) and set(change) <= set(args)
+    with pytest.raises(_hip.AnchorAttnHipError, match=message):
+        _hip.check(_hip.lib().aa_rope(*{**args, **change}.values()))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("batch,n,hq,hkv,d,own_angles", [(1, 1, 32, 8, 64, False), (1, 37, 14, 2, 64, False), (3, 65, 28, 4, 128, False),
