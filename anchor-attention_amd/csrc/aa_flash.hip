@@ -204,7 +204,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
   // 32/8 of 64, 36.1 -> 35.0; 16384 tokens dense and 131072 of the operator +-0.1 %).  Rows of fp16 at 64 spill out of line, and their maxima grow in the first tiles of
   // every chunk but the first, which holds no sink, and everywhere without one (one time in two, in ten and never: 1493 rows, 14/2 heads, in chunks
   // 25.6, 26.2 and 27.5 us; 1700 rows, 32/8 heads, without a sink 37.2, 37.9 and 41.5, with one 30.3, 29.7 and 30.1).  Lists gain 0.8 % from one in two at
-  // 8192 tokens, 14/2 heads of 64, and lose 2 at 4096.
+  // 8192 tokens, 14/2 heads of 64, and lose 2 at 4096.  (The masking alone stays out of line in anchor mode: two registers spill for it at 64, 4096 tokens, 14/2
+  // heads of 64, few keys selected 73.6 -> 72.9 us, 32/8 106.5 -> 105.9.  In dense mode that gives 0.6 % without a sink and costs 0.6 with one: as the rest.)
   constexpr int kGrows = MODE == kAnchor || MODE == kDense ? 2 : MODE == kRows && !kLazyRef && D == 64 && TEAMS == 1 ? 1 : 0;
   static_assert(D == 128 || D == 64, "head dimension");
   constexpr int kKS = D / 16;       // MFMAs per 32-key block of S^T = K Q^T
@@ -565,7 +566,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
         if (!((seen_ >> (8 * (r >> 2) + (r & 3))) & 1u)) sx[r] = -INFINITY;          \
     }                                                                                \
   } else if (MODE != kSparse) {                                                      \
-    if (AA_RARE(key0 + 32 * (kb) + 31 > wave_last_key)) {                            \
+    if (MODE == kAnchor ? __builtin_expect(key0 + 32 * (kb) + 31 > wave_last_key, 0) : AA_RARE(key0 + 32 * (kb) + 31 > wave_last_key)) { \
       _Pragma("unroll") for (int r = 0; r < 16; ++r)                                 \
         if (AA_KEY_OF(kb, r) > my_last_key) sx[r] = -INFINITY;                       \
     }                                                                                \
