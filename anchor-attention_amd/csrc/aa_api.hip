@@ -471,7 +471,7 @@ static int anchor_attn_impl(const char* who, const void* q, int64_t q_sb, int64_
   x.out = out; x.o_sb = o_sb; x.o_sh = o_sh; x.o_sn = o_sn;
   x.rows = rows;
   // (the word for the sum lies where the lists will)
-  const bool sums = selects && ratio != nullptr && select_scores_sums(batch, n_kv_heads, n_ctx);
+  const bool sums = selects && ratio != nullptr && select_scores_sums(batch, n_q_heads, n_kv_heads, n_ctx, head_dim, block_size * step);
   const Ratio r = {ratio, ratio_host, 1.f / (float)denominator, sums ? reinterpret_cast<uint64_t*>(coords) : nullptr};
   x.clear = r.selected;
   if (!selects) { x.zero_counts = counts; x.zero_ratio = ratio; x.zero_ratio_host = ratio_host; }

@@ -130,7 +130,7 @@ struct SelectArgs {
 };
 hipError_t launch_select_thresholds(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_select_scores(SelectArgs a, hipStream_t stream);
-bool select_scores_sums(int batch, int n_kv_heads, int n_ctx);  // whether that is to form the ratio
+bool select_scores_sums(int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim, int big_block);  // whether that is to form the ratio
 hipError_t launch_select_compact(const SelectArgs& a, hipStream_t stream);
 hipError_t launch_ratio(const int32_t* counts, int64_t n, float inverse, float* ratio, hipStream_t stream);
 

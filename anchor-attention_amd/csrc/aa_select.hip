@@ -325,11 +325,15 @@ __global__ void __launch_bounds__(64 * WAVES, AA_SEL_WGS) select_scores_kernel(c
 
 static uint32_t scores_work_groups(int batch, int n_kv_heads, int n_ctx) { return (uint32_t)(n_ctx / (64 * AA_SEL_WAVES)) * n_kv_heads * batch; }
 
-// Up to 128 work-groups (8 KV heads: 4096 tokens, 2: 16384) a call is so short that a logged one's wait for the ratio decides when the next can
-// start: with the ratio from here, a list and a launch sooner than from stage 3, calls in a row take 2048 tokens (14/2 heads of 64, blocks of 64) 55.1
-// -> 52.0 us, 4096 (14/2) 76.7 -> 73.2, (32/8 of 64) 102 -> 98.5, (32/8 of 128) 153.7 -> 151.0, 8192 (14/2) 123 -> 120.  Where the GPU has work for that
-// long, the sums and atomics only cost: 256 work-groups 339 -> 341, 512 721 -> 724 and 1343 -> 1348, 1024 1540 -> 1545 us.
-bool select_scores_sums(int batch, int n_kv_heads, int n_ctx) { return scores_work_groups(batch, n_kv_heads, n_ctx) <= 128; }
+// Where a call is short a logged one's wait for the ratio decides when the next can start: with the ratio from here, a list and a launch sooner
+// than from stage 3, calls in a row take 2048 tokens (14/2 heads of 64, blocks of 64) 54.5 -> 51.5 us, 4096 (14/2) 76.6 -> 73.1, (32/8 of 64) 103.5 -> 100.4,
+// (32/8 of 128) 156.0 -> 153.0, 8192 (14/2) 124 -> 121.  The sums cost this kernel 2 to 3 us, and where stage 3 is long enough that the next call is there
+// before it ends, nothing is left to gain.  That is so from about 11 M elements of output of stage 3 on (22 MB; 15 us where few keys are selected): 28/4 heads of
+// 128 3072 rows of 4096 115.3 us with sums and 118 without, 4096 rows of 6144 220.5 and 218 (all keys selected 468 and 461), of 5120 in blocks of 64 141 and 137.5; 32/8
+// 3072 rows of 4096 in blocks of 64 122 and 121.5; 14/2 of 64 14336 rows of 16384 218.5 and 215.  Beyond 128 work-groups the atomics cost too: 256 339 -> 341, 512 721 -> 724.
+bool select_scores_sums(int batch, int n_q_heads, int n_kv_heads, int n_ctx, int head_dim, int big_block) {
+  return scores_work_groups(batch, n_kv_heads, n_ctx) <= 128 && (int64_t)batch * n_q_heads * (n_ctx - big_block) * head_dim <= 11 << 20;
+}
 
 template <typename T, int D>
 static void launch_select_scores_for(const SelectArgs& a, hipStream_t stream) {

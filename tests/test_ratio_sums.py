@@ -49,6 +49,17 @@ def test_ratio_is_the_sum_of_the_counts(n, hq, hkv, block, step, theta, dtype, b
         assert total > 0
 
 
+@pytest.mark.parametrize("hq", [44, 48])  # 11 * 2^20 elements of stage 3's output: the last that the scores sum for, and more
+def test_ratio_at_the_output_s_size_where_the_scores_stop_summing(hq):
+    from anchor_attn.src.ops import _hip
+    from anchor_attn.src.ops.anchor_attn_v4 import anchor_attn
+    q, k, v = _inputs(3072, hq, 4, 5, d=128)
+    want_out, total, denominator = _by_lists(q, k, v, 64, 16, 12.0, _hip.AA_GEOMETRY_AS_RUN)
+    out, ratio = anchor_attn(q, k, v, block_size=64, difference=12.0)
+    assert torch.equal(out, want_out) and total > 0
+    assert abs(float(ratio) * float(denominator) - total) <= 4 * 2.0 ** -24 * total
+
+
 def test_ratio_on_every_replay_of_a_graph(monkeypatch):
     import my_utils
     from anchor_attn.src.ops.anchor_attn_v4 import anchor_attn
