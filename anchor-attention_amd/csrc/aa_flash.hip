@@ -167,10 +167,10 @@ __device__ __forceinline__ void tile_fetch_one(const int n, const char* kb, cons
 // D is the head dimension, 128 or 64: it sets the LDS row pitch, the number of tile loads, of MFMA steps over the head
 // dimension (kKS per 32 keys of Q.K^T) and of 32-column output blocks (kDB).
 //
-// Work-groups per CU: with 128 two (up to 253 registers, 64 KB of LDS).  With 64 a tile has half the MFMAs but the same soft-max,
-// so the vector ALU bounds it, and a third wave per SIMD (168 registers; around the tile loop 2 of them spill in anchor mode, 9 in sparse,
-// 1 in fp16 rows mode, 2 and in fp16 5 in the launch of both) keeps that busy: 75 % of the cycles, matrix pipe 56 % (16384 tokens, 32/8
-// heads of 64, fp16).  Stage 1 there 470 -> 413 us against two work-groups per CU and 256-byte LDS rows of which half was filled.
+// Work-groups per CU: with 128 two (up to 251 registers, 64 KB of LDS).  With 64 a tile has half the MFMAs but the same soft-max, so that the vector
+// ALU has more to do than the matrix pipe, and a third wave per SIMD (168 registers; around the tile loop 8 of them spill in sparse mode, 9 in fp16, and 1 in fp16 rows
+// mode, alone and beside the anchors) keeps both at work: stage 1 at 16384 tokens, 32/8 heads of 64, fp16, 73 % and 63 % of the cycles, both at once 34 %.  It took 413 us
+// instead of 470 with two work-groups per CU and 256-byte LDS rows of which half was filled (371 now).
 //
 // TEAMS: the waves that own the 128 rows, four to a team.  Two teams take the tiles alternately, each with LDS tiles and accumulators
 // of its own, and are merged through LDS at the end, like two chunks of the keys without a launch between them.  This is for
@@ -354,8 +354,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& p, const uint32_t bl
     for (int ks = 0; ks < kKS; ++ks) qraw[ks] = *reinterpret_cast<const u32x4*>(qrow + 16 * ks);
   };
   // Before all else, so that their way from memory is not added to that of the mask's tile flags, on which the first tile waits, or of that tile: masked
-  // batches of 300 to 4000 tokens 3.5 % on average, up to 24 % (3 x 2500, 32/8 heads of 128, 181.4 -> 175.4 us; 2 x 2000, 14/2 of 64, 46.1 -> 39.4; of 44 sizes
-  // four 1 to 3 % slower, where the end of the launch falls otherwise), dense 1024 tokens, 14/2 heads of 64, 14.1 -> 13.85, 777 rows 19.65 -> 19.55, larger
+  // batches of 300 to 4000 tokens 5 % on average, up to 24 % (3 x 2500, 32/8 heads of 128, 181.4 -> 175.4 us; 2 x 2000, 14/2 of 64, 46.1 -> 39.4; of 96 sizes
+  // one 2 % slower and no other more than 1), dense 1024 tokens, 14/2 heads of 64, 14.1 -> 13.85, 777 rows 19.65 -> 19.55, larger
   // launches +-0.2 %.  fp16 rows at 128, which wait longer for the first tile then, 20.3 -> 21.4, and one team's at 64 (1700 of 32/8 heads 30.3 -> 32.1, 1900 of
   // 14/2 27.4 -> 27.8): after it; two teams' 0.7 % faster (930 of 32/8 16.8 -> 16.6).
   constexpr bool kQueriesFirst = MODE != kSparse && (MODE != kRows || kLazyRef || TEAMS == 2);

@@ -221,7 +221,8 @@ constexpr int kMaxChunks = 64;
 // The bf16 prices were fitted to 192 sizes (20 to 5000 rows over up to 40000 keys, 2 to 32 KV heads in groups of 4 and 7, each with up to twelve
 // numbers of chunks), the fp16 ones to the 2042 of 5 to 3000 rows and 1 to 4 prompts on which both are compared here.  The number taken is slower than the
 // best of about ten measured ones by 1.0 % on average (98 of 100 within 11 %), fp16 0.7 (8) %, at 64 2.3 (27) and 1.4 (15) %, most of it where a
-// call is so short that a second launch costs the host more than it gives the GPU.  The form before, which had the longest chain or the rounds of a full chip at
+// call is so short that a second launch costs the host more than it gives the GPU.  (440 other sizes, some of them masked, on the kernel as it is since: 1.0, 1.1,
+// 1.7 and 0.9 %.)  The form before, which had the longest chain or the rounds of a full chip at
 // one price, came to 2.4, 1.2, 4.3 and 2.5 %: it did not know that a few work-groups more than CUs share them with the lightest ones (1194 rows,
 // 28/4 heads of 128: 36.9 us in three chunks, 30.2 whole); 30 of the 4084 are more than 5 % slower than with it, by 14 % at most.  With the bf16 prices for
 // fp16 those were 92 (22 %): 649 rows over 2890 keys, 32/8 heads of 128, 82.2 us in one chunk, 68.6 in three.
